@@ -95,8 +95,10 @@ def test_m0_belongs_to_the_lds_copies_only(src):
     """The global -> LDS copies are issued from inline assembly that sets M0 (the LDS address)
     itself.  M0 is reserved to the compiler and cannot be declared clobbered, so the sources rely
     on the compiler having no use of M0 of its own in these kernels: on the compiled code, every
-    instruction that names m0 must be the `s_mov_b32 m0, sN` of a copy statement, followed by its
-    `s_nop 0` and its `global_load_lds_*`, and every such load must follow one."""
+    instruction that names m0 must be the `s_mov_b32 m0, <scalar register>` of a copy statement,
+    followed by its `s_nop 0` and its `global_load_lds_*`, and every such load must follow one.  (The
+    register is the statement's "s" operand: the compiler may also hand out the two halves of vcc
+    where no comparison needs them.  An immediate, exec or m0 itself is none of its choices.)"""
     with tempfile.TemporaryDirectory() as tmp:
         out = os.path.join(tmp, "k.s")
         cmd = [B._hipcc()] + B.COMMON + B.PER_FILE.get(src, []) + [
@@ -112,7 +114,7 @@ def test_m0_belongs_to_the_lds_copies_only(src):
     n_copies = 0
     for i, t in enumerate(ins):
         if re.search(r"\bm0\b", t):
-            assert re.match(r"s_mov_b32 m0, s\d+$", t), "compiler-generated use of m0: " + t
+            assert re.match(r"s_mov_b32 m0, (s\d+|vcc_lo|vcc_hi)$", t), "compiler-generated use of m0: " + t
             assert ins[i + 1] == "s_nop 0" and ins[i + 2].startswith("global_load_lds_"), ins[i:i + 3]
         if t.startswith("global_load_lds_"):
             n_copies += 1
