@@ -93,10 +93,6 @@ int launch_mla_decode(const uint8_t *rows, const float *scales, int64_t row_bstr
                       int64_t scale_bstride, int64_t n_rows, int batch, const int32_t *sel, int64_t n_list,
                       const uint16_t *q, int n_heads, float scale, const float *sink, float *out,
                       hipStream_t s, bool fixed_scratch = false);
-// partials of mla_roles.hip's layout, [group][split][16-row block], into out: row block rb = n_hb16 * group + block
-// is heads 16 (rb % nhb) .. of query rb / nhb; blocks from n_rb on are not there
-int launch_mla_merge(const uint32_t *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
-                     int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s);
 int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, int64_t n,
                        const uint16_t *q, int n_heads, float scale, float *out, hipStream_t s);
 int launch_indexer_scores(const uint8_t *keys, const float *kscale, int64_t key_bstride,
@@ -211,6 +207,13 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+
+// partials of mla_roles.hip's layout, [group][split][16-row block], 16-bit fixed point or fp32, into out: row block
+// rb = n_hb16 * group + block is heads 16 (rb % nhb) .. of query rb / nhb; blocks from n_rb on are not there
+int launch_mla_merge(const u32x2 *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
+                     int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s);
+int launch_mla_merge(const f32x4 *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
+                     int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s);
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
     return __builtin_bit_cast(float, (uint32_t)b << 16);

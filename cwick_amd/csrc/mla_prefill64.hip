@@ -10,8 +10,8 @@
 //   takes four consecutive ones (a group): 64 heads of one query, or, with fewer heads, up to four
 //   queries that share the tiles and differ in at most three keys (SPAN).  512 queries of 16 heads
 //   over 5.5K rows: 227 us with one query per workgroup, 101 so.  Where the groups do not fill the
-//   chip a group's keys are cut into slices (plan_slices) whose partials mla_merge_frag16_kernel
-//   combines: 8 queries of 128 heads over 20K rows 453 -> 58 us, 52 over 13.5K 312 -> 172.
+//   chip a group's keys are cut into slices (plan_slices) whose fp32 partials mla_merge_frag32_kernel
+//   combines: 8 queries of 128 heads over 20K rows 453 -> 55 us, 52 over 13.5K 313 -> 170.
 //
 //   workgroup = 8 waves (two per SIMD, 256 registers each), 64 rows x all keys of the group,
 //   walked in tiles of 64 keys, three LDS stages.
@@ -92,7 +92,7 @@ struct WideParams {
     uint32_t n_rest, n_slices, slices_inv;    // groups take n_slices workgroups each and leave partials
     float scale;
     float *part_ml;           // as in mla_roles.hip, [group of n_rest][slice][row block of the group]
-    uint32_t *part_acc;
+    float *part_acc;
 };
 
 // what a position past the end of a query's keys is fetched from (see mla_roles.hip)
@@ -143,11 +143,6 @@ __device__ __forceinline__ float vmax(float a, float b) {
 __device__ __forceinline__ float vmax3(float a, float b, float c) {
     float r;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ uint32_t umax3(uint32_t a, uint32_t b, uint32_t c) {
-    uint32_t r;
-    asm("v_max3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
 #define LDS_AT(type, a) (*(type *)(size_t)(uint32_t)(a))
@@ -715,29 +710,16 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
                     }
                 }
             } else {
-                // the layout, the 16-bit fixed point and the write-through stores of mla_roles.hip's partials
-                uint32_t bm = 0u;
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const u32x4 a = __builtin_bit_cast(u32x4, oacc[0][j]) & 0x7FFFFFFFu;
-                    bm = umax3(bm, a[0], umax3(a[1], a[2], a[3]));
-                }
-                bm = lanes_xor32_max(lanes_xor16_max(bm));
-                const float big = bm > 0x7F7FFFFFu ? __builtin_nanf("") : __builtin_bit_cast(float, bm);
-                const float to_unit = big > 0.0f ? 1.0f / big : 0.0f;
+                // The layout and the write-through stores of mla_roles.hip's partials, but the accumulators as
+                // they are: the sums of an uncut chunk stay in fp32 from the first product to the output, and
+                // so do those that meet in the merge.
                 const size_t pb = ((size_t)grp * n_slices + slice) * p.gsz + h;
-                uint32_t *pq = p.part_acc + (pb * (VDIM / 16) + 8 * cw) * 128 + lane * 2;   // [dim block][lane][4 x i16]
+                float *pq = p.part_acc + ((pb * (VDIM / 16) + 8 * cw) * 64 + lane) * 4;   // [dim block][lane][4]
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const f32x4 v = oacc[0][j] * to_unit;
-                    u32x2 w;
-                    w[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(v[0], v[1]));
-                    w[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(v[2], v[3]));
-                    store_through8(pq + j * 128, w);
-                }
+                for (int j = 0; j < 8; j++) store_through16(pq + j * 256, __builtin_bit_cast(u32x4, oacc[0][j]));
                 if (g == 0)
                     *(f32x4 *)(p.part_ml + ((pb * 4 + cw) * 16 + n) * 4) =
-                        (f32x4){lsum[64 + h * 16 + n] * 0.69314718055994530942f, L, big * unit_f * (1.0f / 32767.0f), 0.0f};
+                        (f32x4){lsum[64 + h * 16 + n] * 0.69314718055994530942f, L, unit_f, 0.0f};
             }
             // the next row block moves up: one copy of the code above serves the four
 #pragma unroll
@@ -751,18 +733,22 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
 // How many of the chunk's `groups` stay whole (the last ones, which have the most keys) and into how
 // many slices the others are cut.  One workgroup runs per compute unit, so whole groups beyond the last
 // full round leave units idle; cut, they fill it.  In steps of one key tile (1.45 us) a workgroup costs
-// its tiles and about five more (Q, the first tiles' way into LDS, the output); partials and their merge
-// cost one, and four for every 256 slices (64 KB each, written and read); and when every compute unit
-// is busy the clock drops by a sixth, so a round that is not full is cheaper than its share.  Fitted to
-// a sweep of slice counts over eleven shapes: 333 queries of 64 heads over 1624 rows 96 us whole, 81 with
-// the last 77 groups in three slices; 666 groups of the same rows 146 us whole, 156 in slices.
+// its tiles and five more (Q, the first tiles' way into LDS, the output; three and two for smaller
+// groups); the merge costs three and a hundredth per slice, the partials one for every 256 row blocks
+// (32 KB each, written and read); and when every compute unit is busy the clock drops by a sixth, so a
+// round that is not full is cheaper than its share.  Fitted to a sweep of group sizes and slice counts
+// over 25 shapes (1 to 512 queries of 16 to 128 heads behind 200 to 28000 rows): what it picks is 0.7 %
+// slower than the best of the sweep on the mean, 7 % at the worst.  333 queries of 64 heads over 1624
+// rows 86 us whole, 80 with the last 77 groups in three slices; 180 groups of 2090 rows 58 us whole, 81
+// in two slices; 20 queries of 64 heads over 320 rows 13.8 us in groups of one row block, 21 in five
+// slices of groups of two.
 struct WidePlan {
     uint32_t whole, slices;
     double time;
 };
 WidePlan plan_slices(int64_t groups, int gsz, int64_t tiles_first, int64_t tiles_last) {
     const int64_t cus = num_cus();
-    const double over = gsz == 4 ? 5.0 : gsz == 2 ? 4.0 : 3.5;
+    const double over = gsz == 4 ? 5.0 : gsz == 2 ? 3.0 : 2.0;
     WidePlan best{(uint32_t)groups, 1, 0.0};
     if (groups > 16 * cus) return best;              // many rounds: what the last one leaves idle is nothing
     auto tiles_at = [&](int64_t i) { return tiles_first + (tiles_last - tiles_first) * i / (groups > 1 ? groups - 1 : 1); };
@@ -780,9 +766,9 @@ WidePlan plan_slices(int64_t groups, int gsz, int64_t tiles_first, int64_t tiles
     const int64_t full = groups / cus * cus;
     for (int64_t whole = full; whole >= 0 && whole >= full - cus; whole -= cus) {
         const int64_t rest = groups - whole, tiles = rest ? tiles_at(rest - 1) : 0;
-        const double base = whole_time(whole) + 1.0;
+        const double base = whole_time(whole) + 3.0;
         for (int64_t s = 2; s <= tiles && rest * s <= 4 * cus && rest; s++) {
-            const double t = base + rounds(rest * s, (tiles + s - 1) / s) + (double)(gsz * rest * s) / (double)cus;
+            const double t = base + 0.01 * (double)s + rounds(rest * s, (tiles + s - 1) / s) + (double)(gsz * rest * s) / (double)cus;
             if (t < best.time) best = WidePlan{(uint32_t)whole, (uint32_t)s, t};
         }
     }
@@ -828,10 +814,10 @@ int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, i
     p.slices_inv = div_inverse(plan.slices);
     if (p.n_rest) {
         const size_t blocks = (size_t)p.n_rest * p.n_slices * p.gsz;
-        const size_t acc_b = blocks * 16 * VDIM * sizeof(int16_t);
+        const size_t acc_b = blocks * 16 * VDIM * sizeof(float);
         char *ws = (char *)workspace(s, acc_b + blocks * 4 * 16 * 4 * sizeof(float));
         if (!ws) return 0;                      // workspace() has recorded why
-        p.part_acc = (uint32_t *)ws;
+        p.part_acc = (float *)ws;
         p.part_ml = (float *)(ws + acc_b);
     }
     {
@@ -842,7 +828,7 @@ int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, i
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (p.n_rest)
-        return launch_mla_merge(p.part_acc, p.part_ml, (int)p.n_slices, (int)p.n_rest, (int)p.gsz, (int)p.nhb, (int64_t)p.n_rb,
+        return launch_mla_merge((const f32x4 *)p.part_acc, p.part_ml, (int)p.n_slices, (int)p.n_rest, (int)p.gsz, (int)p.nhb, (int64_t)p.n_rb,
                                 n_heads, nullptr, out, CWICK_HIP_PROF_MLA_MERGE, s);
     return 1;
 }

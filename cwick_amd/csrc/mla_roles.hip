@@ -728,9 +728,10 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
     }
 }
 
-// merge of fragment-layout partials: values [y][split][16-head block][dim block][lane][4] as
-// 16-bit fixed point, and per 16-head block and quarter of the dims [head][4] floats (running
-// maximum in natural-log units, weight sum, value of one fixed-point step, unused).  With more
+// merge of fragment-layout partials: values [y][split][16-head block][dim block][lane][4], as 16-bit
+// fixed point (the decode's) or fp32 (the chunk prefill's), and per 16-head block and quarter of the
+// dims [head][4] floats (running maximum in natural-log units, weight sum, value of one fixed-point step
+// or unit of the accumulators, unused).  With more
 // than eight splits a workgroup is one dim block of one 16-head block: its waves (eight up to
 // 64 splits, where a wave then has its eight loads in flight at once: 4.55 -> 4.16 us; sixteen
 // beyond) take splits w, w + n_waves, ... and meet in LDS.  With up to eight a wave merges a dim block alone and
@@ -739,19 +740,24 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
 // loads in flight at once (eight splits per batch); which splits exist is uniform per wave, so
 // absent ones cost nothing.
 constexpr int MW = 16;
-__device__ __forceinline__ void merge_add(f32x4 &acc, float &ls, const u32x2 a, const f32x4 v, const float mx) {
+__device__ __forceinline__ f32x4 part_value(const u32x2 a) {
+    return (f32x4){(float)((int32_t)(a[0] << 16) >> 16), (float)((int32_t)a[0] >> 16),
+                   (float)((int32_t)(a[1] << 16) >> 16), (float)((int32_t)a[1] >> 16)};
+}
+__device__ __forceinline__ f32x4 part_value(const f32x4 a) { return a; }
+template <class PART>
+__device__ __forceinline__ void merge_add(f32x4 &acc, float &ls, const PART a, const f32x4 v, const float mx) {
     const float c = v[0] == -INFINITY ? 0.0f : __expf(v[0] - mx);
     ls = __builtin_fmaf(v[1], c, ls);
     const float cs = c * v[2];
-    acc[0] = __builtin_fmaf((float)((int32_t)(a[0] << 16) >> 16), cs, acc[0]);
-    acc[1] = __builtin_fmaf((float)((int32_t)a[0] >> 16), cs, acc[1]);
-    acc[2] = __builtin_fmaf((float)((int32_t)(a[1] << 16) >> 16), cs, acc[2]);
-    acc[3] = __builtin_fmaf((float)((int32_t)a[1] >> 16), cs, acc[3]);
+    const f32x4 x = part_value(a);
+#pragma unroll
+    for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(x[r], cs, acc[r]);
 }
-__global__ void __launch_bounds__(64 * MW)
-mla_merge_frag16_kernel(const uint32_t *__restrict__ part_acc, const float *__restrict__ part_ml,
-                        int n_splits, int n_hb16, int nhb, uint32_t n_rb, int nh, const float *__restrict__ sink,
-                        float *__restrict__ out, int packed) {
+template <class PART>                             // u32x2: four 16-bit values; f32x4
+__device__ __forceinline__ void
+merge_frag(const PART *__restrict__ part_acc, const float *__restrict__ part_ml, int n_splits, int n_hb16, int nhb,
+           uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out, int packed) {
     __shared__ float red_m[MW][64];
     __shared__ float red_l[MW][64];
     __shared__ f32x4 red_a[MW][64];
@@ -774,20 +780,20 @@ mla_merge_frag16_kernel(const uint32_t *__restrict__ part_acc, const float *__re
     const size_t sb = (size_t)y * n_splits;
     const float *ml = part_ml + (((sb * n_hb16 + hb) * 4 + (db >> 3)) * HB + n) * 4;
     const size_t ml_stride = (size_t)n_hb16 * 4 * HB * 4;
-    const uint32_t *pa = part_acc + ((sb * n_hb16 + hb) * NDB + db) * 128 + lane * 2;
-    const size_t pa_stride = (size_t)n_hb16 * NDB * 128;
+    const PART *pa = part_acc + ((sb * n_hb16 + hb) * NDB + db) * 64 + lane;
+    const size_t pa_stride = (size_t)n_hb16 * NDB * 64;
 
     // first batch: everything in flight before anything is waited for
-    u32x2 a0[8];
+    PART a0[8];
     f32x4 v0[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const int s = wv + mw * j;
         v0[j] = (f32x4){-INFINITY, 0.0f, 0.0f, 0.0f};
-        a0[j] = (u32x2){0u, 0u};
+        a0[j] = PART{};
         if (s < n_splits) {
             v0[j] = *(const f32x4 *)(ml + s * ml_stride);
-            a0[j] = *(const u32x2 *)(pa + s * pa_stride);
+            a0[j] = pa[s * pa_stride];
         }
     }
     float mx = -INFINITY;
@@ -805,16 +811,16 @@ mla_merge_frag16_kernel(const uint32_t *__restrict__ part_acc, const float *__re
 #pragma unroll
     for (int j = 0; j < 8; j++) merge_add(acc, ls, a0[j], v0[j], mx);
     for (int s0 = wv + 8 * mw; s0 < n_splits; s0 += 8 * mw) {
-        u32x2 a[8];
+        PART a[8];
         f32x4 v[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int s = s0 + mw * j;
             v[j] = (f32x4){-INFINITY, 0.0f, 0.0f, 0.0f};
-            a[j] = (u32x2){0u, 0u};
+            a[j] = PART{};
             if (s < n_splits) {
                 v[j] = *(const f32x4 *)(ml + s * ml_stride);
-                a[j] = *(const u32x2 *)(pa + s * pa_stride);
+                a[j] = pa[s * pa_stride];
             }
         }
 #pragma unroll
@@ -847,6 +853,16 @@ mla_merge_frag16_kernel(const uint32_t *__restrict__ part_acc, const float *__re
     // accumulator register i <-> dim 16 db + 4 g + i
     *(f32x4 *)(out + ((size_t)yq * nh + head) * VDIM + 16 * db + 4 * g) = r4;
 }
+__global__ void __launch_bounds__(64 * MW)
+mla_merge_frag16_kernel(const u32x2 *__restrict__ part_acc, const float *__restrict__ part_ml, int n_splits, int n_hb16,
+                        int nhb, uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out, int packed) {
+    merge_frag(part_acc, part_ml, n_splits, n_hb16, nhb, n_rb, nh, sink, out, packed);
+}
+__global__ void __launch_bounds__(64 * MW)
+mla_merge_frag32_kernel(const f32x4 *__restrict__ part_acc, const float *__restrict__ part_ml, int n_splits, int n_hb16,
+                        int nhb, uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out, int packed) {
+    merge_frag(part_acc, part_ml, n_splits, n_hb16, nhb, n_rb, nh, sink, out, packed);
+}
 
 // Split-K partials of the entry point that may not allocate (cwick_hip_mla_decode_static_dev):
 // a fixed area in the library's own device image instead of the grow-only workspace.  Host code
@@ -869,15 +885,24 @@ static void *static_scratch() {
 
 }  // namespace
 
-int launch_mla_merge(const uint32_t *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
-                     int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s) {
+template <class PART>
+static int launch_merge_of(void (*kernel)(const PART *, const float *, int, int, int, uint32_t, int, const float *, float *, int),
+                           const PART *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
+                           int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s) {
     const bool packed = n_splits <= 8;
     ProfKernel pk(prof, s);
-    pk.launch(mla_merge_frag16_kernel, dim3(n_hb16 * (packed ? 4 : NDB), n_groups),
-              dim3(64 * (packed || n_splits <= 64 ? 8 : MW)), 0, part_acc, part_ml, n_splits, n_hb16, nhb, (uint32_t)n_rb, nh,
-              sink, out, packed ? 1 : 0);
+    pk.launch(kernel, dim3(n_hb16 * (packed ? 4 : NDB), n_groups), dim3(64 * (packed || n_splits <= 64 ? 8 : MW)), 0,
+              part_acc, part_ml, n_splits, n_hb16, nhb, (uint32_t)n_rb, nh, sink, out, packed ? 1 : 0);
     CWICK_HIP_CALL(hipGetLastError());
     return 1;
+}
+int launch_mla_merge(const u32x2 *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
+                     int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s) {
+    return launch_merge_of(mla_merge_frag16_kernel, part_acc, part_ml, n_splits, n_groups, n_hb16, nhb, n_rb, nh, sink, out, prof, s);
+}
+int launch_mla_merge(const f32x4 *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
+                     int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s) {
+    return launch_merge_of(mla_merge_frag32_kernel, part_acc, part_ml, n_splits, n_groups, n_hb16, nhb, n_rb, nh, sink, out, prof, s);
 }
 
 namespace {
@@ -925,7 +950,7 @@ int run(Params &p, hipStream_t s, bool fixed = false) {
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (p.n_splits > 1)
-        return launch_mla_merge(p.part_acc, p.part_ml, p.n_splits, p.nq, 2 * n_hb, 2 * n_hb, (int64_t)p.nq * 2 * n_hb, p.nh,
+        return launch_mla_merge((const u32x2 *)p.part_acc, p.part_ml, p.n_splits, p.nq, 2 * n_hb, 2 * n_hb, (int64_t)p.nq * 2 * n_hb, p.nh,
                                 p.sink, p.out, fixed ? -1 : CWICK_HIP_PROF_MLA_MERGE, s);
     return 1;
 }

@@ -529,7 +529,7 @@ enum {
     CWICK_HIP_PROF_GQA_DECODE_MERGE,    /* splitk_merge_wide_kernel<256|128> after it (not for lists of up to 192 keys) */
     CWICK_HIP_PROF_GQA_PREFILL,         /* gqa_prefill_kernel, or gqa_prefill_split_kernel without the merge after it */
     CWICK_HIP_PROF_MLA,                 /* mla_roles_kernel (decode, sparse, prefill of at most 32 heads) */
-    CWICK_HIP_PROF_MLA_MERGE,           /* mla_merge_frag16_kernel after it */
+    CWICK_HIP_PROF_MLA_MERGE,           /* mla_merge_frag16_kernel after it; mla_merge_frag32_kernel after a chunk in slices */
     CWICK_HIP_PROF_INDEXER,             /* indexer_scores_kernel, or in a fused select indexer_approx_kernel + topk_mw_hist_kernel + topk_mw_classify_kernel + indexer_rescore_kernel + the exact kernel's fallback pass */
     CWICK_HIP_PROF_TOPK,                /* every kernel of one top-k call: topk_mw_hist_kernel x4 + topk_mw_emit_kernel, or topk_radix[_reg]_kernel; in a fused select topk_band_finish_kernel */
     CWICK_HIP_PROF_MLA_PREFILL,         /* mla_prefill64_kernel (chunked prefill of more than 32 heads) */

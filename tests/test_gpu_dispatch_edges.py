@@ -190,6 +190,27 @@ def test_mla_prefill_groups_and_slices(hip, orc, n, pos0, nh):
     cache.free()
 
 
+@pytest.mark.parametrize("n,pos0,nh", [(8, 20000, 128), (1, 5000, 16), (5, 3000, 24), (300, 700, 64)])
+def test_mla_prefill_slices_keep_their_sums(hip, n, pos0, nh):
+    """The keys of a group in slices: what the slices hand to the merge has all its bits.  A query of zeros
+    weighs every key the same, and rows of small whole numbers with unit scales make every product and
+    every sum exact in fp32 (below 2^24), in a slice and over all of them.  What is left is the
+    reciprocal of the key count and the multiplication by it: half a unit in the last place each, 2^-23
+    together; twice that is allowed.  (Sums handed over in 16 bits are off by 2^-16 of the largest.)"""
+    import torch
+    say("[case] mla prefill, sums of slices", n, pos0, nh)
+    g = synth.rng(88)
+    vals = g.integers(-7, 8, (pos0 + n, synth.KDIM)).astype(np.float32)
+    rows = torch.from_numpy(vals).to(torch.float8_e4m3fn).view(torch.uint8).numpy()
+    cache = hip.LatentCache(1, pos0 + n)
+    cache.write(0, 0, rows, np.ones((pos0 + n, synth.NBLK), np.float32))
+    got = hip.mla_prefill_chunk(cache, 0, pos0, np.zeros((n, nh, synth.KDIM), np.uint16), 0.1).astype(np.float64)
+    sums = np.cumsum(vals[:, :synth.VDIM].astype(np.float64), axis=0)[pos0:]
+    ref = (sums / (pos0 + 1 + np.arange(n))[:, None])[:, None, :]
+    assert (np.abs(got - ref) <= 2.0 ** -22 * np.abs(ref)).all(), "rel %.2e" % (np.abs(got - ref).max() / np.abs(ref).max())
+    cache.free()
+
+
 @pytest.mark.parametrize("pos0", [61, 64, 700])
 def test_mla_prefill_later_rows_stay_out(hip, orc, pos0):
     """Queries that share a workgroup: a later query's row of NaN bytes, or with a scale far above the
