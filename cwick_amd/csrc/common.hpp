@@ -6,6 +6,7 @@
 #include <stddef.h>
 
 #include "../../include/cwick_hip.h"
+#include "band_counter.hpp"
 
 namespace cwick {
 
@@ -104,7 +105,8 @@ int launch_indexer_scores(const uint8_t *keys, const float *kscale, int64_t key_
 struct IndexerBandRow {
     uint32_t n_cand;      // keys inside the band (may exceed the list's capacity)
     uint32_t fallback;    // the band could not be formed (bound not finite, NaN threshold)
-    uint32_t pad[30];     // a row to a 128-byte line: the workgroups of different rows add to n_cand at the same time
+    uint32_t octave;      // the lowest of the octaves that the row's counters resolve (band_counter)
+    uint32_t pad[29];     // a row to a 128-byte line: the workgroups of different rows add to n_cand at the same time
 };
 constexpr int CWICK_INDEXER_BAND_CAP = 4096;   // candidate list entries per row
 constexpr int CWICK_INDEXER_APPROX_KEYS = 2048;   // keys per workgroup (= per bound slot) of the approximate kernel
@@ -115,8 +117,8 @@ int launch_indexer_approx(const uint8_t *keys, const float *kscale, int64_t key_
                           int64_t kscale_bstride, int batch, int64_t n_keys, const uint16_t *q_idx,
                           const float *w, int n_idx_heads, float *scores, float *beta_slots,
                           IndexerBandRow *rows, uint32_t *digits, hipStream_t s);
-// What the approximate kernel leaves for the select, per row and workgroup (slot): how many of its scores'
-// order keys have each leading byte, and each leading twelve bits (16-bit counts).
+// What the approximate kernel leaves for the select, per row and workgroup (slot): how many of its scores
+// each of 4096 counters has (16-bit counts; band_counter), and each sixteen of them together.
 constexpr int CWICK_BAND_DIGITS = 256 + 4096 / 2;         // dwords per slot
 inline size_t indexer_band_digits_dwords(int64_t n_keys) { return (size_t)indexer_approx_slots(n_keys) * CWICK_BAND_DIGITS; }
 __host__ __device__ inline bool indexer_band_failed(const IndexerBandRow &r, int cap) {
@@ -137,7 +139,7 @@ int launch_indexer_banded(const uint8_t *keys, const float *kscale, int64_t key_
                           int64_t kscale_bstride, int batch, int64_t n_keys, const uint16_t *q_idx,
                           const float *w, int n_idx_heads, int64_t k, float *scores, int32_t *out_idx,
                           hipStream_t s);
-// top-k machinery on approximate scores: finds T to twelve bits from the approximate kernel's counts, then
+// top-k machinery on approximate scores: finds the counter that T is in from the approximate kernel's counts, then
 // patches the scores (+inf / -inf / kept) and lists the keys that may lie on either side.
 size_t topk_mw_workspace_bytes(int batch, int64_t n);
 int launch_topk_band_classify(float *scores, int batch, int64_t n, int64_t k, const uint32_t *digits,

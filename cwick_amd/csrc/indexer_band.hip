@@ -18,13 +18,14 @@
 //      and sum_h |w_h| A_h[t] = sum_i |e_ti| c_i with c_i = sum_h |w_h||q_hi|: one more row
 //      through the matrix core, with c rounded up to bf16.  beta[t] = 512 u * ks[t] * that row
 //      (the slack covers the rounding of the bound itself); beta = max_t beta[t].
-//   2. top-k machinery on st: T = the k-th largest approximate score, to the twelve leading bits of its
-//      order key, which the approximate kernel has counted (topk.hip).
+//   2. top-k machinery on st: T = the k-th largest approximate score, to the counter it is in: the
+//      approximate kernel counts its scores in 4096 of them per row, a 128th of an octave wide in the
+//      fourteen octaves where a row's large scores are (topk.hip; band_counter, common.hpp).
 //   3. classify: at most k-1 keys have st > T.  A key with st > T + 2 beta has s > T + beta, and
 //      every key that scores at least as much has st > T: it is among at most k-2 others, so it
 //      is selected whatever the ties do.  At least k keys have st >= T, hence s >= T - beta; a
 //      key with st < T - 2 beta has s < T - beta and is not selected.  The first kind gets +inf,
-//      the second -inf, the rest (a few hundred of 65536) are candidates.
+//      the second -inf, the rest (about a hundred of 65536) are candidates.
 //   4. indexer_rescore_kernel: the reference's arithmetic, instruction for instruction as in
 //      indexer.hip, for the candidates only, spread over heads so that it takes microseconds.
 //   5. the selection is the +inf keys (fewer than k, all selected) and the best k - (their number)
@@ -63,10 +64,11 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
                       uint32_t *__restrict__ digits) {   // or null: [batch][slots][CWICK_BAND_DIGITS]
     __shared__ __attribute__((aligned(16))) float cpart_sh[IB_THREADS / 16][IB_HD];
     __shared__ __attribute__((aligned(16))) uint16_t cb_sh[IB_HD + 64];          // coefficients, then 128 bytes of zeros
-    __shared__ __attribute__((aligned(16))) uint32_t hist12[4096];
+    __shared__ __attribute__((aligned(16))) uint32_t counts[4096];
     __shared__ __attribute__((aligned(16))) uint16_t q_sh[64 * IB_QROW];
     __shared__ float w_sh[64];
     __shared__ float bmax_sh[IB_THREADS / 64];
+    __shared__ uint32_t cmax_sh[2], kexp_sh;
     const int b = blockIdx.y, wg = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint16_t *qb = q + (size_t)b * ih * IB_HD;
@@ -102,6 +104,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     // tid % 16) holds dims 8 part .. +7 of heads group + 16 j, adds up its four heads and leaves
     // the eight sums in LDS; after the barrier thread i < 128 adds the sixteen groups of dim i.
     bf16x8 qa[2][8];
+    uint32_t ks_bits = 0u;              // 64 key scales from all over the row, the same ones in every workgroup
     {
         // (the weights first: a load that is waited for drags every load issued before it along)
         const float w_mine = (tid < 64 && tid < ih) ? wb[tid] : 0.0f;
@@ -120,6 +123,8 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
             stage[j] = *(const u32x4 *)(qb + (size_t)hc * IB_HD + 8 * part);
             if (head >= ih) stage[j] = (u32x4){0u, 0u, 0u, 0u};
         }
+        // (behind the queries, which the first barrier waits for)
+        if (wave == IB_WAVES - 1) ks_bits = __builtin_bit_cast(uint32_t, ksb[(int64_t)lane * n_keys >> 6]);
         load_keys(0, raw_a, kst_a);
         load_keys(1, raw_b, kst_b);
         float cp[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -139,7 +144,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
         if (tid < 64) w_sh[tid] = w_mine;
     }
 #pragma unroll
-    for (int j = 0; j < 4096 / IB_THREADS; j++) hist12[tid + IB_THREADS * j] = 0u;
+    for (int j = 0; j < 4096 / IB_THREADS; j++) counts[tid + IB_THREADS * j] = 0u;
     __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < 2; mb++)
@@ -154,8 +159,33 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
         for (int k = 0; k < IB_THREADS / 16; k++) c += part[k];
         cb_sh[tid] = (uint16_t)((__builtin_bit_cast(uint32_t, c) + 0xFFFFu) >> 16);     // rounded up to bf16
         if (tid < 64) cb_sh[IB_HD + tid] = 0;
+        const uint32_t top = wave_max_u32(__builtin_bit_cast(uint32_t, c));             // (never negative)
+        if (lane == 0) cmax_sh[wave] = top;
+    }
+    if (wave == IB_WAVES - 1) {
+        // the exponent that a quarter of them reach; scales of 0 and 1, which keys of zeros have, do not count
+        const uint32_t e = ks_bits == 0x3F800000u ? 0u : ks_bits >> 23 & 0xFFu;
+        const int quarter = (__builtin_popcountll(__ballot(e != 0u)) + 3) / 4;
+        uint32_t upper = 0u;
+#pragma unroll
+        for (int bit = 7; bit >= 0; bit--)
+            if (__builtin_popcountll(__ballot(e >= (upper | 1u << bit))) >= quarter) upper |= 1u << bit;
+        if (lane == 0) kexp_sh = quarter ? upper : 127u;
     }
     __syncthreads();
+    // The octaves that get most of the counters: a score is at most ks sum_i |e_i| c_i <= ks 448 * 128 max c,
+    // so with the scales above the largest are around 2^16 ks max c, and what threshold a selection has lies
+    // 2 to 13 octaves below that (heads that agree; signed weights that cancel).  Every workgroup of the
+    // row finds the same ones; what they are decides how many candidates there are, not which keys win.
+    uint32_t octave;
+    {
+        const uint32_t c_top = cmax_sh[0] > cmax_sh[1] ? cmax_sh[0] : cmax_sh[1];
+        int lowest = (int)(c_top >> 23 & 0xFFu) + (int)kexp_sh - 127 + 16 - ((int)BAND_OCTAVES - 1);
+        lowest = lowest < 0 ? 0 : lowest;
+        lowest = lowest > 256 - (int)BAND_OCTAVES ? 256 - (int)BAND_OCTAVES : lowest;
+        octave = (uint32_t)__builtin_amdgcn_readfirstlane(lowest);
+    }
+    if (wg == 0 && tid == 0) rows[b].octave = octave;
     // the bound row's A fragments are read from LDS step by step: lanes of row 0 from the
     // coefficients, all others from a stretch of zeros behind them
     const char __attribute__((address_space(3))) *c_lane =
@@ -249,9 +279,8 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
         const float beta = band * fabsf(kst) * (512.0f / 16777216.0f);
         if (live && g == 0) {
             scores[(size_t)b * n_keys + t] = st;
-            // the select's pass over the scores, done here: the leading twelve bits of the order key
-            // (sign, exponent and three more: the scores of an exponent spread over eight counters)
-            atomicAdd(&hist12[topk_key(st) >> 20], 1u);
+            // the select's pass over the scores, done here
+            atomicAdd(&counts[band_counter(st, octave)], 1u);
         }
         if (live) bmax = (beta <= bmax) ? bmax : beta;             // NaN sticks
     };
@@ -281,11 +310,11 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
         beta_slots[(size_t)b * gridDim.x + wg] = m;
     }
     if (digits && tid < 256) {
-        // thread t: the sixteen counters of leading byte t
+        // thread t: counters 16 t .. + 15
         uint32_t *slot = digits + ((size_t)b * gridDim.x + wg) * CWICK_BAND_DIGITS;
         u32x4 c[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) c[j] = *(const u32x4 *)&hist12[16 * tid + 4 * j];
+        for (int j = 0; j < 4; j++) c[j] = *(const u32x4 *)&counts[16 * tid + 4 * j];
         u32x4 w[2];
 #pragma unroll
         for (int j = 0; j < 8; j++) w[j >> 2][j & 3] = c[j >> 1][2 * (j & 1)] | c[j >> 1][2 * (j & 1) + 1] << 16;   // at most 2048 each
@@ -464,11 +493,11 @@ int launch_indexer_banded(const uint8_t *keys, const float *kscale, int64_t key_
     if (!launch_topk_band_classify(scores, batch, n_keys, k, (const uint32_t *)ws, beta_slots, n_wg, cand, cap, rows,
                                    hi_count, s))
         return 0;
-    // Sixteen candidates per workgroup and round, up to a thousand and more per row: 96 workgroups take them
-    // in one round (8 rows of 64K keys: 59.6 us the step with 32 per row, 56.5 with 64, 54.5 with 96, 55 with
-    // 128).  With many rows fewer, because workgroups that find nothing to do cost their launch.
-    const int share = num_cus() / batch, most = 4 * share < 96 ? 4 * share : 96;
-    int rescore_wgs = share > most ? share : most;
+    // Sixteen candidates per workgroup and round, one or two hundred per row: 32 workgroups a row take them in
+    // one (8 rows of 64K keys: 56.4 us the step with 8 per row, 53.3 with 16 or 32, 54.6 with 64 or 96; with
+    // equal weights 60.3, 56.9, 53.7, 54.9).  With few rows there are more, for a row that scores all of its
+    // keys; with many rows fewer, because workgroups that find nothing to do cost their launch.
+    int rescore_wgs = num_cus() / batch;
     rescore_wgs = rescore_wgs < 8 ? 8 : (rescore_wgs > cap / 16 ? cap / 16 : rescore_wgs);
     indexer_rescore_kernel<<<dim3(rescore_wgs, batch), 256, 0, s>>>(
         keys, kscale, key_bstride, kscale_bstride, n_keys, q_idx, w, n_idx_heads, cand, cap, rows, scores, cand_score);

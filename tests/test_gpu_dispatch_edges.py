@@ -281,6 +281,51 @@ def test_dsa_band_of_short_rows(hip, orc, n_keys, batch, topk):
     lat.free()
 
 
+@pytest.mark.parametrize("weights", ["signed", "positive", "equal", "negative"])
+@pytest.mark.parametrize("keys", ["independent", "common", "small with empty rows"])
+def test_dsa_band_takes_every_kind_of_score(hip, orc, weights, keys):
+    """Scores of one sign lie within an octave or two, keys with a common component closer still: the
+    threshold's counter has to be narrow enough for the candidate list there as well.  The scratch
+    scores tell: a row on the band keeps numbers for its candidates alone, a row that fell back for all
+    of its keys.  At 7 bits of fraction the threshold's counter holds 50 to 250 keys of these rows
+    (counted on the CPU), and the error bound's band a few dozen more; 12 leading bits held 400 to 5500."""
+    import torch
+    say("[case] dsa band", weights, keys)
+    n_keys, batch, topk, ih = 65536, 2, 2048, 64
+    c = synth.cfg5_dsa(n_keys=n_keys, batch=batch, ih=ih, topk=topk, nh=16, shared=False, seed=89)
+    g = synth.rng(90)
+    w = c["w"]
+    w = {"signed": w, "positive": np.abs(w), "equal": np.full_like(w, 0.011), "negative": -np.abs(w)}[weights]
+    kb, ks = c["ikeys"], c["ikscale"]
+    if keys != "independent":
+        x = g.standard_normal((batch, n_keys, 128), dtype=np.float32)
+        if keys == "common":
+            x += g.standard_normal((batch, 1, 128), dtype=np.float32)
+        else:
+            x *= np.float32(1e-3)
+            x[:, ::3] = 0.0                                   # quantised to zeros with a scale of 1
+        amax = np.abs(x).max(axis=2)
+        ks = np.where(amax > 0, amax / 448.0, 1.0).astype(np.float32)
+        kb = torch.from_numpy(np.clip(x / ks[:, :, None], -448, 448)).to(torch.float8_e4m3fn).view(torch.uint8).numpy()
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    ops = [d(kb), d(ks), d(c["rows"]), d(c["scales"]), d(c["q_idx"].view(np.int16)), d(w), d(c["q"].view(np.int16))]
+    tmp = torch.empty((batch, n_keys), dtype=torch.float32, device="cuda")
+    sel = torch.empty((batch, topk), dtype=torch.int32, device="cuda")
+    out = torch.empty((batch, 16, synth.VDIM), dtype=torch.float32, device="cuda")
+    hip.dsa_decode_dev(ops[0], ops[1], n_keys * 128, n_keys, ops[2], ops[3], n_keys * synth.KDIM, n_keys * synth.NBLK, batch,
+                       n_keys, ops[4], ops[5], ih, topk, ops[6], 16, c["scale"], tmp, sel, out,
+                       torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    kept = torch.isfinite(tmp).sum(dim=1).tolist()
+    say("[band] candidates", kept)
+    for b in range(batch):
+        sc = orc.indexer_scores(c["q_idx"][b], w[b], kb[b], ks[b], nthreads=0)
+        assert np.array_equal(sel[b].cpu().numpy(), orc.topk_contract(sc, topk)), "query %d" % b
+        # (negative weights and empty rows: 20000 keys tie for the best score, 0, whatever the counters)
+        ties = weights == "negative" and keys == "small with empty rows"
+        assert kept[b] <= 512 or ties, "query %d: %d candidates" % (b, kept[b])
+
+
 @pytest.mark.parametrize("limit,ih,block,keep", [(1, 1, 64, 1), (63, 3, 64, 2), (130, 5, 128, 4), (1000, 2, 100, 3), (66000, 8, 64, 16),
                                                  (70000, 4, 17, 8)])
 def test_mm_select_edges(hip, orc, limit, ih, block, keep):
