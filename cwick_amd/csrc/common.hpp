@@ -39,7 +39,11 @@ int num_cus();
 // Slot WS_NESTED belongs to launchers that other launchers call with operands in slot WS_MAIN
 // (the top-k select inside the block selections).
 constexpr int WS_MAIN = 0, WS_NESTED = 1, WS_SLOTS = 2;
+// A launcher asks for what any smaller call of its kind would need too, so that a stream that has run a
+// shape has room for the smaller ones under capture.
 void *workspace(hipStream_t s, size_t bytes, int slot = WS_MAIN);
+// The same for launchers that can do without: null, and nothing recorded.
+void *workspace_if_free(hipStream_t s, size_t bytes);
 // Where a kernel reports to the host that its results are there: workgroup i writes `epoch` to flags[i]
 // (host memory) when its stores are through.  The launcher says how many workgroups do.
 struct HostFlags {
@@ -49,6 +53,7 @@ struct HostFlags {
 };
 constexpr int HOST_FLAGS_MAX = 1024;
 uint32_t *ticket_counters(hipStream_t s);   // 64 dwords per stream, zero between kernels; null under capture if not there yet
+uint32_t *ticket_counters_if_free(hipStream_t s);   // the same, and nothing recorded
 
 // Phase timer: brackets the launches made while it is alive with two events on
 // `s` when profiling is enabled; does nothing (and records nothing) otherwise.

@@ -365,16 +365,17 @@ static int run_gqa_decode(const uint16_t *k, const uint16_t *v, int64_t n_keys, 
     const int n_splits = (int)((n_keys + per - 1) / per);
     float *part_acc = nullptr, *part_ml = nullptr;
     if (n_splits > 1) {
-        const size_t acc_bytes = (size_t)n_splits * n_heads * HD * sizeof(float);
-        const size_t ml_bytes = (size_t)n_splits * n_heads * 2 * sizeof(float);
-        char *ws = (char *)workspace(s, acc_bytes + ml_bytes);
+        // (asked for: as many splits as any call of up to this many keys has)
+        const int64_t single = 2 * num_cus() / n_kv_heads, most = steps < single ? steps : single;
+        const size_t per_split = (size_t)n_heads * (HD + 2) * sizeof(float);
+        char *ws = (char *)workspace(s, (size_t)(most > n_splits ? most : n_splits) * per_split);
         if (!ws) return 0;                  // workspace() has recorded why
-        part_acc = (float *)ws, part_ml = (float *)(ws + acc_bytes);
+        part_acc = (float *)ws, part_ml = part_acc + (size_t)n_splits * n_heads * HD;
     }
     uint32_t *flags = done ? done->flags : nullptr;
     const uint32_t epoch = done ? done->epoch : 0u;
-    uint32_t *tickets = nullptr;
-    if (n_splits > 1 && n_splits <= GQA_DEC_LAST_MERGE && !(tickets = ticket_counters(s))) return 0;   // the reason is recorded
+    uint32_t *tickets = nullptr;            // (a stream that has none yet and is being captured merges in a second launch)
+    if (n_splits > 1 && n_splits <= GQA_DEC_LAST_MERGE) tickets = ticket_counters_if_free(s);
     const bool one_launch = n_splits == 1 || tickets;
     if (done) done->count = one_launch ? n_kv_heads : n_heads;
     {

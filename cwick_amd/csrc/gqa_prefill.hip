@@ -966,17 +966,11 @@ static hipError_t pf_allow_lds(size_t bytes) {
 
 template <int GROUP, int WAVES>
 static int run_gqa_prefill_split(const uint16_t *k, const uint16_t *v, int64_t pos0, int64_t n, int n_kv_heads, const uint16_t *q,
-                                 float scale, float *out, int64_t n_prec, int pblocks, const PfPlan &plan, uint32_t *tickets,
-                                 hipStream_t s) {
+                                 float scale, float *out, int64_t n_prec, int pblocks, const PfPlan &plan, float *part,
+                                 uint32_t *tickets, hipStream_t s) {
     CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_split_kernel<GROUP, WAVES>>(sizeof(PfSmem<WAVES>))));
     const int slices = plan.first[pblocks] * n_kv_heads;
-    float *part = nullptr, *part_ml = nullptr;
-    if (plan.per) {
-        const size_t acc_bytes = (size_t)slices * PF_PART<WAVES> * sizeof(float);
-        part = (float *)workspace(s, acc_bytes + (size_t)slices * (64 * WAVES * 2) * sizeof(float));
-        if (!part) return 0;
-        part_ml = (float *)((char *)part + acc_bytes);
-    }
+    float *part_ml = part ? part + (size_t)slices * PF_PART<WAVES> : nullptr;
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_PREFILL, s);
         pk.launch(gqa_prefill_split_kernel<GROUP, WAVES>, dim3((unsigned)(slices < num_cus() ? slices : num_cus())), dim3(64 * WAVES),
@@ -989,6 +983,14 @@ static int run_gqa_prefill_split(const uint16_t *k, const uint16_t *v, int64_t p
         part, part_ml, n, n_kv_heads, pblocks, plan, out);
     CWICK_HIP_CALL(hipGetLastError());
     return 1;
+}
+
+// The partials of a plan that cuts blocks.  Null where there is no room for them (a stream that is being captured
+// and has not run the shape before): the blocks then stay whole.
+template <int WAVES>
+static float *pf_partials(const PfPlan &plan, int pblocks, int n_kv_heads, hipStream_t s) {
+    const size_t slices = (size_t)plan.first[pblocks] * n_kv_heads;
+    return (float *)workspace_if_free(s, slices * (PF_PART<WAVES> + 64 * WAVES * 2) * sizeof(float));
 }
 
 template <int GROUP>
@@ -1013,11 +1015,14 @@ static int run_gqa_prefill(const uint16_t *k, const uint16_t *v, int64_t pos0, i
         if (pblocks1 * n_kv_heads <= num_cus() && pblocks1 <= PF_MAX_BLOCKS) {
             PfPlan plan1;
             const int64_t n_prec1 = pf_precise_blocks<GROUP, 1>(pos0, n, pblocks1);
-            if (pf_plan<GROUP, 1>(pos0, n, n_kv_heads, n_prec1, (int)pblocks1, plan1) < t4)
-                return run_gqa_prefill_split<GROUP, 1>(k, v, pos0, n, n_kv_heads, q, scale, out, n_prec1, (int)pblocks1, plan1, tickets, s);
+            if (pf_plan<GROUP, 1>(pos0, n, n_kv_heads, n_prec1, (int)pblocks1, plan1) < t4) {
+                float *part = plan1.per ? pf_partials<1>(plan1, (int)pblocks1, n_kv_heads, s) : nullptr;
+                if (part || !plan1.per)
+                    return run_gqa_prefill_split<GROUP, 1>(k, v, pos0, n, n_kv_heads, q, scale, out, n_prec1, (int)pblocks1, plan1, part, tickets, s);
+            }
         }
-        if (plan.per)
-            return run_gqa_prefill_split<GROUP, PF_WAVES>(k, v, pos0, n, n_kv_heads, q, scale, out, n_prec, (int)pblocks, plan, tickets, s);
+        if (float *part = plan.per ? pf_partials<PF_WAVES>(plan, (int)pblocks, n_kv_heads, s) : nullptr)
+            return run_gqa_prefill_split<GROUP, PF_WAVES>(k, v, pos0, n, n_kv_heads, q, scale, out, n_prec, (int)pblocks, plan, part, tickets, s);
     }
     CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_kernel<GROUP>>(sizeof(PfSmem<PF_WAVES>))));
     const int64_t wgs = items < num_cus() ? items : num_cus();      // the LDS of a compute unit holds one workgroup

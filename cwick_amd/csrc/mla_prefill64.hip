@@ -808,18 +808,19 @@ int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, i
         const WidePlan x = plan_slices(gr, gsz, (pos0 + 1 + TK - 1) / TK, (pos0 + n + TK - 1) / TK);
         if (gsz == NHQ || x.time < plan.time) plan = x, groups = gr, p.gsz = (uint32_t)gsz;
     }
+    if (plan.whole < groups) {
+        const size_t blocks = (size_t)(groups - plan.whole) * plan.slices * p.gsz;
+        const size_t acc_b = blocks * 16 * VDIM * sizeof(float);
+        char *ws = (char *)workspace_if_free(s, acc_b + blocks * 4 * 16 * 4 * sizeof(float));
+        p.part_acc = (float *)ws;
+        p.part_ml = (float *)(ws + acc_b);
+        // no room for partials (a stream that is being captured and has not run the shape before): uncut
+        if (!ws) p.gsz = NHQ, groups = (p.n_rb + NHQ - 1) / NHQ, plan = WidePlan{(uint32_t)groups, 1, 0.0};
+    }
     p.n_whole = plan.whole;
     p.n_rest = (uint32_t)groups - plan.whole;
     p.n_slices = plan.slices;
     p.slices_inv = div_inverse(plan.slices);
-    if (p.n_rest) {
-        const size_t blocks = (size_t)p.n_rest * p.n_slices * p.gsz;
-        const size_t acc_b = blocks * 16 * VDIM * sizeof(float);
-        char *ws = (char *)workspace(s, acc_b + blocks * 4 * 16 * 4 * sizeof(float));
-        if (!ws) return 0;                      // workspace() has recorded why
-        p.part_acc = (float *)ws;
-        p.part_ml = (float *)(ws + acc_b);
-    }
     {
         ProfKernel pk(CWICK_HIP_PROF_MLA_PREFILL, s);
         const dim3 grid(p.n_whole + p.n_rest * p.n_slices);

@@ -908,7 +908,7 @@ int launch_mla_merge(const f32x4 *part_acc, const float *part_ml, int n_splits, 
 namespace {
 
 // fixed == true: partials go to the static area, nothing is allocated and no events are created
-int run(Params &p, hipStream_t s, bool fixed = false) {
+int run(Params &p, int most_splits, hipStream_t s, bool fixed) {
     static std::once_flag attr_once;
     static hipError_t attr_err = hipSuccess;
     const size_t smem = sizeof(Smem);
@@ -937,7 +937,8 @@ int run(Params &p, hipStream_t s, bool fixed = false) {
             ws = (char *)static_scratch();
             if (!ws) return 0;
         } else {
-            ws = (char *)workspace(s, acc_b + ml_b);
+            // (asked for: as many splits as any call of up to this many keys has)
+            ws = (char *)workspace(s, (acc_b + ml_b) / p.n_splits * most_splits);
             if (!ws) return 0;                      // workspace() has recorded why
         }
         p.part_acc = (uint32_t *)ws;
@@ -996,7 +997,8 @@ int launch_mla_decode(const uint8_t *rows, const float *scales, int64_t row_bstr
     per = ((per + TK - 1) / TK) * TK;
     p.keys_per_split = per;
     p.n_splits = (int)((n_list + per - 1) / per);
-    return run(p, s, fixed_scratch);
+    const int64_t tiles = (n_list + TK - 1) / TK;
+    return run(p, (int)(tiles < want ? tiles : want), s, fixed_scratch);
 }
 
 }  // namespace cwick

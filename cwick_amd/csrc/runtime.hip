@@ -175,6 +175,17 @@ uint32_t *ticket_counters(hipStream_t s) {
     return (uint32_t *)p;
 }
 
+void *workspace_if_free(hipStream_t s, size_t bytes) {
+    void *p = workspace(s, bytes, WS_MAIN);
+    if (!p) clear_error();
+    return p;
+}
+uint32_t *ticket_counters_if_free(hipStream_t s) {
+    uint32_t *p = ticket_counters(s);
+    if (!p) clear_error();
+    return p;
+}
+
 // forget (and free) what the library keeps for a stream that is about to be destroyed
 static void drop_workspace(hipStream_t s) {
     std::lock_guard<std::mutex> lk(g_mu);

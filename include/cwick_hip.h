@@ -252,19 +252,26 @@ int cwick_hip_dsa_decode(cwick_hip_ikeys *ik, cwick_hip_latent *lat, int slot0, 
  * old one until cwick_hip_stream_release() or cwick_hip_shutdown(): kernels
  * already enqueued and HIP graphs captured earlier stay valid, and no *_dev
  * call ever waits for the stream or frees memory.  While the stream is being
- * captured into a graph a call that would have to allocate declines instead
- * (the capture stays intact): run each shape once before capturing, or size
- * the workspace up front with cwick_hip_reserve_dev().  The split-K partials and the
- * ticket counters of cwick_hip_gqa_prefill_dev belong to the stream: two calls
+ * captured into a graph nothing is allocated.  The prefills then run without the
+ * slices that a mid-size chunk's keys are otherwise cut into (same results up to
+ * rounding, slower: 8 queries of 128 heads behind 20000 rows 450 us instead of
+ * 54), and a short GQA decode merges its splits in a second launch.  Every other
+ * call that would have to allocate declines (the capture stays intact).  So run
+ * each call once before capturing it, or size the workspace up front with
+ * cwick_hip_reserve_dev().  A decode asks for what any shorter one needs as well;
+ * a prefill may take more than a longer one, which fills the chip uncut: at most
+ * 256 MiB for the GQA prefill (64 for 517 positions behind 7083) and 132 for the
+ * MLA chunk (15 for 8 queries of 128 heads behind 20000 rows).  The split-K partials and the
+ * ticket counters of the GQA prefill and of GQA decodes of up to 16 splits belong to the stream: two calls
  * that use one stream's workspace at the same time (a graph replayed on another stream
  * while eager calls run on the capture stream) race. */
 
 /* No counterpart in the reference (its GPU hooks allocate on demand,
  * src/metal.c:306-319): sizes the workspace of `stream` to at least `bytes`,
- * together with the small fixed-size state the select and prefill kernels keep
- * per stream, so that later *_dev calls whose scratch fits allocate nothing.
+ * together with the small fixed-size state the select, prefill and decode kernels
+ * keep per stream, so that later *_dev calls whose scratch fits allocate nothing.
  * cwick_hip_workspace_bytes_dev() reports what the stream holds now: run the
- * largest shapes once and reserve that figure in the next process. */
+ * shapes in use once and reserve that figure in the next process. */
 int cwick_hip_reserve_dev(void *stream, int64_t bytes);
 int64_t cwick_hip_workspace_bytes_dev(void *stream);
 /* Waits for `stream`, then frees everything the library keeps for it
