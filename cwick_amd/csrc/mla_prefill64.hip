@@ -10,7 +10,7 @@
 //   takes four consecutive ones (a group): 64 heads of one query, or, with fewer heads, up to four
 //   queries that share the tiles and differ in at most three keys (SPAN).  512 queries of 16 heads
 //   over 5.5K rows: 227 us with one query per workgroup, 101 so.  Where the groups do not fill the
-//   chip a group's keys are cut into slices (plan_slices) whose fp32 partials mla_merge_frag32_kernel
+//   chip a group's keys are cut into slices (mla_plan.hpp) whose fp32 partials mla_merge_frag32_kernel
 //   combines: 8 queries of 128 heads over 20K rows 453 -> 55 us, 52 over 13.5K 313 -> 170.
 //
 //   workgroup = 8 waves (two per SIMD, 256 registers each), 64 rows x all keys of the group,
@@ -44,6 +44,7 @@
 //   Every K fragment is read from LDS by all four scoring waves (160 KB per tile); a timing build
 //   that read half of them ran 11 % faster (3 % since the scales are registers).
 #include "common.hpp"
+#include "mla_plan.hpp"
 
 #include <mutex>
 
@@ -730,51 +731,6 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
     }
 }
 
-// How many of the chunk's `groups` stay whole (the last ones, which have the most keys) and into how
-// many slices the others are cut.  One workgroup runs per compute unit, so whole groups beyond the last
-// full round leave units idle; cut, they fill it.  In steps of one key tile (1.45 us) a workgroup costs
-// its tiles and five more (Q, the first tiles' way into LDS, the output; three and two for smaller
-// groups); the merge costs three and a hundredth per slice, the partials one for every 256 row blocks
-// (32 KB each, written and read); and when every compute unit is busy the clock drops by a sixth, so a
-// round that is not full is cheaper than its share.  Fitted to a sweep of group sizes and slice counts
-// over 25 shapes (1 to 512 queries of 16 to 128 heads behind 200 to 28000 rows): what it picks is 0.7 %
-// slower than the best of the sweep on the mean, 7 % at the worst.  333 queries of 64 heads over 1624
-// rows 86 us whole, 80 with the last 77 groups in three slices; 180 groups of 2090 rows 58 us whole, 81
-// in two slices; 20 queries of 64 heads over 320 rows 13.8 us in groups of one row block, 21 in five
-// slices of groups of two.
-struct WidePlan {
-    uint32_t whole, slices;
-    double time;
-};
-WidePlan plan_slices(int64_t groups, int gsz, int64_t tiles_first, int64_t tiles_last) {
-    const int64_t cus = num_cus();
-    const double over = gsz == 4 ? 5.0 : gsz == 2 ? 3.0 : 2.0;
-    WidePlan best{(uint32_t)groups, 1, 0.0};
-    if (groups > 16 * cus) return best;              // many rounds: what the last one leaves idle is nothing
-    auto tiles_at = [&](int64_t i) { return tiles_first + (tiles_last - tiles_first) * i / (groups > 1 ? groups - 1 : 1); };
-    auto rounds = [&](int64_t wgs, int64_t tiles) {  // wgs workgroups of as many tiles
-        const double full = (double)(wgs / cus) * 1.2, last = 1.2 * (double)(wgs % cus) / (double)cus;
-        return (full + (wgs % cus == 0 ? 0.0 : last < 1.0 ? 1.0 : last)) * ((double)tiles + over);
-    };
-    auto whole_time = [&](int64_t whole) {           // whole groups from the last one down
-        double t = 0.0;
-        for (int64_t done = 0; done < whole; done += cus)
-            t += rounds(whole - done < cus ? whole - done : cus, tiles_at(groups - 1 - done));
-        return t;
-    };
-    best.time = whole_time(groups);
-    const int64_t full = groups / cus * cus;
-    for (int64_t whole = full; whole >= 0 && whole >= full - cus; whole -= cus) {
-        const int64_t rest = groups - whole, tiles = rest ? tiles_at(rest - 1) : 0;
-        const double base = whole_time(whole) + 3.0;
-        for (int64_t s = 2; s <= tiles && rest * s <= 4 * cus && rest; s++) {
-            const double t = base + 0.01 * (double)s + rounds(rest * s, (tiles + s - 1) / s) + (double)(gsz * rest * s) / (double)cus;
-            if (t < best.time) best = WidePlan{(uint32_t)whole, (uint32_t)s, t};
-        }
-    }
-    return best;
-}
-
 }  // namespace
 
 int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, int64_t n,
@@ -800,25 +756,19 @@ int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, i
     p.nhb = (uint32_t)(n_heads + 15) / 16;
     p.n_rb = (uint32_t)n * p.nhb;               // below 2^25
     p.nhb_inv = div_inverse(p.nhb);
-    WidePlan plan{};
-    int64_t groups = 0;
-    for (int gsz = NHQ; gsz >= 1; gsz /= 2) {
-        const int64_t gr = ((int64_t)p.n_rb + gsz - 1) / gsz;
-        if (gsz < NHQ && gr > num_cus()) break;
-        const WidePlan x = plan_slices(gr, gsz, (pos0 + 1 + TK - 1) / TK, (pos0 + n + TK - 1) / TK);
-        if (gsz == NHQ || x.time < plan.time) plan = x, groups = gr, p.gsz = (uint32_t)gsz;
-    }
-    if (plan.whole < groups) {
-        const size_t blocks = (size_t)(groups - plan.whole) * plan.slices * p.gsz;
+    WidePlan plan = plan_wide((int64_t)p.n_rb, (pos0 + 1 + TK - 1) / TK, (pos0 + n + TK - 1) / TK, num_cus());
+    if (plan.whole < plan.groups) {
+        const size_t blocks = (size_t)(plan.groups - plan.whole) * plan.slices * plan.gsz;
         const size_t acc_b = blocks * 16 * VDIM * sizeof(float);
         char *ws = (char *)workspace_if_free(s, acc_b + blocks * 4 * 16 * 4 * sizeof(float));
         p.part_acc = (float *)ws;
         p.part_ml = (float *)(ws + acc_b);
         // no room for partials (a stream that is being captured and has not run the shape before): uncut
-        if (!ws) p.gsz = NHQ, groups = (p.n_rb + NHQ - 1) / NHQ, plan = WidePlan{(uint32_t)groups, 1, 0.0};
+        if (!ws) plan = WidePlan{NHQ, (p.n_rb + NHQ - 1) / NHQ, (p.n_rb + NHQ - 1) / NHQ, 1, 0.0f};
     }
+    p.gsz = plan.gsz;
     p.n_whole = plan.whole;
-    p.n_rest = (uint32_t)groups - plan.whole;
+    p.n_rest = plan.groups - plan.whole;
     p.n_slices = plan.slices;
     p.slices_inv = div_inverse(plan.slices);
     {
