@@ -190,6 +190,23 @@ def test_mla_prefill_groups_and_slices(hip, orc, n, pos0, nh):
     cache.free()
 
 
+@pytest.mark.parametrize("nh", [16, 64])
+@pytest.mark.parametrize("n_keys", [191, 192, 193, 256, 257, 320])
+def test_mla_prefill_last_tile(hip, orc, n_keys, nh):
+    """Lengths around a whole tile: the tiles behind the second are copied from constant lane offsets when they
+    are whole, row by row when they are not (the rows past the end then come from a row of zeros)."""
+    n = 5
+    say("[case] mla prefill last tile", n_keys, nh)
+    c = synth.cfg4_mla_prefill(n, n_keys - n, nh, seed=91)
+    cache = hip.LatentCache(1, n_keys + 64)
+    cache.write(0, 0, c["rows"], c["scales"])
+    cache.write(0, n_keys, np.full((64, synth.KDIM), 0x7F, np.uint8), np.full((64, synth.NBLK), np.nan, np.float32))
+    got = hip.mla_prefill_chunk(cache, 0, n_keys - n, c["q"], c["scale"])
+    ref = orc.mla_prefill_chunk(c["q"], c["rows"], c["scales"], n_keys - n, c["scale"], nthreads=0)
+    assert_close(got, ref, "mla prefill, last tile", strict=False)
+    cache.free()
+
+
 @pytest.mark.parametrize("n,pos0,nh", [(8, 20000, 128), (1, 5000, 16), (5, 3000, 24), (300, 700, 64)])
 def test_mla_prefill_slices_keep_their_sums(hip, n, pos0, nh):
     """The keys of a group in slices: what the slices hand to the merge has all its bits.  A query of zeros
