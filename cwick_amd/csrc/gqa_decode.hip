@@ -51,8 +51,9 @@ struct GqaDecTile {
 template <int HD, int GROUP>
 constexpr int GQA_DEC_QUADS = GROUP <= 4 ? 1 : GROUP == 8 && HD == 128 ? 2 : 0;   // (8 x 256: too many accumulators)
 
+// (Two workgroups per compute unit is what the launcher makes at most; where three fit the registers, they do.)
 template <int HD, int GROUP, bool LIST>
-__global__ void __launch_bounds__(GQA_DEC_THREADS, HD == 256 ? 2 : 3)
+__global__ void __launch_bounds__(GQA_DEC_THREADS, HD == 256 || (LIST && GROUP == 8) ? 2 : 3)
 gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
                         const uint16_t *__restrict__ Q, int64_t n_keys, int n_kv_heads,
                         const int32_t *__restrict__ sel, int64_t n_rows,
@@ -76,47 +77,60 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
     const uint16_t *Vg = V + (LIST ? 0 : k_begin * row_stride) + (size_t)g * HD + l16 * 8;
     const int32_t *list = LIST ? sel + k_begin : nullptr;
 
-    // list entries of a tile: of key l16 (whose K row this lane reads) and of keys 4 lg .. +4
-    struct Entries {
-        int32_t k, v[4];
-    };
+    constexpr int STRIDE = NW * GQA_DEC_TILE;
+    int t = wave * GQA_DEC_TILE;
+    // List entries, those of four of the wave's tiles in one register: lane 16 j + i has key i of the j-th.
+    // A tile takes what it needs (key l16, whose K row this lane reads, and keys 4 lg .. +4 of the V rows)
+    // from other lanes when it is requested, and what outlives the request is a bit for each of the four.
+    // (Five entries per tile, in registers beside two tiles and waited for one by one: of eight heads x 128
+    // and of every group x 256 the loop spilled.  16 blocks of 256 on 8 kv heads x 128, eight query heads
+    // each: 10.5 us, 7.2 so; 16 of 128 on 4 x 256, sixteen heads each: 8.4, 7.5.)
+    const uint32_t rows_end = (uint32_t)(n_rows < ((int64_t)1 << 31) ? n_rows : (int64_t)1 << 31);
+    int32_t names = 0, names_next = 0;
+    int j = 4;                                          // tiles of `names` that have been requested
     auto entries = [&](int t) {
-        Entries e;
-        const int i = t + l16;
-        e.k = list[i < count ? i : count - 1];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int j = t + 4 * lg + r;
-            e.v[r] = list[j < count ? j : count - 1];
-        }
-        return e;
+        const int i = t + STRIDE * lg + l16;
+        return list[i < count ? i : count - 1];
     };
-    // keys past the slice and list entries that name no row are read from a row that exists and
-    // carry no weight
-    auto load = [&](GqaDecTile<HD> &x, int t, const Entries &e) {
-        uint32_t row = (uint32_t)(t + l16 < count ? t + l16 : count - 1);
-        if (LIST) row = e.k >= 0 && e.k < n_rows ? (uint32_t)e.k : 0u;
-        const uint16_t *kp = Kg + (uint64_t)row * row_stride;
+    // Requests a tile and returns which of this lane's keys 4 lg .. +4 carry no weight: those past the slice
+    // and list entries that name no row, which are read from a row that exists.
+    auto load = [&](GqaDecTile<HD> &x, int t) {
+        uint32_t k_row, v_row[4], dead = 0;
+        if (LIST) {
+            if (j == 4) {
+                j = 0;
+                names = t + STRIDE * lg + l16 < count && (uint32_t)names_next < rows_end ? names_next : -1;
+                if (t + 4 * STRIDE < count) names_next = entries(t + 4 * STRIDE);
+            }
+            const int32_t k = __builtin_amdgcn_ds_bpermute(4 * (16 * j + l16), names);
+            k_row = k < 0 ? 0u : (uint32_t)k;
 #pragma unroll
-        for (int j = 0; j < NK; j++) x.k[j] = *(const u32x4 *)(kp + 32 * j);
+            for (int r = 0; r < 4; r++) {
+                const int32_t v = __builtin_amdgcn_ds_bpermute(4 * (16 * j + 4 * lg + r), names);
+                v_row[r] = v < 0 ? 0u : (uint32_t)v;
+                if (v < 0) dead |= 1u << r;
+            }
+            j++;
+        } else {
+            k_row = (uint32_t)(t + l16 < count ? t + l16 : count - 1);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int i = t + 4 * lg + r;
+                v_row[r] = (uint32_t)(i < count ? i : count - 1);
+                if (i >= count) dead |= 1u << r;
+            }
+        }
+        const uint16_t *kp = Kg + (uint64_t)k_row * row_stride;
+#pragma unroll
+        for (int i = 0; i < NK; i++) x.k[i] = *(const u32x4 *)(kp + 32 * i);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int i = t + 4 * lg + r;
-            uint32_t vrow = (uint32_t)(i < count ? i : count - 1);
-            if (LIST) vrow = e.v[r] >= 0 && e.v[r] < n_rows ? (uint32_t)e.v[r] : 0u;
-            const uint16_t *vp = Vg + (uint64_t)vrow * row_stride;
+            const uint16_t *vp = Vg + (uint64_t)v_row[r] * row_stride;
 #pragma unroll
             for (int h = 0; h < NV; h++) x.v[r][h] = *(const u32x4 *)(vp + 128 * h);
         }
+        return dead;
     };
-    auto dead_keys = [&](int t, const Entries &e) {
-        uint32_t d = 0;
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (t + 4 * lg + r >= count || (LIST && (e.v[r] < 0 || e.v[r] >= n_rows))) d |= 1u << r;
-        return d;
-    };
-
     // this lane's part of the queries: head `col`, dims 32j + 8 lg .. +8
     const int col = QUADS ? l16 % GROUP : l16;
     bf16x8 q[NK];
@@ -192,27 +206,17 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
         }
     };
 
-    constexpr int STRIDE = NW * GQA_DEC_TILE;
-    int t = wave * GQA_DEC_TILE;
     if (t < count) {
         GqaDecTile<HD> a, b;
-        Entries ea = {}, eb = {};
-        if (LIST) {
-            ea = entries(t);
-            eb = entries(t + STRIDE);
-        }
-        load(a, t, ea);
+        if (LIST) names_next = entries(t);
+        uint32_t dead_a = load(a, t), dead_b = 0;
         for (;;) {
-            uint32_t dead = dead_keys(t, ea);
-            if (LIST) ea = entries(t + 2 * STRIDE);
-            if (t + STRIDE < count) load(b, t + STRIDE, eb);
-            step(a, dead);
+            if (t + STRIDE < count) dead_b = load(b, t + STRIDE);
+            step(a, dead_a);
             t += STRIDE;
             if (t >= count) break;
-            dead = dead_keys(t, eb);
-            if (LIST) eb = entries(t + 2 * STRIDE);
-            if (t + STRIDE < count) load(a, t + STRIDE, ea);
-            step(b, dead);
+            if (t + STRIDE < count) dead_a = load(a, t + STRIDE);
+            step(b, dead_b);
             t += STRIDE;
             if (t >= count) break;
         }

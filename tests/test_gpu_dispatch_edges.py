@@ -171,6 +171,33 @@ def test_gqa_decode_late_maximum_and_dead_lists(hip, orc, nh, nkv, hd):
     cache.free()
 
 
+@pytest.mark.parametrize("nh,nkv,hd,n_list", [
+    (64, 8, 128, 1), (64, 8, 128, 17), (64, 8, 128, 63), (32, 4, 256, 65), (16, 16, 256, 191),    # one workgroup per kv head
+    (64, 64, 128, 1089),     # five tiles a wave: one more than the four whose entries it holds at once
+    (64, 64, 128, 2049),     # nine
+    (128, 64, 128, 3333), (64, 4, 128, 3000),
+])
+def test_gqa_decode_list_lengths(hip, orc, nh, nkv, hd, n_list):
+    """Lists that end inside a tile, a workgroup's step and the four tiles whose entries a wave holds; a fifth of the
+    entries name no row, on either side of the range."""
+    say("[case] gqa decode, list lengths", nh, nkv, hd, n_list)
+    n = 700
+    c = synth.cfg1_gqa_decode(n, nh, nkv, hd, seed=92)
+    g = synth.rng(93)
+    sel = g.integers(0, n, n_list).astype(np.int32)
+    bad = g.permutation(n_list)[:n_list // 5]
+    sel[bad] = np.where(bad % 2 == 0, -1 - bad, n + bad)
+    sel[:n_list:97] = g.integers(0, n, len(sel[:n_list:97]))
+    live = sel[(sel >= 0) & (sel < n)]
+    cache = hip.KVCache(n, nkv, hd)
+    cache.write(0, c["k"], c["v"])
+    got = hip.gqa_decode_sel(cache, sel, c["q"], c["scale"])
+    ref = orc.gqa_decode(c["q"], c["k"][live], c["v"][live], c["scale"], nthreads=0)
+    # fp32 sums of exact products over up to 3333 entries, as in the decode without a list
+    assert np.abs(got - ref).max() < 2e-5 * np.abs(ref).max()
+    cache.free()
+
+
 @pytest.mark.parametrize("n,pos0,nh", [
     (1, 5000, 16),           # a quarter of a group, its keys in slices
     (6, 189, 16),            # groups of four queries that end on either side of a tile, nothing to slice

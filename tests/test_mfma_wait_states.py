@@ -87,6 +87,21 @@ def test_no_valu_write_right_before_an_mfma_reads_it(src):
     assert not early, "MFMA result read before the matrix pipe has written it: %r" % early[:3]
 
 
+def test_decode_kernels_keep_their_tiles_in_registers():
+    """The decode requests a tile while it works on the one before.  Where the two tiles and what belongs to them do
+    not fit the registers, the compiler parks the requested one in scratch memory and waits for it there, and
+    with that the request ahead is gone.  No variant of the kernel may have scratch memory."""
+    with tempfile.TemporaryDirectory() as tmp:
+        out = os.path.join(tmp, "k.s")
+        cmd = [B._hipcc()] + B.COMMON + ["-w", "-S", "--cuda-device-only", os.path.join(B.CSRC, "gqa_decode.hip"), "-o", out]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:]
+        text = open(out).read()
+    seen = re.findall(r"\.name:\s+(\S*gqa_decode_split_kernel\S*)\n\s+\.private_segment_fixed_size:\s+(\d+)", text)
+    assert len(seen) == 20, "ten shapes, with a list and without: %d" % len(seen)
+    assert not [k for k in seen if int(k[1])], [k for k in seen if int(k[1])]
+
+
 LDS_DMA_SOURCES = ["mla_roles.hip", "mla_prefill64.hip", "gqa_prefill.hip"]
 
 
