@@ -2,8 +2,8 @@
 // libcwick_hip.so.  Kernels live in the other .hip files; this file only
 // validates arguments, moves host operands and enqueues.
 #include "common.hpp"
+#include "host_flags.hpp"
 
-#include <atomic>
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
@@ -213,7 +213,6 @@ constexpr size_t PIN_PIECE = 64 << 10, PIN_DATA = PIN_PIECE - HOST_FLAGS_MAX * s
 constexpr size_t PIN_SLAB = 1 << 20, PIN_SLABS = 64;
 static std::mutex g_pin_mu;
 static std::vector<void *> g_pin_slabs, g_pin_free;
-static std::atomic<uint32_t> g_pin_epoch{0};      // never the same twice: a piece's old flags mean nothing to its next call
 
 static char *pin_take() {
     std::lock_guard<std::mutex> lk(g_pin_mu);
@@ -224,12 +223,12 @@ static char *pin_take() {
             (void)hipGetLastError();
             return nullptr;
         }
-        memset(p, 0, PIN_SLAB);
         g_pin_slabs.push_back(p);
         for (size_t o = 0; o < PIN_SLAB; o += PIN_PIECE) g_pin_free.push_back((char *)p + o);
     }
     char *p = (char *)g_pin_free.back();
     g_pin_free.pop_back();
+    memset(p + PIN_DATA, 0, HOST_FLAGS_MAX * sizeof(uint32_t));    // the last context's numbers
     return p;
 }
 static void pin_give(void *p) {
@@ -252,6 +251,7 @@ struct HostCtx {
     hipStream_t stream = nullptr;
     Scratch stage;
     char *pin = nullptr;
+    FlagNumbers numbers;
     bool pin_asked = false;
     // the context's piece of pinned memory, if a call of `bytes` fits it
     char *pinned(size_t bytes) {
@@ -259,7 +259,10 @@ struct HostCtx {
         if (!pin_asked) pin = pin_take(), pin_asked = true;
         return pin;
     }
-    HostFlags flags() { return HostFlags{(uint32_t *)(pin + PIN_DATA), ++g_pin_epoch, 0}; }
+    HostFlags flags() {
+        uint32_t *f = (uint32_t *)(pin + PIN_DATA);
+        return HostFlags{f, numbers.next(f, HOST_FLAGS_MAX), 0};
+    }
     // every flag is there; a call that takes long stops watching and waits for the stream
     bool watch(const HostFlags &f) {
         const auto start = std::chrono::steady_clock::now();
@@ -287,6 +290,7 @@ struct HostCtx {
         }
         if (pin) pin_give(pin);
         pin = nullptr;
+        numbers = FlagNumbers();
         pin_asked = false;
         stage.free_all();
     }

@@ -123,3 +123,26 @@ int main() {
     return slowest < 5.0 ? 0 : 1;
 }""")
     print(out)
+
+
+def test_flag_numbers_never_meet_an_old_flag(tmp_path):
+    """Around the end of 32 bits: a call's number is never 0 (a flag never written) nor what any flag still holds,
+    whether the calls before wrote all of their flags, some, or none."""
+    run_cpp(tmp_path, "host_flags.hpp", r"""
+int main() {
+    for (uint32_t start : {0u, 0xFFFFFFF0u, 0xFFFFFFFEu, 0xFFFFFFFFu}) {
+        uint32_t flags[8] = {0};
+        FlagNumbers numbers;
+        numbers.last = start;
+        for (int i = 0; i < 8 && start; i++) flags[i] = i < 4 ? start : i - 3;     // old calls, and long ago the first ones
+        for (int call = 0; call < 64; call++) {
+            const uint32_t e = numbers.next(flags, 8);
+            if (e == 0u) { printf("start %u call %d: number 0\n", start, call); return 1; }
+            // (numbers of long ago: only once they run again)
+            for (int i = 0; i < 8; i++)
+                if (flags[i] == e) { printf("start %u call %d: flag %d holds %u\n", start, call, i, e); return 1; }
+            for (int i = 0; i < call % 9; i++) flags[i] = e;
+        }
+    }
+    return 0;
+}""")
