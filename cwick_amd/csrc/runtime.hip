@@ -4,7 +4,6 @@
 #include "common.hpp"
 #include "host_flags.hpp"
 
-#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -263,19 +262,9 @@ struct HostCtx {
         uint32_t *f = (uint32_t *)(pin + PIN_DATA);
         return HostFlags{f, numbers.next(f, HOST_FLAGS_MAX), 0};
     }
-    // every flag is there; a call that takes long stops watching and waits for the stream
+    // every flag is there
     bool watch(const HostFlags &f) {
-        const auto start = std::chrono::steady_clock::now();
-        for (int i = 0, spins = 0; i < f.count;) {
-            if (__atomic_load_n(f.flags + i, __ATOMIC_ACQUIRE) == f.epoch) {
-                i++;
-                continue;
-            }
-            __builtin_ia32_pause();
-            if ((++spins & 1023) == 0 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(5))
-                return hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize(handle)");
-        }
-        return true;
+        return flags_arrive(f.flags, f.count, f.epoch) || hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize(handle)");
     }
     bool init() {
         return hip_ok(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate(handle)");

@@ -146,3 +146,24 @@ int main() {
     }
     return 0;
 }""")
+
+
+def test_watching_for_flags_ends(tmp_path):
+    """Flags that arrive while they are watched are seen; where one does not arrive, the watch ends at its limit of
+    half a millisecond (the best of five in less than two, on a loaded machine): no call keeps a core for longer."""
+    run_cpp(tmp_path, "host_flags.hpp", r"""
+int main() {
+    using namespace std::chrono;
+    uint32_t flags[4] = {7, 7, 7, 7};
+    if (!flags_arrive(flags, 4, 7) || !flags_arrive(flags, 0, 9)) return 1;
+    flags[3] = 6;
+    double best = 1e9;
+    for (int rep = 0; rep < 5; rep++) {
+        const auto t0 = steady_clock::now();
+        if (flags_arrive(flags, 4, 7)) return 2;
+        const double us = duration<double, std::micro>(steady_clock::now() - t0).count();
+        if (us < best) best = us;
+    }
+    printf("%.0f us\n", best);
+    return best >= 500.0 && best < 2000.0 ? 0 : 3;
+}""")
