@@ -7,22 +7,17 @@
 // (-0.0 folded into +0.0, NaN below everything), so the selection is integer
 // work and bit-exact by construction:
 //
-//   1. four 8-bit histogram passes, most significant digit first, find the key
-//      T of the k-th best element and r = how many elements equal to T belong
-//      to the selection;
+//   1. histogram passes, most significant digit first, find the key T of the k-th best
+//      element and r = how many elements equal to T belong to the selection;
 //   2. one ordered pass emits every index with key > T and the first r indices
-//      with key == T, in ascending index order, through a block-wide scan.
+//      with key == T, in ascending index order.
 //
-// Rows of 32 K to 128 K scores are split over many
+// Rows of up to 32 K scores take one workgroup of 1024 threads that reads them once, up to 32
+// consecutive keys per thread in registers, with digits of twelve, twelve and eight bits
+// (topk_radix_reg_row, topk_row.hpp).  Rows of 32 K to 128 K are split over many
 // workgroups that meet at kernel boundaries: four digit-histogram launches and
-// one ordered emit (see topk_mw_hist_kernel below).  Other rows take one
-// workgroup of 1024 threads.  Up to 65536 scores
-// are read once: every thread keeps its 64 consecutive keys in
-// registers for all five passes, the first histogram pass counts into one of 32
-// lane-indexed copies (scores cluster in a few exponent buckets, and same-address
-// LDS atomics serialise), and the ordered emit places elements with ballots
-// inside a wave and one pass over the wave totals.  Longer rows take the streaming kernel,
-// which reads the row five times from L2.  Rows past min(k, n) are filled with -1.
+// one ordered emit (topk_mw_hist_kernel below).  Longer rows take the streaming kernel, one
+// workgroup that reads the row five times from L2.  Entries past min(k, n) are filled with -1.
 #include "common.hpp"
 #include "topk_row.hpp"
 
@@ -645,8 +640,6 @@ int launch_topk(const float *scores, int batch, int64_t n, int64_t k, int32_t *o
             topk_radix_reg_kernel<24><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
         else if (n <= (int64_t)TOPK_THREADS * 32)
             topk_radix_reg_kernel<32><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else if (n <= (int64_t)TOPK_THREADS * TOPK_EPT)
-            topk_radix_reg_kernel<TOPK_EPT><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
         else
             topk_radix_kernel<<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
     }

@@ -127,12 +127,10 @@ __device__ __forceinline__ void topk_radix_row(const float *__restrict__ sc, int
     }
 }
 
-// ---- rows that fit the register file: n <= TOPK_THREADS * TOPK_EPT ----
+// ---- rows that fit the register file: n <= TOPK_THREADS * EPT ----
 // Wave w owns the consecutive elements [w * 64 * ept, (w + 1) * 64 * ept); inside it lane l
 // holds elements base + 64 j + l, so the loads are coalesced and index order is (j, lane):
 // positions inside a wave come from ballots, positions of the waves from one block scan.
-constexpr int TOPK_EPT = 64;                   // keys per thread at most; shorter rows take a kernel unrolled for fewer
-
 //
 // The threshold comes from digits of twelve, twelve and eight bits: a pass costs its barriers more than
 // its work (four passes of eight bits: 12.6 us for 512 of 9001 scores, these 9.0), and 4096 buckets spread
