@@ -13,8 +13,9 @@
  *   - cwick_hip_last_error() says why the last call on this thread declined.
  *   - called from the request thread, one generation at a time
  *     (src/attention.c:353-354); calls on one handle must not overlap.  Every
- *     cache handle owns a HIP stream and a staging buffer for the operands of
- *     its host-pointer calls, so calls on different handles may run on different
+ *     cache handle owns a HIP stream, a staging buffer and, for calls of up to
+ *     60 KB, a piece of pinned memory for the operands of its host-pointer
+ *     calls, so calls on different handles may run on different
  *     threads (the per-slot model of src/metal.c:306-319).  The two host-pointer
  *     calls that take no handle (cwick_hip_topk, cwick_hip_e4m3_table) take
  *     turns under a lock.  The *_dev calls use the caller's stream and a
@@ -533,14 +534,14 @@ int cwick_hip_ikeys_read_f32(cwick_hip_ikeys *c, int slot, int64_t pos0, int64_t
  * sections since the last reset.  Off by default (no events are recorded). */
 enum {
     CWICK_HIP_PROF_GQA_DECODE = 0,      /* gqa_decode_split_kernel */
-    CWICK_HIP_PROF_GQA_DECODE_MERGE,    /* splitk_merge_wide_kernel<256|128> after it (not for lists of up to 192 keys) */
-    CWICK_HIP_PROF_GQA_PREFILL,         /* gqa_prefill_kernel, or gqa_prefill_split_kernel without the merge after it */
-    CWICK_HIP_PROF_MLA,                 /* mla_roles_kernel (decode, sparse, prefill of at most 32 heads) */
+    CWICK_HIP_PROF_GQA_DECODE_MERGE,    /* splitk_merge_wide_kernel<256|128> after it (more than 16 splits: up to 16 are merged by gqa_decode_split_kernel itself) */
+    CWICK_HIP_PROF_GQA_PREFILL,         /* gqa_prefill_kernel, or gqa_prefill_split_kernel without gqa_prefill_merge_kernel after it */
+    CWICK_HIP_PROF_MLA,                 /* mla_roles_kernel (decode, sparse) */
     CWICK_HIP_PROF_MLA_MERGE,           /* mla_merge_frag16_kernel after it; mla_merge_frag32_kernel after a chunk in slices */
-    CWICK_HIP_PROF_INDEXER,             /* indexer_scores_kernel, or in a fused select indexer_approx_kernel + topk_mw_hist_kernel + topk_mw_classify_kernel + indexer_rescore_kernel + the exact kernel's fallback pass */
+    CWICK_HIP_PROF_INDEXER,             /* indexer_scores[_rows|_ds]_kernel, or in a fused select indexer_approx_kernel + topk_mw_classify_kernel + indexer_rescore_kernel */
     CWICK_HIP_PROF_TOPK,                /* every kernel of one top-k call: topk_mw_hist_kernel x4 + topk_mw_emit_kernel, or topk_radix[_reg]_kernel; in a fused select topk_band_finish_kernel */
-    CWICK_HIP_PROF_MLA_PREFILL,         /* mla_prefill64_kernel (chunked prefill of more than 32 heads) */
-    CWICK_HIP_PROF_MM_SELECT,           /* mm_index_scores[_long]_kernel + mm_pick_kernel; for block sizes that are not a multiple of 64 mm_blockmax_kernel and mm_expand_kernel, with the block top-k between them under CWICK_HIP_PROF_TOPK */
+    CWICK_HIP_PROF_MLA_PREFILL,         /* mla_prefill64_kernel (chunked prefill) */
+    CWICK_HIP_PROF_MM_SELECT,           /* mm_index_scores[_long|128]_kernel + mm_pick_kernel; for block sizes that are not a multiple of 64 mm_blockmax_kernel and mm_expand_kernel, with the block top-k between them under CWICK_HIP_PROF_TOPK */
     CWICK_HIP_PROF_INDEXER_APPROX,      /* indexer_approx_kernel alone (also counted inside CWICK_HIP_PROF_INDEXER) */
     CWICK_HIP_PROF_COUNT
 };
