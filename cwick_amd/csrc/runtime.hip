@@ -31,6 +31,8 @@ void clear_error() { g_err[0] = 0; }
 
 bool hip_ok(hipError_t e, const char *what) {
     if (e == hipSuccess) return true;
+    // taken from the runtime too, which would hand it to the next call's check of its launches
+    (void)hipGetLastError();
     set_error("HIP error %d (%s) in %s", (int)e, hipGetErrorString(e), what);
     return false;
 }

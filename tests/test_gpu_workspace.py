@@ -102,6 +102,24 @@ def test_capture_declines_instead_of_allocating_and_reserve_prevents_it(hip):
     assert hip.stream_release(sp) == 1
 
 
+def test_a_failed_allocation_stays_with_its_call(hip):
+    """A reservation larger than the device's memory declines; the calls behind it run, whether or not they need
+    workspace of their own."""
+    import torch
+    print("[case] workspace: a reservation of a tebibyte, then ordinary calls", flush=True)
+    c = synth.cfg1_gqa_decode(500, 16, 4, 256, seed=3207)
+    k, v, q = (torch.from_numpy(c[x].view(np.int16)).cuda() for x in "kvq")
+    out = torch.empty((16, 256), dtype=torch.float32, device="cuda")
+    s = torch.cuda.Stream()
+    for n in (100, 500):                                  # one split, then eight
+        assert hip.reserve_dev(s.cuda_stream, 1 << 40, raw=True) == 0
+        assert "hipMalloc" in hip.last_error()
+        hip.gqa_decode_dev(k, v, n, 4, 256, q, 16, c["scale"], out, s.cuda_stream)
+        s.synchronize()
+        assert torch.isfinite(out).all() and hip.last_error() == ""
+    assert hip.stream_release(s.cuda_stream) == 1
+
+
 def _captured(torch, stream, call, out):
     """`call` as the only work of a graph captured on `stream`; the result after two replays."""
     g = torch.cuda.CUDAGraph()
