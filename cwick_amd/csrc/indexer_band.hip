@@ -68,7 +68,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     __shared__ __attribute__((aligned(16))) uint16_t q_sh[64 * IB_QROW];
     __shared__ float w_sh[64];
     __shared__ float bmax_sh[IB_THREADS / 64];
-    __shared__ uint32_t cmax_sh[2], kexp_sh;
+    __shared__ uint32_t cmax_sh[2];
     const int b = blockIdx.y, wg = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint16_t *qb = q + (size_t)b * ih * IB_HD;
@@ -104,7 +104,9 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     // tid % 16) holds dims 8 part .. +7 of heads group + 16 j, adds up its four heads and leaves
     // the eight sums in LDS; after the barrier thread i < 128 adds the sixteen groups of dim i.
     bf16x8 qa[2][8];
-    uint32_t ks_bits = 0u;              // 64 key scales from all over the row, the same ones in every workgroup
+    // Key scales from four places of the row, the same ones in every workgroup.  (From 64 places, a cache line
+    // each in front of the first keys, the kernel takes 0.3 us longer.)
+    uint32_t ks_bits;
     {
         // (the weights first: a load that is waited for drags every load issued before it along)
         const float w_mine = (tid < 64 && tid < ih) ? wb[tid] : 0.0f;
@@ -123,8 +125,8 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
             stage[j] = *(const u32x4 *)(qb + (size_t)hc * IB_HD + 8 * part);
             if (head >= ih) stage[j] = (u32x4){0u, 0u, 0u, 0u};
         }
-        // (behind the queries, which the first barrier waits for)
-        if (wave == IB_WAVES - 1) ks_bits = __builtin_bit_cast(uint32_t, ksb[(int64_t)lane * n_keys >> 6]);
+        const int64_t ks_at = ((int64_t)(lane >> 4) * n_keys >> 2) + (lane & 15);
+        ks_bits = __builtin_bit_cast(uint32_t, ksb[ks_at < n_keys ? ks_at : n_keys - 1]);
         load_keys(0, raw_a, kst_a);
         load_keys(1, raw_b, kst_b);
         float cp[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -162,30 +164,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
         const uint32_t top = wave_max_u32(__builtin_bit_cast(uint32_t, c));             // (never negative)
         if (lane == 0) cmax_sh[wave] = top;
     }
-    if (wave == IB_WAVES - 1) {
-        // the exponent that a quarter of them reach; scales of 0 and 1, which keys of zeros have, do not count
-        const uint32_t e = ks_bits == 0x3F800000u ? 0u : ks_bits >> 23 & 0xFFu;
-        const int quarter = (__builtin_popcountll(__ballot(e != 0u)) + 3) / 4;
-        uint32_t upper = 0u;
-#pragma unroll
-        for (int bit = 7; bit >= 0; bit--)
-            if (__builtin_popcountll(__ballot(e >= (upper | 1u << bit))) >= quarter) upper |= 1u << bit;
-        if (lane == 0) kexp_sh = quarter ? upper : 127u;
-    }
     __syncthreads();
-    // The octaves that get most of the counters: a score is at most ks sum_i |e_i| c_i <= ks 448 * 128 max c,
-    // so with the scales above the largest are around 2^16 ks max c, and what threshold a selection has lies
-    // 2 to 13 octaves below that (heads that agree; signed weights that cancel).  Every workgroup of the
-    // row finds the same ones; what they are decides how many candidates there are, not which keys win.
-    uint32_t octave;
-    {
-        const uint32_t c_top = cmax_sh[0] > cmax_sh[1] ? cmax_sh[0] : cmax_sh[1];
-        int lowest = (int)(c_top >> 23 & 0xFFu) + (int)kexp_sh - 127 + 16 - ((int)BAND_OCTAVES - 1);
-        lowest = lowest < 0 ? 0 : lowest;
-        lowest = lowest > 256 - (int)BAND_OCTAVES ? 256 - (int)BAND_OCTAVES : lowest;
-        octave = (uint32_t)__builtin_amdgcn_readfirstlane(lowest);
-    }
-    if (wg == 0 && tid == 0) rows[b].octave = octave;
     // the bound row's A fragments are read from LDS step by step: lanes of row 0 from the
     // coefficients, all others from a stretch of zeros behind them
     const char __attribute__((address_space(3))) *c_lane =
@@ -197,6 +176,28 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     for (int mb = 0; mb < 2; mb++)
 #pragma unroll
         for (int i = 0; i < 16; i++) wl[mb][i] = w_sh[mb * 32 + (i >> 2) * 8 + 4 * g + (i & 3)];
+
+    // The octaves that get most of the counters: a score is at most ks sum_i |e_i| c_i <= ks 448 * 128 max c,
+    // so the largest are around 2^16 ks max c, for the ks whose exponent a quarter of the sample reaches
+    // (scales of 0 and 1, which keys of zeros have, left out), and what threshold a selection has lies
+    // 2 to 13 octaves below that (heads that agree; signed weights that cancel).  Every wave of the row
+    // finds the same ones; what they are decides how many candidates there are, not which keys win.  (Here,
+    // where the keys are still on their way: each wave for itself, so that no barrier waits for the sample.)
+    uint32_t octave;
+    {
+        const uint32_t e = ks_bits == 0x3F800000u ? 0u : ks_bits >> 23 & 0xFFu;
+        const int quarter = (__builtin_popcountll(__ballot(e != 0u)) + 3) / 4;
+        uint32_t upper = 0u;
+#pragma unroll
+        for (int bit = 7; bit >= 0; bit--)
+            if (__builtin_popcountll(__ballot(e >= (upper | 1u << bit))) >= quarter) upper |= 1u << bit;
+        const uint32_t c_top = cmax_sh[0] > cmax_sh[1] ? cmax_sh[0] : cmax_sh[1];
+        int lowest = (int)(c_top >> 23 & 0xFFu) + (int)(quarter ? upper : 127u) - 127 + 16 - ((int)BAND_OCTAVES - 1);
+        lowest = lowest < 0 ? 0 : lowest;
+        lowest = lowest > 256 - (int)BAND_OCTAVES ? 256 - (int)BAND_OCTAVES : lowest;
+        octave = (uint32_t)__builtin_amdgcn_readfirstlane(lowest);
+    }
+    if (wg == 0 && tid == 0) rows[b].octave = octave;
 
     float bmax = 0.0f;
     auto iteration = [&](int it, const u32x4 (&raw)[4], float kst) {
