@@ -844,9 +844,13 @@ gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restr
 }
 
 // Combines the slices of a block: out = sum_s 2^(m_s - M) acc_s / sum_s 2^(m_s - M) l_s.  A wave
-// takes 32 rows x 32 dims (the partials of output block db of one column block: 4 KiB per slice in
-// four coalesced loads), a workgroup four of the eight output blocks.
-template <int GROUP, int WAVES>
+// takes 32 rows x 8 dims (one KiB of the partials per slice, one load), a workgroup a 32-dim output block.
+// What it waits for is the partials' way from memory, so the loads of BATCH slices are in flight at once and
+// few rows make many waves: 16 positions behind 16000 on four kv heads (64 slices) took 46.6 us of which this
+// kernel had 17, and take 32.3 (a wave for four times the dims, four slices at a time, before).  Blocks of up
+// to eight slices are shorter with eight (2500 positions 103 us against 108): the registers of sixteen cost
+// waves.
+template <int GROUP, int WAVES, int BATCH>
 __global__ void __launch_bounds__(256)
 gqa_prefill_merge_kernel(const float *__restrict__ part, const float *__restrict__ part_ml, int64_t n,
                          int n_kv_heads, int pblocks, const PfPlan plan, float *__restrict__ out) {
@@ -854,38 +858,45 @@ gqa_prefill_merge_kernel(const float *__restrict__ part, const float *__restrict
     const int rank = blockIdx.x / n_kv_heads, kvh = blockIdx.x % n_kv_heads;
     const int n_slices = plan.first[rank + 1] - plan.first[rank];
     if (n_slices < 2) return;                           // its workgroup wrote the output
-    const int cb = blockIdx.y >> 1;                     // column block: 32 rows
+    const int cb = blockIdx.y >> 3, db = blockIdx.y & 7;        // column block: 32 rows; output block: 32 dims
     const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
-    const int db = (blockIdx.y & 1) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const size_t item0 = (size_t)plan.first[rank] * n_kv_heads + kvh, step = n_kv_heads;
     const float *ml = part_ml + item0 * (64 * WAVES * 2) + (cb * 32 + l32) * 2;
-    const float *pa = part + item0 * PF_PART<WAVES> + ((size_t)(cb * 8 + db) * 4 * 64 + lane) * 4;
-    float mx = -INFINITY;
-#pragma unroll 8
-    for (int s = 0; s < n_slices; s++) mx = fmaxf(mx, ml[s * step * (64 * WAVES * 2)]);
-    float l = 0.0f;
-    f32x4 acc[4];
+    const float *pa = part + item0 * PF_PART<WAVES> + ((size_t)((cb * 8 + db) * 4 + b4) * 64 + lane) * 4;
+    float mx = -INFINITY, l = 0.0f;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < n_slices; s0 += BATCH) {
+        f32x2 v[BATCH];
+        f32x4 a[BATCH];
+        float top = mx;
 #pragma unroll
-    for (int b = 0; b < 4; b++) acc[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-    for (int s = 0; s < n_slices; s++) {
-        const f32x2 v = *(const f32x2 *)(ml + s * step * (64 * WAVES * 2));
-        const float c = __builtin_amdgcn_exp2f(v[0] - mx);
-        l = __builtin_fmaf(v[1], c, l);
+        for (int j = 0; j < BATCH; j++) {
+            v[j] = (f32x2){-INFINITY, 0.0f};
+            a[j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            if (s0 + j < n_slices) {
+                v[j] = *(const f32x2 *)(ml + (s0 + j) * step * (64 * WAVES * 2));
+                a[j] = *(const f32x4 *)(pa + (s0 + j) * step * PF_PART<WAVES>);
+            }
+        }
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const f32x4 a = *(const f32x4 *)(pa + s * step * PF_PART<WAVES> + b * 256);
+        for (int j = 0; j < BATCH; j++) top = fmaxf(top, v[j][0]);
+        const float keep = __builtin_amdgcn_exp2f(mx - top);    // the first slices: exp2(-inf) = 0
+        mx = top;
+        l *= keep;
+        acc *= keep;
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[b][i] = __builtin_fmaf(a[i], c, acc[b][i]);
+        for (int j = 0; j < BATCH; j++) {
+            const float c = __builtin_amdgcn_exp2f(v[j][0] - mx);
+            l = __builtin_fmaf(v[j][1], c, l);
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(a[j][i], c, acc[i]);
         }
     }
     const int r = cb * 32 + l32;
     const int64_t t = (int64_t)(pblocks - 1 - rank) * P + r % P;
     if (t >= n) return;
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    float *o = out + (t * n_kv_heads * GROUP + kvh * GROUP + r / P) * PF_HD + 32 * db + 4 * g;
-#pragma unroll
-    for (int b = 0; b < 4; b++) *(f32x4 *)(o + 8 * b) = acc[b] * inv;
+    *(f32x4 *)(out + (t * n_kv_heads * GROUP + kvh * GROUP + r / P) * PF_HD + 32 * db + 8 * b4 + 4 * g) = acc * (l > 0.0f ? 1.0f / l : 0.0f);
 }
 
 // Position blocks that take the PRECISE body: those whose rows see at most this many keys.  Short
@@ -979,8 +990,9 @@ static int run_gqa_prefill_split(const uint16_t *k, const uint16_t *v, int64_t p
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (!plan.per) return 1;
-    gqa_prefill_merge_kernel<GROUP, WAVES><<<dim3((unsigned)(pblocks * n_kv_heads), 4 * WAVES), 256, 0, s>>>(
-        part, part_ml, n, n_kv_heads, pblocks, plan, out);
+    const bool many = plan.first[1] > 8;                // (no block has more slices than the last)
+    (many ? gqa_prefill_merge_kernel<GROUP, WAVES, 16> : gqa_prefill_merge_kernel<GROUP, WAVES, 8>)<<<
+        dim3((unsigned)(pblocks * n_kv_heads), 16 * WAVES), 256, 0, s>>>(part, part_ml, n, n_kv_heads, pblocks, plan, out);
     CWICK_HIP_CALL(hipGetLastError());
     return 1;
 }

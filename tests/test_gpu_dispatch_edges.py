@@ -49,6 +49,8 @@ def test_absorb_expand_edges(hip, orc, nh, batch, nope, rope, vdim):
     (300, 700, 16, 4),       # blocks on either side of the two-term weights' 1024 keys
     (130, 5000, 16, 2),      # eight heads per kv head
     (33, 0, 16, 4),          # nothing to split
+    (16, 16001, 16, 4),      # sixty slices and more: batches of sixteen in the merge, the last one short
+    (16, 1100, 16, 4),       # more than eight slices, fewer than sixteen
 ])
 def test_gqa_prefill_slices(hip, orc, n, pos0, nh, nkv):
     """Chunks whose position blocks do not fill the chip: the keys of a block in several slices."""
