@@ -43,17 +43,18 @@
 //   simpler two-stage schedule: scores of tile t+1, then its softmax next to
 //   the value products of tile t.
 //
-//   Problems that do not fill the chip take workgroups of one wave (64 rows, on one of a compute unit's
-//   four matrix cores): what an item costs besides its tiles goes with its rows.
+//   Problems that do not fill the chip take gqa_prefill_team_kernel: four waves on 64 rows, each on key tiles of
+//   its own.
 #include "common.hpp"
+#include "gqa_plan.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 namespace cwick {
 
-constexpr int PF_TK = 32;
 constexpr int PF_HD = 256;
-constexpr int PF_WAVES = 4;                 // waves per workgroup; small problems take one (see the launcher)
+constexpr int PF_WAVES = 4;                 // waves per workgroup
 constexpr int PF_PAIR = 1024 + 32;          // bytes between pairs of rows in LDS
 constexpr int PF_TILE = 16 * PF_PAIR;       // one K or V tile, or the 32 query rows of a column block, in LDS
 constexpr int PF_PRE = 4;                   // k-steps of fragment prefetch in the score loop
@@ -62,13 +63,12 @@ typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef __attribute__((address_space(3))) void pf_lds_void;
 
-template <int WAVES>
 struct PfSmem {
     unsigned char k[2][PF_TILE];
     unsigned char v[3][PF_TILE];                // the pipelined body keeps three V tiles, the other two
     // the query rows of column block B: the register file holds 256 accumulators + 64 Q registers +
     // the working set, not 128 Q registers
-    unsigned char q[WAVES][PF_TILE];
+    unsigned char q[PF_WAVES][PF_TILE];
 };
 
 // A tile in LDS is sixteen pairs of rows, m and m + 16, each row whole (512 bytes), 32 bytes between the
@@ -93,15 +93,15 @@ __device__ __forceinline__ uint32_t pf_swap(uint32_t row) { return (row >> 3) & 
 struct PfSlice {
     float *part, *part_ml;                      // part is null for a block that is one slice
 };
-template <int GROUP, int WAVES, bool PRECISE, bool SPLIT>
+template <int GROUP, bool PRECISE, bool SPLIT>
 __device__ __forceinline__ void
 gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
                  const uint16_t *__restrict__ Q, int64_t pos0, int64_t n, int64_t wg_keys, int n_kv_heads,
                  float scale_log2e, float *__restrict__ out, int64_t pblk, int kvh,
                  const PfSlice *slice = nullptr) {
-    constexpr int P = 64 * WAVES / GROUP;   // positions per workgroup
-    constexpr int NI = 16 / WAVES;          // copies of a tile that each wave issues
-    PfSmem<WAVES> &sm = *reinterpret_cast<PfSmem<WAVES> *>(smem_raw);
+    constexpr int P = 64 * PF_WAVES / GROUP;    // positions per workgroup
+    constexpr int NI = 16 / PF_WAVES;       // copies of a tile that each wave issues
+    PfSmem &sm = *reinterpret_cast<PfSmem *>(smem_raw);
 
     // The thread's number is opaque to the compiler here, and the copy's key below: what it knows of
     // their ranges and of the loop over items around this body it turns into per-lane constants that
@@ -144,7 +144,7 @@ gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const 
     };
     auto copy_one = [&](const CopySrc &src, uint32_t lds_tile, int i) {
         const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_tile + (uint32_t)((NI * wave + i) * PF_PAIR));
-        uint32_t off = (NI == 16 && i >= 8 ? cp_off ^ 16 : cp_off) + (uint32_t)i * row_bytes;
+        uint32_t off = cp_off + (uint32_t)i * row_bytes;
         off = off < src.last ? off : src.last;
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src.base), "s"(m0) : "memory");
     };
@@ -719,11 +719,9 @@ __device__ __forceinline__ void pf_tickets_done(uint32_t *__restrict__ tickets) 
     }
 }
 
-// keys a position block attends to: 0 .. its last position (clipped to the chunk)
 template <int GROUP, int WAVES>
 __host__ __device__ inline int64_t pf_block_keys(int64_t pos0, int64_t n, int64_t pblk) {
-    const int64_t last = (pblk + 1) * (64 * WAVES / GROUP);
-    return pos0 + (last < n ? last : n);
+    return pf_keys(pos0, n, 64 * WAVES / GROUP, pblk);
 }
 
 // One launch: position blocks below n_prec take the PRECISE body.
@@ -763,8 +761,8 @@ gqa_prefill_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ 
         }
         if (pblk < 0) pblk = pblocks - 1 - (rank - before);
         const int64_t keys = pf_block_keys<GROUP, PF_WAVES>(pos0, n, pblk);
-        if (pblk < n_prec) gqa_prefill_body<GROUP, PF_WAVES, true, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh);
-        else gqa_prefill_body<GROUP, PF_WAVES, false, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh);
+        if (pblk < n_prec) gqa_prefill_body<GROUP, true, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh);
+        else gqa_prefill_body<GROUP, false, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh);
         // nothing of the last item may still be on its way into LDS
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (threadIdx.x == 0) sh_item = gridDim.x + atomicAdd(&tickets[0], 1u);
@@ -779,27 +777,11 @@ gqa_prefill_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ 
 // workgroups, each with whole tiles, and gqa_prefill_merge_kernel combines what they leave.
 // What it costs is the partials: 256 KB written and read per slice of 256 rows, 252 slices of 34 tiles
 // for 517 positions behind 7083 on four kv heads.  That chunk took 310 us on its 36 workgroups and takes
-// 92 (with the preparation of its rows); 2048 positions at position 0 101 -> 83.  (Partials by
-// non-temporal stores: 3 us slower.)  With workgroups of one wave 17 positions behind 1706 take 26 us
-// (36 with four waves), 16 behind 16000 47 (61), 45 at position 0 12.7 (18.9).
-// A plan names the slices: block rank r (rank 0 is the last position block) has slices
-// first[r] .. first[r + 1], of `per` tiles each, the last one with the rest of the block.
-constexpr int PF_MAX_BLOCKS = 512;
-struct PfPlan {
-    int per;                                    // tiles per slice
-    uint16_t first[PF_MAX_BLOCKS + 1];
-};
+// 90 (with the preparation of its rows).  (Partials by non-temporal stores: 3 us slower.)
 template <int WAVES> constexpr size_t PF_PART = (size_t)64 * WAVES * PF_HD;     // floats of one slice's accumulators
 
-// Slices of a block of `tiles` tiles whose first `plain` need no mask: as many as `per` fit, every
-// slice beginning below the diagonal (the first tile of a slice must give every row its reference).
-__host__ __device__ inline int pf_slices(int tiles, int plain, int per) {
-    const int by_tiles = (tiles + per - 1) / per, by_plain = 1 + plain / per;
-    return by_tiles < by_plain ? by_tiles : by_plain;
-}
-
-template <int GROUP, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES, 1)
+template <int GROUP>
+__global__ void __launch_bounds__(64 * PF_WAVES, 1)
 gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
                          const uint16_t *__restrict__ Q, int64_t pos0, int64_t n, int n_kv_heads,
                          float scale_log2e, float *__restrict__ out, int64_t n_prec, int pblocks,
@@ -822,18 +804,470 @@ gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restr
         const int64_t pblk = pblocks - 1 - lo;
         const int slice = slice_no - plan.first[lo], n_slices = plan.first[lo + 1] - plan.first[lo];
         const int64_t k0 = (int64_t)slice * plan.per * PF_TK;
-        int64_t keys = pf_block_keys<GROUP, WAVES>(pos0, n, pblk) - k0;
+        int64_t keys = pf_block_keys<GROUP, PF_WAVES>(pos0, n, pblk) - k0;
         if (slice + 1 < n_slices) keys = (int64_t)plan.per * PF_TK;
         const size_t row0 = (size_t)k0 * n_kv_heads * PF_HD;
         // (read behind the body's barriers; the last item's reads are behind the draw's)
-        if (threadIdx.x == 0) sh_slice = {n_slices > 1 ? part + item * PF_PART<WAVES> : nullptr, part_ml + (size_t)item * (64 * WAVES * 2)};
+        if (threadIdx.x == 0) sh_slice = {n_slices > 1 ? part + item * PF_PART<PF_WAVES> : nullptr, part_ml + (size_t)item * (64 * PF_WAVES * 2)};
         if (pblk < n_prec)
-            gqa_prefill_body<GROUP, WAVES, true, true>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads,
+            gqa_prefill_body<GROUP, true, true>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads,
                                                 scale_log2e, out, pblk, kvh, &sh_slice);
         else
-            gqa_prefill_body<GROUP, WAVES, false, true>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads,
+            gqa_prefill_body<GROUP, false, true>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads,
                                                  scale_log2e, out, pblk, kvh, &sh_slice);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (gridDim.x >= total) break;                  // one item each: nothing to draw
+        if (threadIdx.x == 0) sh_item = gridDim.x + atomicAdd(&tickets[0], 1u);
+        __syncthreads();
+        item = __builtin_amdgcn_readfirstlane(sh_item);
+        __syncthreads();
+    }
+    if (gridDim.x < total) pf_tickets_done(tickets);
+}
+
+// ---- workgroups whose four waves share one block of 64 rows ----
+// For problems of few rows or few keys.  What 256 rows cost besides their tiles (18 us: query rows, first
+// tiles, the tiles at either end of the pipeline in sequence, 256 KB of output) and what slices of them leave
+// behind (256 KB of partials each, written and read) is most of such a problem's time.  Here a wave takes every
+// fourth key tile of the same 64 rows, copies it into its own part of LDS and works on it alone, without
+// barriers; the four meet in LDS at the end.  A tile serves 64 rows instead of 256: a step of four tiles takes
+// 1.65 us, 2.1 with every compute unit at it (2048 cycles of it matrix instructions), and what is in the way is
+// the copies.  One buffer each for K and V: K(u + 1) is on its way during the softmax and the value products of
+// tile u, V(u + 1) during the next scores.
+// 1000 positions of 16 heads 47.7 -> 31.5 us, 360: 22.9 -> 17.5, 100: 16.5 -> 11.7, 16: 10.2 -> 7.6 (the
+// launches of a call); 1000 of 8 / 8 heads 41.4 -> 24.5; 2500 of 16 105 -> 87; 29 behind 3219 29 -> 21.8 (23.4 with
+// the merge of the slices alone), 128 of 8 / 8 behind 1800 30.4 -> 22.6.  Long chunks go the other way: 517
+// behind 7083 take 115 us on 132 such workgroups, 104 in two slices each.
+struct PfTeamSmem {
+    unsigned char k[PF_WAVES][PF_TILE], v[PF_WAVES][PF_TILE];   // at the end: the accumulators that change hands
+    unsigned char q[PF_TILE];                                   // query rows 32 .. 63 (block B)
+    f32x2 ml[PF_WAVES][64];                                     // a wave's reference and weight sum of every row
+};
+
+template <int GROUP, bool PRECISE>
+__device__ __forceinline__ void
+gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
+                      const uint16_t *__restrict__ Q, int64_t pos0, int64_t n, int64_t wg_keys, int n_kv_heads,
+                      float scale_log2e, float *__restrict__ out, int64_t pblk, int kvh, float *part, float *part_ml) {
+    constexpr int P = 64 / GROUP;           // positions per workgroup
+    constexpr int NI = 16;                  // copies of a tile
+    PfTeamSmem &sm = *reinterpret_cast<PfTeamSmem *>(smem_raw);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));           // (see gqa_prefill_body)
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31;
+    const int g = lane >> 5;                // 0/1
+
+    const int64_t t0 = pblk * P;
+    const int n_heads = n_kv_heads * GROUP;
+    const int64_t q_stride = (int64_t)n_heads * PF_HD;
+    const int n_tiles = (int)((wg_keys + PF_TK - 1) / PF_TK);
+    const int my_tiles = (n_tiles - wave + PF_WAVES - 1) / PF_WAVES;        // tiles wave, wave + 4, ...
+    const int64_t first_masked_key = pos0 + t0;
+
+    const uint32_t row_bytes = (uint32_t)n_kv_heads * (PF_HD * 2);
+    uint32_t cp_off = (uint32_t)(16 * g) * row_bytes + (uint32_t)l32 * 16;
+    asm volatile("" : "+v"(cp_off));
+    const unsigned char *Kg = (const unsigned char *)(K + (size_t)kvh * PF_HD);
+    const unsigned char *Vg = (const unsigned char *)(V + (size_t)kvh * PF_HD);
+    const uint32_t lds_k = (uint32_t)(uintptr_t)(pf_lds_void *)&sm.k[wave][0];
+    const uint32_t lds_v = (uint32_t)(uintptr_t)(pf_lds_void *)&sm.v[wave][0];
+    // copy i of a tile takes rows i and i + 16 (gqa_prefill_body's copies)
+    auto issue = [&](const unsigned char *base, uint32_t lds_tile, int tile) {
+        const uint32_t key0 = (uint32_t)tile * PF_TK;
+        const uint32_t left = (uint32_t)wg_keys - 1 - key0;
+        const uint64_t first = (uint64_t)base + (uint64_t)key0 * row_bytes;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)first), hi = __builtin_amdgcn_readfirstlane((uint32_t)(first >> 32));
+        const unsigned char *src = (const unsigned char *)((uint64_t)hi << 32 | lo);
+        const uint32_t last = (left < PF_TK ? left : PF_TK - 1) * row_bytes + (PF_HD * 2 - 16);
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_tile + (uint32_t)(i * PF_PAIR));
+            uint32_t off = (i >= 8 ? cp_off ^ 16 : cp_off) + (uint32_t)i * row_bytes;
+            off = off < last ? off : last;
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src), "s"(m0) : "memory");
+        }
+    };
+
+    // Query rows, sixteen pairs of rows of either block, dealt to the waves; block A goes through the last
+    // wave's V buffer on its way into fragments.  The first tiles are requested with them.
+    {
+        const int c = wave >> 1;
+        const uint32_t lds_q = (uint32_t)(uintptr_t)(pf_lds_void *)(c ? &sm.q[0] : &sm.v[PF_WAVES - 1][0]);
+        const int64_t left = n - 1 - t0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int m = 8 * (wave & 1) + j;
+            const int r = 32 * c + m + 16 * g;
+            const uint32_t t = (uint32_t)(r % P) < left ? (uint32_t)(r % P) : (uint32_t)left;
+            const unsigned char *src = (const unsigned char *)(Q + t0 * q_stride + (size_t)kvh * GROUP * PF_HD) +
+                                       (uint64_t)t * ((uint32_t)n_heads * (PF_HD * 2)) + (r / P) * (PF_HD * 2) + ((uint32_t)l32 ^ pf_swap(m)) * 16;
+            const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_q + (uint32_t)(m * PF_PAIR));
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory");
+        }
+    }
+    const bool single = n_tiles == 1 && !part;
+    const int first_tile = single ? 0 : wave;
+    if (first_tile < n_tiles) {
+        issue(Kg, lds_k, first_tile);
+        if (wave != PF_WAVES - 1) issue(Vg, lds_v, first_tile);
+    }
+    f32x16 oacc[2][8];
+    auto clear = [&]() {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int db = 0; db < 8; db++) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) oacc[c][db][i] = 0.0f;
+                asm volatile("" : "+a"(oacc[c][db]));
+            }
+    };
+    clear();                                // (while the copies are on their way)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    PF_LDS_BARRIER();
+    bf16x8 qf[16];
+    {
+        const unsigned char *a = &sm.v[PF_WAVES - 1][pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) qf[ks] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(a + 32 * ks));
+    }
+    PF_LDS_BARRIER();
+    if (wave == PF_WAVES - 1 && first_tile < n_tiles) issue(Vg, lds_v, first_tile);
+
+    const unsigned char *kfrag = &sm.k[wave][pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
+    const unsigned char *qfrag = &sm.q[pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
+    const int grp = lane >> 4, gi = lane & 15;
+    const int v_key0 = 4 * (grp >> 1) + (gi >> 2);
+    const int v_col = 2 * (grp & 1) + ((gi & 3) >> 1);
+    const unsigned char *vfrag[2] = {&sm.v[wave][pf_row(v_key0) + (v_col << 4) + (gi & 1) * 8],
+                                     &sm.v[wave][pf_row(v_key0 + 8) + ((v_col ^ 1) << 4) + (gi & 1) * 8]};
+    auto vread = [&](int st, int half) -> s16x4 {
+        return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vfrag[half] + (st & 7) * 64 + (st >> 3) * 512));
+    };
+
+    float m_ref[2] = {-INFINITY, -INFINITY}, l_part[2] = {0.0f, 0.0f};
+
+    auto scores = [&](f32x16 (&s)[2]) {
+        u32x4 ka[PF_PRE], qa[PF_PRE];
+#pragma unroll
+        for (int ks = 0; ks < PF_PRE; ks++) {
+            ka[ks] = *(const u32x4 *)(kfrag + 32 * ks);
+            qa[ks] = *(const u32x4 *)(qfrag + 32 * ks);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) {
+            const bf16x8 kf = __builtin_bit_cast(bf16x8, ka[ks % PF_PRE]);
+            const bf16x8 q1 = __builtin_bit_cast(bf16x8, qa[ks % PF_PRE]);
+            if (ks + PF_PRE < 16) {
+                ka[ks % PF_PRE] = *(const u32x4 *)(kfrag + 32 * (ks + PF_PRE));
+                qa[ks % PF_PRE] = *(const u32x4 *)(qfrag + 32 * (ks + PF_PRE));
+            }
+            if (ks == 0) {
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s[0]) : "v"(kf), "v"(qf[ks]));
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s[1]) : "v"(kf), "v"(q1));
+            } else {
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[0]) : "v"(kf), "v"(qf[ks]));
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[1]) : "v"(kf), "v"(q1));
+            }
+        }
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    };
+    // masks the raw scores of a tile and returns this lane's maximum in log2 units
+    auto prep = [&](int tile, int c, f32x16 &s) -> float {
+        const int64_t key0 = (int64_t)tile * PF_TK;
+        float tmax = -INFINITY;
+        if (key0 + PF_TK - 1 > first_masked_key) {
+            const int left = (int)(n - 1 - t0 < P ? n - 1 - t0 : P), tr = (32 * c + l32) % P;
+            const int lim = (int)(first_masked_key - key0) + (tr < left ? tr : left) - 4 * g;
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if ((i >> 2) * 8 + (i & 3) > lim) s[i] = -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) tmax = fmaxf(tmax, s[i]);
+        return tmax * scale_log2e;
+    };
+    auto finish = [&](int c, f32x16 &s, u32x4 (&pw)[2], u32x4 (&pl)[2]) {
+        const float m_use = m_ref[c] == -INFINITY ? 0.0f : m_ref[c];
+        float psum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], scale_log2e, -m_use));
+            if (PRECISE) psum += s[i];
+        }
+#pragma unroll
+        for (int ks2 = 0; ks2 < 2; ks2++)
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                pw[ks2][h] = pack_bf16_rne(s[8 * ks2 + 2 * h], s[8 * ks2 + 2 * h + 1]);
+                if (PRECISE)
+                    pl[ks2][h] = pack_bf16_rne(s[8 * ks2 + 2 * h] - bf16lo_to_f32(pw[ks2][h]),
+                                               s[8 * ks2 + 2 * h + 1] - bf16hi_to_f32(pw[ks2][h]));
+                else
+                    psum = pair_sum_bf16(pw[ks2][h], psum);
+            }
+        l_part[c] += psum;
+    };
+    constexpr float SLACK = 64.0f;
+    auto move_ref = [&](int c, float tmax) -> float {
+        tmax = xor32_max(tmax);
+        float corr = 1.0f;
+        if (tmax > m_ref[c] + 8.0f) {
+            corr = __builtin_amdgcn_exp2f(m_ref[c] - tmax);
+            m_ref[c] = tmax;
+            l_part[c] *= corr;
+        }
+        return corr;
+    };
+    // (the accumulators pinned to AGPRs: left to the allocator, some of them change sides in every tile)
+    auto value_mfma = [&](f32x16 &acc, bf16x8 a, const u32x4 &b) {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+    };
+    auto values = [&](u32x4 (&pw)[2][2], u32x4 (&pl)[2][2]) {
+        s16x4 lo[PF_PRE], hi[PF_PRE];
+#pragma unroll
+        for (int st = 0; st < PF_PRE; st++) lo[st] = vread(st, 0), hi[st] = vread(st, 1);
+        // all weights are in their registers, two wait states in front of the first product
+        if (PRECISE) asm volatile("" : "+v"(pl[0][0]), "+v"(pl[0][1]), "+v"(pl[1][0]), "+v"(pl[1][1]));
+        asm volatile("s_nop 1" : "+v"(pw[0][0]), "+v"(pw[0][1]), "+v"(pw[1][0]), "+v"(pw[1][1])::"memory");
+#pragma unroll
+        for (int st = 0; st < 16; st++) {
+            const int ks2 = st >> 3, db = st & 7;
+            typedef __attribute__((ext_vector_type(8))) short s16x8;
+            const bf16x8 va = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo[st % PF_PRE], hi[st % PF_PRE], 0, 1, 2, 3, 4, 5, 6, 7));
+            if (st + PF_PRE < 16) lo[st % PF_PRE] = vread(st + PF_PRE, 0), hi[st % PF_PRE] = vread(st + PF_PRE, 1);
+            value_mfma(oacc[0][db], va, pw[0][ks2]);
+            value_mfma(oacc[1][db], va, pw[1][ks2]);
+            if (PRECISE) {
+                value_mfma(oacc[0][db], va, pl[0][ks2]);
+                value_mfma(oacc[1][db], va, pl[1][ks2]);
+            }
+        }
+    };
+    auto values_done = [&]() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); };     // before a VALU read of the accumulators
+    auto rescale = [&](const float (&corr)[2]) {            // in place (see gqa_prefill_body)
+        values_done();
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int db = 0; db < 8; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    float tmp;
+                    asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\ts_nop 0\n\t"
+                                 "v_accvgpr_write_b32 %0, %1"
+                                 : "+a"(oacc[c][db][i]), "=&v"(tmp)
+                                 : "v"(corr[c]));
+                }
+    };
+    // The oldest tile in flight has landed: behind it the copies of at most one other are on their way.
+    auto landed = [&](bool other) {
+        if (other) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    // the fragments of a buffer have been read: its next tile may come
+    auto next_tile = [&](const unsigned char *base, uint32_t lds_tile, int u) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (u < my_tiles) issue(base, lds_tile, wave + PF_WAVES * u);
+    };
+
+    // A block of one tile: every wave scores it, and takes a quarter of the dims of the value products to the output
+    // (16 positions: 7.6 us, 11.0 where one wave takes them all and the meeting below follows).
+    if (single) {
+        f32x16 s[2], acc[2][2];
+        u32x4 pw[2][2], pl[2][2];
+        landed(false);
+        scores(s);
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            (void)move_ref(c, prep(0, c, s[c]));
+            finish(c, s[c], pw[c], pl[c]);
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[c][d][i] = 0.0f;
+        }
+        typedef __attribute__((ext_vector_type(8))) short s16x8;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            const int ks2 = st >> 1, d = st & 1, off = wave * 128 + d * 64 + ks2 * 512;
+            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vfrag[0] + off));
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vfrag[1] + off));
+            const bf16x8 va = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                acc[c][d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8, pw[c][ks2]), acc[c][d], 0, 0, 0);
+                if (PRECISE)
+                    acc[c][d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8, pl[c][ks2]), acc[c][d], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const float l = xor32_sum(l_part[c]), inv = l > 0.0f ? 1.0f / l : 0.0f;
+            const int r = 32 * c + l32;
+            if (t0 + r % P < n) {
+                float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 64 * wave + 4 * g;
+#pragma unroll
+                for (int d = 0; d < 2; d++)
+#pragma unroll
+                    for (int b = 0; b < 4; b++) {
+                        f32x4 w;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) w[i] = acc[c][d][4 * b + i] * inv;
+                        *(f32x4 *)(o + 32 * d + 8 * b) = w;
+                    }
+            }
+        }
+        return;
+    }
+
+    // All of the wave's tiles.  FOLLOW: the reference follows the maximum and the accumulators are rescaled every
+    // tile; without, the reference stays at the first tile's maximum, and a tile with a row that outgrew it ends the
+    // attempt (false).  (A row whose keys of a tile are all masked sees nothing of later tiles either: every row
+    // has its reference from the first tile.)
+    auto tiles = [&](auto follow) -> bool {
+        constexpr bool FOLLOW = decltype(follow)::value;
+        for (int u = 0;;) {
+            f32x16 s[2];
+            u32x4 pw[2][2], pl[2][2];
+            landed(true);
+            scores(s);
+            next_tile(Kg, lds_k, u + 1);
+            const int tile = wave + PF_WAVES * u;
+            const float x[2] = {prep(tile, 0, s[0]), prep(tile, 1, s[1])};
+            if constexpr (FOLLOW) {
+                const float corr[2] = {move_ref(0, x[0]), move_ref(1, x[1])};
+                rescale(corr);
+            } else if (__any(x[0] > m_ref[0] + SLACK || x[1] > m_ref[1] + SLACK)) {
+                if (u > 0) return false;
+                (void)move_ref(0, x[0]);                    // nothing accumulated yet
+                (void)move_ref(1, x[1]);
+            }
+            finish(0, s[0], pw[0], pl[0]);
+            finish(1, s[1], pw[1], pl[1]);
+            landed(u + 1 < my_tiles);
+            values(pw, pl);
+            next_tile(Vg, lds_v, u + 1);
+            if (++u == my_tiles) return true;
+        }
+    };
+    if (my_tiles > 0 && !tiles(std::false_type{})) {
+        // a row outgrew its reference (rare): from the first tile again
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+        clear();
+        m_ref[0] = m_ref[1] = -INFINITY;
+        l_part[0] = l_part[1] = 0.0f;
+        issue(Kg, lds_k, wave);
+        issue(Vg, lds_v, wave);
+        (void)tiles(std::true_type{});
+    }
+
+    // ---- the waves meet: a quarter of the dims at a time, in two places of LDS in turn; of a quarter's sixteen
+    // pieces (a column block, 32 dims, 8 of them) a wave adds up those of one column block and 32 dims ----
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const float l = xor32_sum(l_part[c]);
+        if (g == 0) sm.ml[wave][32 * c + l32] = (f32x2){m_ref[c], l};
+    }
+    values_done();
+    PF_LDS_BARRIER();                                       // (and all waves are done with their tiles)
+    const int cw = wave >> 1, dw = wave & 1, r = 32 * cw + l32;
+    float f[2], top = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        f32x2 ml[PF_WAVES];
+        float t = -INFINITY, l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < PF_WAVES; w++) {
+            ml[w] = sm.ml[w][32 * c + l32];
+            t = fmaxf(t, ml[w][0]);
+        }
+#pragma unroll
+        for (int w = 0; w < PF_WAVES; w++)
+            if (ml[w][0] > -INFINITY) l = __builtin_fmaf(ml[w][1], __builtin_amdgcn_exp2f(ml[w][0] - t), l);
+        f[c] = m_ref[c] > -INFINITY ? __builtin_amdgcn_exp2f(m_ref[c] - t) : 0.0f;
+        if (c == cw) top = t, sum = l;
+    }
+    const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+    const bool row = t0 + r % P < n;
+    float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 32 * dw + 4 * g;
+    float *po = part + ((cw * 8 + dw) * 4 * 64 + lane) * 4;
+    const int live = n_tiles < PF_WAVES ? n_tiles : PF_WAVES;       // waves that had tiles
+    f32x4 *put = (f32x4 *)smem_raw + wave * 16 * 64 + lane;
+    const f32x4 *get = (const f32x4 *)smem_raw + (cw * 2 + dw) * 4 * 64 + lane;
+    // (of one or two waves' accumulators all quarters have a place at once)
+    const bool few = live <= 2;
+    auto place = [&](int qd) { return (few ? 2 * qd : PF_WAVES * (qd & 1)) * 16 * 64; };
+#pragma unroll
+    for (int qd = 0; qd < 4; qd++) {
+        if (wave < live)
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    f32x4 w;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        float x;
+                        asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(oacc[c][2 * qd + d][4 * b + i]));
+                        w[i] = x * f[c];
+                    }
+                    put[place(qd) + ((c * 2 + d) * 4 + b) * 64] = w;
+                }
+        if (few && qd < 3) continue;
+        PF_LDS_BARRIER();
+        for (int q = few ? 0 : qd; q <= qd; q++) {
+            f32x4 w[4];
+#pragma unroll
+            for (int b = 0; b < 4; b++) w[b] = get[place(q) + b * 64];
+#pragma unroll
+            for (int v = 1; v < PF_WAVES; v++)
+                if (v < live)
+#pragma unroll
+                    for (int b = 0; b < 4; b++) w[b] += get[place(q) + (v * 16 + b) * 64];
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                if (part) *(f32x4 *)(po + (2 * q * 4 + b) * 256) = w[b];
+                else if (row) *(f32x4 *)(o + 64 * q + 8 * b) = w[b] * inv;
+            }
+        }
+    }
+    if (part && dw == 0 && g == 0) *(f32x2 *)(part_ml + r * 2) = (f32x2){top, sum};
+}
+
+template <int GROUP>
+__global__ void __launch_bounds__(64 * PF_WAVES, 1)
+gqa_prefill_team_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
+                        const uint16_t *__restrict__ Q, int64_t pos0, int64_t n, int n_kv_heads,
+                        float scale_log2e, float *__restrict__ out, int64_t n_prec, int pblocks,
+                        const PfPlan plan, float *__restrict__ part, float *__restrict__ part_ml,
+                        uint32_t *__restrict__ tickets) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    __shared__ uint32_t sh_item;
+    const uint32_t total = (uint32_t)plan.first[pblocks] * (uint32_t)n_kv_heads;
+    uint32_t item = blockIdx.x;
+    for (;;) {
+        if (item >= total) break;
+        const int slice_no = (int)(item / (uint32_t)n_kv_heads), kvh = (int)(item % (uint32_t)n_kv_heads);
+        int lo = 0, hi = pblocks;                       // the rank with first[rank] <= slice_no < first[rank + 1]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if ((int)plan.first[mid] <= slice_no) lo = mid;
+            else hi = mid;
+        }
+        const int64_t pblk = pblocks - 1 - lo;
+        const int slice = slice_no - plan.first[lo], n_slices = plan.first[lo + 1] - plan.first[lo];
+        const int64_t k0 = (int64_t)slice * plan.per * PF_TK;
+        int64_t keys = pf_block_keys<GROUP, 1>(pos0, n, pblk) - k0;
+        if (slice + 1 < n_slices) keys = (int64_t)plan.per * PF_TK;
+        const size_t row0 = (size_t)k0 * n_kv_heads * PF_HD;
+        float *p = n_slices > 1 ? part + item * PF_PART<1> : nullptr, *pml = part_ml + (size_t)item * (64 * 2);
+        if (pblk < n_prec) gqa_prefill_team_body<GROUP, true>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh, p, pml);
+        else gqa_prefill_team_body<GROUP, false>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh, p, pml);
         if (gridDim.x >= total) break;                  // one item each: nothing to draw
         if (threadIdx.x == 0) sh_item = gridDim.x + atomicAdd(&tickets[0], 1u);
         __syncthreads();
@@ -917,53 +1351,6 @@ static int64_t pf_precise_blocks(int64_t pos0, int64_t n, int64_t pblocks) {
     return n_prec;
 }
 
-// Cuts the blocks into slices of plan.per tiles (0: whole blocks are as good) and returns what that
-// takes, in units of one key tile of one workgroup (about 1.2 us): an item costs its tiles and ITEM more
-// (first tiles, query rows, output: these go with the rows), a tile of a PRECISE block 1.6; the partials
-// of a slice are written and read once.  The launch takes the longest item, or the chip's even share, or
-// k + 1 of the items that some compute unit must take k + 1 of; the smallest of these over the slice
-// lengths tried wins.  (More than two items for each compute unit are never worth it.)
-template <int GROUP, int WAVES>
-static float pf_plan(int64_t pos0, int64_t n, int n_kv_heads, int64_t n_prec, int pblocks, PfPlan &best) {
-    constexpr float ITEM = WAVES == 4 ? 13.0f : 6.0f, SLICE = WAVES == 4 ? 0.065f : 0.015f, MERGE = WAVES == 4 ? 2.0f : 4.0f;
-    constexpr int P = 64 * WAVES / GROUP;
-    const int cus = num_cus();
-    float best_t = INFINITY;
-    best.per = 0;
-    const int most = (int)((pf_block_keys<GROUP, WAVES>(pos0, n, pblocks - 1) + PF_TK - 1) / PF_TK);
-    for (int ns = 1; ns <= 64 && (ns == 1 || (ns - 1) * pblocks * n_kv_heads < 2 * cus); ns = ns < 8 ? ns + 1 : ns * 5 / 4) {
-        const int per = (most + ns - 1) / ns;
-        if (ns > 1 && per < (WAVES == 4 ? 4 : 2)) break;
-        float sum = 0.0f, longest = 0.0f, rounds = 0.0f;
-        int items = 0, parts = 0;
-        for (int pb = pblocks - 1; pb >= 0; pb--) {
-            const int tiles = (int)((pf_block_keys<GROUP, WAVES>(pos0, n, pb) + PF_TK - 1) / PF_TK);
-            const int plain = (int)((pos0 + (int64_t)pb * P + 1) / PF_TK);
-            const int k = ns == 1 ? 1 : pf_slices(tiles, plain, per);
-            const float tile = pb < n_prec ? 1.6f : 1.0f;
-            const float cost = ITEM + tile * (float)tiles / (float)k;
-            const float last = k > 1 ? ITEM + tile * (float)(tiles - (k - 1) * per) : cost;
-            longest = fmaxf(longest, fmaxf(last, k > 1 ? ITEM + tile * (float)per : cost));
-            sum += cost * (float)(k * n_kv_heads);
-            const int before = items;
-            items += k * n_kv_heads;
-            if (k > 1) parts += k * n_kv_heads;
-            const int round = (items + cus - 1) / cus;
-            if (round > 1 && round != (before + cus - 1) / cus) rounds = fmaxf(rounds, (float)round * cost);
-        }
-        const float t = fmaxf(fmaxf(longest, sum / (float)cus), rounds) + (parts ? MERGE + SLICE * (float)parts : 0.0f);
-        if (t < best_t) best_t = t, best.per = ns == 1 ? 0 : per;
-    }
-    best.first[0] = 0;
-    for (int r = 0; r < pblocks; r++) {
-        const int pb = pblocks - 1 - r;
-        const int tiles = (int)((pf_block_keys<GROUP, WAVES>(pos0, n, pb) + PF_TK - 1) / PF_TK);
-        const int plain = (int)((pos0 + (int64_t)pb * P + 1) / PF_TK);
-        best.first[r + 1] = (uint16_t)(best.first[r] + (best.per ? pf_slices(tiles, plain, best.per) : 1));
-    }
-    return best_t;
-}
-
 // the dynamic LDS a kernel asks for is allowed once
 template <auto KERNEL>
 static hipError_t pf_allow_lds(size_t bytes) {
@@ -975,24 +1362,46 @@ static hipError_t pf_allow_lds(size_t bytes) {
     return err;
 }
 
-template <int GROUP, int WAVES>
-static int run_gqa_prefill_split(const uint16_t *k, const uint16_t *v, int64_t pos0, int64_t n, int n_kv_heads, const uint16_t *q,
-                                 float scale, float *out, int64_t n_prec, int pblocks, const PfPlan &plan, float *part,
-                                 uint32_t *tickets, hipStream_t s) {
-    CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_split_kernel<GROUP, WAVES>>(sizeof(PfSmem<WAVES>))));
+template <int GROUP>
+static int run_gqa_prefill_team(const uint16_t *k, const uint16_t *v, int64_t pos0, int64_t n, int n_kv_heads, const uint16_t *q,
+                                float scale, float *out, int64_t n_prec, int pblocks, const PfPlan &plan, float *part,
+                                uint32_t *tickets, hipStream_t s) {
+    CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_team_kernel<GROUP>>(sizeof(PfTeamSmem))));
     const int slices = plan.first[pblocks] * n_kv_heads;
-    float *part_ml = part ? part + (size_t)slices * PF_PART<WAVES> : nullptr;
+    float *part_ml = part ? part + (size_t)slices * PF_PART<1> : nullptr;
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_PREFILL, s);
-        pk.launch(gqa_prefill_split_kernel<GROUP, WAVES>, dim3((unsigned)(slices < num_cus() ? slices : num_cus())), dim3(64 * WAVES),
-                  sizeof(PfSmem<WAVES>), k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, plan,
+        pk.launch(gqa_prefill_team_kernel<GROUP>, dim3((unsigned)(slices < num_cus() ? slices : num_cus())), dim3(64 * PF_WAVES),
+                  sizeof(PfTeamSmem), k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, plan,
                   part, part_ml, tickets);
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (!plan.per) return 1;
     const bool many = plan.first[1] > 8;                // (no block has more slices than the last)
-    (many ? gqa_prefill_merge_kernel<GROUP, WAVES, 16> : gqa_prefill_merge_kernel<GROUP, WAVES, 8>)<<<
-        dim3((unsigned)(pblocks * n_kv_heads), 16 * WAVES), 256, 0, s>>>(part, part_ml, n, n_kv_heads, pblocks, plan, out);
+    (many ? gqa_prefill_merge_kernel<GROUP, 1, 16> : gqa_prefill_merge_kernel<GROUP, 1, 8>)<<<
+        dim3((unsigned)(pblocks * n_kv_heads), 16), 256, 0, s>>>(part, part_ml, n, n_kv_heads, pblocks, plan, out);
+    CWICK_HIP_CALL(hipGetLastError());
+    return 1;
+}
+
+template <int GROUP>
+static int run_gqa_prefill_split(const uint16_t *k, const uint16_t *v, int64_t pos0, int64_t n, int n_kv_heads, const uint16_t *q,
+                                 float scale, float *out, int64_t n_prec, int pblocks, const PfPlan &plan, float *part,
+                                 uint32_t *tickets, hipStream_t s) {
+    CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_split_kernel<GROUP>>(sizeof(PfSmem))));
+    const int slices = plan.first[pblocks] * n_kv_heads;
+    float *part_ml = part ? part + (size_t)slices * PF_PART<PF_WAVES> : nullptr;
+    {
+        ProfKernel pk(CWICK_HIP_PROF_GQA_PREFILL, s);
+        pk.launch(gqa_prefill_split_kernel<GROUP>, dim3((unsigned)(slices < num_cus() ? slices : num_cus())), dim3(64 * PF_WAVES),
+                  sizeof(PfSmem), k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, plan,
+                  part, part_ml, tickets);
+    }
+    CWICK_HIP_CALL(hipGetLastError());
+    if (!plan.per) return 1;
+    const bool many = plan.first[1] > 8;                // (no block has more slices than the last)
+    (many ? gqa_prefill_merge_kernel<GROUP, PF_WAVES, 16> : gqa_prefill_merge_kernel<GROUP, PF_WAVES, 8>)<<<
+        dim3((unsigned)(pblocks * n_kv_heads), 16 * PF_WAVES), 256, 0, s>>>(part, part_ml, n, n_kv_heads, pblocks, plan, out);
     CWICK_HIP_CALL(hipGetLastError());
     return 1;
 }
@@ -1016,31 +1425,28 @@ static int run_gqa_prefill(const uint16_t *k, const uint16_t *v, int64_t pos0, i
     uint32_t *tickets = ticket_counters(s);
     if (!tickets) return 0;                 // ticket_counters() has recorded why
     // From two items per compute unit on the tickets even the blocks out; below that some units
-    // would have one item, or none.
-    if (items < 2 * num_cus() && pblocks <= PF_MAX_BLOCKS) {
-        PfPlan plan;
-        const float t4 = pf_plan<GROUP, PF_WAVES>(pos0, n, n_kv_heads, n_prec, (int)pblocks, plan);
-        // Workgroups of one wave, a quarter of the rows each, use one of a compute unit's four matrix
-        // cores, but start and end four times as fast: they are for problems that do not fill the chip.
-        constexpr int P1 = 64 / GROUP;
-        const int64_t pblocks1 = (n + P1 - 1) / P1;
-        if (pblocks1 * n_kv_heads <= num_cus() && pblocks1 <= PF_MAX_BLOCKS) {
-            PfPlan plan1;
-            const int64_t n_prec1 = pf_precise_blocks<GROUP, 1>(pos0, n, pblocks1);
-            if (pf_plan<GROUP, 1>(pos0, n, n_kv_heads, n_prec1, (int)pblocks1, plan1) < t4) {
-                float *part = plan1.per ? pf_partials<1>(plan1, (int)pblocks1, n_kv_heads, s) : nullptr;
-                if (part || !plan1.per)
-                    return run_gqa_prefill_split<GROUP, 1>(k, v, pos0, n, n_kv_heads, q, scale, out, n_prec1, (int)pblocks1, plan1, part, tickets, s);
-            }
-        }
-        if (float *part = plan.per ? pf_partials<PF_WAVES>(plan, (int)pblocks, n_kv_heads, s) : nullptr)
-            return run_gqa_prefill_split<GROUP, PF_WAVES>(k, v, pos0, n, n_kv_heads, q, scale, out, n_prec, (int)pblocks, plan, part, tickets, s);
+    // would have one item, or none.  The plans of both ways to deal the chunk are priced, and a plan that
+    // cuts blocks needs room for the partials.
+    PfPlan plan, team_plan;
+    constexpr int TEAM_P = 64 / GROUP;
+    const int64_t team_blocks = (n + TEAM_P - 1) / TEAM_P, team_prec = pf_precise_blocks<GROUP, 1>(pos0, n, team_blocks);
+    float t = INFINITY;
+    if (items < 2 * num_cus() && pblocks <= PF_MAX_BLOCKS)
+        t = pf_plan(pos0, n, P, n_kv_heads, n_prec, num_cus(), PF_COST_WIDE, t, plan);
+    else plan.per = 0;
+    if (team_blocks <= PF_MAX_BLOCKS && t < INFINITY &&
+        pf_plan(pos0, n, TEAM_P, n_kv_heads, team_prec, num_cus(), PF_COST_TEAM, t, team_plan) < t) {
+        float *part = team_plan.per ? pf_partials<1>(team_plan, (int)team_blocks, n_kv_heads, s) : nullptr;
+        if (part || !team_plan.per)
+            return run_gqa_prefill_team<GROUP>(k, v, pos0, n, n_kv_heads, q, scale, out, team_prec, (int)team_blocks, team_plan, part, tickets, s);
     }
-    CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_kernel<GROUP>>(sizeof(PfSmem<PF_WAVES>))));
+    if (float *part = plan.per ? pf_partials<PF_WAVES>(plan, (int)pblocks, n_kv_heads, s) : nullptr)
+        return run_gqa_prefill_split<GROUP>(k, v, pos0, n, n_kv_heads, q, scale, out, n_prec, (int)pblocks, plan, part, tickets, s);
+    CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_kernel<GROUP>>(sizeof(PfSmem))));
     const int64_t wgs = items < num_cus() ? items : num_cus();      // the LDS of a compute unit holds one workgroup
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_PREFILL, s);
-        pk.launch(gqa_prefill_kernel<GROUP>, dim3((unsigned)wgs), dim3(64 * PF_WAVES), sizeof(PfSmem<PF_WAVES>),
+        pk.launch(gqa_prefill_kernel<GROUP>, dim3((unsigned)wgs), dim3(64 * PF_WAVES), sizeof(PfSmem),
                   k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, tickets);
     }
     CWICK_HIP_CALL(hipGetLastError());

@@ -89,6 +89,34 @@ def test_gqa_prefill_one_wave(hip, orc, n, pos0, nh, nkv):
     cache.free()
 
 
+@pytest.mark.parametrize("n,pos0,nh,nkv", [
+    (1, 0, 16, 4), (31, 0, 16, 2), (32, 0, 4, 2),       # one tile: every wave scores it, a quarter of the dims each
+    (33, 0, 16, 4),                                     # one tile for the first blocks, two for the last
+    (70, 0, 8, 8), (97, 0, 16, 4), (129, 0, 16, 2),     # three, four and five tiles; diagonals of three tiles
+    (64, 192, 16, 4), (63, 1, 8, 8),                    # blocks that end at and before a tile's border
+    (1025, 0, 16, 4), (1060, 0, 8, 8),                  # two-term weights and plain ones, more than one round of blocks
+    (40, 4000, 8, 8), (24, 2500, 4, 2),                 # slices, some of fewer tiles than waves
+    (64, 1000, 16, 4), (237, 627, 16, 4),               # slices of a single tile
+])
+@pytest.mark.parametrize("late", [False, True])
+def test_gqa_prefill_four_waves_a_block(hip, orc, n, pos0, nh, nkv, late):
+    """Workgroups whose four waves share a block of 64 rows; with a key that outgrows every reference before it,
+    for which the waves that meet it start over."""
+    say("[case] gqa prefill, four waves a block", n, pos0, nh, nkv, late)
+    c = synth.cfg2_gqa_prefill(n, nh, nkv, 256, pos0, seed=81)
+    k = c["k"]
+    if late:
+        k = synth.bf16_to_f32(k)
+        k[(pos0 + n) * 2 // 3] = 30.0 * synth.bf16_to_f32(c["q"])[n - 1].reshape(nkv, nh // nkv, 256)[:, 0]
+        k = synth.f32_to_bf16(k)
+    cache = hip.KVCache(pos0 + n, nkv, 256)
+    cache.write(0, k.reshape(pos0 + n, -1), c["v"].reshape(pos0 + n, -1))
+    got = hip.gqa_prefill(cache, pos0, c["q"], c["scale"])
+    ref = orc.gqa_prefill(c["q"], k, c["v"], pos0, c["scale"], nthreads=0)
+    assert_close(got, ref, "gqa prefill, four waves a block", strict=pos0 >= 200 and not late)
+    cache.free()
+
+
 @pytest.mark.parametrize("HD,rotary", [(256, 256), (256, 36), (128, 24), (128, 6)])
 def test_gqa_prepare_head_sizes(hip, orc, HD, rotary):
     """The rotation over all and a part of a head, its halves in fours (four dims a lane) and not."""

@@ -125,6 +125,70 @@ int main() {
     print(out)
 
 
+def test_gqa_prefill_plans_are_sound_and_quick(tmp_path):
+    """The plans of both prefill kernels: the slices of every block cover its tiles, each begins below the
+    diagonal and none is empty, there is room for the partials' numbers; less than a
+    fifth behind the best of all slice lengths by its own cost (a dozen of them are tried, a quarter apart; here 17 %
+    at the worst, where the other kernel's plan is a third shorter); a limit is kept; and a plan is made in a
+    fraction of the kernel behind it: at most 10 us and an eighth of its time (on a loaded machine; here 1 us for
+    200 positions, 5 for 1000, 11 for 4000, which take 160)."""
+    out = run_cpp(tmp_path, "gqa_plan.hpp", r"""
+int main() {
+    float worst = 0.0f;
+    const int cus = 256;
+    for (int kv : {1, 2, 4, 8, 6})
+            for (int rows : {64, 256})
+                for (int group : {1, 4, 8})
+                    for (int64_t n = 1; n <= 9000; n = n < 4 ? n + 1 : n * 17 / 10)
+                        for (int64_t pos0 : {0, 31, 700, 5000, 16384, 1000000}) {
+                            const PfCost &c = rows == 64 ? PF_COST_TEAM : PF_COST_WIDE;
+                            const int P = rows / group;
+                            const int64_t blocks = (n + P - 1) / P;
+                            if (blocks > PF_MAX_BLOCKS) continue;
+                            int64_t prec = 0;
+                            while (prec < blocks && pf_keys(pos0, n, P, prec) <= 1024) prec++;
+                            PfPlan p;
+                            const float t = pf_plan(pos0, n, P, kv, prec, cus, c, INFINITY, p);
+                            PfBlocks b;
+                            b.count = (int)blocks, b.n_kv_heads = kv, b.n_prec = (int)prec, b.cus = cus;
+                            bool ok = t > 0.0f && t < INFINITY && p.first[0] == 0;
+                            for (int r = 0; r < b.count; r++) {
+                                const int64_t pb = b.count - 1 - r;
+                                b.tiles[r] = (int)((pf_keys(pos0, n, P, pb) + PF_TK - 1) / PF_TK);
+                                b.plain[r] = (int)((pos0 + pb * P + 1) / PF_TK);
+                                const int k = p.first[r + 1] - p.first[r];
+                                ok = ok && k >= 1 && (p.per || k == 1);
+                                if (k > 1) ok = ok && (int64_t)(k - 1) * p.per < b.tiles[r] && (int64_t)(k - 1) * p.per * PF_TK <= pos0 + pb * P + 1;
+                            }
+                            if (!ok) { printf("bad plan: %d rows, %d at %d, %d kv heads of %d\n", rows, (int)n, (int)pos0, kv, group); return 1; }
+                            PfPlan q;
+                            if (pf_plan(pos0, n, P, kv, prec, cus, c, 0.5f * t, q) != 0.5f * t) { printf("limit not kept\n"); return 1; }
+                            if (b.tiles[0] > 600 || b.count == cus / kv) continue;      // (those stay whole)
+                            float best = pf_time(b, c, 0, INFINITY);
+                            for (int per = c.least; per < b.tiles[0]; per += c.waves) best = std::fmin(best, pf_time(b, c, per, best));
+                            if (t / best > worst) worst = t / best;
+                            if (t > 1.2f * best) { printf("%.3f: %d rows, %d at %d, %d kv heads of %d, %d units\n", t / best, rows, (int)n, (int)pos0, kv, group, cus); return 1; }
+                        }
+    double slowest = 0.0;
+    for (int64_t n : {16, 128, 360, 1000, 2500, 4000, 6000, 8000})
+        for (int64_t pos0 : {0, 2000, 12000}) {
+            double us = 1e9;
+            float t = 0.0f;
+            for (int rep = 0; rep < 20; rep++) {
+                const auto t0 = std::chrono::steady_clock::now();
+                PfPlan a, b;
+                t = pf_plan(pos0, n, 64, 4, 0, 256, PF_COST_WIDE, INFINITY, a);
+                if (n <= 8192) t = pf_plan(pos0, n, 16, 4, 0, 256, PF_COST_TEAM, t, b);
+                us = std::fmin(us, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count());
+            }
+            slowest = std::fmax(slowest, us / (10.0 + t / 8));
+        }
+    printf("worst %.3f, slowest %.2f of what it may take\n", worst, slowest);
+    return slowest < 1.0 ? 0 : 1;
+}""")
+    print(out)
+
+
 def test_flag_numbers_never_meet_an_old_flag(tmp_path):
     """Around the end of 32 bits: a call's number is never 0 (a flag never written) nor what any flag still holds,
     whether the calls before wrote all of their flags, some, or none."""
