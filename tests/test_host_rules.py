@@ -164,8 +164,9 @@ int main() {
                             PfPlan q;
                             if (pf_plan(pos0, n, P, kv, prec, cus, c, 0.5f * t, q) != 0.5f * t) { printf("limit not kept\n"); return 1; }
                             if (b.tiles[0] > 600 || b.count == cus / kv) continue;      // (those stay whole)
-                            float best = pf_time(b, c, 0, INFINITY);
-                            for (int per = c.least; per < b.tiles[0]; per += c.waves) best = std::fmin(best, pf_time(b, c, per, best));
+                            int parts;
+                            float best = pf_time(b, c, 0, INFINITY, parts);
+                            for (int per = c.least; per < b.tiles[0]; per += c.waves) best = std::fmin(best, pf_time(b, c, per, best, parts));
                             if (t / best > worst) worst = t / best;
                             if (t > 1.2f * best) { printf("%.3f: %d rows, %d at %d, %d kv heads of %d, %d units\n", t / best, rows, (int)n, (int)pos0, kv, group, cus); return 1; }
                         }
