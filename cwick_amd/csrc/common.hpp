@@ -130,13 +130,14 @@ __host__ __device__ inline bool indexer_band_failed(const IndexerBandRow &r, int
     return r.fallback != 0u || r.n_cand > (uint32_t)cap;
 }
 // shapes the banded path takes: rows that the many-workgroup top-k handles, k < n
-// The banded select is four launches, 26 us for a few rows and 34 for eight of 64K keys; every key scored
-// exactly and one workgroup's select take 10 us, 4 us more per million key-head pairs of the batch and
-// 0.4 per 1024 keys of a row (batch 1, 64 heads: 26000 keys 42.7 us with the attention against 41, 20000
-// 36.9 against 40; 8 x 14400: 68 against 46).
+// The banded select is four launches, about the same for any row; every key scored exactly and one
+// workgroup's select take 5.4 us per million key-head pairs of the batch and 0.43 per 1024 keys of a row: the
+// difference is 24.3 less than these (19 shapes on either side of the line, off by 2.5 us at most).  With the
+// attention, batch 1, 64 heads: 24000 keys 34.1 us against 41.1, 32000 42.0 against 41.2; 4 x 10000 36.8 against
+// 43.2, 4 x 16000 48.3 against 43.8; 8 x 8300 51.9 against 48.8.
 inline bool indexer_band_applies(int64_t n_keys, int64_t k, int n_idx_heads, int batch) {
     return n_keys >= 8192 && n_keys <= 131072 && k < n_keys && n_idx_heads >= 1 && n_idx_heads <= 64 &&
-           10.3 + 4e-6 * (double)(n_keys * batch * n_idx_heads) + 4.2e-4 * (double)n_keys > 26.0;
+           5.4e-6 * (double)(n_keys * batch * n_idx_heads) + 4.3e-4 * (double)n_keys > 24.3;
 }
 // indexer and top-k in one: `scores` is scratch (its contents afterwards are not scores), the
 // selected indices of every row go to out_idx[batch][k] in ascending order
@@ -201,11 +202,9 @@ int run_probe_mfma(int kind, int reps, double *tflops);
 // order-preserving 32-bit key of a score for the radix select: larger score, larger key; NaN
 // sorts below everything (key 0), -0.0 equals +0.0, and no number maps to 0
 __device__ __forceinline__ uint32_t topk_key(float f) {
-    if (f != f) return 0u;
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if ((u << 1) == 0u) u = 0u;                       // -0.0 -> +0.0
-    u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-    return u == 0u ? 1u : u;
+    const uint32_t u = __builtin_bit_cast(uint32_t, f + 0.0f);        // -0.0 + 0.0 is +0.0
+    const uint32_t key = u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+    return f != f ? 0u : key;                                         // (only a NaN's bits would give key 0)
 }
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;

@@ -608,8 +608,8 @@ int launch_topk(const float *scores, int batch, int64_t n, int64_t k, int32_t *o
     CWICK_REQUIRE(batch >= 1 && batch <= 65535, "topk: batch %d", batch);
     CWICK_REQUIRE(n >= 1 && n <= ((int64_t)1 << 24), "topk: n %lld (1..2^24)", (long long)n);
     CWICK_REQUIRE(k >= 1 && k <= 65536, "topk: k %lld (1..65536)", (long long)k);
-    // One workgroup takes 3.3 us and 0.4 per 1024 scores, whatever the batch; the five launches of the
-    // many-workgroup select 21 us (32768 scores: 16.1 and 20.8; 65536: 21.1).
+    // One workgroup takes 3.1 us and 0.4 per 1024 scores, whatever the batch; the five launches of the
+    // many-workgroup select 21 us (30000 scores: 15.3; 65536: 21.1).
     const int64_t n_wg = topk_mw_wgs(n);
     if (n > (int64_t)TOPK_THREADS * 32 && n_wg <= TOPK_MW_MAX_WGS) {
         const size_t ws_row = topk_mw_row_dwords(n_wg);             // dwords: slices, four states, above counts
@@ -626,21 +626,10 @@ int launch_topk(const float *scores, int batch, int64_t n, int64_t k, int32_t *o
     }
     {
         ProfScope ps(CWICK_HIP_PROF_TOPK, s);
-        if (n <= (int64_t)TOPK_THREADS)
-            topk_radix_reg_kernel<1><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else if (n <= (int64_t)TOPK_THREADS * 4)
-            topk_radix_reg_kernel<4><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else if (n <= (int64_t)TOPK_THREADS * 8)
-            topk_radix_reg_kernel<8><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else if (n <= (int64_t)TOPK_THREADS * 12)
-            topk_radix_reg_kernel<12><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else if (n <= (int64_t)TOPK_THREADS * 16)
-            topk_radix_reg_kernel<16><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else if (n <= (int64_t)TOPK_THREADS * 24)
-            topk_radix_reg_kernel<24><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else if (n <= (int64_t)TOPK_THREADS * 32)
-            topk_radix_reg_kernel<32><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
-        else
+#define CWICK_TOPK_REG(E) \
+    if (n <= (int64_t)TOPK_THREADS * (E)) topk_radix_reg_kernel<E><<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx); else
+        CWICK_TOPK_REG(1) CWICK_TOPK_REG(4) CWICK_TOPK_REG(8) CWICK_TOPK_REG(12) CWICK_TOPK_REG(16) CWICK_TOPK_REG(24) CWICK_TOPK_REG(32)
+#undef CWICK_TOPK_REG
             topk_radix_kernel<<<batch, TOPK_THREADS, 0, s>>>(scores, n, k, out_idx);
     }
     CWICK_HIP_CALL(hipGetLastError());
