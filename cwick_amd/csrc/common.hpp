@@ -5,6 +5,8 @@
 #include <stdint.h>
 #include <stddef.h>
 
+#include <initializer_list>
+
 #include "../../include/cwick_hip.h"
 #include "band_counter.hpp"
 
@@ -114,9 +116,21 @@ struct IndexerBandRow {
     uint32_t pad[29];     // a row to a 128-byte line: the workgroups of different rows add to n_cand at the same time
 };
 constexpr int CWICK_INDEXER_BAND_CAP = 4096;   // candidate list entries per row
-constexpr int CWICK_INDEXER_APPROX_KEYS = 2048;   // keys per workgroup (= per bound slot) of the approximate kernel
-inline int indexer_approx_slots(int64_t n_keys) {
-    return (int)((n_keys + CWICK_INDEXER_APPROX_KEYS - 1) / CWICK_INDEXER_APPROX_KEYS);
+// Keys per workgroup (= per slot of bounds and counts) of the approximate kernel: 2048, or fewer where that
+// leaves compute units without one (a workgroup takes 5 us and 1.2 per 256 keys; what the select adds up of a
+// row grows with its slots, so at most 128).  With the attention, rows of 64K keys: one 44.7 us with 2048, 38.6
+// with 512; two 48.3, 41.1; four 49.2, 46.6 with 1024; eight of 16000 49.3, 43.9 with 512.
+constexpr int CWICK_INDEXER_APPROX_KEYS = 2048, CWICK_INDEXER_APPROX_SLOTS = 128;
+inline int indexer_approx_keys(int64_t n_keys, int batch) {
+    for (int keys : {512, 768, 1024, 1536}) {
+        const int64_t slots = (n_keys + keys - 1) / keys;
+        if (slots * batch <= num_cus() && slots <= CWICK_INDEXER_APPROX_SLOTS) return keys;
+    }
+    return CWICK_INDEXER_APPROX_KEYS;
+}
+inline int indexer_approx_slots(int64_t n_keys, int batch) {
+    const int keys = indexer_approx_keys(n_keys, batch);
+    return (int)((n_keys + keys - 1) / keys);
 }
 int launch_indexer_approx(const uint8_t *keys, const float *kscale, int64_t key_bstride,
                           int64_t kscale_bstride, int batch, int64_t n_keys, const uint16_t *q_idx,
@@ -125,19 +139,23 @@ int launch_indexer_approx(const uint8_t *keys, const float *kscale, int64_t key_
 // What the approximate kernel leaves for the select, per row and workgroup (slot): how many of its scores
 // each of 4096 counters has (16-bit counts; band_counter), and each sixteen of them together.
 constexpr int CWICK_BAND_DIGITS = 256 + 4096 / 2;         // dwords per slot
-inline size_t indexer_band_digits_dwords(int64_t n_keys) { return (size_t)indexer_approx_slots(n_keys) * CWICK_BAND_DIGITS; }
+// (of a call: as much as any call of fewer rows or keys needs)
+inline size_t indexer_band_digits_dwords(int64_t n_keys, int batch) {
+    const size_t slots = (size_t)indexer_approx_slots(n_keys, batch) * batch, few = (size_t)num_cus();
+    return (slots > few ? slots : few) * CWICK_BAND_DIGITS;
+}
 __host__ __device__ inline bool indexer_band_failed(const IndexerBandRow &r, int cap) {
     return r.fallback != 0u || r.n_cand > (uint32_t)cap;
 }
 // shapes the banded path takes: rows that the many-workgroup top-k handles, k < n
 // The banded select is four launches, about the same for any row; every key scored exactly and one
-// workgroup's select take 5.4 us per million key-head pairs of the batch and 0.43 per 1024 keys of a row: the
-// difference is 24.3 less than these (19 shapes on either side of the line, off by 2.5 us at most).  With the
-// attention, batch 1, 64 heads: 24000 keys 34.1 us against 41.1, 32000 42.0 against 41.2; 4 x 10000 36.8 against
-// 43.2, 4 x 16000 48.3 against 43.8; 8 x 8300 51.9 against 48.8.
+// workgroup's select take 5.05 us per million key-head pairs of the batch and 0.37 per 1024 keys of a row: the
+// difference is 15.8 less than these (26 shapes on either side of the line, off by 2.5 us at most).  With the
+// attention, 64 heads: one row of 24000 keys 33.7 us against 33.8, of 28000 39.7 against 34.0; 2 x 14000 32.1 against
+// 34.0, 2 x 18000 38.3 against 35.0; 4 x 8300 35.1 against 36.4, 4 x 13000 42.5 against 36.4; 8 x 8300 51.4 against 41.9.
 inline bool indexer_band_applies(int64_t n_keys, int64_t k, int n_idx_heads, int batch) {
-    return n_keys >= 8192 && n_keys <= 131072 && k < n_keys && n_idx_heads >= 1 && n_idx_heads <= 64 &&
-           5.4e-6 * (double)(n_keys * batch * n_idx_heads) + 4.3e-4 * (double)n_keys > 24.3;
+    return n_keys > 6144 && n_keys <= 131072 && k < n_keys && n_idx_heads >= 1 && n_idx_heads <= 64 &&
+           5.05e-6 * (double)(n_keys * batch * n_idx_heads) + 3.7e-4 * (double)n_keys > 15.8;
 }
 // indexer and top-k in one: `scores` is scratch (its contents afterwards are not scores), the
 // selected indices of every row go to out_idx[batch][k] in ascending order

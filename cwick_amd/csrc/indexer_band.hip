@@ -41,7 +41,6 @@ namespace cwick {
 constexpr int IB_THREADS = 512;
 constexpr int IB_WAVES = IB_THREADS / 64;
 constexpr int IB_QROW = 128 + 8;                 // bf16 per head row of q in LDS (padded: 272 bytes)
-constexpr int IB_KEYS = CWICK_INDEXER_APPROX_KEYS;   // keys per workgroup of the approximate kernel
 constexpr int IB_HD = CWICK_HIP_INDEX_DIM;    // 128
 
 typedef __attribute__((ext_vector_type(2))) float ib_f32x2;
@@ -54,6 +53,7 @@ __device__ __forceinline__ float ib_half_sum(float v) {
     return a + b;
 }
 
+template <int IB_KEYS>                          // keys per workgroup
 __global__ void __launch_bounds__(IB_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict__ kscale,
                       int64_t key_bstride, int64_t kscale_bstride, int64_t n_keys,
@@ -89,7 +89,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     u32x4 raw_a[4], raw_b[4], raw_c[4];
     float kst_a, kst_b, kst_c;
     auto load_keys = [&](int it, u32x4 (&raw)[4], float &kst) {
-        int64_t tc = wbase + (it < N_IT ? it : N_IT - 1) * 32 + row;
+        int64_t tc = wbase + it * 32 + row;
         tc = tc < n_keys ? tc : n_keys - 1;
         const uint8_t *krow = kb + (size_t)tc * IB_HD + 64 * g;
 #pragma unroll
@@ -291,13 +291,13 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
 #pragma unroll
     for (int it = 0; it < N_IT; it += 3) {
         if (wbase + it * 32 >= n_keys) break;                      // wave-uniform
-        load_keys(it + 2, raw_c, kst_c);
+        if (it + 2 < N_IT) load_keys(it + 2, raw_c, kst_c);
         iteration(it, raw_a, kst_a);
         if (it + 1 >= N_IT || wbase + (it + 1) * 32 >= n_keys) break;
-        load_keys(it + 3, raw_a, kst_a);
+        if (it + 3 < N_IT) load_keys(it + 3, raw_a, kst_a);
         iteration(it + 1, raw_b, kst_b);
         if (it + 2 >= N_IT || wbase + (it + 2) * 32 >= n_keys) break;
-        load_keys(it + 4, raw_b, kst_b);
+        if (it + 4 < N_IT) load_keys(it + 4, raw_b, kst_b);
         iteration(it + 2, raw_c, kst_c);
     }
     // (never negative: the bit patterns order like the values as unsigned integers, NaNs on top)
@@ -450,10 +450,11 @@ int launch_indexer_approx(const uint8_t *keys, const float *kscale, int64_t key_
     CWICK_REQUIRE(n_keys >= 1 && n_idx_heads >= 1 && n_idx_heads <= 64, "indexer_approx: shape out of range");
     CWICK_REQUIRE((uintptr_t)keys % 16 == 0 && key_bstride % 16 == 0 && (uintptr_t)q_idx % 16 == 0,
                   "indexer_approx: keys and q must be 16-byte aligned");
-    const int n_wg = indexer_approx_slots(n_keys);
+    const int n_wg = indexer_approx_slots(n_keys, batch), per = indexer_approx_keys(n_keys, batch);
     {
         ProfKernel pk(CWICK_HIP_PROF_INDEXER_APPROX, s);
-        pk.launch(indexer_approx_kernel, dim3(n_wg, batch), dim3(IB_THREADS), 0,
+        pk.launch(per == 512 ? indexer_approx_kernel<512> : per == 768 ? indexer_approx_kernel<768> : per == 1024 ? indexer_approx_kernel<1024> :
+                  per == 1536 ? indexer_approx_kernel<1536> : indexer_approx_kernel<CWICK_INDEXER_APPROX_KEYS>, dim3(n_wg, batch), dim3(IB_THREADS), 0,
                   keys, kscale, key_bstride, kscale_bstride, n_keys, q_idx, w, n_idx_heads, scores, beta_slots, rows,
                   digits);
     }
@@ -469,10 +470,10 @@ int launch_indexer_banded(const uint8_t *keys, const float *kscale, int64_t key_
     CWICK_REQUIRE(indexer_band_applies(n_keys, k, n_idx_heads, batch), "indexer_banded: shape out of range");
     CWICK_REQUIRE((uintptr_t)keys % 16 == 0 && key_bstride % 16 == 0 && (uintptr_t)q_idx % 16 == 0,
                   "indexer_banded: keys and q must be 16-byte aligned");
-    const int n_wg = indexer_approx_slots(n_keys);
+    const int n_wg = indexer_approx_slots(n_keys, batch);
     constexpr int cap = CWICK_INDEXER_BAND_CAP;
     // workspace: [digit counts][beta slots][row states][+inf counts][candidate lists][their exact scores]
-    const size_t digit_bytes = batch * indexer_band_digits_dwords(n_keys) * sizeof(uint32_t);
+    const size_t digit_bytes = indexer_band_digits_dwords(n_keys, batch) * sizeof(uint32_t);
     size_t off_beta = (digit_bytes + 255) & ~(size_t)255;
     size_t off_rows = off_beta + (((size_t)batch * n_wg * sizeof(float) + 255) & ~(size_t)255);
     size_t off_hi = off_rows + (((size_t)batch * sizeof(IndexerBandRow) + 255) & ~(size_t)255);

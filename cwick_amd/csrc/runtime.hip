@@ -1158,7 +1158,7 @@ int cwick_hip_indexer_scores_approx(cwick_hip_ikeys *c, int slot, int64_t n_keys
                   (long long)n_keys, (long long)c->capacity);
     CWICK_REQUIRE(n_idx_heads >= 1 && n_idx_heads <= 64, "indexer_scores_approx: n_idx_heads %d (1..64)",
                   n_idx_heads);
-    const int n_slots = indexer_approx_slots(n_keys);
+    const int n_slots = indexer_approx_slots(n_keys, 1);
     size_t qb = (size_t)n_idx_heads * CWICK_HIP_INDEX_DIM * 2, wb = (size_t)n_idx_heads * 4;
     size_t ob = (size_t)n_keys * 4, bb = (size_t)n_slots * 4;
     Stager st(c->ctx, pad256(qb) + pad256(wb) + pad256(ob) + pad256(bb) + 256);

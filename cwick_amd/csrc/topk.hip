@@ -74,9 +74,9 @@ __device__ __forceinline__ uint32_t topk_mw_colsum(const uint32_t *__restrict__ 
 // key; all threads return the new (prefix, remaining)
 __device__ __forceinline__ TopkMwState
 topk_mw_pick(const uint32_t *__restrict__ slices, int n_wg, int shift, TopkMwState st,
-             uint32_t *hist /* LDS, 256 */, TopkMwState *sh_state /* LDS */, int stride = 256) {
+             uint32_t *hist /* LDS, 256 */, TopkMwState *sh_state /* LDS */) {
     const int tid = threadIdx.x;
-    hist[tid] = topk_mw_colsum(slices + tid, n_wg, stride);
+    hist[tid] = topk_mw_colsum(slices + tid, n_wg);
     __syncthreads();
     if (tid < 64) {
         // walk the 256 buckets from the largest digit down; lane b owns buckets 255-4b .. 252-4b
@@ -271,10 +271,12 @@ topk_mw_classify_kernel(float *__restrict__ scores, int64_t n, int64_t k, int n_
                         const float *__restrict__ beta_slots, int n_beta,
                         int32_t *__restrict__ cand, int cap, IndexerBandRow *__restrict__ rows,
                         uint32_t *__restrict__ hi_count) {   // [row][TOPK_MW_MAX_WGS]: keys set to +inf per workgroup
-    __shared__ uint32_t hist[256];
+    __shared__ uint32_t hist[TOPK_MW_THREADS];
+    __shared__ __attribute__((aligned(16))) uint32_t part[TOPK_MW_THREADS / 64][256];
     __shared__ TopkMwState sh_state;
     __shared__ float sh_beta[TOPK_MW_THREADS / 64];
     __shared__ uint32_t sh_digit;
+    static_assert(TOPK_MW_THREADS == 256, "four waves add up, sixteen threads per counter");
     const int row = blockIdx.y, wg = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const uint32_t *slots = digits + (size_t)row * n_beta * CWICK_BAND_DIGITS;
     float *sc = scores + (size_t)row * n;
@@ -297,22 +299,53 @@ topk_mw_classify_kernel(float *__restrict__ scores, int64_t n, int64_t k, int n_
     // (5 us).  (Counters by the twelve leading bits of the order key, an eighth of an octave: a thousand
     // keys with weights of both signs, and with weights of one sign more than the list holds: the whole
     // row scored exactly, 304 us for eight rows of 64K keys and equal weights where this takes 53.)
-    TopkMwState st = topk_mw_pick(slots, n_beta, 24, TopkMwState{0u, (uint32_t)k}, hist, &sh_state, CWICK_BAND_DIGITS);
-    {   // the sixteen counters behind the byte, largest first: a lane each, their pairs summed over the slots
-        uint32_t c = 0u;
-        const uint32_t bin = (st.prefix >> 20) + 15u - (uint32_t)(tid & 15);      // (the byte's low end is the prefix)
-        if (tid < 128) {
-            // eight threads per counter, every eighth slot each
-            const int part = tid >> 4;
-            const uint32_t *p = slots + 256 + (bin >> 1);
-            for (int w0 = part; w0 < n_beta; w0 += 8) c += p[(size_t)w0 * CWICK_BAND_DIGITS] >> (16 * (bin & 1)) & 0xFFFFu;
-            hist[tid] = c;
+    {   // the sixteenths, four neighbours and every fourth slot a thread, thirty-two slots of them in flight
+        u32x4 c = {0u, 0u, 0u, 0u};
+        for (int w0 = tid >> 6; w0 < n_beta; w0 += 32) {
+            u32x4 x[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int w = w0 + 4 * j;
+                x[j] = *(const u32x4 *)&slots[(size_t)(w < n_beta ? w : w0) * CWICK_BAND_DIGITS + 4 * lane];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (w0 + 4 * j < n_beta) c += x[j];
         }
+        *(u32x4 *)&part[tid >> 6][4 * lane] = c;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        // from the largest down; lane b owns 255 - 4b .. 252 - 4b
+        const u32x4 c = (*(const u32x4 *)&part[0][252 - 4 * lane] + *(const u32x4 *)&part[1][252 - 4 * lane]) +
+                        (*(const u32x4 *)&part[2][252 - 4 * lane] + *(const u32x4 *)&part[3][252 - 4 * lane]);
+        const uint32_t sum = (c[0] + c[1]) + (c[2] + c[3]);
+        uint32_t before = wave_scan_u32(sum) - sum;
+#pragma unroll
+        for (int j = 3; j >= 0; j--) {
+            if (before < (uint32_t)k && (uint32_t)k <= before + c[j]) sh_state = TopkMwState{(uint32_t)(252 - 4 * lane + j), (uint32_t)k - before};
+            before += c[j];
+        }
+    }
+    __syncthreads();
+    {   // the sixteen counters behind it, largest first: sixteen threads each, every sixteenth slot
+        const TopkMwState st = sh_state;
+        const uint32_t bin = (st.prefix << 4) + 15u - (uint32_t)(tid & 15);
+        const uint32_t *p = slots + 256 + (bin >> 1);
+        uint32_t c = 0u;
+        for (int w0 = tid >> 4; w0 < n_beta; w0 += 64) {
+            uint32_t x[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = p[(size_t)(w0 + 16 * j < n_beta ? w0 + 16 * j : w0) * CWICK_BAND_DIGITS];
+#pragma unroll
+            for (int j = 0; j < 4; j++) c += w0 + 16 * j < n_beta ? x[j] >> (16 * (bin & 1)) & 0xFFFFu : 0u;
+        }
+        hist[tid] = c;
         __syncthreads();
         if (tid < 16) {
             c = 0u;
 #pragma unroll
-            for (int p = 0; p < 8; p++) c += hist[tid + 16 * p];
+            for (int j = 0; j < 16; j++) c += hist[tid + 16 * j];
             const uint32_t inc = wave_scan_u32(c), before = inc - c;      // (of the first sixteen lanes: a row)
             if (before < st.remaining && st.remaining <= inc) sh_digit = bin;
         }

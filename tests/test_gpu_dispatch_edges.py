@@ -338,7 +338,10 @@ def test_topk_register_rows(hip, orc, n, kind):
         assert np.array_equal(hip.topk(x, k), orc.topk_contract(x, k)), "k %d" % k
 
 
-@pytest.mark.parametrize("n_keys,batch,topk", [(8192, 8, 512), (8193, 9, 2048), (14337, 4, 700)])
+@pytest.mark.parametrize("n_keys,batch,topk", [(8192, 8, 512), (8193, 9, 2048), (14337, 4, 700),
+                                               (6145, 8, 1000), (65537, 1, 2048), (40003, 2, 512),    # 512 keys a workgroup
+                                               (60001, 3, 1024), (65536, 4, 512), (33000, 10, 512),   # 768, 1024, 1536
+                                               (33000, 17, 300)])                                     # 2048
 def test_dsa_band_of_short_rows(hip, orc, n_keys, batch, topk):
     """The banded select at its shortest rows: four and five stretches of keys per row."""
     say("[case] dsa band, short rows", n_keys, batch, topk)
