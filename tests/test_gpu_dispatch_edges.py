@@ -358,6 +358,30 @@ def test_dsa_band_of_short_rows(hip, orc, n_keys, batch, topk):
     lat.free()
 
 
+@pytest.mark.parametrize("repeats", [2, 7, 60, 400])
+def test_dsa_band_ties(hip, orc, repeats):
+    """Every key several times over, in places all over the row: the last selected position is one of several with
+    the same score, among a candidate list of less and of more than 256."""
+    n_keys, batch, topk = 21000, 3, 1024
+    say("[case] dsa band, ties", repeats)
+    c = synth.cfg5_dsa(n_keys=n_keys, batch=batch, ih=64, topk=topk, nh=16, seed=88)
+    ik, lat = hip.IndexKeys(batch, n_keys), hip.LatentCache(batch, n_keys)
+    g = np.random.default_rng(3)
+    keys, scales = [], []
+    for b in range(batch):
+        of = g.permutation(n_keys) // repeats
+        keys.append(np.ascontiguousarray(c["ikeys"][b][of]))
+        scales.append(np.ascontiguousarray(c["ikscale"][b][of]))
+        ik.write(b, 0, keys[b], scales[b])
+        lat.write(b, 0, c["rows"][b], c["scales"][b])
+    _, sel = hip.dsa_decode(ik, lat, 0, 1, n_keys, c["q_idx"], c["w"], topk, c["q"], c["scale"])
+    for b in range(batch):
+        sc = orc.indexer_scores(c["q_idx"][b], c["w"][b], keys[b], scales[b], nthreads=0)
+        assert np.array_equal(sel[b], orc.topk_contract(sc, topk)), "query %d" % b
+    ik.free()
+    lat.free()
+
+
 @pytest.mark.parametrize("weights", ["signed", "positive", "equal", "negative"])
 @pytest.mark.parametrize("keys", ["independent", "common", "small with empty rows"])
 def test_dsa_band_takes_every_kind_of_score(hip, orc, weights, keys):
