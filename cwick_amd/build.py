@@ -1,4 +1,5 @@
-"""Build libcwick_hip.so for gfx950 with hipcc (cross-compiles without a GPU).
+"""Build libcwick_hip.so for gfx950 with hipcc (cross-compiles without a GPU), and the extension
+that hip.py makes its step calls through.
 
     python -m cwick_amd.build            # compile what changed, link
     python -m cwick_amd.build --force    # recompile everything
@@ -9,12 +10,15 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(LIBDIR, "obj")
 LIB = os.path.join(LIBDIR, "libcwick_hip.so")
+# the step calls of hip.py as a CPython extension (host code only)
+CALLS = os.path.join(LIBDIR, "_cwick_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 SOURCES = ["runtime.hip", "misc.hip", "gqa_decode.hip", "gqa_prefill.hip", "mla_roles.hip",
            "indexer.hip", "indexer_band.hip", "topk.hip", "probe.hip", "prep.hip", "mla_prefill64.hip", "mm_select.hip"]
@@ -55,6 +59,18 @@ def _compile(src, force):
     return obj, log
 
 
+def _build_calls(force):
+    src = os.path.join(CSRC, "binding.cpp")
+    deps = [src, os.path.join(HERE, "..", "include", "cwick_hip.h"), os.path.abspath(__file__)]
+    if not force and os.path.exists(CALLS) and all(os.path.getmtime(CALLS) >= os.path.getmtime(d) for d in deps):
+        return
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-Wall", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-I" + sysconfig.get_path("include"), src, "-o", CALLS]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("compiling %s failed:\n%s" % (src, r.stdout + r.stderr))
+
+
 def build(force=False, verbose=True):
     os.makedirs(OBJDIR, exist_ok=True)
     with cf.ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
@@ -72,6 +88,7 @@ def build(force=False, verbose=True):
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link failed:\n" + r.stdout + r.stderr)
+    _build_calls(force)
     if verbose:
         print("built", LIB)
     return LIB

@@ -1,5 +1,6 @@
-"""ctypes binding of libcwick_hip.so (include/cwick_hip.h), one Python function
-per C entry point with the same name, argument meaning and 1/0 convention.
+"""Binding of libcwick_hip.so (include/cwick_hip.h), one Python function per C entry
+point with the same name, argument meaning and 1/0 convention: ctypes, and for the
+calls of a step a CPython extension (binding.cpp).
 
 There is no CPU fallback here: if the library is missing the import of any
 function raises, and a call that the library declines raises Declined with the
@@ -7,12 +8,16 @@ library's own reason (cwick_hip_last_error) unless the caller asks for the raw
 return code.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
+import types
 
 import numpy as np
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libcwick_hip.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_cwick_calls" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 KDIM, VDIM, NBLK, BLOCK, IDIM = 576, 512, 5, 128, 128
 
@@ -21,7 +26,7 @@ class Declined(RuntimeError):
     """The GPU backend returned 0: the engine would run its CPU path."""
 
 
-_lib = None
+_lib = _c = None
 
 _u8p, _u16p, _i32p, _f32p = (C.POINTER(C.c_uint8), C.POINTER(C.c_uint16),
                              C.POINTER(C.c_int32), C.POINTER(C.c_float))
@@ -131,6 +136,23 @@ def lib():
     return _lib
 
 
+def _calls():
+    """The calls of a step (binding.cpp), by name: they take tensors and arrays as they are, in 0.3 to 0.6 us where
+    ctypes and the addresses taken in Python need 2 (one decode over 4096 keys, which the host's launches bound: 10.6 us
+    through ctypes, 9.9 through these; one step on state in host memory, 760 keys: 33.1, 29.6)."""
+    global _c
+    if _c is None:
+        L = lib()
+        if not os.path.exists(CALLS_PATH):
+            raise ImportError("%s is missing: build it with `python -m cwick_amd.build`" % CALLS_PATH)
+        spec = importlib.util.spec_from_file_location("_cwick_calls", CALLS_PATH)
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        _c = types.SimpleNamespace(**{name: m.bind(name, C.cast(getattr(L, "cwick_hip_" + name), _vp).value)
+                                      for name in m.names()})
+    return _c
+
+
 def last_error():
     return lib().cwick_hip_last_error().decode("utf-8", "replace")
 
@@ -186,15 +208,15 @@ class KVCache:
             raise Declined("kv_create: " + last_error())
 
     def write(self, pos0, k_rows, v_rows):
-        k, kp = _np(k_rows, np.uint16)
-        v, vp = _np(v_rows, np.uint16)
+        k = np.ascontiguousarray(k_rows, np.uint16)
+        v = np.ascontiguousarray(v_rows, np.uint16)
         n = k.shape[0]
-        _check(lib().cwick_hip_kv_write(self.h, pos0, n, kp, vp), "kv_write")
+        _check(_calls().kv_write(self.h, pos0, n, k, v), "kv_write")
 
     def write_f32(self, pos0, k_rows, v_rows):
-        k, kp = _np(k_rows, np.float32)
-        v, vp = _np(v_rows, np.float32)
-        _check(lib().cwick_hip_kv_write_f32(self.h, pos0, k.shape[0], kp, vp), "kv_write_f32")
+        k = np.ascontiguousarray(k_rows, np.float32)
+        v = np.ascontiguousarray(v_rows, np.float32)
+        _check(_calls().kv_write_f32(self.h, pos0, k.shape[0], k, v), "kv_write_f32")
 
     def read(self, pos0, n):
         row = self.n_kv_heads * self.head_dim
@@ -234,15 +256,15 @@ class LatentCache:
             raise Declined("latent_create: " + last_error())
 
     def write(self, slot, pos0, rows, scales):
-        r, rp = _np(rows, np.uint8)
-        s, sp = _np(scales, np.float32)
+        r = np.ascontiguousarray(rows, np.uint8)
+        s = np.ascontiguousarray(scales, np.float32)
         assert r.shape[1] == KDIM and s.shape == (r.shape[0], NBLK)
-        _check(lib().cwick_hip_latent_write(self.h, slot, pos0, r.shape[0], rp, sp), "latent_write")
+        _check(_calls().latent_write(self.h, slot, pos0, r.shape[0], r, s), "latent_write")
 
     def write_f32(self, slot, pos0, rows):
-        r, rp = _np(rows, np.float32)
+        r = np.ascontiguousarray(rows, np.float32)
         assert r.shape[1] == KDIM
-        _check(lib().cwick_hip_latent_write_f32(self.h, slot, pos0, r.shape[0], rp),
+        _check(_calls().latent_write_f32(self.h, slot, pos0, r.shape[0], r),
                "latent_write_f32")
 
     def read(self, slot, pos0, n):
@@ -281,14 +303,14 @@ class IndexKeys:
             raise Declined("ikeys_create: " + last_error())
 
     def write(self, slot, pos0, rows, scales):
-        r, rp = _np(rows, np.uint8)
-        s, sp = _np(scales, np.float32)
+        r = np.ascontiguousarray(rows, np.uint8)
+        s = np.ascontiguousarray(scales, np.float32)
         assert r.shape[1] == IDIM and s.size == r.shape[0]
-        _check(lib().cwick_hip_ikeys_write(self.h, slot, pos0, r.shape[0], rp, sp), "ikeys_write")
+        _check(_calls().ikeys_write(self.h, slot, pos0, r.shape[0], r, s), "ikeys_write")
 
     def write_f32(self, slot, pos0, rows):
-        r, rp = _np(rows, np.float32)
-        _check(lib().cwick_hip_ikeys_write_f32(self.h, slot, pos0, r.shape[0], rp),
+        r = np.ascontiguousarray(rows, np.float32)
+        _check(_calls().ikeys_write_f32(self.h, slot, pos0, r.shape[0], r),
                "ikeys_write_f32")
 
     def read(self, slot, pos0, n):
@@ -326,10 +348,10 @@ class IndexKeys:
 
 # ------------------------------------------------------------------ host-pointer ops
 def gqa_decode(cache, n_keys, q, scale, raw=False):
-    q, qp = _np(q, np.uint16)
+    q = np.ascontiguousarray(q, np.uint16)
     nh, hd = q.shape
     out = np.empty((nh, hd), np.float32)
-    rc = lib().cwick_hip_gqa_decode(cache.h, n_keys, qp, nh, scale, out.ctypes.data)
+    rc = _calls().gqa_decode(cache.h, n_keys, q, nh, scale, out)
     if raw:
         return rc, out
     _check(rc, "gqa_decode")
@@ -337,11 +359,11 @@ def gqa_decode(cache, n_keys, q, scale, raw=False):
 
 
 def gqa_decode_sel(cache, sel, q, scale, raw=False):
-    q, qp = _np(q, np.uint16)
-    sel, sp = _np(sel, np.int32)
+    q = np.ascontiguousarray(q, np.uint16)
+    sel = np.ascontiguousarray(sel, np.int32)
     nh, hd = q.shape
     out = np.empty((nh, hd), np.float32)
-    rc = lib().cwick_hip_gqa_decode_sel(cache.h, sp, sel.size, qp, nh, scale, out.ctypes.data)
+    rc = _calls().gqa_decode_sel(cache.h, sel, sel.size, q, nh, scale, out)
     if raw:
         return rc, out
     _check(rc, "gqa_decode_sel")
@@ -349,15 +371,15 @@ def gqa_decode_sel(cache, sel, q, scale, raw=False):
 
 
 def gqa_decode_sel_dev(k, v, n_rows, n_kv_heads, head_dim, sel, n_list, q, n_heads, scale, out, stream=None):
-    return _check(lib().cwick_hip_gqa_decode_sel_dev(_dp(k), _dp(v), n_rows, n_kv_heads, head_dim, _dp(sel), n_list,
-                                                     _dp(q), n_heads, scale, _dp(out), stream), "gqa_decode_sel_dev")
+    return _check(_calls().gqa_decode_sel_dev(k, v, n_rows, n_kv_heads, head_dim, sel, n_list, q, n_heads, scale,
+                                              out, stream), "gqa_decode_sel_dev")
 
 
 def gqa_prefill(cache, pos0, q, scale, raw=False):
-    q, qp = _np(q, np.uint16)
+    q = np.ascontiguousarray(q, np.uint16)
     n, nh, hd = q.shape
     out = np.empty((n, nh, hd), np.float32)
-    rc = lib().cwick_hip_gqa_prefill(cache.h, pos0, n, qp, nh, scale, out.ctypes.data)
+    rc = _calls().gqa_prefill(cache.h, pos0, n, q, nh, scale, out)
     if raw:
         return rc, out
     _check(rc, "gqa_prefill")
@@ -365,21 +387,19 @@ def gqa_prefill(cache, pos0, q, scale, raw=False):
 
 
 def mla_decode(cache, slot, q, scale, sel=None, n_list=None, raw=False, sink=None):
-    q, qp = _np(q, np.uint16)
+    q = np.ascontiguousarray(q, np.uint16)
     nh = q.shape[0]
     assert q.shape[1] == KDIM
-    selp = None
     if sel is not None:
-        sel, selp = _np(sel, np.int32)
+        sel = np.ascontiguousarray(sel, np.int32)
         n_list = sel.size if n_list is None else n_list
     out = np.empty((nh, VDIM), np.float32)
     if sink is not None:
-        sink, sinkp = _np(sink, np.float32)
+        sink = np.ascontiguousarray(sink, np.float32)
         assert sink.size == nh
-        rc = lib().cwick_hip_mla_decode_sink(cache.h, slot, selp, n_list, qp, nh, scale, sinkp,
-                                             out.ctypes.data)
+        rc = _calls().mla_decode_sink(cache.h, slot, sel, n_list, q, nh, scale, sink, out)
     else:
-        rc = lib().cwick_hip_mla_decode(cache.h, slot, selp, n_list, qp, nh, scale, out.ctypes.data)
+        rc = _calls().mla_decode(cache.h, slot, sel, n_list, q, nh, scale, out)
     if raw:
         return rc, out
     _check(rc, "mla_decode")
@@ -387,11 +407,11 @@ def mla_decode(cache, slot, q, scale, sel=None, n_list=None, raw=False, sink=Non
 
 
 def mla_prefill_chunk(cache, slot, pos0, q, scale, raw=False):
-    q, qp = _np(q, np.uint16)
+    q = np.ascontiguousarray(q, np.uint16)
     n, nh, kd = q.shape
     assert kd == KDIM
     out = np.empty((n, nh, VDIM), np.float32)
-    rc = lib().cwick_hip_mla_prefill_chunk(cache.h, slot, pos0, n, qp, nh, scale, out.ctypes.data)
+    rc = _calls().mla_prefill_chunk(cache.h, slot, pos0, n, q, nh, scale, out)
     if raw:
         return rc, out
     _check(rc, "mla_prefill_chunk")
@@ -440,15 +460,15 @@ def topk(scores, k, raw=False):
 
 
 def dsa_decode(ikeys, latent, slot0, slot_step, n_keys, q_idx, w, topk_k, q, scale, raw=False):
-    qi, qip = _np(q_idx, np.uint16)
-    w, wp = _np(w, np.float32)
-    q, qp = _np(q, np.uint16)
+    qi = np.ascontiguousarray(q_idx, np.uint16)
+    w = np.ascontiguousarray(w, np.float32)
+    q = np.ascontiguousarray(q, np.uint16)
     batch, ih, _ = qi.shape
     nh = q.shape[1]
     out = np.empty((batch, nh, VDIM), np.float32)
     sel = np.empty((batch, topk_k), np.int32)
-    rc = lib().cwick_hip_dsa_decode(ikeys.h, latent.h, slot0, slot_step, batch, n_keys, qip, wp,
-                                    ih, topk_k, qp, nh, scale, out.ctypes.data, sel.ctypes.data)
+    rc = _calls().dsa_decode(ikeys.h, latent.h, slot0, slot_step, batch, n_keys, qi, w, ih, topk_k, q, nh, scale,
+                             out, sel)
     if raw:
         return rc, out, sel
     _check(rc, "dsa_decode")
@@ -488,84 +508,77 @@ def e4m3_table():
 # Arguments are torch CUDA tensors (or raw device addresses); `stream` is a raw
 # hipStream_t address (torch.cuda.current_stream().cuda_stream) or None.
 def gqa_decode_dev(k, v, n_keys, n_kv_heads, head_dim, q, n_heads, scale, out, stream=None):
-    return _check(lib().cwick_hip_gqa_decode_dev(_dp(k), _dp(v), n_keys, n_kv_heads, head_dim,
-                                                 _dp(q), n_heads, scale, _dp(out), stream),
+    return _check(_calls().gqa_decode_dev(k, v, n_keys, n_kv_heads, head_dim, q, n_heads, scale, out, stream),
                   "gqa_decode_dev")
 
 
 def gqa_prefill_dev(k, v, pos0, n, n_kv_heads, head_dim, q, n_heads, scale, out, stream=None):
-    return _check(lib().cwick_hip_gqa_prefill_dev(_dp(k), _dp(v), pos0, n, n_kv_heads, head_dim,
-                                                  _dp(q), n_heads, scale, _dp(out), stream),
+    return _check(_calls().gqa_prefill_dev(k, v, pos0, n, n_kv_heads, head_dim, q, n_heads, scale, out, stream),
                   "gqa_prefill_dev")
 
 
 def mla_decode_dev(rows, scales, row_bstride, scale_bstride, n_rows, batch, sel, n_list, q,
                    n_heads, scale, out, stream=None, raw=False):
-    rc = lib().cwick_hip_mla_decode_dev(_dp(rows), _dp(scales), row_bstride, scale_bstride, n_rows, batch,
-                                        _dp(sel), n_list, _dp(q), n_heads, scale, _dp(out), stream)
+    rc = _calls().mla_decode_dev(rows, scales, row_bstride, scale_bstride, n_rows, batch, sel, n_list, q,
+                                 n_heads, scale, out, stream)
     return rc if raw else _check(rc, "mla_decode_dev")
 
 
 def mla_decode_static_dev(rows, scales, row_bstride, scale_bstride, n_rows, batch, sel, n_list, q,
                           n_heads, scale, out, stream=None, raw=False):
     """cwick_hip_mla_decode_dev that allocates nothing (fixed scratch inside the library)."""
-    rc = lib().cwick_hip_mla_decode_static_dev(_dp(rows), _dp(scales), row_bstride, scale_bstride,
-                                               n_rows, batch, _dp(sel), n_list, _dp(q), n_heads,
-                                               scale, _dp(out), stream)
+    rc = _calls().mla_decode_static_dev(rows, scales, row_bstride, scale_bstride, n_rows, batch, sel, n_list, q,
+                                        n_heads, scale, out, stream)
     return rc if raw else _check(rc, "mla_decode_static_dev")
 
 
 def mla_prefill_chunk_dev(rows, scales, pos0, n, q, n_heads, scale, out, stream=None):
-    return _check(lib().cwick_hip_mla_prefill_chunk_dev(_dp(rows), _dp(scales), pos0, n, _dp(q),
-                                                        n_heads, scale, _dp(out), stream),
+    return _check(_calls().mla_prefill_chunk_dev(rows, scales, pos0, n, q, n_heads, scale, out, stream),
                   "mla_prefill_chunk_dev")
 
 
 def indexer_scores_dev(keys, kscale, key_bstride, kscale_bstride, batch, n_keys, q_idx, w,
                        n_idx_heads, scores, stream=None):
-    return _check(lib().cwick_hip_indexer_scores_dev(_dp(keys), _dp(kscale), key_bstride,
-                                                     kscale_bstride, batch, n_keys, _dp(q_idx),
-                                                     _dp(w), n_idx_heads, _dp(scores), stream),
+    return _check(_calls().indexer_scores_dev(keys, kscale, key_bstride, kscale_bstride, batch, n_keys, q_idx, w,
+                                              n_idx_heads, scores, stream),
                   "indexer_scores_dev")
 
 
 def topk_dev(scores, batch, n, k, out_idx, stream=None):
-    return _check(lib().cwick_hip_topk_dev(_dp(scores), batch, n, k, _dp(out_idx), stream),
+    return _check(_calls().topk_dev(scores, batch, n, k, out_idx, stream),
                   "topk_dev")
 
 
 def dsa_decode_dev(ikeys, ikscale, key_bstride, kscale_bstride, rows, scales, row_bstride,
                    scale_bstride, batch, n_keys, q_idx, w, n_idx_heads, topk_k, q, n_heads, scale,
                    scores_tmp, sel_out, out, stream=None):
-    return _check(lib().cwick_hip_dsa_decode_dev(
-        _dp(ikeys), _dp(ikscale), key_bstride, kscale_bstride, _dp(rows), _dp(scales),
-        row_bstride, scale_bstride, batch, n_keys, _dp(q_idx), _dp(w), n_idx_heads, topk_k,
-        _dp(q), n_heads, scale, _dp(scores_tmp), _dp(sel_out), _dp(out), stream),
+    return _check(_calls().dsa_decode_dev(ikeys, ikscale, key_bstride, kscale_bstride, rows, scales, row_bstride,
+                                          scale_bstride, batch, n_keys, q_idx, w, n_idx_heads, topk_k, q,
+                                          n_heads, scale, scores_tmp, sel_out, out, stream),
         "dsa_decode_dev")
 
 
 def mla_absorb_dev(kv_b_proj, q, q_bstride, batch, n_heads, q_dim, nope, rope, kv_dim, kv_lora, q_abs,
                    stream=None):
-    return _check(lib().cwick_hip_mla_absorb_dev(_dp(kv_b_proj), _dp(q), q_bstride, batch, n_heads, q_dim,
-                                                 nope, rope, kv_dim, kv_lora, _dp(q_abs), stream),
+    return _check(_calls().mla_absorb_dev(kv_b_proj, q, q_bstride, batch, n_heads, q_dim, nope, rope, kv_dim,
+                                          kv_lora, q_abs, stream),
                   "mla_absorb_dev")
 
 
 def mla_expand_dev(kv_b_proj, c_acc, batch, n_heads, nope, vdim, kv_dim, kv_lora, out, stream=None):
-    return _check(lib().cwick_hip_mla_expand_dev(_dp(kv_b_proj), _dp(c_acc), batch, n_heads, nope, vdim,
-                                                 kv_dim, kv_lora, _dp(out), stream), "mla_expand_dev")
+    return _check(_calls().mla_expand_dev(kv_b_proj, c_acc, batch, n_heads, nope, vdim, kv_dim, kv_lora, out,
+                                          stream), "mla_expand_dev")
 
 
 def gqa_prepare_dev(q_proj, q_head_stride, k_proj, v_proj, n, pos0, n_heads, n_kv_heads, head_dim,
                     q_norm, k_norm, eps, rope_cos, rope_sin, rotary_dim, q_out, cache, stream=None, raw=False):
-    rc = lib().cwick_hip_gqa_prepare_dev(_dp(q_proj), q_head_stride, _dp(k_proj), _dp(v_proj), n, pos0,
-                                         n_heads, n_kv_heads, head_dim, _dp(q_norm), _dp(k_norm), eps,
-                                         _dp(rope_cos), _dp(rope_sin), rotary_dim, _dp(q_out), cache.h, stream)
+    rc = _calls().gqa_prepare_dev(q_proj, q_head_stride, k_proj, v_proj, n, pos0, n_heads, n_kv_heads, head_dim,
+                                  q_norm, k_norm, eps, rope_cos, rope_sin, rotary_dim, q_out, cache.h, stream)
     return rc if raw else _check(rc, "gqa_prepare_dev")
 
 
 def candidate_select_dev(scores, batch, n, block, keep_blocks, cand, stream=None, raw=False):
-    rc = lib().cwick_hip_candidate_select_dev(_dp(scores), batch, n, block, keep_blocks, _dp(cand), stream)
+    rc = _calls().candidate_select_dev(scores, batch, n, block, keep_blocks, cand, stream)
     return rc if raw else _check(rc, "candidate_select_dev")
 
 
@@ -582,9 +595,8 @@ def mm_select(idx_cache, limit, iq, block, keep_blocks, max_sel):
 
 def mm_select_dev(idx_keys, iq, batch, limit0, index_heads, index_dim, block, keep_blocks, scores, score_stride,
                   blk_out, sel, max_sel, n_sel, stream=None, raw=False):
-    rc = lib().cwick_hip_mm_select_dev(_dp(idx_keys), _dp(iq), batch, limit0, index_heads, index_dim, block,
-                                       keep_blocks, _dp(scores), score_stride, _dp(blk_out), _dp(sel), max_sel,
-                                       _dp(n_sel), stream)
+    rc = _calls().mm_select_dev(idx_keys, iq, batch, limit0, index_heads, index_dim, block, keep_blocks, scores,
+                                score_stride, blk_out, sel, max_sel, n_sel, stream)
     return rc if raw else _check(rc, "mm_select_dev")
 
 
@@ -603,13 +615,13 @@ def stream_release(stream, raw=False):
 
 
 def glm_select_dev(scores, batch, n_comp, npos, kpool, topk, strict, sel, max_sel, n_sel, stream=None, raw=False):
-    rc = lib().cwick_hip_glm_select_dev(_dp(scores), batch, n_comp, npos, kpool, topk, 1 if strict else 0, _dp(sel),
-                                        max_sel, _dp(n_sel), stream)
+    rc = _calls().glm_select_dev(scores, batch, n_comp, npos, kpool, topk, 1 if strict else 0, sel, max_sel,
+                                 n_sel, stream)
     return rc if raw else _check(rc, "glm_select_dev")
 
 
 def candidate_apply_dev(scores, cand, batch, n, stream=None):
-    return _check(lib().cwick_hip_candidate_apply_dev(_dp(scores), _dp(cand), batch, n, stream),
+    return _check(_calls().candidate_apply_dev(scores, cand, batch, n, stream),
                   "candidate_apply_dev")
 
 
