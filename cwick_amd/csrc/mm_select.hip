@@ -15,10 +15,10 @@
 //      one thread per position.)
 //   2. block maxima, started from -1e30 like the reference.  The scoring kernel leaves the
 //      maximum of every group of 64 positions; when a block is a whole number of groups (128 in
-//      the reference's configuration) mm_pick_kernel, one workgroup per query, makes the block
-//      maxima from them, selects the `keep` best blocks (the one-workgroup radix select, lowest
-//      index first among equal maxima -- the reference's heap makes that choice on tie-free
-//      input) and writes the list: one launch.  Other block sizes take mm_blockmax_kernel (one
+//      the reference's configuration) mm_pick_few_kernel (up to 2048 blocks, 64 kept) or
+//      mm_pick_kernel, one workgroup per query, makes the block maxima from them, selects the
+//      `keep` best blocks (the radix select in the second, lowest index first among equal maxima --
+//      the reference's heap makes that choice on tie-free input) and writes the list: one launch.  Other block sizes take mm_blockmax_kernel (one
 //      wave per block over the scores; blocks past a query's last one get -inf so that rows of
 //      a chunk with different block counts share one top-k launch), launch_topk and
 //      mm_expand_kernel.
@@ -247,31 +247,15 @@ mm_blockmax_kernel(const float *__restrict__ scores, int64_t score_stride, int64
     if (lane == 0) bsc[(size_t)row * nblk_max + b] = mx;
 }
 
-// The list of one query, by all NT threads of a workgroup: `mine` holds the kb chosen blocks in
-// ascending order, -1 padded.
+// The list of one query, by all NT threads of a workgroup: the first `nv` of `mine` are the chosen blocks in
+// ascending order, the newest block among them (`has`) or not.
 template <int NT>
-__device__ __forceinline__ void mm_expand_row(const int32_t *__restrict__ mine, int kb, int64_t limit, int bs,
-                                              int32_t *__restrict__ blk_out, int32_t *__restrict__ sel, int64_t max_sel,
-                                              int32_t *__restrict__ n_sel) {
-    __shared__ uint32_t sh_nv, sh_has;
+__device__ __forceinline__ void mm_write_row(const int32_t *__restrict__ mine, int nv, bool has, int kb, int64_t limit, int bs,
+                                             int32_t *__restrict__ blk_out, int32_t *__restrict__ sel, int64_t max_sel,
+                                             int32_t *__restrict__ n_sel) {
     const int tid = threadIdx.x;
-    const int64_t nblk = (limit + bs - 1) / bs;
     const int32_t newest = (int32_t)(limit / bs);
-    if (tid == 0) sh_nv = 0, sh_has = 0;
-    __syncthreads();
-    // the chosen blocks come in ascending order, blocks this query does not have (and the -1
-    // padding of a short row) after the ones it has: the valid entries are a prefix
-    for (int j0 = 0; j0 < kb; j0 += NT) {
-        const int j = j0 + tid;
-        const int32_t b = j < kb ? mine[j] : -1;
-        const uint32_t ok = b >= 0 && b < nblk;
-        const uint32_t cnt = wave_sum_u32(ok), has = wave_sum_u32(ok && b == newest);
-        if ((tid & 63) == 0 && cnt) atomicAdd(&sh_nv, cnt);
-        if ((tid & 63) == 0 && has) atomicAdd(&sh_has, has);
-    }
-    __syncthreads();
-    const int nv = (int)sh_nv;
-    const int nb = nv + (sh_has ? 0 : 1);
+    const int nb = nv + (has ? 0 : 1);
     if (blk_out)
         for (int j = tid; j <= kb; j += NT) blk_out[j] = j < nv ? mine[j] : j < nb ? newest : -1;
     // every block of the list but its last is full
@@ -294,6 +278,31 @@ __device__ __forceinline__ void mm_expand_row(const int32_t *__restrict__ mine, 
     }
 }
 
+// The same where `mine` holds kb chosen blocks in ascending order, -1 padded.
+template <int NT>
+__device__ __forceinline__ void mm_expand_row(const int32_t *__restrict__ mine, int kb, int64_t limit, int bs,
+                                              int32_t *__restrict__ blk_out, int32_t *__restrict__ sel, int64_t max_sel,
+                                              int32_t *__restrict__ n_sel) {
+    __shared__ uint32_t sh_nv, sh_has;
+    const int tid = threadIdx.x;
+    const int64_t nblk = (limit + bs - 1) / bs;
+    const int32_t newest = (int32_t)(limit / bs);
+    if (tid == 0) sh_nv = 0, sh_has = 0;
+    __syncthreads();
+    // the chosen blocks come in ascending order, blocks this query does not have (and the -1
+    // padding of a short row) after the ones it has: the valid entries are a prefix
+    for (int j0 = 0; j0 < kb; j0 += NT) {
+        const int j = j0 + tid;
+        const int32_t b = j < kb ? mine[j] : -1;
+        const uint32_t ok = b >= 0 && b < nblk;
+        const uint32_t cnt = wave_sum_u32(ok), has = wave_sum_u32(ok && b == newest);
+        if ((tid & 63) == 0 && cnt) atomicAdd(&sh_nv, cnt);
+        if ((tid & 63) == 0 && has) atomicAdd(&sh_has, has);
+    }
+    __syncthreads();
+    mm_write_row<NT>(mine, (int)sh_nv, sh_has != 0u, kb, limit, bs, blk_out, sel, max_sel, n_sel);
+}
+
 __global__ void __launch_bounds__(MM_THREADS)
 mm_expand_kernel(const int32_t *__restrict__ blk, int kb, int64_t limit0, int bs, int32_t *__restrict__ blk_out,
                  int32_t *__restrict__ sel, int64_t max_sel, int32_t *__restrict__ n_sel) {
@@ -303,7 +312,143 @@ mm_expand_kernel(const int32_t *__restrict__ blk, int kb, int64_t limit0, int bs
                               n_sel ? n_sel + row : nullptr);
 }
 
-// Block maxima, the kept blocks and the list of one query in one workgroup, for blocks that are
+// Block maxima, the kept blocks and the list of one query in one workgroup, for up to 2048 blocks that are a whole
+// number of the scoring kernel's 64-position groups, of which at most 64 are kept.
+//
+// Nothing here but the trip to the group maxima takes long by itself, so what counts is the chain: the radix select
+// has ten barriers of sixteen waves between that trip and the list, this four of eight.  The kk-th largest of 64
+// maxima, each of every 64th block, is a bound that kk blocks reach and few others do, found bit by bit from counts of
+// ballots, by every wave for itself.  Where the blocks that reach it are at most 64 (nearly always) they go
+// into a lane each of the first wave, in order, which finds the threshold in the same way, until as many as are wanted
+// reach it; otherwise it does so on all blocks.  65536 positions in blocks of 128, sixteen kept: 5.2 us by the radix
+// select, 3.5; 131072 in blocks of 64: 5.8, 3.6.  (The first wave alone with a lane for every 64th block: 4.1 and 8.2.)
+constexpr int MM_PICK_THREADS = 512, MM_PICK_WAVES = MM_PICK_THREADS / 64, MM_PICK_KEEP = 64, MM_PICK_BLOCKS = 2048;
+template <int EPT>
+__global__ void __launch_bounds__(MM_PICK_THREADS)
+mm_pick_few_kernel(const float *__restrict__ gmax, int64_t gmax_stride, int64_t limit0, int bs, int kb,
+                   int32_t *__restrict__ blk_out, int32_t *__restrict__ sel, int64_t max_sel, int32_t *__restrict__ n_sel) {
+    __shared__ uint32_t sh_key[MM_PICK_THREADS * EPT], sh_top[MM_PICK_WAVES][64], sh_cand[64];
+    __shared__ int32_t sh_idx[64], sh_blk[MM_PICK_KEEP];
+    __shared__ uint32_t sh_cnt[MM_PICK_WAVES], sh_has;
+    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int limit = (int)(limit0 + row);
+    const int nblk = (limit + bs - 1) / bs, ngrp = (limit + 63) / 64, gpb = bs / 64;
+    const int kk = kb < nblk ? kb : nblk, newest = limit / bs;
+    const float *gm = gmax + (size_t)row * gmax_stride;
+    // element j of this lane is block first + 64 j
+    const int first = wave * (64 * EPT) + lane;
+    float v[EPT];
+#pragma unroll
+    for (int j = 0; j < EPT; j++) v[j] = -1e30f;
+    for (int u = 0; u < gpb; u += 4)                                    // four groups of each block at a time
+#pragma unroll
+        for (int j = 0; j < EPT; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int b = first + 64 * j < nblk ? first + 64 * j : nblk - 1;     // (past the end: the last block's)
+                const int g = b * gpb + (u + i < gpb ? u + i : gpb - 1);
+                v[j] = fmaxf(v[j], gm[g < ngrp ? g : ngrp - 1]);
+            }
+    uint32_t key[EPT], top = 0u;                                        // (no block's key is 0)
+#pragma unroll
+    for (int j = 0; j < EPT; j++) {
+        key[j] = first + 64 * j < nblk ? topk_key(v[j]) : 0u;
+        sh_key[first + 64 * j] = key[j];
+        top = key[j] > top ? key[j] : top;
+    }
+    sh_top[wave][lane] = top;
+    __syncthreads();
+    auto count = [](bool x) { return __builtin_popcountll(__ballot(x)); };
+    auto below = [](uint64_t m) {                                       // lanes below this one in m
+        return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    };
+    // the largest T that at least kk of what `reach` counts reach, or the first found that exactly kk do (`all`)
+    auto threshold = [&](auto reach, bool &all) {
+        uint32_t T = 0u;
+        all = false;
+        for (uint32_t bit = 0x80000000u; bit; bit >>= 1) {
+            const int c = reach(T | bit);
+            if (c >= kk) T |= bit;
+            if (c == kk) {
+                all = true;
+                break;
+            }
+        }
+        return T;
+    };
+    bool all;
+#pragma unroll
+    for (int w = 0; w < MM_PICK_WAVES; w++) top = sh_top[w][lane] > top ? sh_top[w][lane] : top;
+    const uint32_t bound = threshold([&](uint32_t x) { return count(top >= x); }, all);
+    uint64_t in[EPT];
+    int n_in = 0;
+#pragma unroll
+    for (int j = 0; j < EPT; j++) {
+        in[j] = __ballot(key[j] >= bound && key[j]);
+        n_in += __builtin_popcountll(in[j]);
+    }
+    if (lane == 0) sh_cnt[wave] = (uint32_t)n_in;
+    __syncthreads();
+    int at = 0, n_cand = 0;
+#pragma unroll
+    for (int w = 0; w < MM_PICK_WAVES; w++) {
+        if (w < wave) at += (int)sh_cnt[w];
+        n_cand += (int)sh_cnt[w];
+    }
+    if (n_cand <= 64) {                                                 // uniform
+#pragma unroll
+        for (int j = 0; j < EPT; j++) {
+            if (in[j] >> lane & 1) {
+                sh_cand[at + below(in[j])] = key[j];
+                sh_idx[at + below(in[j])] = first + 64 * j;
+            }
+            at += __builtin_popcountll(in[j]);
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+        bool has = false;
+        if (n_cand <= 64) {
+            const uint32_t mine = lane < n_cand ? sh_cand[lane] : 0u;
+            const uint32_t T = threshold([&](uint32_t x) { return count(mine >= x); }, all);
+            // ties at T that do not all fit: the smaller indices win
+            const int r = kk - count(mine > T);
+            const bool tied = mine == T && mine, take = mine && (all ? mine >= T : mine > T || (tied && below(__ballot(tied)) < r));
+            const uint64_t m = __ballot(take);
+            if (take) {
+                const int idx = sh_idx[lane];
+                sh_blk[below(m)] = idx;
+                has = idx == newest;
+            }
+        } else {
+            const int steps = (nblk + 63) / 64;
+            auto over = [&](uint32_t x) {
+                int c = 0;
+                for (int j = 0; j < steps; j++) c += count(sh_key[64 * j + lane] >= x);
+                return c;
+            };
+            const uint32_t T = threshold(over, all);
+            int r = kk - (T == 0xFFFFFFFFu ? 0 : over(T + 1u)), to = 0;
+            for (int j = 0; j < steps; j++) {
+                const uint32_t x = sh_key[64 * j + lane];
+                const bool tied = x == T && x, take = x && (all ? x >= T : x > T || (tied && below(__ballot(tied)) < r));
+                r -= count(tied);
+                const uint64_t m = __ballot(take);
+                if (take) sh_blk[to + below(m)] = 64 * j + lane;
+                to += __builtin_popcountll(m);
+                has = has || (take && 64 * j + lane == newest);
+            }
+        }
+        const uint64_t any = __ballot(has);
+        if (lane == 0) sh_has = any != 0u;
+    }
+    __syncthreads();
+    mm_write_row<MM_PICK_THREADS>(sh_blk, kk, sh_has != 0u, kb, limit, bs, blk_out ? blk_out + (size_t)row * (kb + 1) : nullptr,
+                                  sel + (size_t)row * max_sel, max_sel, n_sel ? n_sel + row : nullptr);
+}
+
+// The same for any number of blocks, of which any number is kept: blocks that are
 // a whole number of the scoring kernel's 64-position groups: a block's maximum is that of its
 // groups (a few KB per query instead of the scores themselves), the selection is the
 // one-workgroup radix select, the list follows.  Three launches less than the general path.
@@ -395,7 +540,10 @@ int launch_mm_select(const uint16_t *idx_keys, const float *iq, int batch, int64
         else
             mm_index_scores_long_kernel<<<sgrid, MM_SCORE_THREADS, 0, s>>>(idx_keys, iq, limit0, index_heads, index_dim,
                                                                        scores, score_stride, gmax, ng_max);
-        if (fused)
+        if (fused && nblk_max <= MM_PICK_BLOCKS && keep_blocks <= MM_PICK_KEEP)
+            (nblk_max <= MM_PICK_THREADS ? mm_pick_few_kernel<1> : mm_pick_few_kernel<MM_PICK_BLOCKS / MM_PICK_THREADS>)<<<dim3(batch), MM_PICK_THREADS, 0, s>>>(
+                gmax, ng_max, limit0, block, keep_blocks, blk_out, sel, max_sel, n_sel);
+        else if (fused)
             mm_pick_kernel<<<dim3(batch), TOPK_THREADS, 0, s>>>(gmax, ng_max, limit0, block, nblk_max, keep_blocks, bsc,
                                                                 blk, blk_out, sel, max_sel, n_sel);
         else

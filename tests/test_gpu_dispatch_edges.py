@@ -452,3 +452,44 @@ def test_mm_select_edges(hip, orc, limit, ih, block, keep):
     want = [p for b in blocks for p in range(b * block, min(limit, (b + 1) * block))]
     have = sel[0].cpu().numpy()
     assert have[have >= 0].tolist() == want[:max_sel]
+
+
+@pytest.mark.parametrize("limit,block,keep,kind", [
+    (1, 64, 16, "random"), (4095, 64, 64, "random"), (4096, 64, 64, "random"), (4097, 64, 65, "random"),     # 64 blocks, 64 and 65 kept
+    (32768, 64, 8, "few levels"), (32769, 64, 8, "few levels"),             # 512 and 513 blocks: eight, thirty-two a lane
+    (131072, 64, 16, "random"), (131073, 64, 16, "random"),                 # 2048 blocks, and one too many for a wave
+    (65536, 256, 16, "ascending"), (65500, 128, 16, "equal"), (9000, 64, 64, "few levels"), (9000, 128, 3, "negative")])
+def test_mm_pick_by_one_wave(hip, orc, limit, block, keep, kind):
+    """A selection of blocks by one wave: as many blocks as lanes, candidates for the threshold that fit its lanes and
+    that do not, ties that do not all fit, and the line to the workgroup's radix select; three queries of growing
+    limits.  The scores are set by one dimension, so that whole blocks agree."""
+    import torch
+    say("[case] mm pick", limit, block, keep, kind)
+    g = synth.rng(91)
+    n, nq = limit + 2, 3
+    nb = (n + block - 1) // block
+    level = {"random": g.standard_normal(nb), "few levels": g.integers(0, 4, nb) - 1.0, "ascending": np.arange(nb) / 64.0 + 1.0,
+             "equal": np.ones(nb), "negative": -np.ones(nb)}[kind]
+    keys = np.zeros((n, 128), np.float32)
+    keys[:, 5] = level.repeat(block)[:n]
+    keys = synth.f32_to_bf16(keys)
+    iq = np.ones((nq, 1, 128), np.float32)
+    d_k, d_q = torch.from_numpy(keys.view(np.int16)).cuda(), torch.from_numpy(iq).cuda()
+    scores = torch.empty((nq, n), dtype=torch.float32, device="cuda")
+    max_sel = (keep + 1) * block
+    sel = torch.empty((nq, max_sel), dtype=torch.int32, device="cuda")
+    blk = torch.empty((nq, keep + 1), dtype=torch.int32, device="cuda")
+    n_sel = torch.empty(nq, dtype=torch.int32, device="cuda")
+    hip.mm_select_dev(d_k, d_q, nq, limit, 1, 128, block, keep, scores, n, blk, sel, max_sel, n_sel,
+                      torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for y in range(nq):
+        lim = limit + y
+        ref = orc.mm_index_scores(iq[y], keys, lim)
+        assert np.array_equal(scores[y, :lim].cpu().numpy(), ref)
+        best = orc.topk_contract(np.array([max(ref[b:b + block].max(), -1e30) for b in range(0, lim, block)], np.float32), keep)
+        blocks = sorted({int(b) for b in best if b >= 0} | {lim // block})
+        assert [b for b in blk[y].tolist() if b >= 0] == blocks, "query %d" % y
+        want = [p for b in blocks for p in range(b * block, min(lim, (b + 1) * block))][:max_sel]
+        have = sel[y].cpu().numpy()
+        assert have[have >= 0].tolist() == want and int(n_sel[y]) == len(want), "query %d" % y
