@@ -14,6 +14,8 @@
 // loop, so results agree to rounding, not bit for bit.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace cwick {
 namespace {
 
@@ -30,19 +32,58 @@ constexpr int PROJ_ROWS = 8;             // 16-byte pieces of the weights per th
 typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
 typedef f32x4 __attribute__((aligned(4))) f32x4_a4;
 
-// workgroup (4 head + block, queries): columns 128 block .. +128 of the 512-wide latent.  Sixteen
+// Sums over the lanes of pairs of values at a time: in each pair one of two lane groups gets the first value's
+// sum and the other the second's, for one swap and one addition.
+// x[i] and x[i + N / 2] -> x[i], lanes 0 .. 31 and 32 .. 63
+template <int N>
+__device__ __forceinline__ void halve32(float (&x)[N]) {
+#pragma unroll
+    for (int i = 0; i < N / 2; i++) {
+        uint32_t a = __builtin_bit_cast(uint32_t, x[i]), b = __builtin_bit_cast(uint32_t, x[i + N / 2]);
+        lanes_swap32(a, b);
+        x[i] = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+    }
+}
+// the same for the rows of sixteen lanes, even and odd
+template <int N>
+__device__ __forceinline__ void halve16(float (&x)[N], int n) {
+#pragma unroll
+    for (int i = 0; i < N / 2; i++)
+        if (i < n / 2) {
+            uint32_t a = __builtin_bit_cast(uint32_t, x[i]), b = __builtin_bit_cast(uint32_t, x[i + n / 2]);
+            lanes_swap16(a, b);
+            x[i] = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+        }
+}
+
+// within the rows: the value of the lane opposite in a group of sixteen, eight (bit 3 or 2 of the lane differs, and
+// the bits below it) or four lanes (bit 1 does)
+template <int WIDTH>
+__device__ __forceinline__ float opposite(float v) {
+    constexpr int CTRL = WIDTH == 4 ? 0x4E : WIDTH == 8 ? 0x141 : 0x140;
+    return __builtin_bit_cast(float, dpp_u32<CTRL, 0xF>(__builtin_bit_cast(uint32_t, v)));
+}
+
+// workgroup (4 head + block, NY queries): columns 128 block .. +128 of the 512-wide latent.  Sixteen
 // lanes read a row's 256 bytes, so the 256 threads hold sixteen rows, PROJ_ROWS times; the sixteen
-// partial sums of a column meet through two lane swaps and, between the waves, in LDS.
+// partial sums of a column meet through lane swaps and, between the waves, in LDS.
+// Bound by the weights for one query (8.4 MB at 64 heads: 3.8 us, 4.3 with the rope dims fetched at the end).  For more of them it is the instructions of the one
+// or two waves that a SIMD has: so a weight is widened once for all NY queries, their values of a row are one read,
+// and the swaps sum two values at a time.  (A query after the other, each with its own sums, and the rope dims
+// fetched at the end: 7.6 us for four queries of 64 heads, 4.8 now; of 128 heads 9.4, 6.5.)
+template <int NY>
 __global__ void __launch_bounds__(256)
 mla_absorb_kernel(const uint16_t *__restrict__ kvb_w, const float *__restrict__ q, int64_t q_stride, int batch,
                   int q_dim, int nope, int rope, int kv_dim, int kv_lora, uint16_t *__restrict__ out) {
-    constexpr int COLS = CWICK_HIP_LATENT_VDIM / PROJ_SPLIT, ROWS = 16;
+    constexpr int COLS = CWICK_HIP_LATENT_VDIM / PROJ_SPLIT, ROWS = 16, STEP = ROWS * PROJ_ROWS;
     static_assert(COLS == 16 * 8, "sixteen lanes of eight columns");
+    static_assert(STEP == 128 && CWICK_HIP_LATENT_KDIM - CWICK_HIP_LATENT_VDIM == 64 && NY <= 4, "rows and rope dims by the thread");
+    typedef float vec __attribute__((ext_vector_type(NY)));
     const int h = blockIdx.x / PROJ_SPLIT, blk = blockIdx.x % PROJ_SPLIT, nh = gridDim.x / PROJ_SPLIT;
-    const int y0 = blockIdx.y * PROJ_QUERIES, ny = batch - y0 < PROJ_QUERIES ? batch - y0 : PROJ_QUERIES;
+    const int y0 = blockIdx.y * PROJ_QUERIES, ny = batch - y0 < NY ? batch - y0 : NY;
     const int tid = threadIdx.x, c8 = tid & 15, rg = tid >> 4;
-    __shared__ float qs[PROJ_QUERIES][512];
-    __shared__ __attribute__((aligned(16))) float part[PROJ_QUERIES][4][COLS];
+    __shared__ __attribute__((aligned(16))) float qs[512][NY];
+    __shared__ __attribute__((aligned(16))) float part[NY][4][COLS];
     const uint16_t *wk = kvb_w + (size_t)h * kv_dim * kv_lora + blk * COLS + c8 * 8;
     u32x4 w[PROJ_ROWS];
 #pragma unroll
@@ -50,104 +91,136 @@ mla_absorb_kernel(const uint16_t *__restrict__ kvb_w, const float *__restrict__ 
         const int r = rg + ROWS * j;
         w[j] = *(const u32x4_a4 *)(wk + (size_t)(r < nope ? r : 0) * kv_lora);     // nope >= 1 (the launcher)
     }
-    // rows past `nope` meet a zero
-    const int qn = (nope + ROWS * PROJ_ROWS - 1) / (ROWS * PROJ_ROWS) * (ROWS * PROJ_ROWS);
-    for (int y = 0; y < ny; y++)
-        for (int i = tid; i < qn; i += 256)
-            qs[y][i] = i < nope ? q[(size_t)(y0 + y) * q_stride + (size_t)h * q_dim + i] : 0.0f;
+    // the rope dims of the query pass through (zero when the model has none): wave y has query y's
+    const float *qh = q + (size_t)y0 * q_stride + (size_t)h * q_dim;
+    const int yr = tid >> 6, ir = tid & 63;
+    float x_rope = 0.0f;
+    if (blk == 0 && yr < ny && ir < rope) x_rope = qh[(size_t)yr * q_stride + nope + ir];
+    // rows past `nope` and queries past the batch meet a zero
+    for (int i = tid & 127; i < nope + STEP - 1; i += STEP)
+#pragma unroll
+        for (int k = 0; k < (NY + 1) / 2; k++) {
+            const int y = (tid >> 7) + 2 * k;
+            if (i < 512 && y < NY) qs[i][y] = i < nope && y < ny ? qh[(size_t)y * q_stride + i] : 0.0f;
+        }
     __syncthreads();
-    for (int y = 0; y < ny; y++) {
-        float a[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        for (int r0 = 0; r0 < nope; r0 += ROWS * PROJ_ROWS) {
-            u32x4 wr[PROJ_ROWS];
+    float a[NY * 8];                                                // [query][column]
+#pragma unroll
+    for (int i = 0; i < NY * 8; i++) a[i] = 0.0f;
+    for (int r0 = 0; r0 < nope; r0 += STEP) {
+        if (r0)
 #pragma unroll
             for (int j = 0; j < PROJ_ROWS; j++) {
                 const int r = r0 + rg + ROWS * j;
-                wr[j] = r0 == 0 ? w[j] : *(const u32x4_a4 *)(wk + (size_t)(r < nope ? r : 0) * kv_lora);
+                w[j] = *(const u32x4_a4 *)(wk + (size_t)(r < nope ? r : 0) * kv_lora);
             }
 #pragma unroll
-            for (int j = 0; j < PROJ_ROWS; j++) {
-                const float x = qs[y][r0 + rg + ROWS * j];
+        for (int j = 0; j < PROJ_ROWS; j++) {
+            const vec x = *(const vec *)qs[r0 + rg + ROWS * j];
 #pragma unroll
-                for (int d = 0; d < 4; d++) {
-                    a[2 * d] = __builtin_fmaf(x, bf16lo_to_f32(wr[j][d]), a[2 * d]);
-                    a[2 * d + 1] = __builtin_fmaf(x, bf16hi_to_f32(wr[j][d]), a[2 * d + 1]);
+            for (int d = 0; d < 4; d++) {
+                const float lo = bf16lo_to_f32(w[j][d]), hi = bf16hi_to_f32(w[j][d]);
+#pragma unroll
+                for (int y = 0; y < NY; y++) {
+                    a[8 * y + 2 * d] = __builtin_fmaf(x[y], lo, a[8 * y + 2 * d]);
+                    a[8 * y + 2 * d + 1] = __builtin_fmaf(x[y], hi, a[8 * y + 2 * d + 1]);
                 }
             }
         }
+    }
+    // row g of sixteen lanes ends with the eight columns of query g (of two queries: g / 2, of one: every row)
+    if (NY > 1) halve32(a);
+    if (NY > 2) halve16(a, NY * 4);
 #pragma unroll
-        for (int d = 0; d < 8; d++) a[d] = xor32_sum(xor16_sum(a[d]));
-        if ((tid & 63) < 16) {
-            float *dst = &part[y][tid >> 6][c8 * 8];
-            *(f32x4 *)dst = (f32x4){a[0], a[1], a[2], a[3]};
-            *(f32x4 *)(dst + 4) = (f32x4){a[4], a[5], a[6], a[7]};
-        }
+    for (int d = 0; d < 8; d++) {
+        if (NY == 1) a[d] = xor32_sum(a[d]);
+        if (NY <= 2) a[d] = xor16_sum(a[d]);
+    }
+    const int g = (tid & 63) >> 4;
+    if (NY == 4 || (g & (NY == 2 ? 1 : 3)) == 0) {
+        float *dst = &part[NY == 4 ? g : NY == 2 ? g >> 1 : 0][tid >> 6][c8 * 8];
+        *(f32x4 *)dst = (f32x4){a[0], a[1], a[2], a[3]};
+        *(f32x4 *)(dst + 4) = (f32x4){a[4], a[5], a[6], a[7]};
     }
     __syncthreads();
+    uint16_t *o = out + ((size_t)y0 * nh + h) * CWICK_HIP_LATENT_KDIM;
+    const size_t o_query = (size_t)nh * CWICK_HIP_LATENT_KDIM;
     for (int i = tid; i < ny * COLS / 2; i += 256) {
         const int y = i / (COLS / 2), c = i % (COLS / 2) * 2;
         f32x2 t = *(const f32x2 *)&part[y][0][c];
 #pragma unroll
         for (int v = 1; v < 4; v++) {
-            const f32x2 o = *(const f32x2 *)&part[y][v][c];
-            t[0] += o[0], t[1] += o[1];
+            const f32x2 x = *(const f32x2 *)&part[y][v][c];
+            t[0] += x[0], t[1] += x[1];
         }
-        *(uint32_t *)(out + ((size_t)(y0 + y) * nh + h) * CWICK_HIP_LATENT_KDIM + blk * COLS + c) = pack_bf16_rne(t[0], t[1]);
+        *(uint32_t *)(o + y * o_query + blk * COLS + c) = pack_bf16_rne(t[0], t[1]);
     }
-    // the rope dims of the query pass through (zero when the model has none)
-    if (blk == 0)
-        for (int y = 0; y < ny; y++)
-            for (int i = tid; i < CWICK_HIP_LATENT_KDIM - kv_lora; i += 256)
-                out[((size_t)(y0 + y) * nh + h) * CWICK_HIP_LATENT_KDIM + kv_lora + i] = (uint16_t)f32_to_bf16_rne(
-                    i < rope ? q[(size_t)(y0 + y) * q_stride + (size_t)h * q_dim + nope + i] : 0.0f);
+    if (blk == 0 && yr < ny) o[yr * o_query + kv_lora + ir] = (uint16_t)f32_to_bf16_rne(x_rope);
 }
 
-// workgroup (4 head + block, queries): the rows of W_v with (row / 8) % 16 = 4 block + wave.  A lane
-// reads eight bf16 of a row (16 bytes, a wave the row's KiB) and keeps the matching eight floats of
-// c_acc; the eight dots of a wave are summed over the lanes together.
+// workgroup (4 head + block, NY queries): the rows of W_v with (row / 8) % 16 = 4 block + wave.  A lane
+// reads eight bf16 of a row (16 bytes, a wave the row's KiB) and keeps the matching eight floats of the
+// queries' c_acc; the 8 NY dots of a wave are summed over the lanes two at a time, so that every lane ends with one.
+// (Each query by itself, its sums in all lanes: 6.0 us for four queries of 64 heads, 3.9 now; one query 3.8, 3.4.)
+template <int NY>
 __global__ void __launch_bounds__(256)
 mla_expand_kernel(const uint16_t *__restrict__ kvb_w, const float *__restrict__ c_acc, int batch, int nope, int vdim,
                   int kv_dim, int kv_lora, float *__restrict__ out) {
-    static_assert(CWICK_HIP_LATENT_VDIM == 64 * 8, "a wave's lanes cover a row");
+    static_assert(CWICK_HIP_LATENT_VDIM == 64 * 8 && PROJ_ROWS == 8, "a wave's lanes cover a row");
     const int h = blockIdx.x / PROJ_SPLIT, blk = blockIdx.x % PROJ_SPLIT, nh = gridDim.x / PROJ_SPLIT;
-    const int y0 = blockIdx.y * PROJ_QUERIES, ny = batch - y0 < PROJ_QUERIES ? batch - y0 : PROJ_QUERIES;
+    const int y0 = blockIdx.y * PROJ_QUERIES, ny = batch - y0 < NY ? batch - y0 : NY;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint16_t *wv = kvb_w + ((size_t)h * kv_dim + nope) * kv_lora + 8 * lane;
+    f32x4 c[NY][2];
+#pragma unroll
+    for (int y = 0; y < NY; y++) {
+        const float *p = c_acc + ((size_t)(y0 + (y < ny ? y : 0)) * nh + h) * kv_lora + 8 * lane;
+        c[y][0] = *(const f32x4_a4 *)p, c[y][1] = *(const f32x4_a4 *)(p + 4);
+    }
     for (int r0 = (blk * 4 + wave) * PROJ_ROWS; r0 < vdim; r0 += PROJ_SPLIT * 4 * PROJ_ROWS) {
         u32x4 w[PROJ_ROWS];
 #pragma unroll
         for (int j = 0; j < PROJ_ROWS; j++)
             w[j] = *(const u32x4_a4 *)(wv + (size_t)(r0 + j < vdim ? r0 + j : 0) * kv_lora);
-        for (int y = 0; y < ny; y++) {
-            const float *c = c_acc + ((size_t)(y0 + y) * nh + h) * kv_lora + 8 * lane;
-            const f32x4 c0 = *(const f32x4_a4 *)c, c1 = *(const f32x4_a4 *)(c + 4);
-            float s[PROJ_ROWS];
+        float s[NY * 8];                                            // [query][row]
 #pragma unroll
-            for (int j = 0; j < PROJ_ROWS; j++) {
-                float t = bf16lo_to_f32(w[j][0]) * c0[0];
-                t = __builtin_fmaf(bf16hi_to_f32(w[j][0]), c0[1], t);
-                t = __builtin_fmaf(bf16lo_to_f32(w[j][1]), c0[2], t);
-                t = __builtin_fmaf(bf16hi_to_f32(w[j][1]), c0[3], t);
-                t = __builtin_fmaf(bf16lo_to_f32(w[j][2]), c1[0], t);
-                t = __builtin_fmaf(bf16hi_to_f32(w[j][2]), c1[1], t);
-                t = __builtin_fmaf(bf16lo_to_f32(w[j][3]), c1[2], t);
-                s[j] = __builtin_fmaf(bf16hi_to_f32(w[j][3]), c1[3], t);
+        for (int j = 0; j < PROJ_ROWS; j++) {
+            float e[8];
+#pragma unroll
+            for (int d = 0; d < 4; d++) e[2 * d] = bf16lo_to_f32(w[j][d]), e[2 * d + 1] = bf16hi_to_f32(w[j][d]);
+#pragma unroll
+            for (int y = 0; y < NY; y++) {
+                float t = e[0] * c[y][0][0];
+#pragma unroll
+                for (int d = 1; d < 8; d++) t = __builtin_fmaf(e[d], c[y][d >> 2][d & 3], t);
+                s[8 * y + j] = t;
             }
-#pragma unroll
-            for (int j = 0; j < PROJ_ROWS; j++) s[j] = group_step_sum<2>(s[j]);
-#pragma unroll
-            for (int j = 0; j < PROJ_ROWS; j++) s[j] = group_step_sum<4>(s[j]);
-#pragma unroll
-            for (int j = 0; j < PROJ_ROWS; j++) s[j] = group_step_sum<8>(s[j]);
-#pragma unroll
-            for (int j = 0; j < PROJ_ROWS; j++) s[j] = group_step_sum<16>(s[j]);
-#pragma unroll
-            for (int j = 0; j < PROJ_ROWS; j++) s[j] = xor32_sum(xor16_sum(s[j]));
-            float t = s[0];
-#pragma unroll
-            for (int j = 1; j < PROJ_ROWS; j++) t = lane == j ? s[j] : t;
-            if (lane < PROJ_ROWS && r0 + lane < vdim) out[((size_t)(y0 + y) * nh + h) * vdim + r0 + lane] = t;
         }
+        // Lane bits 5, 4, 3, 2, 1 (as many as there are halvings) pick the value that the lane ends with, the first one
+        // the upper half of the list; what is left of the lanes adds up the same value.
+        halve32(s);
+        halve16(s, NY * 4);
+        constexpr int LEFT = NY * 2;                                // values a lane has now
+        auto halve = [&](auto width, int n) {
+            constexpr int W = decltype(width)::value;
+            const bool upper = lane & (W / 2);                      // (the lanes of a group that differ in lower bits hold the same values)
+#pragma unroll
+            for (int i = 0; i < LEFT / 2; i++)
+                if (i < n / 2) {
+                    const float keep = upper ? s[i + n / 2] : s[i], give = upper ? s[i] : s[i + n / 2];
+                    s[i] = keep + opposite<W>(give);
+                }
+        };
+        if (LEFT == 8) halve(std::integral_constant<int, 16>{}, 8);
+        if (LEFT >= 4) halve(std::integral_constant<int, LEFT == 8 ? 8 : 16>{}, 4);
+        halve(std::integral_constant<int, LEFT == 8 ? 4 : LEFT == 4 ? 8 : 16>{}, 2);
+        float t = s[0];
+        if (LEFT <= 2) t = group_step_sum<8>(group_step_sum<4>(group_step_sum<2>(t)));
+        else if (LEFT == 4) t = group_step_sum<4>(group_step_sum<2>(t));
+        else t = group_step_sum<2>(t);
+        const int bits = NY == 4 ? lane >> 1 : NY == 2 ? lane >> 2 : lane >> 3, y = bits >> 3, j = bits & 7;
+        const bool first = (lane & (NY == 4 ? 1 : NY == 2 ? 3 : 7)) == 0;
+        if (first && y < ny && r0 + j < vdim) out[((size_t)(y0 + y) * nh + h) * vdim + r0 + j] = t;
     }
 }
 
@@ -304,7 +377,8 @@ int launch_mla_absorb(const uint16_t *kvb_w, const float *q, int64_t q_stride, i
                       nope + rope <= 512 && nope <= kv_dim,
                   "mla_absorb: nope %d rope %d q_dim %d kv_dim %d", nope, rope, q_dim, kv_dim);
     CWICK_REQUIRE((uintptr_t)kvb_w % 4 == 0 && (uintptr_t)q_abs % 4 == 0, "mla_absorb: operands must be 4-byte aligned");
-    mla_absorb_kernel<<<dim3(n_heads * PROJ_SPLIT, (batch + PROJ_QUERIES - 1) / PROJ_QUERIES), 256, 0, s>>>(
+    (batch == 1 ? mla_absorb_kernel<1> : batch == 2 ? mla_absorb_kernel<2> : mla_absorb_kernel<PROJ_QUERIES>)<<<
+        dim3(n_heads * PROJ_SPLIT, (batch + PROJ_QUERIES - 1) / PROJ_QUERIES), 256, 0, s>>>(
         kvb_w, q, q_stride, batch, q_dim, nope, rope, kv_dim, kv_lora, q_abs);
     CWICK_HIP_CALL(hipGetLastError());
     return 1;
@@ -318,7 +392,8 @@ int launch_mla_expand(const uint16_t *kvb_w, const float *c_acc, int batch, int 
     CWICK_REQUIRE(kv_lora == CWICK_HIP_LATENT_VDIM, "mla_expand: kv_lora %d (the latent cache holds 512)", kv_lora);
     CWICK_REQUIRE(vdim >= 1 && nope >= 0 && nope + vdim <= kv_dim, "mla_expand: nope %d vdim %d kv_dim %d", nope, vdim, kv_dim);
     CWICK_REQUIRE((uintptr_t)kvb_w % 16 == 0, "mla_expand: kv_b_proj must be 16-byte aligned");
-    mla_expand_kernel<<<dim3(n_heads * PROJ_SPLIT, (batch + PROJ_QUERIES - 1) / PROJ_QUERIES), 256, 0, s>>>(
+    (batch == 1 ? mla_expand_kernel<1> : batch == 2 ? mla_expand_kernel<2> : mla_expand_kernel<PROJ_QUERIES>)<<<
+        dim3(n_heads * PROJ_SPLIT, (batch + PROJ_QUERIES - 1) / PROJ_QUERIES), 256, 0, s>>>(
         kvb_w, c_acc, batch, nope, vdim, kv_dim, kv_lora, out);
     CWICK_HIP_CALL(hipGetLastError());
     return 1;

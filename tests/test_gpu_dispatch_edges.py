@@ -14,7 +14,8 @@ def say(*a):
 
 
 @pytest.mark.parametrize("nh,batch,nope,rope,vdim", [(1, 1, 1, 0, 1), (3, 4, 127, 64, 31), (2, 5, 128, 64, 128),
-                                                      (5, 3, 129, 8, 130), (2, 9, 300, 64, 192)])
+                                                      (5, 3, 129, 8, 130), (2, 9, 300, 64, 192),
+                                                      (4, 2, 512, 0, 65), (3, 2, 64, 17, 9), (2, 6, 448, 64, 8)])
 def test_absorb_expand_edges(hip, orc, nh, batch, nope, rope, vdim):
     """Row counts around the 128 that a workgroup holds at a time, batches around its four queries."""
     import torch
