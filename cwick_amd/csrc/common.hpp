@@ -391,6 +391,17 @@ __device__ __forceinline__ float group_step_sum(float v) {
     constexpr int CTRL = WIDTH == 2 ? 0xB1 : WIDTH == 4 ? 0x4E : WIDTH == 8 ? 0x141 : 0x140;
     return v + __builtin_bit_cast(float, dpp_u32<CTRL, 0xF>(__builtin_bit_cast(uint32_t, v)));
 }
+// the maximum over each row of sixteen lanes
+__device__ __forceinline__ float row_max(float v) {
+#define CWICK_ROW_MAX(ctrl)                                                                                   \
+    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, false)))
+    CWICK_ROW_MAX(0xB1);     // quad_perm [1, 0, 3, 2]
+    CWICK_ROW_MAX(0x4E);     // quad_perm [2, 3, 0, 1]
+    CWICK_ROW_MAX(0x141);    // row_half_mirror
+    CWICK_ROW_MAX(0x140);    // row_mirror
+#undef CWICK_ROW_MAX
+    return v;
+}
 // the maximum over the wave in every lane
 __device__ __forceinline__ float wave_max(float v) {
 #define CWICK_DPP_MAX(ctrl)                                                                                   \

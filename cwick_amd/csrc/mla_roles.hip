@@ -63,6 +63,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 namespace cwick {
 namespace {
@@ -740,31 +741,36 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
 // loads in flight at once (eight splits per batch); which splits exist is uniform per wave, so
 // absent ones cost nothing.
 constexpr int MW = 16;
+// (the kernel goes by these too: an argument behind the first fourteen dwords, or the launch's own sizes, would be a
+// trip to memory in front of the first load)
+__host__ __device__ inline bool merge_packed(int n_splits) { return n_splits <= 8; }
+__host__ __device__ inline int merge_waves(int n_splits) { return n_splits <= 64 ? 8 : MW; }
 __device__ __forceinline__ f32x4 part_value(const u32x2 a) {
     return (f32x4){(float)((int32_t)(a[0] << 16) >> 16), (float)((int32_t)a[0] >> 16),
                    (float)((int32_t)(a[1] << 16) >> 16), (float)((int32_t)a[1] >> 16)};
 }
 __device__ __forceinline__ f32x4 part_value(const f32x4 a) { return a; }
-template <class PART>
-__device__ __forceinline__ void merge_add(f32x4 &acc, float &ls, const PART a, const f32x4 v, const float mx) {
-    const float c = v[0] == -INFINITY ? 0.0f : __expf(v[0] - mx);
-    ls = __builtin_fmaf(v[1], c, ls);
-    const float cs = c * v[2];
-    const f32x4 x = part_value(a);
-#pragma unroll
-    for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(x[r], cs, acc[r]);
+// what each row of sixteen lanes holds, in all of them
+__device__ __forceinline__ void rows_to_all(float x, float (&out)[4]) {
+    uint32_t a = __builtin_bit_cast(uint32_t, x), b = a;
+    lanes_swap32(a, b);                                 // a: rows 0, 1, 0, 1; b: rows 2, 3, 2, 3
+    uint32_t c = a, d = b;
+    lanes_swap16(a, c);
+    lanes_swap16(b, d);
+    out[0] = __builtin_bit_cast(float, a), out[1] = __builtin_bit_cast(float, c);
+    out[2] = __builtin_bit_cast(float, b), out[3] = __builtin_bit_cast(float, d);
 }
 template <class PART>                             // u32x2: four 16-bit values; f32x4
 __device__ __forceinline__ void
 merge_frag(const PART *__restrict__ part_acc, const float *__restrict__ part_ml, int n_splits, int n_hb16, int nhb,
-           uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out, int packed) {
+           uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out) {
     __shared__ float red_m[MW][64];
     __shared__ float red_l[MW][64];
     __shared__ f32x4 red_a[MW][64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), y = blockIdx.y;
     int wv, mw, db, hb;
-    if (packed) {
+    if (merge_packed(n_splits)) {
         // up to eight splits: a wave merges a dim block by itself, and the workgroup's eight
         // waves take the eight dim blocks of one quarter
         wv = 0, mw = 1, db = 8 * (int)(blockIdx.x & 3) + wave, hb = (int)(blockIdx.x >> 2);
@@ -773,7 +779,7 @@ merge_frag(const PART *__restrict__ part_acc, const float *__restrict__ part_ml,
         // [head][4] floats sit on one XCD, so that only one L2 fetches them (with an odd number of
         // row blocks on two)
         const int b = (int)blockIdx.x, grp = n_hb16 & 1 ? (b & 3) + 4 * (b >> 5) : (b & 7) + 8 * (b >> 6);
-        wv = wave, mw = (int)blockDim.x >> 6;
+        wv = wave, mw = merge_waves(n_splits);
         db = 8 * (grp & 3) + ((n_hb16 & 1 ? b >> 2 : b >> 3) & 7), hb = grp >> 2;
     }
     const int n = lane & 15, g = lane >> 4;
@@ -783,49 +789,70 @@ merge_frag(const PART *__restrict__ part_acc, const float *__restrict__ part_ml,
     const PART *pa = part_acc + ((sb * n_hb16 + hb) * NDB + db) * 64 + lane;
     const size_t pa_stride = (size_t)n_hb16 * NDB * 64;
 
-    // first batch: everything in flight before anything is waited for
+    // Four slices come with one load of [head][4] floats, a row of sixteen lanes for each (a load of the same
+    // sixteen heads for all four rows takes the memory pipeline as long), and what the values are weighted by goes to
+    // the other rows by swaps.  48 slices of 64 heads: 4.0 us with a load for each slice, 3.5 so.
     PART a0[8];
-    f32x4 v0[8];
+    f32x4 v0[2];
+    auto fetch = [&](int s0, auto count) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int s = wv + mw * j;
-        v0[j] = (f32x4){-INFINITY, 0.0f, 0.0f, 0.0f};
-        a0[j] = PART{};
-        if (s < n_splits) {
-            v0[j] = *(const f32x4 *)(ml + s * ml_stride);
-            a0[j] = pa[s * pa_stride];
+        for (int i = 0; i < decltype(count)::value / 4; i++) {
+            const int s = s0 + mw * (4 * i + g);
+            v0[i] = *(const f32x4 *)(ml + (s < n_splits ? s : n_splits - 1) * ml_stride);
         }
-    }
-    float mx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < 8; j++) mx = fmaxf(mx, v0[j][0]);
-    for (int s = wv + 8 * mw; s < n_splits; s += mw) mx = fmaxf(mx, ml[s * ml_stride]);
-    if (mw > 1) {
-        red_m[wv][lane] = mx;
-        __syncthreads();
-        for (int w = 0; w < mw; w++) mx = fmaxf(mx, red_m[w][lane]);
-    }
-
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    float ls = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) merge_add(acc, ls, a0[j], v0[j], mx);
-    for (int s0 = wv + 8 * mw; s0 < n_splits; s0 += 8 * mw) {
-        PART a[8];
-        f32x4 v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
+        for (int j = 0; j < decltype(count)::value; j++) {
             const int s = s0 + mw * j;
-            v[j] = (f32x4){-INFINITY, 0.0f, 0.0f, 0.0f};
-            a[j] = PART{};
-            if (s < n_splits) {
-                v[j] = *(const f32x4 *)(ml + s * ml_stride);
-                a[j] = pa[s * pa_stride];
+            a0[j] = pa[(s < n_splits ? s : n_splits - 1) * pa_stride];
+        }
+#pragma unroll
+        for (int i = 0; i < decltype(count)::value / 4; i++)
+            if (s0 + mw * (4 * i + g) >= n_splits) v0[i] = (f32x4){-INFINITY, 0.0f, 0.0f, 0.0f};
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float ls = 0.f, mx = -INFINITY;                   // ls: of this row's slices
+    auto add = [&](auto count) {
+#pragma unroll
+        for (int i = 0; i < decltype(count)::value / 4; i++) {
+            const float c = v0[i][0] == -INFINITY ? 0.0f : __expf(v0[i][0] - mx);
+            ls = __builtin_fmaf(v0[i][1], c, ls);
+            float cs[4];
+            rows_to_all(c * v0[i][2], cs);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const f32x4 x = part_value(a0[4 * i + j]);
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(x[r], cs[j], acc[r]);
             }
         }
-#pragma unroll
-        for (int j = 0; j < 8; j++) merge_add(acc, ls, a[j], v[j], mx);
+    };
+    auto meet = [&] {
+        mx = xor32_max(xor16_max(mx));
+        if (mw > 1) {
+            red_m[wv][lane] = mx;
+            __syncthreads();
+            for (int w = 0; w < mw; w++) mx = fmaxf(mx, red_m[w][lane]);
+        }
+    };
+    const std::integral_constant<int, 4> four;
+    const std::integral_constant<int, 8> eight;
+    if (n_splits <= 4 * mw) {
+        fetch(wv, four);
+        mx = v0[0][0];
+        meet();
+        add(four);
+    } else {
+        fetch(wv, eight);
+        mx = fmaxf(v0[0][0], v0[1][0]);
+        for (int s = wv + mw * (8 + g); s < n_splits; s += 4 * mw) mx = fmaxf(mx, ml[s * ml_stride]);
+        meet();
+        add(eight);
+        for (int s0 = wv + 8 * mw; s0 < n_splits; s0 += 8 * mw) {
+            fetch(s0, eight);
+            add(eight);
+        }
     }
+    ls = xor32_sum(xor16_sum(ls));
     float l = ls;
     f32x4 r4 = acc;
     if (mw > 1) {
@@ -855,13 +882,13 @@ merge_frag(const PART *__restrict__ part_acc, const float *__restrict__ part_ml,
 }
 __global__ void __launch_bounds__(64 * MW)
 mla_merge_frag16_kernel(const u32x2 *__restrict__ part_acc, const float *__restrict__ part_ml, int n_splits, int n_hb16,
-                        int nhb, uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out, int packed) {
-    merge_frag(part_acc, part_ml, n_splits, n_hb16, nhb, n_rb, nh, sink, out, packed);
+                        int nhb, uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out) {
+    merge_frag(part_acc, part_ml, n_splits, n_hb16, nhb, n_rb, nh, sink, out);
 }
 __global__ void __launch_bounds__(64 * MW)
 mla_merge_frag32_kernel(const f32x4 *__restrict__ part_acc, const float *__restrict__ part_ml, int n_splits, int n_hb16,
-                        int nhb, uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out, int packed) {
-    merge_frag(part_acc, part_ml, n_splits, n_hb16, nhb, n_rb, nh, sink, out, packed);
+                        int nhb, uint32_t n_rb, int nh, const float *__restrict__ sink, float *__restrict__ out) {
+    merge_frag(part_acc, part_ml, n_splits, n_hb16, nhb, n_rb, nh, sink, out);
 }
 
 // Split-K partials of the entry point that may not allocate (cwick_hip_mla_decode_static_dev):
@@ -886,13 +913,12 @@ static void *static_scratch() {
 }  // namespace
 
 template <class PART>
-static int launch_merge_of(void (*kernel)(const PART *, const float *, int, int, int, uint32_t, int, const float *, float *, int),
+static int launch_merge_of(void (*kernel)(const PART *, const float *, int, int, int, uint32_t, int, const float *, float *),
                            const PART *part_acc, const float *part_ml, int n_splits, int n_groups, int n_hb16, int nhb,
                            int64_t n_rb, int nh, const float *sink, float *out, int prof, hipStream_t s) {
-    const bool packed = n_splits <= 8;
     ProfKernel pk(prof, s);
-    pk.launch(kernel, dim3(n_hb16 * (packed ? 4 : NDB), n_groups), dim3(64 * (packed || n_splits <= 64 ? 8 : MW)), 0,
-              part_acc, part_ml, n_splits, n_hb16, nhb, (uint32_t)n_rb, nh, sink, out, packed ? 1 : 0);
+    pk.launch(kernel, dim3(n_hb16 * (merge_packed(n_splits) ? 4 : NDB), n_groups), dim3(64 * merge_waves(n_splits)), 0,
+              part_acc, part_ml, n_splits, n_hb16, nhb, (uint32_t)n_rb, nh, sink, out);
     CWICK_HIP_CALL(hipGetLastError());
     return 1;
 }

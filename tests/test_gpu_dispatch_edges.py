@@ -494,3 +494,25 @@ def test_mm_pick_by_one_wave(hip, orc, limit, block, keep, kind):
         want = [p for b in blocks for p in range(b * block, min(lim, (b + 1) * block))][:max_sel]
         have = sel[y].cpu().numpy()
         assert have[have >= 0].tolist() == want and int(n_sel[y]) == len(want), "query %d" % y
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4, 5, 8, 9, 16, 17, 31, 32, 33, 64, 65, 127, 128, 129, 200, 255])
+def test_merges_of_every_number_of_slices(hip, orc, splits):
+    """As many 64-key slices as the merges take at a time, one more and one fewer: of a GQA decode (one kv head) and of
+    an MLA decode (16 heads), the last slice a single key, one slice far above the others."""
+    say("[case] merges", splits)
+    n = 64 * (splits - 1) + 1
+    c = synth.cfg1_gqa_decode(n_keys=n, nh=8, nkv=1, hd=128, seed=splits)
+    top = synth.bf16_to_f32(c["q"][3]) * np.float32(3.0)          # a key that one head agrees with
+    c["k"][n // 2, 0] = synth.f32_to_bf16(top)
+    kv = hip.KVCache(n, 1, 128)
+    kv.write(0, c["k"].reshape(n, -1), c["v"].reshape(n, -1))
+    got = hip.gqa_decode(kv, n, c["q"], c["scale"])
+    ref = orc.gqa_decode(c["q"], c["k"], c["v"], c["scale"], nthreads=0)
+    assert np.isfinite(got).all() and np.abs(got - ref).max() <= 2e-3
+    c = synth.cfg3_mla_decode(n, 16, seed=splits)
+    lat = hip.LatentCache(1, n)
+    lat.write(0, 0, c["rows"], c["scales"])
+    got = hip.mla_decode(lat, 0, c["q"], c["scale"], n_list=n)
+    ref = orc.mla_decode(c["q"], c["rows"], c["scales"], c["scale"], nthreads=0)
+    assert np.isfinite(got).all() and (np.abs(got - ref) <= 2e-3 + 1e-2 * np.abs(ref)).all()
