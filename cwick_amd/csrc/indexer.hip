@@ -56,7 +56,7 @@ indexer_scores_rows_kernel(const uint8_t *__restrict__ keys, const float *__rest
                            const uint16_t *__restrict__ q, const float *__restrict__ w, int ih,
                            float *__restrict__ scores) {
     constexpr int KEYS = 16 * (16 / ROWS);          // per workgroup
-    __shared__ float terms[KEYS][4 * ROWS + 1];
+    __shared__ __attribute__((aligned(16))) float terms[KEYS][4 * ROWS + 4];
     const int b = blockIdx.y, tid = threadIdx.x, j = tid & 15, row = tid >> 4;
     const int kg = row / ROWS, hg = row % ROWS;
     const int64_t t0 = (int64_t)blockIdx.x * KEYS, t = t0 + 16 * kg + j;
@@ -86,6 +86,7 @@ indexer_scores_rows_kernel(const uint8_t *__restrict__ keys, const float *__rest
             e[c * 16 + i * 4 + 2] = hi[0];
             e[c * 16 + i * 4 + 3] = hi[1];
         }
+    f32x4 mine;
 #pragma unroll
     for (int hh = 0; hh < 4; hh++) {
         float qv[8];
@@ -115,12 +116,20 @@ indexer_scores_rows_kernel(const uint8_t *__restrict__ keys, const float *__rest
         float d = (s0 + s1) + (s2 + s3);
         d = d * ks;
         d = d < 0.0f ? 0.0f : d;
-        terms[16 * kg + j][4 * hg + hh] = d * wh[hh];
+        const float prod = d * wh[hh];
+        mine[hh] = 4 * hg + hh < ih ? prod : 0.0f;
     }
+    *(f32x4 *)&terms[16 * kg + j][4 * hg] = mine;
     __syncthreads();
     if (tid < KEYS && t0 + tid < n_keys) {
+        // (all terms read at once; past the last head a zero is added, which changes nothing: the sum is never -0.
+        // Eight by eight, and written one by one: 9001 keys of 64 heads 7.8 us, now 7.4.)
+        f32x4 x[ROWS];
+#pragma unroll
+        for (int h = 0; h < ROWS; h++) x[h] = *(const f32x4 *)&terms[tid][4 * h];
         float s = 0.0f;
-        for (int h = 0; h < ih; h++) s = s + terms[tid][h];
+#pragma unroll
+        for (int h = 0; h < 4 * ROWS; h++) s = s + x[h >> 2][h & 3];
         scores[(size_t)b * n_keys + t0 + tid] = s;
     }
 }

@@ -338,7 +338,7 @@ indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict
                        const int32_t *__restrict__ cand, int cap,
                        const IndexerBandRow *__restrict__ rows, float *__restrict__ scores,
                        float *__restrict__ cand_score) {   // [batch][cap]: the same scores in list order
-    __shared__ float terms[16][65];
+    __shared__ __attribute__((aligned(16))) float terms[16][68];
     const int b = blockIdx.y, tid = threadIdx.x;
     int c0 = blockIdx.x * 16;
     const int j = tid & 15, hg = tid >> 4;                          // candidate, head group
@@ -394,6 +394,7 @@ indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict
         qraw[hh] = *(const u32x4 *)(qb + (size_t)hc * IB_HD + 8 * j);
         wh[hh] = wb[hc];
     }
+    f32x4 mine;
 #pragma unroll
     for (int hh = 0; hh < 4; hh++) {
         const int h = hg * 4 + hh;
@@ -426,12 +427,17 @@ indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict
         d = d * ks;
         d = d < 0.0f ? 0.0f : d;
         const float prod = d * wh[hh];
-        terms[j][h] = h < ih ? prod : 0.0f;
+        mine[hh] = h < ih ? prod : 0.0f;
     }
+    *(f32x4 *)&terms[j][4 * hg] = mine;
     __syncthreads();
     if (tid < 16 && c0 + tid < (int)st.n_cand) {
+        f32x4 x[16];                                                // (all terms at once; past the last head a zero)
+#pragma unroll
+        for (int h = 0; h < 16; h++) x[h] = *(const f32x4 *)&terms[tid][4 * h];
         float s = 0.0f;
-        for (int h = 0; h < ih; h++) s = s + terms[tid][h];
+#pragma unroll
+        for (int h = 0; h < 64; h++) s = s + x[h >> 2][h & 3];
         scores[(size_t)b * n_keys + cand[(size_t)b * cap + c0 + tid]] = s;
         cand_score[(size_t)b * cap + c0 + tid] = s;
     }
