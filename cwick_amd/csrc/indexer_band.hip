@@ -16,8 +16,9 @@
 //      each relative to A_h = sum_i |e_i||q_hi| >= |q_h . e_t|, so
 //          |st - s| <= 450 u * ks[t] * sum_h |w_h| A_h[t],   u = 2^-24,
 //      and sum_h |w_h| A_h[t] = sum_i |e_ti| c_i with c_i = sum_h |w_h||q_hi|: one more row
-//      through the matrix core, with c rounded up to bf16.  beta[t] = 512 u * ks[t] * that row
-//      (the slack covers the rounding of the bound itself); beta = max_t beta[t].
+//      through the matrix core, the key bytes as they are without their signs against c rounded up
+//      to E4M3 (at most an eighth more).  beta[t] = 512 u * ks[t] * that row (the slack covers the
+//      rounding of the bound itself); beta = max_t beta[t].
 //   2. top-k machinery on st: T = the k-th largest approximate score, to the counter it is in: the
 //      approximate kernel counts its scores in 4096 of them per row, a 128th of an octave wide in the
 //      fourteen octaves where a row's large scores are (topk.hip; band_counter, common.hpp).
@@ -44,7 +45,15 @@ constexpr int IB_QROW = 128 + 8;                 // bf16 per head row of q in LD
 constexpr int IB_HD = CWICK_HIP_INDEX_DIM;    // 128
 
 typedef __attribute__((ext_vector_type(2))) float ib_f32x2;
+typedef __attribute__((ext_vector_type(8))) int ib_i32x8;
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+
+// The (biased) exponent that the bound row's E4M3 coefficients are laid out by, from the largest one's
+// bits: kept where 2^(e - 7) and a bound's 512 u times it are normal numbers.
+__device__ __forceinline__ uint32_t ib_bound_exponent(uint32_t top) {
+    const uint32_t e = top >> 23;
+    return e < 24u ? 24u : (e > 254u ? 254u : e);
+}
 
 // v[l] + v[l ^ 32] in every lane: the two halves of the wave trade places between two copies
 __device__ __forceinline__ float ib_half_sum(float v) {
@@ -53,7 +62,13 @@ __device__ __forceinline__ float ib_half_sum(float v) {
     return a + b;
 }
 
-template <int IB_KEYS>                          // keys per workgroup
+// What bounds this kernel is the matrix and the vector instructions of an iteration, which two waves
+// per SIMD do one after the other.  The bound row on the FP8 matrix core takes 64 cycles per 32 keys (as a
+// row of a bf16 product, 31 others of which were zero, 256, and four instructions per k-step to clear
+// the signs of the converted keys), and up to 32 heads take one block of them, not one of zeros beside it.
+// Sparse decode, 8 rows of 65536 keys 52.0 -> 51.0 us, of 32 heads 50.8 -> 49.3; 4 rows 37.6 -> 35.9.
+// (The keys of a third iteration in flight: 51.4 and 49.5.)
+template <int IB_KEYS, int NB>                  // keys per workgroup, blocks of 32 heads
 __global__ void __launch_bounds__(IB_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict__ kscale,
                       int64_t key_bstride, int64_t kscale_bstride, int64_t n_keys,
@@ -63,7 +78,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
                       IndexerBandRow *__restrict__ rows,
                       uint32_t *__restrict__ digits) {   // or null: [batch][slots][CWICK_BAND_DIGITS]
     __shared__ __attribute__((aligned(16))) float cpart_sh[IB_THREADS / 16][IB_HD];
-    __shared__ __attribute__((aligned(16))) uint16_t cb_sh[IB_HD + 64];          // coefficients, then 128 bytes of zeros
+    __shared__ __attribute__((aligned(16))) uint8_t cb_sh[IB_HD + 64];           // coefficients in E4M3, then 64 zeros
     __shared__ __attribute__((aligned(16))) uint32_t counts[4096];
     __shared__ __attribute__((aligned(16))) uint16_t q_sh[64 * IB_QROW];
     __shared__ float w_sh[64];
@@ -103,7 +118,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     // c_i = sum_h |w_h| |q_hi| starts from the same registers: thread (group = tid / 16, part =
     // tid % 16) holds dims 8 part .. +7 of heads group + 16 j, adds up its four heads and leaves
     // the eight sums in LDS; after the barrier thread i < 128 adds the sixteen groups of dim i.
-    bf16x8 qa[2][8];
+    bf16x8 qa[NB][8];
     // Key scales from four places of the row, the same ones in every workgroup.  (From 64 places, a cache line
     // each in front of the first keys, the kernel takes 0.3 us longer.)
     uint32_t ks_bits;
@@ -149,31 +164,36 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     for (int j = 0; j < 4096 / IB_THREADS; j++) counts[tid + IB_THREADS * j] = 0u;
     __syncthreads();
 #pragma unroll
-    for (int mb = 0; mb < 2; mb++)
+    for (int mb = 0; mb < NB; mb++)
 #pragma unroll
         for (int ks = 0; ks < 8; ks++)
             qa[mb][ks] = *(const bf16x8 *)&q_sh[(mb * 32 + row) * IB_QROW + 64 * g + 8 * ks];
+    float c = 0.0f;                                                                     // never negative
     if (tid < IB_HD) {
-        float part[IB_THREADS / 16], c = 0.0f;
+        float part[IB_THREADS / 16];
 #pragma unroll
         for (int k = 0; k < IB_THREADS / 16; k++) part[k] = cpart_sh[k][tid];
 #pragma unroll
         for (int k = 0; k < IB_THREADS / 16; k++) c += part[k];
-        cb_sh[tid] = (uint16_t)((__builtin_bit_cast(uint32_t, c) + 0xFFFFu) >> 16);     // rounded up to bf16
-        if (tid < 64) cb_sh[IB_HD + tid] = 0;
-        const uint32_t top = wave_max_u32(__builtin_bit_cast(uint32_t, c));             // (never negative)
+        const uint32_t top = wave_max_u32(__builtin_bit_cast(uint32_t, c));
         if (lane == 0) cmax_sh[wave] = top;
     }
     __syncthreads();
-    // the bound row's A fragments are read from LDS step by step: lanes of row 0 from the
-    // coefficients, all others from a stretch of zeros behind them
-    const char __attribute__((address_space(3))) *c_lane =
-        (const char __attribute__((address_space(3))) *)&cb_sh[row == 0 ? 64 * g : IB_HD];
+    const uint32_t c_top = cmax_sh[0] > cmax_sh[1] ? cmax_sh[0] : cmax_sh[1];
+    const uint32_t c_exp = ib_bound_exponent(c_top);
+    if (tid < IB_HD) {
+        // The coefficients over 2^(exponent of the largest - 7), 128 <= largest < 256.  What is below 2^-13 of
+        // the largest becomes 2^-6, the smallest normal number of E4M3; the rest is rounded up.
+        float x = c * __builtin_bit_cast(float, (261u - c_exp) << 23);
+        x = x > 0.015625f ? x : 0.015625f;                                              // (NaN: see bound_unit)
+        cb_sh[tid] = (uint8_t)(((__builtin_bit_cast(uint32_t, x) + 0xFFFFFu) >> 20) - (120u << 3));
+        if (tid < 64) cb_sh[IB_HD + tid] = 0;
+    }
     // the heads this lane holds after the MFMAs: register i of block mb is head
     // 32 mb + 8 (i / 4) + 4 g + i % 4
-    float wl[2][16];
+    float wl[NB][16];
 #pragma unroll
-    for (int mb = 0; mb < 2; mb++)
+    for (int mb = 0; mb < NB; mb++)
 #pragma unroll
         for (int i = 0; i < 16; i++) wl[mb][i] = w_sh[mb * 32 + (i >> 2) * 8 + 4 * g + (i & 3)];
 
@@ -191,13 +211,31 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
 #pragma unroll
         for (int bit = 7; bit >= 0; bit--)
             if (__builtin_popcountll(__ballot(e >= (upper | 1u << bit))) >= quarter) upper |= 1u << bit;
-        const uint32_t c_top = cmax_sh[0] > cmax_sh[1] ? cmax_sh[0] : cmax_sh[1];
         int lowest = (int)(c_top >> 23 & 0xFFu) + (int)(quarter ? upper : 127u) - 127 + 16 - ((int)BAND_OCTAVES - 1);
         lowest = lowest < 0 ? 0 : lowest;
         lowest = lowest > 256 - (int)BAND_OCTAVES ? 256 - (int)BAND_OCTAVES : lowest;
         octave = (uint32_t)__builtin_amdgcn_readfirstlane(lowest);
     }
     if (wg == 0 && tid == 0) rows[b].octave = octave;
+    __syncthreads();                                                // cb_sh
+
+    // The bound row's A fragments.  As operand of a 16x16x128 product a lane's key bytes are column
+    // lane % 16, contraction block lane / 16: blocks 0 and 2 hold key `column`, dims 0.. and 64..,
+    // blocks 1 and 3 the same dims of key column + 16.  Rows 0 and 8 have coefficients in blocks 0 and 2,
+    // rows 4 and 12 in blocks 1 and 3, so that the first register of every lane is the sum of its own key.
+    const int arow = lane & 15, ablk = lane >> 4;
+    const bool has_c = (arow & 3) == 0 && ((arow >> 2 ^ ablk) & 1) == 0;
+    ib_i32x8 ca[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const lds_u32x4 *src = (const lds_u32x4 *)(const char __attribute__((address_space(3))) *)&cb_sh[
+            has_c ? 64 * (ablk >> 1) + 32 * h : IB_HD + 32 * h];
+        const u32x4 lo = src[0], hi = src[1];
+        ca[h] = (ib_i32x8){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+    }
+    // 512 u in the coefficients' scale; an infinite or NaN coefficient makes every bound of the row NaN
+    const float bound_unit = c_top >= 0x7F800000u ? __builtin_bit_cast(float, 0x7FC00000u)
+                                                  : 512.0f / 16777216.0f * __builtin_bit_cast(float, (c_exp - 7u) << 23);
 
     float bmax = 0.0f;
     auto iteration = [&](int it, const u32x4 (&raw)[4], float kst) {
@@ -210,74 +248,87 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
         // an MFMA and a VALU read of its result.  The first is met by converting the keys
         // of k-step ks + 1 before the MFMAs of k-step ks are issued (which also puts the
         // conversions in the shadow of the matrix pipe), the second by the s_nop behind the loop.
-        f32x16 d0, d1, ab;
+        f32x16 d0, d1;
+        // The bound row: a product the compiler knows, in front of the others and read behind them.  Its
+        // operands and its result are tied to the assembly below, or it would be moved behind the loop,
+        // under the branch of the keys that exist.
+        f32x4 ab = {0.0f, 0.0f, 0.0f, 0.0f};
+        ib_i32x8 em;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) em[j] = (int)(raw[2 * h + (j >> 2)][j & 3] & 0x7F7F7F7Fu);
+            ab = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ca[h], em, ab, 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+        }
+        __builtin_amdgcn_sched_barrier(0);
         typedef __attribute__((ext_vector_type(2))) __bf16 ib_bf16x2;
-        u32x4 e[2], ea[2], cfrag[2];
-        auto convert = [&](int ks, u32x4 &eo, u32x4 &eao) {
+        u32x4 e[2];
+        auto convert = [&](int ks, u32x4 &eo) {
 #pragma unroll
             for (int j = 0; j < 2; j++) {                          // exact: E4M3 fits bf16
                 const int dw = raw[ks >> 1][2 * (ks & 1) + j];
                 eo[2 * j] = __builtin_bit_cast(uint32_t, (ib_bf16x2)__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(dw, 1.0f, false));
                 eo[2 * j + 1] = __builtin_bit_cast(uint32_t, (ib_bf16x2)__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(dw, 1.0f, true));
             }
-#pragma unroll
-            for (int j = 0; j < 4; j++) eao[j] = eo[j] & 0x7FFF7FFFu;
         };
-        convert(0, e[0], ea[0]);
-        cfrag[0] = *(const lds_u32x4 *)(c_lane);
+        convert(0, e[0]);
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) {
             const int cur = ks & 1, nxt = cur ^ 1;
-            const u32x4 ea_before = ea[nxt], c_before = cfrag[nxt];   // operands of the last MFMA issued
-            if (ks + 1 < 8) {
-                convert(ks + 1, e[nxt], ea[nxt]);
-                cfrag[nxt] = *(const lds_u32x4 *)(c_lane + 16 * (ks + 1));
-            }
+            const u32x4 e_before = e[nxt];                          // an operand of the last MFMA issued
+            if (ks + 1 < 8) convert(ks + 1, e[nxt]);
             // Everything above is in its registers before the first MFMA below is issued; the
             // operands of the step before stay allocated up to here (an MFMA goes on reading its
             // operands for a while after it has been issued, and the compiler, which does not
             // know, would hand their registers to the conversions above).
             if (ks == 0)
-                asm volatile("s_nop 1" : "+v"(e[nxt]), "+v"(ea[nxt]), "+v"(e[cur]), "+v"(ea[cur]), "+v"(cfrag[cur]));
+                asm volatile("s_nop 1" : "+v"(e[nxt]), "+v"(e[cur]), "+v"(ab) : "v"(em));
             else
-                asm volatile("" : "+v"(e[nxt]), "+v"(ea[nxt]), "+v"(e[cur]), "+v"(ea[cur]), "+v"(cfrag[cur])
-                             : "v"(ea_before), "v"(c_before));
+                asm volatile("" : "+v"(e[nxt]), "+v"(e[cur]) : "v"(e_before));
             if (ks == 0) {
                 asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d0) : "v"(qa[0][ks]), "v"(e[cur]));
-                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d1) : "v"(qa[1][ks]), "v"(e[cur]));
-                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(ab) : "v"(cfrag[cur]), "v"(ea[cur]), "v"(e[cur]));
+                if constexpr (NB == 2)
+                    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d1) : "v"(qa[NB - 1][ks]), "v"(e[cur]));
             } else {
                 asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d0) : "v"(qa[0][ks]), "v"(e[cur]));
-                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d1) : "v"(qa[1][ks]), "v"(e[cur]));
-                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(ab) : "v"(cfrag[cur]), "v"(ea[cur]), "v"(e[cur]));
+                if constexpr (NB == 2)
+                    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d1) : "v"(qa[NB - 1][ks]), "v"(e[cur]));
             }
         }
         // Nothing may read the results or write a register that these MFMAs read before the last
         // one is through: the wait carries the accumulators, so that nothing that reads them can
         // be scheduled above it either.
-        asm volatile("s_nop 15\n\ts_nop 2" : "+v"(d0), "+v"(d1), "+v"(ab)::"memory");
+        if constexpr (NB == 2)
+            asm volatile("s_nop 15\n\ts_nop 2" : "+v"(d0), "+v"(d1), "+v"(ab) : "v"(e[1]) : "memory");
+        else
+            asm volatile("s_nop 15\n\ts_nop 2" : "+v"(d0), "+v"(ab) : "v"(e[1]) : "memory");
         float sp = 0.0f, sq = 0.0f, sr = 0.0f, ss = 0.0f;      // four chains: a dependent FMA waits for the one before it
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             // one instruction per ReLU (through fmaxf or fmed3 the compiler adds a second one
             // that quiets NaNs; a NaN dot counts as 0 here, and the bound row turns NaN with it)
-            float r0, r1;
+            float r0;
             asm("v_max_f32 %0, 0, %1" : "=v"(r0) : "v"(d0[i]));
-            asm("v_max_f32 %0, 0, %1" : "=v"(r1) : "v"(d1[i]));
-            if (i & 1) {
-                sr = __builtin_fmaf(wl[0][i], r0, sr);
-                ss = __builtin_fmaf(wl[1][i], r1, ss);
+            if constexpr (NB == 2) {
+                float r1;
+                asm("v_max_f32 %0, 0, %1" : "=v"(r1) : "v"(d1[i]));
+                if (i & 1) {
+                    sr = __builtin_fmaf(wl[0][i], r0, sr);
+                    ss = __builtin_fmaf(wl[NB - 1][i], r1, ss);
+                } else {
+                    sp = __builtin_fmaf(wl[0][i], r0, sp);
+                    sq = __builtin_fmaf(wl[NB - 1][i], r1, sq);
+                }
             } else {
-                sp = __builtin_fmaf(wl[0][i], r0, sp);
-                sq = __builtin_fmaf(wl[1][i], r1, sq);
+                float &chain = (i & 3) == 0 ? sp : (i & 3) == 1 ? sr : (i & 3) == 2 ? sq : ss;
+                chain = __builtin_fmaf(wl[0][i], r0, chain);
             }
         }
         sp = (sp + sq) + (sr + ss);
         // lane l + lane l ^ 32 without a trip through LDS
         sp = ib_half_sum(sp);
-        const float band = ib_half_sum(ab[0]);                     // row 0 sits in the g = 0 lanes
         const float st = sp * kst;
-        const float beta = band * fabsf(kst) * (512.0f / 16777216.0f);
+        const float beta = ab[0] * fabsf(kst) * bound_unit;
         if (live && g == 0) {
             scores[(size_t)b * n_keys + t] = st;
             // the select's pass over the scores, done here
@@ -445,6 +496,13 @@ indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict
     }
 }
 
+template <int NB>
+static auto indexer_approx_of(int per) {
+    return per == 512 ? indexer_approx_kernel<512, NB> : per == 768 ? indexer_approx_kernel<768, NB> :
+           per == 1024 ? indexer_approx_kernel<1024, NB> : per == 1536 ? indexer_approx_kernel<1536, NB> :
+           indexer_approx_kernel<CWICK_INDEXER_APPROX_KEYS, NB>;
+}
+
 // the approximate scores and the per-workgroup maxima of their error bound (the first stage of
 // the banded select on its own; n_keys / IB_KEYS slots per row, rounded up)
 int launch_indexer_approx(const uint8_t *keys, const float *kscale, int64_t key_bstride,
@@ -459,10 +517,9 @@ int launch_indexer_approx(const uint8_t *keys, const float *kscale, int64_t key_
     const int n_wg = indexer_approx_slots(n_keys, batch), per = indexer_approx_keys(n_keys, batch);
     {
         ProfKernel pk(CWICK_HIP_PROF_INDEXER_APPROX, s);
-        pk.launch(per == 512 ? indexer_approx_kernel<512> : per == 768 ? indexer_approx_kernel<768> : per == 1024 ? indexer_approx_kernel<1024> :
-                  per == 1536 ? indexer_approx_kernel<1536> : indexer_approx_kernel<CWICK_INDEXER_APPROX_KEYS>, dim3(n_wg, batch), dim3(IB_THREADS), 0,
-                  keys, kscale, key_bstride, kscale_bstride, n_keys, q_idx, w, n_idx_heads, scores, beta_slots, rows,
-                  digits);
+        const auto kernel = n_idx_heads > 32 ? indexer_approx_of<2>(per) : indexer_approx_of<1>(per);
+        pk.launch(kernel, dim3(n_wg, batch), dim3(IB_THREADS), 0, keys, kscale, key_bstride, kscale_bstride,
+                  n_keys, q_idx, w, n_idx_heads, scores, beta_slots, rows, digits);
     }
     CWICK_HIP_CALL(hipGetLastError());
     return 1;

@@ -516,3 +516,33 @@ def test_merges_of_every_number_of_slices(hip, orc, splits):
     got = hip.mla_decode(lat, 0, c["q"], c["scale"], n_list=n)
     ref = orc.mla_decode(c["q"], c["rows"], c["scales"], c["scale"], nthreads=0)
     assert np.isfinite(got).all() and (np.abs(got - ref) <= 2e-3 + 1e-2 * np.abs(ref)).all()
+
+
+@pytest.mark.parametrize("n_keys,ih,kind", [(31, 32, "normal"), (513, 33, "normal"), (4111, 1, "normal"),
+                                            (777, 32, "one dim"), (777, 64, "tiny"), (777, 32, "huge")])
+def test_indexer_bound_row(hip, orc, n_keys, ih, kind):
+    """The bound of the approximate scores where its E4M3 coefficients have an edge: one or two blocks of
+    heads, a coefficient far above the others, magnitudes near the ends of fp32."""
+    import torch
+    say("[case] indexer bound row", n_keys, ih, kind)
+    g = synth.rng(640 + n_keys + ih)
+    keys, ks = synth.index_keys(g, n_keys)
+    q = synth.normal_bf16(g, (ih, synth.IDIM))
+    w = (g.standard_normal(ih, dtype=np.float32) / np.float32(np.sqrt(128.0 * ih))).astype(np.float32)
+    if kind == "one dim":
+        qf = synth.bf16_to_f32(q)
+        qf[:, 77] *= np.float32(2.0 ** 20)
+        q = synth.f32_to_bf16(qf)
+    elif kind in ("tiny", "huge"):
+        w = (w * np.float32(2.0 ** (-100 if kind == "tiny" else 100))).astype(np.float32)
+    cache = hip.IndexKeys(1, n_keys)
+    cache.write(0, 0, keys, ks)
+    approx, bound = hip.indexer_scores_approx(cache, 0, n_keys, q, w)
+    ref = orc.indexer_scores(q, w, keys, ks, nthreads=0)
+    # the bound in 64 bits; a coefficient is rounded up by an eighth at most, one below 2^-13 of the largest to that
+    e = np.abs(torch.from_numpy(keys.reshape(n_keys, 128).copy()).view(torch.float8_e4m3fn).double().numpy())
+    c = (np.abs(w.astype(np.float64))[:, None] * np.abs(synth.bf16_to_f32(q).astype(np.float64))).sum(axis=0)
+    least = ((e @ c) * np.abs(ks.astype(np.float64))).max() * 512.0 / 2 ** 24
+    most = ((e @ np.maximum(c * 1.125, c.max() / 2 ** 12)) * np.abs(ks.astype(np.float64))).max() * 512.0 / 2 ** 24
+    assert least * (1 - 1e-4) <= bound <= most * (1 + 1e-4)
+    assert np.abs(approx.astype(np.float64) - ref.astype(np.float64)).max() <= bound
