@@ -82,7 +82,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     __shared__ __attribute__((aligned(16))) uint32_t counts[4096];
     __shared__ __attribute__((aligned(16))) uint16_t q_sh[64 * IB_QROW];
     __shared__ float w_sh[64];
-    __shared__ float bmax_sh[IB_THREADS / 64];
+    __shared__ uint32_t bmax_sh[IB_THREADS / 64];
     __shared__ uint32_t cmax_sh[2];
     const int b = blockIdx.y, wg = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -237,7 +237,7 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     const float bound_unit = c_top >= 0x7F800000u ? __builtin_bit_cast(float, 0x7FC00000u)
                                                   : 512.0f / 16777216.0f * __builtin_bit_cast(float, (c_exp - 7u) << 23);
 
-    float bmax = 0.0f;
+    uint32_t bmax = 0u;      // bits of the largest bound: never negative, they order like the values, NaNs on top
     auto iteration = [&](int it, const u32x4 (&raw)[4], float kst) {
         const int64_t t = wbase + it * 32 + row;
         const bool live = t < n_keys;
@@ -334,7 +334,8 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
             // the select's pass over the scores, done here
             atomicAdd(&counts[band_counter(st, octave)], 1u);
         }
-        if (live) bmax = (beta <= bmax) ? bmax : beta;             // NaN sticks
+        const uint32_t bits = __builtin_bit_cast(uint32_t, beta);
+        if (live) bmax = bits > bmax ? bits : bmax;
     };
     // three register sets in turn, so that the loads of iteration it + 2 go out before
     // iteration it computes and nothing is copied between sets (a copy waits for its load);
@@ -351,15 +352,14 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
         if (it + 4 < N_IT) load_keys(it + 4, raw_b, kst_b);
         iteration(it + 2, raw_c, kst_c);
     }
-    // (never negative: the bit patterns order like the values as unsigned integers, NaNs on top)
-    bmax = __builtin_bit_cast(float, wave_max_u32(__builtin_bit_cast(uint32_t, bmax)));
+    bmax = wave_max_u32(bmax);
     if (lane == 0) bmax_sh[wave] = bmax;
     __syncthreads();
     if (tid == 0) {
-        float m = bmax_sh[0];
+        uint32_t m = bmax_sh[0];
 #pragma unroll
-        for (int i = 1; i < IB_THREADS / 64; i++) m = (bmax_sh[i] <= m) ? m : bmax_sh[i];
-        beta_slots[(size_t)b * gridDim.x + wg] = m;
+        for (int i = 1; i < IB_THREADS / 64; i++) m = bmax_sh[i] > m ? bmax_sh[i] : m;
+        beta_slots[(size_t)b * gridDim.x + wg] = __builtin_bit_cast(float, m);
     }
     if (digits && tid < 256) {
         // thread t: counters 16 t .. + 15

@@ -1175,7 +1175,7 @@ int cwick_hip_indexer_scores_approx(cwick_hip_ikeys *c, int slot, int64_t n_keys
     std::vector<float> hb((size_t)n_slots);
     if (!st.out(scores, dout, ob) || !st.out(hb.data(), dbeta, bb) || !st.wait()) return 0;
     float m = hb[0];
-    for (int i = 1; i < n_slots; i++) m = (hb[i] <= m) ? m : hb[i];      // NaN sticks
+    for (int i = 1; i < n_slots; i++) m = (hb[i] <= m || m != m) ? m : hb[i];      // NaN sticks
     *bound = m;
     return 1;
 }

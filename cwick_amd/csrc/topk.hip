@@ -354,7 +354,7 @@ topk_mw_classify_kernel(float *__restrict__ scores, int64_t n, int64_t k, int n_
     const uint32_t counter = sh_digit;
     beta = sh_beta[0];
 #pragma unroll
-    for (int i = 1; i < TOPK_MW_THREADS / 64; i++) beta = (sh_beta[i] <= beta) ? beta : sh_beta[i];
+    for (int i = 1; i < TOPK_MW_THREADS / 64; i++) beta = (sh_beta[i] <= beta || beta != beta) ? beta : sh_beta[i];
     float T_lo, T_hi;
     band_range(counter, octave, T_lo, T_hi);
     const bool ok = counter != 0u && beta >= 0.0f && beta < INFINITY && T_lo == T_lo && T_hi == T_hi;

@@ -519,10 +519,11 @@ def test_merges_of_every_number_of_slices(hip, orc, splits):
 
 
 @pytest.mark.parametrize("n_keys,ih,kind", [(31, 32, "normal"), (513, 33, "normal"), (4111, 1, "normal"),
-                                            (777, 32, "one dim"), (777, 64, "tiny"), (777, 32, "huge")])
+                                            (777, 32, "one dim"), (777, 64, "tiny"), (777, 32, "huge"),
+                                            (600, 32, "infinite"), (600, 64, "nan key")])
 def test_indexer_bound_row(hip, orc, n_keys, ih, kind):
     """The bound of the approximate scores where its E4M3 coefficients have an edge: one or two blocks of
-    heads, a coefficient far above the others, magnitudes near the ends of fp32."""
+    heads, a coefficient far above the others, magnitudes near the ends of fp32, an infinite query, a NaN key."""
     import torch
     say("[case] indexer bound row", n_keys, ih, kind)
     g = synth.rng(640 + n_keys + ih)
@@ -535,9 +536,18 @@ def test_indexer_bound_row(hip, orc, n_keys, ih, kind):
         q = synth.f32_to_bf16(qf)
     elif kind in ("tiny", "huge"):
         w = (w * np.float32(2.0 ** (-100 if kind == "tiny" else 100))).astype(np.float32)
+    elif kind == "infinite":
+        q = q.copy()
+        q[ih - 1, 5] = 0x7F80
+    elif kind == "nan key":
+        keys = keys.copy()
+        keys.reshape(n_keys, 128)[n_keys - 1, 100] = 0x7F
     cache = hip.IndexKeys(1, n_keys)
     cache.write(0, 0, keys, ks)
     approx, bound = hip.indexer_scores_approx(cache, 0, n_keys, q, w)
+    if kind in ("infinite", "nan key"):
+        assert not np.isfinite(bound)                       # the row is scored exactly
+        return
     ref = orc.indexer_scores(q, w, keys, ks, nthreads=0)
     # the bound in 64 bits; a coefficient is rounded up by an eighth at most, one below 2^-13 of the largest to that
     e = np.abs(torch.from_numpy(keys.reshape(n_keys, 128).copy()).view(torch.float8_e4m3fn).double().numpy())
