@@ -5,9 +5,14 @@
 // HBM-bound: every K and V row is read exactly once, and nothing but the loads may be in the way.
 //
 //   grid  = (n_splits, n_kv_heads), 256 threads (4 waves)
-//   A workgroup owns one kv head and one contiguous slice of keys and serves the `group` query
+//   A workgroup owns one kv head and every n_splits-th step of 64 keys and serves the `group` query
 //   heads that share the kv head (the reference walks cache rows for the same reason: one row
 //   serves every head of its group, src/q35_model.c:1417-1423).  A wave takes tiles of 16 keys.
+//   At any time the workgroups read neighbouring steps, which lie in all channels of the memory.
+//   (A contiguous slice each: where its length is a multiple of a power of two, the slices are in the same
+//   channels at the same time.  64 heads on 8 x 128: 65536 keys 57.0 us, 51.8 so; 131072 102.0 and 96.3; 36500
+//   34.6 and 32.3; 100003 77.4 and 75.3.  Slices of 15 and 17 steps are the better ones of the two: 30000 keys
+//   26.5 and 27.2, 33000 29.0 and 29.9; 16 on 4 x 256 at 33000 30.0 and 28.8.)
 //
 //   scores:  S[key][head] = K Q^T, v_mfma_f32_16x16x32_bf16 straight from registers: lane l reads
 //            16 bytes of key l%16 per load, which is the A operand as it lies in the cache.  The
@@ -60,7 +65,7 @@ __global__ void __launch_bounds__(GQA_DEC_THREADS, HD == 256 || (LIST && GROUP =
 gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
                         const uint16_t *__restrict__ Q, int64_t n_keys, int n_kv_heads,
                         const int32_t *__restrict__ sel, int64_t n_rows,
-                        int keys_per_split, float scale_log2e,
+                        float scale_log2e,
                         float *__restrict__ part_acc,   // [n_splits][n_heads][HD]
                         float *__restrict__ part_ml,    // [n_splits][n_heads][2]
                         float *__restrict__ out,        // [n_heads][HD], one split only; host memory where there are flags
@@ -74,13 +79,13 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, lg = lane >> 4;
     const uint32_t row_stride = (uint32_t)n_kv_heads * HD;
-    const int64_t k_begin = (int64_t)split * keys_per_split;
-    const int count = (int)(n_keys - k_begin < keys_per_split ? n_keys - k_begin : keys_per_split);
+    const int64_t k_begin = (int64_t)split * (NW * GQA_DEC_TILE);
+    const int count = (int)(n_keys - k_begin);          // from its first key to the end (negative: none)
     const uint16_t *Kg = K + (LIST ? 0 : k_begin * row_stride) + (size_t)g * HD + lg * 8;
     const uint16_t *Vg = V + (LIST ? 0 : k_begin * row_stride) + (size_t)g * HD + l16 * 8;
     const int32_t *list = LIST ? sel + k_begin : nullptr;
 
-    constexpr int STRIDE = NW * GQA_DEC_TILE;
+    const int STRIDE = (int)gridDim.x * (NW * GQA_DEC_TILE);
     int t = wave * GQA_DEC_TILE;
     // List entries, those of four of the wave's tiles in one register: lane 16 j + i has key i of the j-th.
     // A tile takes what it needs (key l16, whose K row this lane reads, and keys 4 lg .. +4 of the V rows)
@@ -95,7 +100,7 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
         const int i = t + STRIDE * lg + l16;
         return list[i < count ? i : count - 1];
     };
-    // Requests a tile and returns which of this lane's keys 4 lg .. +4 carry no weight: those past the slice
+    // Requests a tile and returns which of this lane's keys 4 lg .. +4 carry no weight: those past the end
     // and list entries that name no row, which are read from a row that exists.
     auto load = [&](GqaDecTile<HD> &x, int t) {
         uint32_t k_row, v_row[4], dead = 0;
@@ -368,8 +373,7 @@ static int run_gqa_decode(const uint16_t *k, const uint16_t *v, int64_t n_keys, 
         const int64_t want = num_cus() > n_kv_heads ? num_cus() / n_kv_heads : 1;
         per_steps = (steps + want - 1) / want;
     }
-    const int64_t per = per_steps * step;
-    const int n_splits = (int)((n_keys + per - 1) / per);
+    const int n_splits = (int)((steps + per_steps - 1) / per_steps);
     float *part_acc = nullptr, *part_ml = nullptr;
     if (n_splits > 1) {
         // (asked for: as many splits as any call of up to this many keys has)
@@ -388,7 +392,7 @@ static int run_gqa_decode(const uint16_t *k, const uint16_t *v, int64_t n_keys, 
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_DECODE, s);
         pk.launch(sel ? gqa_decode_split_kernel<HD, GROUP, true> : gqa_decode_split_kernel<HD, GROUP, false>,
-                  dim3(n_splits, n_kv_heads), dim3(GQA_DEC_THREADS), 0, k, v, q, n_keys, n_kv_heads, sel, n_rows, (int)per,
+                  dim3(n_splits, n_kv_heads), dim3(GQA_DEC_THREADS), 0, k, v, q, n_keys, n_kv_heads, sel, n_rows,
                   scale * 1.44269504088896340736f, part_acc, part_ml, out, flags, epoch, tickets);
     }
     CWICK_HIP_CALL(hipGetLastError());

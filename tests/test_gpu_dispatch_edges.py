@@ -177,6 +177,25 @@ def test_gqa_decode_edges(hip, orc, n_keys, nh, nkv, hd):
     cache.free()
 
 
+@pytest.mark.parametrize("n_keys,nh,nkv,hd", [
+    (4161, 64, 8, 128),      # 66 steps for 22 workgroups a kv head, a key in the last
+    (8193, 16, 4, 256),      # 129 for 43
+    (8256, 8, 4, 128),       # 129 whole ones for 43
+    (700, 64, 64, 128),      # 11 for 4: one of them has a step less, and their last workgroup merges
+])
+def test_gqa_decode_steps_in_turn(hip, orc, n_keys, nh, nkv, hd):
+    """Several steps per workgroup, dealt in turn: as many for each, one less for some, one that ends in it."""
+    say("[case] gqa decode, steps in turn", n_keys, nh, nkv, hd)
+    c = synth.cfg1_gqa_decode(n_keys, nh, nkv, hd, seed=95)
+    cache = hip.KVCache(n_keys, nkv, hd)
+    cache.write(0, c["k"], c["v"])
+    got = hip.gqa_decode(cache, n_keys, c["q"], c["scale"])
+    ref = orc.gqa_decode(c["q"], c["k"], c["v"], c["scale"], nthreads=0)
+    # fp32 sums of exact products, as at the other lengths
+    assert np.abs(got - ref).max() < 2e-5 * np.abs(ref).max()
+    cache.free()
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(16, 4, 256), (64, 8, 128), (64, 4, 128)])
 def test_gqa_decode_late_maximum_and_dead_lists(hip, orc, nh, nkv, hd):
     """A score far above its wave's first tile (the reference moves), and lists whose first tiles, or
