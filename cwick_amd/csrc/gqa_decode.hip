@@ -10,9 +10,8 @@
 //   serves every head of its group, src/q35_model.c:1417-1423).  A wave takes tiles of 16 keys.
 //   At any time the workgroups read neighbouring steps, which lie in all channels of the memory.
 //   (A contiguous slice each: where its length is a multiple of a power of two, the slices are in the same
-//   channels at the same time.  64 heads on 8 x 128: 65536 keys 57.0 us, 51.8 so; 131072 102.0 and 96.3; 36500
-//   34.6 and 32.3; 100003 77.4 and 75.3.  Slices of 15 and 17 steps are the better ones of the two: 30000 keys
-//   26.5 and 27.2, 33000 29.0 and 29.9; 16 on 4 x 256 at 33000 30.0 and 28.8.)
+//   channels at the same time.  64 heads on 8 x 128: 65536 keys 57.1 us, 50.5 so; 131072 103.0 and 95.3; 100003
+//   77.8 and 73.9; 33000 29.1 and 28.5.)
 //
 //   scores:  S[key][head] = K Q^T, v_mfma_f32_16x16x32_bf16 straight from registers: lane l reads
 //            16 bytes of key l%16 per load, which is the A operand as it lies in the cache.  The
@@ -59,9 +58,10 @@ struct GqaDecTile {
 template <int HD, int GROUP>
 constexpr int GQA_DEC_QUADS = GROUP <= 4 ? 1 : GROUP == 8 && HD == 128 ? 2 : 0;   // (8 x 256: too many accumulators)
 
-// (Two workgroups per compute unit is what the launcher makes at most; where three fit the registers, they do.)
+// (Two workgroups per compute unit is what the launcher makes at most; where three fit the registers, they do.
+// Eight heads x 128 need 171 registers: held to three, 12 bytes of scratch in the loop, 30000 keys 27.6 us, 26.2 so.)
 template <int HD, int GROUP, bool LIST>
-__global__ void __launch_bounds__(GQA_DEC_THREADS, HD == 256 || (LIST && GROUP == 8) ? 2 : 3)
+__global__ void __launch_bounds__(GQA_DEC_THREADS, HD == 256 || GROUP == 8 ? 2 : 3)
 gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
                         const uint16_t *__restrict__ Q, int64_t n_keys, int n_kv_heads,
                         const int32_t *__restrict__ sel, int64_t n_rows,
