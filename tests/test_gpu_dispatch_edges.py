@@ -575,3 +575,20 @@ def test_indexer_bound_row(hip, orc, n_keys, ih, kind):
     most = ((e @ np.maximum(c * 1.125, c.max() / 2 ** 12)) * np.abs(ks.astype(np.float64))).max() * 512.0 / 2 ** 24
     assert least * (1 - 1e-4) <= bound <= most * (1 + 1e-4)
     assert np.abs(approx.astype(np.float64) - ref.astype(np.float64)).max() <= bound
+
+
+@pytest.mark.parametrize("n,nh", [
+    (128, 16), (129, 16),            # two tiles in one workgroup, three in three
+    (8192, 16),                      # two tiles each instead of one
+    (4097, 128), (12288, 128),       # a last workgroup of one tile; four tiles each instead of three
+])
+def test_mla_decode_fewer_workgroups(hip, orc, n, nh):
+    """The lengths at which a workgroup of the MLA decode takes more tiles than a full round of workgroups needs."""
+    say("[case] mla decode, fewer workgroups", n, nh)
+    c = synth.cfg3_mla_decode(n, nh, seed=n)
+    lat = hip.LatentCache(1, n)
+    lat.write(0, 0, c["rows"], c["scales"])
+    got = hip.mla_decode(lat, 0, c["q"], c["scale"], n_list=n)
+    ref = orc.mla_decode(c["q"], c["rows"], c["scales"], c["scale"], nthreads=0)
+    assert_close(got, ref, "mla decode, fewer workgroups", strict=False)
+    lat.free()
