@@ -1028,9 +1028,9 @@ int launch_mla_decode(const uint8_t *rows, const float *scales, int64_t row_bstr
     if (want > MERGE_MAX_SPLITS) want = MERGE_MAX_SPLITS;
     const int64_t tiles = (n_list + TK - 1) / TK;
     int64_t per_tiles = (tiles + want - 1) / want;
-    if (splits_per_cu() > 1) {}                         // (asked for: as many as that makes)
-    else if (tiles <= 2) per_tiles = tiles;
-    else if (per_tiles <= 3) {
+    const bool choose = splits_per_cu() == 1;           // (more are asked for: as many as that makes)
+    if (choose && tiles <= 2) per_tiles = tiles;
+    else if (choose && per_tiles <= 3) {
         const float step = sel ? 1.5f : 1.1f;
         float best = INFINITY;
         for (int64_t t = per_tiles, end = per_tiles + 3; t <= end; t++) {
