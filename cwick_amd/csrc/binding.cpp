@@ -8,7 +8,11 @@
 //
 // Arguments are what ctypes took: integers by their low bits, anything with __float__ for a float, and for a
 // pointer None, an address, or (calls on device memory) a contiguous device tensor, (calls on host memory) an
-// object with a buffer, such as a NumPy array.  The interpreter lock is released during the call.
+// object with a buffer, such as a NumPy array.  A stream, the last argument of every call on device memory, is
+// None, an address or whatever else ctypes makes a void pointer of (an object with _as_parameter_, such as
+// torch.cuda.Stream), and never a tensor.  What cannot be converted is a ctypes.ArgumentError, as it is there,
+// and a TypeError besides.
+// The interpreter lock is released during the call.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -23,6 +27,7 @@
 namespace {
 
 PyObject *s_is_cuda, *s_is_contiguous, *s_data_ptr, *s_value;
+PyObject *argument_error, *ctypes_error, *ctypes_cast, *void_pointer;
 
 struct Buffers {                            // of the arrays in a call: held until it is over
     Py_buffer held[8];
@@ -32,31 +37,29 @@ struct Buffers {                            // of the arrays in a call: held unt
     }
 };
 
+// what is not an integer or a number where one is needed (any other error stays as it is)
+bool not_an_argument() {
+    if (PyErr_ExceptionMatches(PyExc_TypeError) || PyErr_ExceptionMatches(PyExc_OverflowError) || PyErr_ExceptionMatches(ctypes_error)) {
+        PyObject *type, *value, *trace;
+        PyErr_Fetch(&type, &value, &trace);
+        PyErr_Format(argument_error, "%S", value ? value : type);
+        Py_XDECREF(type), Py_XDECREF(value), Py_XDECREF(trace);
+    }
+    return false;
+}
+
 bool address(PyObject *o, uintptr_t &out) { // None or an integer
     if (o == Py_None) {
         out = 0;
         return true;
     }
     out = (uintptr_t)PyLong_AsUnsignedLongLongMask(o);
-    return !(out == (uintptr_t)-1 && PyErr_Occurred());
+    return !(out == (uintptr_t)-1 && PyErr_Occurred()) || not_an_argument();
 }
 
 bool device_address(PyObject *o, uintptr_t &out) {
     PyObject *cuda = PyObject_GetAttr(o, s_is_cuda);
-    if (!cuda) {                            // a ctypes pointer, where a stream was given as one
-        if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return false;
-        PyObject *type, *value, *trace;
-        PyErr_Fetch(&type, &value, &trace);
-        PyObject *p = PyObject_GetAttr(o, s_value);
-        if (!p) {
-            PyErr_Restore(type, value, trace);
-            return false;
-        }
-        Py_XDECREF(type), Py_XDECREF(value), Py_XDECREF(trace);
-        const bool ok = address(p, out);
-        Py_DECREF(p);
-        return ok;
-    }
+    if (!cuda) return false;
     const int is_cuda = PyObject_IsTrue(cuda);
     Py_DECREF(cuda);
     if (is_cuda < 0) return false;
@@ -76,11 +79,25 @@ bool device_address(PyObject *o, uintptr_t &out) {
     return got;
 }
 
-template <bool DEV, class T>
+bool stream_address(PyObject *o, uintptr_t &out) {
+    if (o == Py_None || PyLong_Check(o)) return address(o, out);
+    PyObject *p = PyObject_CallFunctionObjArgs(ctypes_cast, o, void_pointer, nullptr);
+    if (!p) return not_an_argument();
+    PyObject *value = PyObject_GetAttr(p, s_value);
+    Py_DECREF(p);
+    if (!value) return false;
+    const bool ok = address(value, out);
+    Py_DECREF(value);
+    return ok;
+}
+
+template <bool DEV, bool STREAM, class T>
 bool convert(PyObject *o, T &out, Buffers &b) {
     if constexpr (std::is_pointer_v<T>) {
         uintptr_t a = 0;
-        if (o == Py_None || PyLong_Check(o)) {
+        if constexpr (STREAM) {
+            if (!stream_address(o, a)) return false;
+        } else if (o == Py_None || PyLong_Check(o)) {
             if (!address(o, a)) return false;
         } else if constexpr (DEV) {
             if (!device_address(o, a)) return false;
@@ -95,11 +112,11 @@ bool convert(PyObject *o, T &out, Buffers &b) {
         out = (T)a;
     } else if constexpr (std::is_floating_point_v<T>) {
         const double x = PyFloat_AsDouble(o);
-        if (x == -1.0 && PyErr_Occurred()) return false;
+        if (x == -1.0 && PyErr_Occurred()) return not_an_argument();
         out = (T)x;
     } else {
         const unsigned long long x = PyLong_AsUnsignedLongLongMask(o);
-        if (x == (unsigned long long)-1 && PyErr_Occurred()) return false;
+        if (x == (unsigned long long)-1 && PyErr_Occurred()) return not_an_argument();
         out = (T)x;
     }
     return true;
@@ -109,7 +126,7 @@ template <bool DEV, class... A, size_t... I>
 PyObject *invoke(int (*fn)(A...), PyObject *const *args, std::index_sequence<I...>) {
     std::tuple<A...> v;
     Buffers b;
-    if (!(convert<DEV>(args[I], std::get<I>(v), b) && ...)) return nullptr;
+    if (!(convert<DEV, DEV && I + 1 == sizeof...(A)>(args[I], std::get<I>(v), b) && ...)) return nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = fn(std::get<I>(v)...);
@@ -185,6 +202,15 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_cwick_calls", nullptr, -1, method
 }  // namespace
 
 PyMODINIT_FUNC PyInit__cwick_calls(void) {
+    PyObject *ctypes = PyImport_ImportModule("ctypes");
+    if (!ctypes) return nullptr;
+    ctypes_error = PyObject_GetAttrString(ctypes, "ArgumentError");
+    ctypes_cast = ctypes_error ? PyObject_GetAttrString(ctypes, "cast") : nullptr;
+    void_pointer = ctypes_cast ? PyObject_GetAttrString(ctypes, "c_void_p") : nullptr;
+    PyObject *bases = void_pointer ? PyTuple_Pack(2, ctypes_error, PyExc_TypeError) : nullptr;
+    argument_error = bases ? PyErr_NewException("_cwick_calls.ArgumentError", bases, nullptr) : nullptr;
+    Py_XDECREF(bases), Py_DECREF(ctypes);
+    if (!argument_error) return nullptr;
     s_is_cuda = PyUnicode_InternFromString("is_cuda");
     s_is_contiguous = PyUnicode_InternFromString("is_contiguous");
     s_data_ptr = PyUnicode_InternFromString("data_ptr");

@@ -24,6 +24,13 @@ class Tensor:
         return self.address
 
 
+class Stream:
+    """What torch.cuda.Stream is to ctypes."""
+
+    def __init__(self, address):
+        self._as_parameter_ = C.c_void_p(address)
+
+
 def _recorder(name):
     res, types = hip.SIGNATURES["cwick_hip_" + name]
     seen = []
@@ -60,7 +67,8 @@ def test_arguments_arrive_as_through_ctypes(name):
                 kind = (turn + i) % 3
                 a = None if kind == 0 else 0x7F0000001000 + 64 * i if kind == 1 else arrays[i].ctypes.data
                 plain.append(a)
-                given.append(a if kind < 2 else Tensor(a) if name.endswith("_dev") else arrays[i])
+                device = Stream if i == len(types) - 1 else Tensor
+                given.append(a if kind < 2 else device(a) if name.endswith("_dev") else arrays[i])
             elif t is C.c_float:
                 plain.append((0.125, 3, -1.0, 1e300, np.float32(0.1), float("nan"), True, 0.1)[turn])
                 given.append(plain[-1])
@@ -91,6 +99,44 @@ def test_what_is_no_argument_is_refused():
     with pytest.raises(ValueError):
         _module().bind("no_such_call", 1)
     assert len(seen) == 2
+
+
+def test_a_stream_is_what_ctypes_takes_as_one():
+    """The last argument of a call on device memory: all that ctypes makes a void pointer of, and nothing else.  A tensor
+    there would be a stream whose state is the tensor's bytes."""
+    fn, types, seen = _recorder("topk_dev")
+    call = _module().bind("topk_dev", C.cast(fn, C.c_void_p).value)
+    head = [64, 1, 2, 3, 128]
+    block = C.create_string_buffer(8)
+    for stream in (None, 0, 4096, C.c_void_p(), C.c_void_p(4096), Stream(0), Stream(4096), C.cast(block, C.POINTER(C.c_char)), block):
+        assert call(*head, stream) == fn(*head, stream) - 1
+        assert seen[-1] == seen[-2]
+    n = len(seen)
+    for bad in (Tensor(64), object(), 2.5, np.zeros(3), np.int64(4096)):
+        for f in (call, fn):
+            with pytest.raises(C.ArgumentError):
+                f(*head, bad)
+    with pytest.raises(AttributeError):                     # and a pointer is no tensor
+        call(C.c_void_p(64), *head[1:], None)
+    assert len(seen) == n
+
+
+@pytest.mark.parametrize("at,bad", [(1, 2.5), (1, None), (2, "3"), (3, np.zeros(2))])
+def test_refused_arguments_raise_what_ctypes_raises(at, bad):
+    fn, types, seen = _recorder("topk_dev")
+    call = _module().bind("topk_dev", C.cast(fn, C.c_void_p).value)
+    given = [64, 1, 2, 3, 128, None]
+    given[at] = bad
+    for f in (call, fn):
+        with pytest.raises(C.ArgumentError):
+            f(*given)
+    fn, types, seen = _recorder("gqa_decode")
+    call = _module().bind("gqa_decode", C.cast(fn, C.c_void_p).value)
+    for bad in ("0.5", None, 10 ** 400):
+        for f in (call, fn):
+            with pytest.raises(C.ArgumentError):
+                f(64, 1, None, 2, bad, None)
+    assert not seen
 
 
 def test_the_interpreter_runs_during_a_call():
