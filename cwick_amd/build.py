@@ -8,6 +8,7 @@ The library lands in cwick_amd/lib/ so that it travels with the source tree.
 """
 import concurrent.futures as cf
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -60,11 +61,20 @@ def _compile(src, force):
 
 
 def _build_calls(force):
+    """Needs this interpreter's headers and a host compiler; without them hip.py makes its calls through ctypes."""
     src = os.path.join(CSRC, "binding.cpp")
     deps = [src, os.path.join(HERE, "..", "include", "cwick_hip.h"), os.path.abspath(__file__)]
     if not force and os.path.exists(CALLS) and all(os.path.getmtime(CALLS) >= os.path.getmtime(d) for d in deps):
         return
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-Wall", "-fPIC", "-shared", "-fvisibility=hidden",
+    cxx = os.environ.get("CXX", "g++").split()
+    missing = [what for what, there in (("Python.h", os.path.exists(os.path.join(sysconfig.get_path("include"), "Python.h"))),
+                                        (cxx[0], shutil.which(cxx[0]))) if not there]
+    if missing:
+        print("no %s: the step calls of hip.py go through ctypes" % " and no ".join(missing))
+        if os.path.exists(CALLS):
+            os.remove(CALLS)                    # (of other sources)
+        return
+    cmd = cxx + ["-O2", "-std=c++17", "-Wall", "-fPIC", "-shared", "-fvisibility=hidden",
            "-I" + sysconfig.get_path("include"), src, "-o", CALLS]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

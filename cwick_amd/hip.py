@@ -136,15 +136,41 @@ def lib():
     return _lib
 
 
+def _through_ctypes(name, fn):
+    """A call of a step through ctypes: takes what the extension's takes, in some 2 us."""
+    types = SIGNATURES["cwick_hip_" + name][1]
+    stream = len(types) - 1 if name.endswith("_dev") else None
+    pointers = [i for i, t in enumerate(types) if t is _vp and i != stream]
+    address = _hp if stream is None else _dp
+
+    def call(*args):
+        args = list(args)
+        for i in pointers:
+            args[i] = address(args[i])
+        return fn(*args)
+    return call
+
+
+class _CtypesCalls:
+    """The calls of a step where the extension has not been built for this interpreter."""
+
+    def __getattr__(self, name):
+        call = _through_ctypes(name, getattr(lib(), "cwick_hip_" + name))
+        setattr(self, name, call)
+        return call
+
+
 def _calls():
     """The calls of a step (binding.cpp), by name: they take tensors and arrays as they are, in 0.3 to 0.6 us where
-    ctypes and the addresses taken in Python need 2 (one decode over 4096 keys, which the host's launches bound: 10.6 us
-    through ctypes, 9.9 through these; one step on state in host memory, 760 keys: 33.1, 29.6)."""
+    ctypes and the addresses taken in Python need 2 (one step on state in host memory, 760 keys: 33.1 us through ctypes,
+    29.6 through these).  Through ctypes all the same where the extension is missing: it is built for one interpreter,
+    from its headers, and the library serves any."""
     global _c
     if _c is None:
         L = lib()
         if not os.path.exists(CALLS_PATH):
-            raise ImportError("%s is missing: build it with `python -m cwick_amd.build`" % CALLS_PATH)
+            _c = _CtypesCalls()
+            return _c
         spec = importlib.util.spec_from_file_location("_cwick_calls", CALLS_PATH)
         m = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(m)
@@ -195,6 +221,14 @@ def _dp(t):
         return t
     assert t.is_cuda and t.is_contiguous()
     return t.data_ptr()
+
+
+def _hp(a):
+    """Host address of a contiguous NumPy array (or a raw integer address / None)."""
+    if a is None or isinstance(a, int):
+        return a
+    assert a.flags.c_contiguous
+    return a.ctypes.data
 
 
 # ------------------------------------------------------------------ caches

@@ -4,11 +4,12 @@ hands over."""
 import ctypes as C
 import importlib.util
 import threading
+import types as _types
 
 import numpy as np
 import pytest
 
-from cwick_amd import hip
+from cwick_amd import build, hip
 
 
 class Tensor:
@@ -149,3 +150,38 @@ def test_the_interpreter_runs_during_a_call():
     t.start()
     assert call(None, 1, 2, 3, None, None) == 1
     t.join()
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_calls_go_through_ctypes_without_the_extension(name, monkeypatch, tmp_path):
+    """The extension is built for one interpreter; the library serves any other through ctypes."""
+    fn, types, seen = _recorder(name)
+    bound = _module().bind(name, C.cast(fn, C.c_void_p).value)
+    monkeypatch.setattr(hip, "CALLS_PATH", str(tmp_path / "missing.so"))
+    monkeypatch.setattr(hip, "_c", None)
+    monkeypatch.setattr(hip, "_lib", _types.SimpleNamespace(**{"cwick_hip_" + name: fn}))
+    call = getattr(hip._calls(), name)
+    arrays = [np.arange(4 + i, dtype=np.float32) for i in range(len(types))]
+    for turn in range(3):
+        given = []
+        for i, t in enumerate(types):
+            if t is C.c_void_p:
+                device = Stream if i == len(types) - 1 else Tensor
+                given.append((None, 4096 + i, device(64 * i + 64) if name.endswith("_dev") else arrays[i])[(turn + i) % 3])
+            else:
+                given.append(0.25 if t is C.c_float else 11 + i)
+        assert call(*given) == bound(*given) - 1
+        assert repr(seen[-2]) == repr(seen[-1])
+
+
+def test_the_library_builds_without_the_headers_of_python(monkeypatch, tmp_path, capsys):
+    monkeypatch.setattr(build, "CALLS", str(tmp_path / "calls.so"))
+    with monkeypatch.context() as m:
+        m.setattr(build.sysconfig, "get_path", lambda name: str(tmp_path))
+        build._build_calls(force=True)
+    with monkeypatch.context() as m:
+        m.setenv("CXX", str(tmp_path / "no-compiler"))
+        build._build_calls(force=True)
+    out = capsys.readouterr().out
+    assert "no Python.h: the step calls" in out and "no-compiler: the step calls" in out
+    assert not (tmp_path / "calls.so").exists()
