@@ -15,7 +15,7 @@
 //      one thread per position.)
 //   2. block maxima, started from -1e30 like the reference.  The scoring kernel leaves the
 //      maximum of every group of 64 positions; when a block is a whole number of groups (128 in
-//      the reference's configuration) mm_pick_few_kernel (up to 2048 blocks, 64 kept) or
+//      the reference's configuration) mm_pick_few_kernel (up to 2048 blocks, 32 kept) or
 //      mm_pick_kernel, one workgroup per query, makes the block maxima from them, selects the
 //      `keep` best blocks (the radix select in the second, lowest index first among equal maxima --
 //      the reference's heap makes that choice on tie-free input) and writes the list: one launch.  Other block sizes take mm_blockmax_kernel (one
@@ -313,21 +313,32 @@ mm_expand_kernel(const int32_t *__restrict__ blk, int kb, int64_t limit0, int bs
 }
 
 // Block maxima, the kept blocks and the list of one query in one workgroup, for up to 2048 blocks that are a whole
-// number of the scoring kernel's 64-position groups, of which at most 64 are kept.
+// number of the scoring kernel's 64-position groups, of which at most 32 are kept.
 //
 // Nothing here but the trip to the group maxima takes long by itself, so what counts is the chain: the radix select
 // has ten barriers of sixteen waves between that trip and the list, this four of eight.  The kk-th largest of 64
-// maxima, each of every 64th block, is a bound that kk blocks reach and few others do, found bit by bit from counts of
-// ballots, by every wave for itself.  Where the blocks that reach it are at most 64 (nearly always) they go
+// maxima, each of every 64th block, is a bound that kk blocks reach and few others do (32 of them: some 44), found bit
+// by bit from counts of ballots, by every wave for itself.  Where the blocks that reach it are at most 64 they go
 // into a lane each of the first wave, in order, which finds the threshold in the same way, until as many as are wanted
-// reach it; otherwise it does so on all blocks.  65536 positions in blocks of 128, sixteen kept: 5.2 us by the radix
-// select, 3.5; 131072 in blocks of 64: 5.8, 3.6.  (The first wave alone with a lane for every 64th block: 4.1 and 8.2.)
-constexpr int MM_PICK_THREADS = 512, MM_PICK_WAVES = MM_PICK_THREADS / 64, MM_PICK_KEEP = 64, MM_PICK_BLOCKS = 2048;
+// reach it.  65536 positions in blocks of 128, sixteen kept: 5.2 us by the radix select, 3.5; 131072 in blocks of 64: 5.8,
+// 3.6.  (The first wave alone with a lane for every 64th block: 4.1 and 8.2.)
+//
+// Where more blocks reach it, by ties or because the largest share lanes, the whole workgroup counts, three bits of
+// the threshold to a barrier.  The whole selection of 16 of 2048 blocks, us, by the radix select and so: all
+// equal 19.9 and 11.1, eight levels 15.5 and 11.1, a hundred equal above the rest 15.3 and 14.7, four in one lane
+// of every wave 13.5 and 12.9, distinct 13.7 and 10.9; of 512 blocks 13.4 and 9.2, 12.4 and 9.2, 12.6 and 9.2, 12.4 and
+// 9.3, 11.4 and 9.5.  (The first wave alone, bit by bit, all equal: 63 and 22.6.)
+//
+// More than 32 are kept by the radix select: the 36th largest of 64 maxima has 53 blocks above it on the average
+// and the 64th nearly all, so that counting is what is left.  64 of 2048 distinct blocks 14.3 us by the radix select and
+// 17.8 by counts of the workgroup, of 512 blocks 12.3 and 13.3.
+constexpr int MM_PICK_THREADS = 512, MM_PICK_WAVES = MM_PICK_THREADS / 64, MM_PICK_KEEP = 32, MM_PICK_BLOCKS = 2048;
 template <int EPT>
 __global__ void __launch_bounds__(MM_PICK_THREADS)
 mm_pick_few_kernel(const float *__restrict__ gmax, int64_t gmax_stride, int64_t limit0, int bs, int kb,
                    int32_t *__restrict__ blk_out, int32_t *__restrict__ sel, int64_t max_sel, int32_t *__restrict__ n_sel) {
-    __shared__ uint32_t sh_key[MM_PICK_THREADS * EPT], sh_top[MM_PICK_WAVES][64], sh_cand[64];
+    __shared__ uint32_t sh_top[MM_PICK_WAVES][64], sh_cand[64], sh_of[MM_PICK_WAVES][2];
+    __shared__ __attribute__((aligned(16))) uint32_t sh_digit[2][MM_PICK_WAVES][4];
     __shared__ int32_t sh_idx[64], sh_blk[MM_PICK_KEEP];
     __shared__ uint32_t sh_cnt[MM_PICK_WAVES], sh_has;
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
@@ -354,10 +365,10 @@ mm_pick_few_kernel(const float *__restrict__ gmax, int64_t gmax_stride, int64_t 
 #pragma unroll
     for (int j = 0; j < EPT; j++) {
         key[j] = first + 64 * j < nblk ? topk_key(v[j]) : 0u;
-        sh_key[first + 64 * j] = key[j];
         top = key[j] > top ? key[j] : top;
     }
     sh_top[wave][lane] = top;
+    if (tid == 0) sh_has = 0u;
     __syncthreads();
     auto count = [](bool x) { return __builtin_popcountll(__ballot(x)); };
     auto below = [](uint64_t m) {                                       // lanes below this one in m
@@ -407,41 +418,81 @@ mm_pick_few_kernel(const float *__restrict__ gmax, int64_t gmax_stride, int64_t 
         }
         __syncthreads();
     }
-    if (wave == 0) {
-        bool has = false;
-        if (n_cand <= 64) {
+    if (n_cand <= 64) {
+        if (wave == 0) {
             const uint32_t mine = lane < n_cand ? sh_cand[lane] : 0u;
             const uint32_t T = threshold([&](uint32_t x) { return count(mine >= x); }, all);
             // ties at T that do not all fit: the smaller indices win
             const int r = kk - count(mine > T);
             const bool tied = mine == T && mine, take = mine && (all ? mine >= T : mine > T || (tied && below(__ballot(tied)) < r));
             const uint64_t m = __ballot(take);
+            bool has = false;
             if (take) {
                 const int idx = sh_idx[lane];
                 sh_blk[below(m)] = idx;
                 has = idx == newest;
             }
-        } else {
-            const int steps = (nblk + 63) / 64;
-            auto over = [&](uint32_t x) {
-                int c = 0;
-                for (int j = 0; j < steps; j++) c += count(sh_key[64 * j + lane] >= x);
-                return c;
-            };
-            const uint32_t T = threshold(over, all);
-            int r = kk - (T == 0xFFFFFFFFu ? 0 : over(T + 1u)), to = 0;
-            for (int j = 0; j < steps; j++) {
-                const uint32_t x = sh_key[64 * j + lane];
-                const bool tied = x == T && x, take = x && (all ? x >= T : x > T || (tied && below(__ballot(tied)) < r));
-                r -= count(tied);
-                const uint64_t m = __ballot(take);
-                if (take) sh_blk[to + below(m)] = 64 * j + lane;
-                to += __builtin_popcountll(m);
-                has = has || (take && 64 * j + lane == newest);
-            }
+            const uint64_t any = __ballot(has);
+            if (lane == 0) sh_has = any != 0u;
         }
-        const uint64_t any = __ballot(has);
-        if (lane == 0) sh_has = any != 0u;
+    } else {
+        // Three bits at a time, from the first in which the bound and the largest maximum differ (equal scores: none at
+        // all).  Every lane counts its blocks by digit, a nibble each; what is added up over the workgroup
+        // are the blocks up to each digit, digits d and d + 4 in the halves of word d.
+        const uint32_t most = wave_max_u32(top);
+        int bits = bound == most ? 0 : 32 - __builtin_clz(bound ^ most);
+        uint32_t T = bits == 32 ? 0u : bound >> bits << bits;
+        for (int turn = 0; bits > 0; turn ^= 1) {
+            const int shift = bits > 3 ? bits - 3 : 0;                  // (fewer bits left: no block reaches the values past them)
+            uint32_t seen = 0u;
+#pragma unroll
+            for (int j = 0; j < EPT; j++) {
+                const uint32_t d = (key[j] - T) >> shift;
+                seen += 1u << 4 * (key[j] < T ? 0u : d < 7u ? d : 7u);
+            }
+            seen *= 0x11111111u;
+            u32x4 up_to;
+#pragma unroll
+            for (int d = 0; d < 4; d++) up_to[d] = wave_sum_u32(seen >> 4 * d & 0x000F000Fu);
+            if (lane == 0) *(u32x4 *)sh_digit[turn][wave] = up_to;
+            __syncthreads();
+            uint32_t sum = 0u;                                          // for lanes 1 .. 7: blocks below the value of this digit
+#pragma unroll
+            for (int w = 0; w < MM_PICK_WAVES; w++) sum += sh_digit[turn][w][(lane - 1) & 3];
+            const int reach = MM_PICK_THREADS * EPT - (int)(lane > 4 ? sum >> 16 : sum & 0xFFFFu);
+            const int digit = count(lane > 0 && lane < 8 && reach >= kk);       // (more blocks reach the smaller values)
+            T += (uint32_t)digit << shift;
+            bits = digit && __builtin_amdgcn_readlane(reach, digit) == kk ? 0 : shift;
+        }
+        int over = 0, ties = 0;                                         // of this wave
+        uint64_t m_eq[EPT];
+#pragma unroll
+        for (int j = 0; j < EPT; j++) {
+            over += count(key[j] > T);
+            m_eq[j] = __ballot(key[j] == T);
+            ties += __builtin_popcountll(m_eq[j]);
+        }
+        if (lane == 0) sh_of[wave][0] = (uint32_t)over, sh_of[wave][1] = (uint32_t)ties;
+        __syncthreads();
+        int r = kk, to = 0, tied = 0;                                   // ties that are selected; places and ties in front of this wave
+#pragma unroll
+        for (int w = 0; w < MM_PICK_WAVES; w++) {
+            const int o = (int)sh_of[w][0], e = (int)sh_of[w][1];
+            r -= o;
+            if (w < wave) to += o, tied += e;
+        }
+        to += tied < r ? tied : r;
+#pragma unroll
+        for (int j = 0; j < EPT; j++) {
+            const bool take = key[j] > T || (key[j] == T && tied + below(m_eq[j]) < r);
+            const uint64_t m = __ballot(take);
+            if (take) {
+                sh_blk[to + below(m)] = first + 64 * j;
+                if (first + 64 * j == newest) sh_has = 1u;
+            }
+            to += __builtin_popcountll(m);
+            tied += __builtin_popcountll(m_eq[j]);
+        }
     }
     __syncthreads();
     mm_write_row<MM_PICK_THREADS>(sh_blk, kk, sh_has != 0u, kb, limit, bs, blk_out ? blk_out + (size_t)row * (kb + 1) : nullptr,

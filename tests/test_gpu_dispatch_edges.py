@@ -515,6 +515,90 @@ def test_mm_pick_by_one_wave(hip, orc, limit, block, keep, kind):
         assert have[have >= 0].tolist() == want and int(n_sel[y]) == len(want), "query %d" % y
 
 
+def _mm_pick(hip, torch, level, limit, block, keep):
+    """A selection over keys whose scores are `level`, one value a block; as a call to repeat, and its list of blocks."""
+    keys = np.zeros((limit, 128), np.float32)
+    keys[:, 5] = np.asarray(level, np.float32).repeat(block)[:limit]
+    keys = synth.f32_to_bf16(keys)
+    d_k, d_q = torch.from_numpy(keys.view(np.int16)).cuda(), torch.ones((1, 1, 128), device="cuda")
+    scores = torch.empty((1, limit), dtype=torch.float32, device="cuda")
+    sel = torch.empty((1, (keep + 1) * block), dtype=torch.int32, device="cuda")
+    blk = torch.empty((1, keep + 1), dtype=torch.int32, device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+    call = lambda: hip.mm_select_dev(d_k, d_q, 1, limit, 1, 128, block, keep, scores, limit, blk, sel, (keep + 1) * block,
+                                     None, s)
+    return keys, call, blk, sel
+
+
+@pytest.mark.parametrize("limit,block,keep,kind", [
+    (131072, 64, 32, "random"), (131072, 64, 33, "random"), (65536, 128, 64, "random"),     # the line to the radix select
+    (131072, 64, 32, "same lanes"), (65536, 64, 32, "same lanes"),          # three bits a turn down to the last ones
+    (32768, 64, 32, "same lanes"), (131072, 64, 32, "next to one another"), (32768, 64, 31, "next to one another"),
+    (131072, 64, 16, "equal"), (32768, 64, 16, "zero"), (131072, 64, 1, "equal"), (4161, 64, 32, "equal"),
+    (131072, 64, 16, "100 top"), (32768, 64, 16, "100 top"),                # ties above all others, spread over the waves
+    (131072, 64, 32, "20 above 100"), (32768, 64, 32, "20 above 100"),      # some above the ties, twelve of the ties
+    (131072, 64, 16, "late")])                                              # ties in the last wave only
+def test_mm_pick_of_many_candidates(hip, orc, limit, block, keep, kind):
+    """A selection in which more than 64 blocks reach its bound, by counts of the whole workgroup, and the line to
+    the radix select."""
+    import torch
+    say("[case] mm pick, many candidates", limit, block, keep, kind)
+    g = synth.rng(92)
+    nb = (limit + block - 1) // block
+    level = np.ones(nb)
+    some = g.permutation(nb)
+    if kind == "random":
+        level = 1.0 + np.abs(g.standard_normal(nb))
+    elif kind == "zero":
+        level = np.zeros(nb)
+    elif kind == "100 top":
+        level[some[:100]] = 2.0
+    elif kind == "20 above 100":
+        level[some[:20]], level[some[20:120]] = 3.0 + g.integers(0, 3, 20), 2.0
+    elif kind == "same lanes": # the best in one lane of every wave
+        level = 1.0 + 0.5 * g.random(nb)
+        level[17::64] = 2.0 ** g.integers(1, 20, len(level[17::64])) * (1.0 + 0.9 * g.random(len(level[17::64])))
+    elif kind == "next to one another":
+        level = 1.0 + g.integers(0, 128, nb) / 128.0                        # neighbours in bf16
+    elif kind == "late":
+        level[-100:] = 2.0
+    keys, call, blk, sel = _mm_pick(hip, torch, level, limit, block, keep)
+    call()
+    torch.cuda.synchronize()
+    ref = orc.mm_index_scores(np.ones((1, 128), np.float32), keys, limit)
+    best = orc.topk_contract(np.array([ref[b:b + block].max() for b in range(0, limit, block)], np.float32), keep)
+    blocks = sorted({int(b) for b in best if b >= 0} | {limit // block})
+    assert [b for b in blk[0].tolist() if b >= 0] == blocks
+    want = [p for b in blocks for p in range(b * block, min(limit, (b + 1) * block))]
+    have = sel[0].cpu().numpy()
+    assert have[have >= 0].tolist() == want
+
+
+@pytest.mark.parametrize("keep,kind", [(16, "equal"), (64, "random")])
+def test_mm_pick_of_many_candidates_is_no_slow_path(hip, keep, kind):
+    """2048 blocks that all tie, and 64 kept of 2048, in less than 2.5 times what sixteen of distinct ones take (1.0 and 1.3
+    times; by counts of one wave alone 5.8 and 4)."""
+    import torch
+    say("[case] mm pick, time of many candidates", keep, kind)
+
+    def us(level, keep):
+        _, call, _, _ = _mm_pick(hip, torch, level, 131072, 64, keep)
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = []
+        for _ in range(7):
+            a.record()
+            for _ in range(100):
+                call()
+            b.record()
+            torch.cuda.synchronize()
+            best.append(a.elapsed_time(b) * 10.0)
+        return min(best)
+    distinct = np.random.default_rng(93).permutation(2048) / 2048.0 + 1.0
+    base, many = us(distinct, 16), us(np.ones(2048) if kind == "equal" else distinct, keep)
+    say("[time]", base, many)
+    assert many < 2.5 * base
+
+
 @pytest.mark.parametrize("splits", [1, 2, 4, 5, 8, 9, 16, 17, 31, 32, 33, 64, 65, 127, 128, 129, 200, 255])
 def test_merges_of_every_number_of_slices(hip, orc, splits):
     """As many 64-key slices as the merges take at a time, one more and one fewer: of a GQA decode (one kv head) and of
