@@ -661,6 +661,46 @@ def test_indexer_bound_row(hip, orc, n_keys, ih, kind):
     assert np.abs(approx.astype(np.float64) - ref.astype(np.float64)).max() <= bound
 
 
+@pytest.mark.parametrize("n_keys,ih,kind", [(1111, 32, "normal"), (2049, 64, "normal"), (300, 7, "one dim"), (333, 64, "one dim off"),
+                                            (500, 33, "subnormal keys"), (97, 16, "halves"), (97, 40, "nothing")])
+def test_indexer_bound_has_twelve_bits(hip, orc, n_keys, ih, kind):
+    """The bound of the approximate scores against its coefficients in 64 bits: rounded up by a 2048th of their own or by
+    2^-21 of the largest at most, less than a coefficient in bf16 is."""
+    import torch
+    say("[case] indexer bound, twelve bits", n_keys, ih, kind)
+    g = synth.rng(660 + n_keys + ih)
+    keys, ks = synth.index_keys(g, n_keys)
+    qf = synth.bf16_to_f32(synth.normal_bf16(g, (ih, synth.IDIM)))
+    w = (g.standard_normal(ih, dtype=np.float32) / np.float32(np.sqrt(128.0 * ih))).astype(np.float32)
+    if kind.startswith("one dim"):
+        qf[:, 77] *= np.float32(2.0 ** 12)
+        if kind == "one dim off":                           # only the other coefficients, and their terms, count
+            keys.reshape(n_keys, 128)[:, 77] = 0
+    elif kind == "subnormal keys":
+        keys = (g.integers(0, 8, (n_keys, 128)) | g.integers(0, 2, (n_keys, 128)) << 7).astype(np.uint8)
+    elif kind == "halves":                                  # c = 1/2, 1/4 .. 2^-12: each exact in one term
+        qf[:] = 2.0 ** -(1.0 + np.arange(128) % 12) / ih
+        w[:] = 1.0
+    elif kind == "nothing":
+        w[:] = 0.0
+    q = synth.f32_to_bf16(qf.astype(np.float32))
+    cache = hip.IndexKeys(1, n_keys)
+    cache.write(0, 0, keys, ks)
+    approx, bound = hip.indexer_scores_approx(cache, 0, n_keys, q, w)
+    ref = orc.indexer_scores(q, w, keys, ks, nthreads=0)
+    e = np.abs(torch.from_numpy(np.ascontiguousarray(keys).reshape(n_keys, 128).copy()).view(torch.float8_e4m3fn).double().numpy())
+    c = (np.abs(w.astype(np.float64))[:, None] * np.abs(synth.bf16_to_f32(q).astype(np.float64))).sum(axis=0)
+    unit = np.abs(ks.astype(np.float64)) * 512.0 / 2 ** 24
+    least = ((e @ c) * unit).max()
+    most = ((e @ (c * (1 + 2.0 ** -11) + (c > 0) * c.max() * 2.0 ** -21)) * unit).max()
+    say("[bound]", bound, least, most)
+    # Below: of eight products that the FP8 matrix core adds up at a time, each loses its bits under 2^-13 of the largest,
+    # so that a sum of products of one sign may lack 7 x 2^-13 of itself (no more than 1.3e-4 was seen over coefficients
+    # of twelve octaves).  1e-5: fp32 sums of 3 x 128 terms, and of up to 64 heads in a coefficient.
+    assert least * (1 - 7 * 2.0 ** -13 - 1e-5) <= bound <= most * (1 + 1e-5)
+    assert np.abs(approx.astype(np.float64) - ref.astype(np.float64)).max() <= bound
+
+
 @pytest.mark.parametrize("n,nh", [
     (128, 16), (129, 16),            # two tiles in one workgroup, three in three
     (8192, 16),                      # two tiles each instead of one
