@@ -164,9 +164,11 @@ inline float pf_plan(int64_t pos0, int64_t n, int positions, int n_kv_heads, int
     };
     look(0);
     const int room = cus / n_kv_heads;      // slices for one round
-    // (One round of whole blocks stays whole: 4096 positions of 16 / 4 heads take no memory for partials, wherever
-    // they run.  Cut, they would be a tenth shorter.)
-    const bool whole = b.count == room;
+    // (A prompt of one round of whole blocks, at the beginning of a cache, stays whole and takes no memory for partials:
+    // 4096 positions of 16 / 4 heads 176 us, cut 164; 8192 of 8 / 8 330 and 275.  Behind earlier keys it is a chunk
+    // like its neighbours, whole and cut: 4096 of 16 / 4 behind 500 keys 207 and 195, 2048 295 and 274, 4096 402 and
+    // 370, 8192 615 and 595; of 16 / 2 behind 2048 292 and 260; 8192 of 8 / 8 behind 2048 510 and 377.)
+    const bool whole = pos0 == 0 && b.count == room;
     if (!whole && (b.count < room || (room > 0 && 2 * b.tiles[b.count - 1] > most))) {
         auto round_up = [&](int64_t per) { return (int)(c.waves == 1 ? per : (per + 3) / 4 * 4); };
         const int first = b.count / room + 1;

@@ -125,6 +125,29 @@ int main() {
     print(out)
 
 
+def test_gqa_prefill_plan_of_one_round_of_blocks(tmp_path):
+    """A chunk of exactly one round of whole blocks behind earlier keys is priced like its neighbours: no more than one
+    of a position or a block more, and by both kernels."""
+    print(run_cpp(tmp_path, "gqa_plan.hpp", r"""
+int main() {
+    for (int kv : {2, 4, 8})
+        for (int rows : {64, 256}) {
+            const PfCost &c = rows == 64 ? PF_COST_TEAM : PF_COST_WIDE;
+            const int group = 16 / kv, P = rows / group, room = 256 / kv;
+            for (int64_t pos0 : {1, 500, 2048, 4096, 8192, 16384})
+                for (int64_t n : {(int64_t)room * P - P + 1, (int64_t)room * P}) {
+                    PfPlan p;
+                    const float t = pf_plan(pos0, n, P, kv, 0, 256, c, INFINITY, p);
+                    for (int64_t more : {1, P}) {
+                        const float u = pf_plan(pos0, room * P + more, P, kv, 0, 256, c, INFINITY, p);
+                        if (t > 1.02f * u) { printf("%d kv heads, %d rows: %d at %d %.1f, %d %.1f\n", kv, rows, (int)n, (int)pos0, t, (int)(room * P + more), u); return 1; }
+                    }
+                }
+        }
+    return 0;
+}"""))
+
+
 def test_gqa_prefill_plans_are_sound_and_quick(tmp_path):
     """The plans of both prefill kernels: the slices of every block cover its tiles, each begins below the
     diagonal and none is empty, there is room for the partials' numbers; less than a
@@ -163,7 +186,7 @@ int main() {
                             if (!ok) { printf("bad plan: %d rows, %d at %d, %d kv heads of %d\n", rows, (int)n, (int)pos0, kv, group); return 1; }
                             PfPlan q;
                             if (pf_plan(pos0, n, P, kv, prec, cus, c, 0.5f * t, q) != 0.5f * t) { printf("limit not kept\n"); return 1; }
-                            if (b.tiles[0] > 600 || b.count == cus / kv) continue;      // (those stay whole)
+                            if (b.tiles[0] > 600 || (pos0 == 0 && b.count == cus / kv)) continue;      // (a prompt of one round stays whole)
                             int parts;
                             float best = pf_time(b, c, 0, INFINITY, parts);
                             for (int per = c.least; per < b.tiles[0]; per += c.waves) best = std::fmin(best, pf_time(b, c, per, best, parts));
