@@ -223,12 +223,13 @@ gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const 
     // Score MFMA with its accumulator pinned to VGPRs: through the builtin the allocator places
     // every MFMA result in AGPRs, which the 256 output accumulators fill, and moves registers
     // back and forth every tile.  Opaque to the compiler's hazard tracking: score_done() goes
-    // between the last MFMA and the first VALU read of the result.
+    // between the last MFMA and the first VALU read of the result, and carries the result (without,
+    // nothing keeps the first instruction that reads it behind the wait).
     auto score_mfma = [&](f32x16 &acc, bf16x8 a, bf16x8 b, bool first) {
         if (first) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
         else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
     };
-    auto score_done = [&]() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); };
+    auto score_done = [&](f32x16 (&s)[2]) { asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s[0]), "+v"(s[1])::"memory"); };
     // ck / cv >= 0: the copies of K(ck) and V(cv) are issued between the MFMAs (an LDS-DMA
     // instruction occupies the issue slot for about as long as two MFMAs run).  Tile u of K or V
     // lives in buffer u & 1.
@@ -260,7 +261,7 @@ gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const 
                 else if (do_v) copy_one(src_v, dst_v, i);
             }
         }
-        score_done();
+        score_done(s);
     };
     // the same from global memory (the slow loop of the pipelined body: its K tile has already
     // been overwritten in LDS)
@@ -275,7 +276,7 @@ gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const 
             score_mfma(s[0], kf, qf[ks], ks == 0);
             score_mfma(s[1], kf, q1, ks == 0);
         }
-        score_done();
+        score_done(s);
     };
     // softmax bookkeeping of one tile and column block, in two parts.
     // register i holds key (i/4)*8 + 4g + i%4 of the tile for this lane's row.
@@ -587,6 +588,7 @@ gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const 
                 t++;
                 t3 = next3(t3);
                 if (!more()) {
+                    score_done(sb);
 #pragma unroll
                     for (int c = 0; c < 2; c++) {
                         sa[c] = sb[c];
@@ -603,7 +605,7 @@ gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const 
                 t3 = next3(t3);
                 if (!more()) break;
             }
-            score_done();
+            score_done(sa);
         }
         // the tiles on the diagonal and the tail, in sequence
         if (!slow)
@@ -972,7 +974,8 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
                 asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[1]) : "v"(kf), "v"(q1));
             }
         }
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        // (the wait carries the scores: without, nothing keeps the first instruction that reads them behind it)
+        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s[0]), "+v"(s[1])::"memory");
     };
     // masks the raw scores of a tile and returns this lane's maximum in log2 units
     auto prep = [&](int tile, int c, f32x16 &s) -> float {

@@ -87,6 +87,35 @@ def test_no_valu_write_right_before_an_mfma_reads_it(src):
     assert not early, "MFMA result read before the matrix pipe has written it: %r" % early[:3]
 
 
+@pytest.mark.parametrize("src,kernel", [("gqa_prefill.hip", "gqa_prefill_team_kernel"), ("indexer_band.hip", "indexer_approx_kernel")])
+def test_the_wait_behind_the_matrix_instructions_carries_their_results(src, kernel):
+    """The rule above holds for what the compiler happened to schedule.  That it may not schedule otherwise takes the results
+    through the wait: in the compiler's input to the scheduler, nothing but a further MFMA or the `s_nop 15` statement
+    may use what an MFMA from assembly leaves in VGPRs."""
+    with tempfile.TemporaryDirectory() as tmp:
+        out = os.path.join(tmp, "k.ll")
+        cmd = [B._hipcc()] + B.COMMON + B.PER_FILE.get(src, []) + [
+            "-w", "-S", "-emit-llvm", "--cuda-device-only", os.path.join(B.CSRC, src), "-o", out]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:]
+        functions = [f.splitlines() for f in open(out).read().split("\ndefine ")[1:]]
+    n_mfma, loose = 0, []
+    for lines in functions:
+        if kernel not in lines[0]:
+            continue
+        users = {}
+        for t in lines[1:]:
+            for name in set(re.findall(r"%[\w.]+", t.split(" = ", 1)[-1])):
+                users.setdefault(name, []).append(t.strip())
+        for t in lines:
+            m = re.match(r'\s+(%\w+) = .*\basm .*"v_mfma.*", "=&?v', t)
+            if m:
+                n_mfma += 1
+                loose += [u for u in users.get(m.group(1), ()) if not re.search(r'\basm .*"(v_mfma|s_nop 15)', u)]
+    assert n_mfma > 0
+    assert not loose, "an MFMA's result is used by what no wait is in front of: %r" % loose[:3]
+
+
 def test_decode_kernels_keep_their_tiles_in_registers():
     """The decode requests a tile while it works on the one before.  Where the two tiles and what belongs to them do
     not fit the registers, the compiler parks the requested one in scratch memory and waits for it there, and
