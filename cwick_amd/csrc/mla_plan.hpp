@@ -1,5 +1,6 @@
-// mla_plan.hpp -- how a chunk of the latent prefill (mla_prefill64.hip) is dealt to workgroups.  Plain C++:
-// the plan is made anew for every call, in front of kernels that may take 20 us, so it may not take long.
+// mla_plan.hpp -- how a chunk of the latent prefill (mla_prefill64.hip) and a latent decode (mla_roles.hip) are dealt
+// to workgroups.  Plain C++: a plan is made anew for every call, in front of kernels that may take 10 us, so it may
+// not take long.
 #pragma once
 #include <stdint.h>
 
@@ -93,6 +94,36 @@ inline WidePlan plan_wide(int64_t n_rb, int64_t tiles_first, int64_t tiles_last,
         if (x.time < best.time) best = x;
     }
     return best;
+}
+
+// The decode: how many slices the keys of one query can be cut into.  `blocks` are its blocks of 32 heads, of all
+// queries; one workgroup is resident per compute unit (per_cu: more are asked for), so one round of them at most.
+constexpr int MLA_MAX_SPLITS = 1024;
+inline int64_t mla_decode_most_splits(int64_t blocks, int per_cu, int cus) {
+    const int64_t want = (int64_t)per_cu * cus / blocks;
+    return want < 1 ? 1 : want > MLA_MAX_SPLITS ? MLA_MAX_SPLITS : want;
+}
+// The tiles of 64 keys of a workgroup.  With up to three of them each, fewer workgroups of a tile or more in addition
+// are often the shorter ones: a further tile takes 1.1 us (out of a list 1.5), while all workgroups start, write their
+// partials and have them merged at the same time, 2.5 us for 128 of them and 6.2 for 256 (fitted to 150 times; left
+// alone from four tiles on, where the end of the workgroups spreads).  us, with the workgroups of a full round and as
+// chosen here: 64 heads, 8192 keys 16.5 and 12.7, 16384 17.1 and 15.5; 128 heads, 4096 15.8 and 12.6, 12288 17.1 and
+// 16.2; 16 heads, 32768 18.9 and 16.2; 8 x 600 keys of 64 heads 13.5 and 11.6; 4 x 2048 selected keys of 64 heads, the
+// whole step, 31.9 and 29.7.  (A percent behind the full round where it is closest, 16 heads x 49000 and
+// 2 x 12000 of 64.)  Two tiles in one workgroup take less than the merge (100 keys of 16 heads: 8.8 and 7.8).
+inline int64_t mla_decode_tiles(int64_t tiles, int64_t blocks, bool list, int per_cu, int cus) {
+    const int64_t want = mla_decode_most_splits(blocks, per_cu, cus);
+    int64_t per = (tiles + want - 1) / want;
+    if (per_cu != 1) return per;                            // (as many as that makes)
+    if (tiles <= 2) return tiles;
+    if (per > 3) return per;
+    const float step = list ? 1.5f : 1.1f;
+    float best = 1e30f;
+    for (int64_t t = per, end = per + 3; t <= end; t++) {
+        const float wgs = (float)((tiles + t - 1) / t * blocks), cost = step * (float)t + (0.014f + 4e-5f * wgs) * wgs;
+        if (cost < best) best = cost, per = t;
+    }
+    return per;
 }
 
 }  // namespace cwick

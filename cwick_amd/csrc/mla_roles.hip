@@ -59,6 +59,7 @@
 //   [split][16-head block][dim block][lane][4] (every store 1 KiB contiguous);
 //   mla_merge_frag16_kernel reads them in the same order with all loads in flight.
 #include "common.hpp"
+#include "mla_plan.hpp"
 
 #include <cstdlib>
 #include <cstring>
@@ -81,7 +82,6 @@ constexpr int NDB = VDIM / 16;                // 32 sixteen-dim output blocks
 constexpr float LAZY = 4.0f;                  // the reference moves when a tile exceeds it by 2^LAZY
 constexpr int WEXP = 10;                      // fp16 weights are p * scale * 2^(WEXP - e), scale < 2^e
 constexpr int E_NONE = -1000;                 // no scale seen yet
-constexpr int MERGE_MAX_SPLITS = 1024;
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
@@ -1014,31 +1014,9 @@ int launch_mla_decode(const uint8_t *rows, const float *scales, int64_t row_bstr
     p.rows = rows; p.scales = scales; p.row_bstride = row_bstride; p.scale_bstride = scale_bstride;
     p.n_rows = n_rows; p.sel = sel; p.n_list = n_list;
     p.q = q; p.nh = n_heads; p.nq = batch; p.scale = scale; p.out = out; p.sink = sink;
-    // One workgroup is resident per CU: one round of workgroups at most.  With up to three tiles each, fewer
-    // workgroups of a tile or more in addition are often the shorter ones: a further tile takes 1.1 us (out of a
-    // list 1.5), while all workgroups start, write their partials and have them merged at the same time, 2.5 us for
-    // 128 of them and 6.2 for 256 (fitted to 150 times; left alone from four tiles on, where the end of the
-    // workgroups spreads).  us, with the workgroups of a full round and as chosen here: 64 heads, 8192 keys 16.5
-    // and 12.7, 16384 17.1 and 15.5; 128 heads, 4096 15.8 and 12.6, 12288 17.1 and 16.2; 16 heads, 32768 18.9 and
-    // 16.2; 8 x 600 keys of 64 heads 13.5 and 11.6; 4 x 2048 selected keys of 64 heads, the whole step, 31.9 and
-    // 29.7.  Two tiles in one workgroup take less than the merge (100 keys of 16 heads: 8.8 and 7.8).
     const int n_hb = (n_heads + HW - 1) / HW;
-    int64_t want = (int64_t)splits_per_cu() * num_cus() / ((int64_t)n_hb * batch);
-    if (want < 1) want = 1;
-    if (want > MERGE_MAX_SPLITS) want = MERGE_MAX_SPLITS;
-    const int64_t tiles = (n_list + TK - 1) / TK;
-    int64_t per_tiles = (tiles + want - 1) / want;
-    const bool choose = splits_per_cu() == 1;           // (more are asked for: as many as that makes)
-    if (choose && tiles <= 2) per_tiles = tiles;
-    else if (choose && per_tiles <= 3) {
-        const float step = sel ? 1.5f : 1.1f;
-        float best = INFINITY;
-        for (int64_t t = per_tiles, end = per_tiles + 3; t <= end; t++) {
-            const float wgs = (float)((tiles + t - 1) / t * n_hb * batch), cost = step * (float)t + (0.014f + 4e-5f * wgs) * wgs;
-            if (cost < best) best = cost, per_tiles = t;
-        }
-    }
-    int64_t per = per_tiles * TK;
+    const int64_t tiles = (n_list + TK - 1) / TK, want = mla_decode_most_splits(n_hb * batch, splits_per_cu(), num_cus());
+    const int64_t per = (int64_t)TK * mla_decode_tiles(tiles, n_hb * batch, sel != nullptr, splits_per_cu(), num_cus());
     p.keys_per_split = per;
     p.n_splits = (int)((n_list + per - 1) / per);
     return run(p, (int)(tiles < want ? tiles : want), s, fixed_scratch);

@@ -601,8 +601,9 @@ def test_mm_pick_of_many_candidates_is_no_slow_path(hip, keep, kind):
 
 @pytest.mark.parametrize("splits", [1, 2, 4, 5, 8, 9, 16, 17, 31, 32, 33, 64, 65, 127, 128, 129, 200, 255])
 def test_merges_of_every_number_of_slices(hip, orc, splits):
-    """As many 64-key slices as the merges take at a time, one more and one fewer: of a GQA decode (one kv head) and of
-    an MLA decode (16 heads), the last slice a single key, one slice far above the others."""
+    """As many 64-key slices as the merge of a GQA decode (one kv head) takes at a time, one more and one fewer, the last
+    slice a single key, one slice far above the others; and an MLA decode (16 heads) over as many keys, which
+    it cuts into fewer slices from 108 tiles on (their numbers: MLA_SLICES)."""
     say("[case] merges", splits)
     n = 64 * (splits - 1) + 1
     c = synth.cfg1_gqa_decode(n_keys=n, nh=8, nkv=1, hd=128, seed=splits)
@@ -619,6 +620,38 @@ def test_merges_of_every_number_of_slices(hip, orc, splits):
     got = hip.mla_decode(lat, 0, c["q"], c["scale"], n_list=n)
     ref = orc.mla_decode(c["q"], c["rows"], c["scales"], c["scale"], nthreads=0)
     assert np.isfinite(got).all() and (np.abs(got - ref) <= 2e-3 + 1e-2 * np.abs(ref)).all()
+
+
+# Keys, heads and queries of an MLA decode, and the slices that they are cut into with 256 compute units
+# (test_host_rules.py has the rule give these numbers).  Where there is one query, the last slice is a single key.
+MLA_SLICES = [
+    (193, 32, 64, 2), (385, 16, 1, 7), (449, 16, 1, 8), (513, 16, 1, 9),        # up to eight: a wave by itself
+    (2049, 16, 1, 33), (4033, 16, 1, 64), (4097, 16, 1, 65),                    # four of eight waves each, eight, sixteen waves
+    (16129, 16, 1, 127), (16257, 16, 1, 128), (16385, 16, 1, 129),              # eight of sixteen waves each, and one more
+    (17281, 16, 1, 136), (18433, 32, 1, 97), (30529, 16, 1, 160), (49153, 16, 1, 193), (65281, 32, 1, 256),
+]
+
+
+@pytest.mark.parametrize("n,nh,batch,slices", MLA_SLICES)
+def test_mla_merge_of_every_number_of_slices(hip, orc, n, nh, batch, slices):
+    """The merge of an MLA decode: as many slices as it takes at a time, one more and one fewer, up to a full round of
+    them; a key in the middle whose slice has the greatest maximum by far."""
+    import torch
+    say("[case] mla merge", n, nh, batch, slices)
+    c = synth.cfg3_mla_decode(n, nh, seed=n + nh)
+    c["scales"][n // 2] *= np.float32(6.0)
+    g = synth.rng(n)
+    q = synth.f32_to_bf16(g.standard_normal((batch, nh, synth.KDIM), dtype=np.float32))
+    d_rows, d_scales = torch.from_numpy(c["rows"]).cuda(), torch.from_numpy(c["scales"]).cuda()
+    out = torch.full((batch, nh, synth.VDIM), float("nan"), device="cuda")
+    # (a stride of 0: the queries share the rows)
+    hip.mla_decode_dev(d_rows, d_scales, 0, 0, n, batch, None, n, torch.from_numpy(q.view(np.int16)).cuda(), nh, c["scale"],
+                       out, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for y in {0, batch // 2, batch - 1}:
+        ref = orc.mla_decode(q[y], c["rows"], c["scales"], c["scale"], nthreads=0)
+        got = out[y].cpu().numpy()
+        assert np.isfinite(got).all() and (np.abs(got - ref) <= 2e-3 * np.abs(ref).max() + 1e-2 * np.abs(ref)).all()
 
 
 @pytest.mark.parametrize("n_keys,ih,kind", [(31, 32, "normal"), (513, 33, "normal"), (4111, 1, "normal"),

@@ -255,3 +255,35 @@ int main() {
     printf("%.0f us\n", best);
     return best >= 500.0 && best < 2000.0 ? 0 : 3;
 }""")
+
+
+def test_mla_decode_slices(tmp_path):
+    """The slices of an MLA decode: as many as the merge's test says; never more than the workspace is asked for, none
+    empty; and by the rule's own figures never slower than a full round of workgroups."""
+    from tests.test_gpu_dispatch_edges import MLA_SLICES
+    cases = ", ".join("{%d, %d, %d, %d}" % c for c in MLA_SLICES)
+    assert {s for _, _, _, s in MLA_SLICES} >= {2, 8, 9, 64, 65, 128, 129, 193, 256}
+    run_cpp(tmp_path, "mla_plan.hpp", r"""
+int main() {
+    const int known[][4] = {CASES};
+    for (auto &c : known) {
+        const int64_t blocks = (c[1] + 31) / 32 * c[2], per = 64 * mla_decode_tiles((c[0] + 63) / 64, blocks, false, 1, 256);
+        if ((c[0] + per - 1) / per != c[3]) { printf("%d keys of %d heads x %d: %d slices\n", c[0], c[1], c[2], (int)((c[0] + per - 1) / per)); return 1; }
+    }
+    for (int cus : {256, 304, 64})
+        for (int per_cu : {1, 2, 8})
+            for (bool list : {false, true})
+                for (int64_t blocks : {1, 2, 3, 4, 8, 31, 32, 100, 256, 300, 16384})
+                    for (int64_t tiles = 1; tiles < 40000000; tiles = tiles < 3000 ? tiles + 1 : tiles * 9 / 8) {
+                        const int64_t per = mla_decode_tiles(tiles, blocks, list, per_cu, cus), most = mla_decode_most_splits(blocks, per_cu, cus);
+                        const int64_t slices = (tiles + per - 1) / per, room = tiles < most ? tiles : most;
+                        const int64_t full = (tiles + most - 1) / most, round = (tiles + full - 1) / full;
+                        auto time = [&](int64_t t, int64_t n) { return (list ? 1.5 : 1.1) * t + (0.014 + 4e-5 * n * blocks) * n * blocks; };
+                        if (per < 1 || slices < 1 || slices > room || slices > 1024 || (slices - 1) * per >= tiles ||
+                            (per_cu == 1 && full <= 3 && tiles > 2 && time(per, slices) > time(full, round) * 1.0001)) {
+                            printf("%d tiles, %d blocks, list %d, %d x %d: %d a slice, %d slices\n", (int)tiles, (int)blocks, list, per_cu, cus, (int)per, (int)slices);
+                            return 1;
+                        }
+                    }
+    return 0;
+}""".replace("CASES", cases))
