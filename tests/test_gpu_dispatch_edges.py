@@ -66,16 +66,16 @@ def test_gqa_prefill_slices(hip, orc, n, pos0, nh, nkv):
 
 
 @pytest.mark.parametrize("n,pos0,nh,nkv", [
-    (16, 0, 16, 4),          # one workgroup of one wave for each kv head, all its rows live
+    (16, 0, 16, 4),          # one workgroup for each kv head, all its rows live
     (17, 2000, 16, 4),       # a second block of one position; slices
     (9, 1015, 16, 2),        # eight heads: blocks of eight positions on either side of the 1024 keys
     (65, 1500, 8, 8),        # one head: blocks of 64 positions, the second of one
-    (600, 4000, 16, 4),      # too many blocks for one wave each
+    (600, 4000, 16, 4),      # more rows than that
 ])
-def test_gqa_prefill_one_wave(hip, orc, n, pos0, nh, nkv):
-    """Problems that do not fill the chip: workgroups of one wave, with a key that outgrows every
-    reference before it (the slow loop)."""
-    say("[case] gqa prefill, one wave", n, pos0, nh, nkv)
+def test_gqa_prefill_small_problems(hip, orc, n, pos0, nh, nkv):
+    """Problems that do not fill the chip: blocks of 64 rows, whole and in slices, with a key that outgrows every
+    reference before it (the tiles that follow the maximum)."""
+    say("[case] gqa prefill, small problems", n, pos0, nh, nkv)
     c = synth.cfg2_gqa_prefill(n, nh, nkv, 256, pos0, seed=80)
     k = synth.bf16_to_f32(c["k"])
     late = (pos0 + n) * 2 // 3
@@ -86,7 +86,7 @@ def test_gqa_prefill_one_wave(hip, orc, n, pos0, nh, nkv):
     cache.write(0, k.reshape(pos0 + n, -1), c["v"].reshape(pos0 + n, -1))
     got = hip.gqa_prefill(cache, pos0, c["q"], c["scale"])
     ref = orc.gqa_prefill(c["q"], k, c["v"], pos0, c["scale"], nthreads=0)
-    assert_close(got, ref, "gqa prefill, one wave", strict=False)
+    assert_close(got, ref, "gqa prefill, small problems", strict=False)
     cache.free()
 
 
@@ -476,13 +476,17 @@ def test_mm_select_edges(hip, orc, limit, ih, block, keep):
 
 @pytest.mark.parametrize("limit,block,keep,kind", [
     (1, 64, 16, "random"), (4095, 64, 64, "random"), (4096, 64, 64, "random"), (4097, 64, 65, "random"),     # 64 blocks, 64 and 65 kept
-    (32768, 64, 8, "few levels"), (32769, 64, 8, "few levels"),             # 512 and 513 blocks: eight, thirty-two a lane
-    (131072, 64, 16, "random"), (131073, 64, 16, "random"),                 # 2048 blocks, and one too many for a wave
+    (32766, 64, 8, "few levels"), (32767, 64, 8, "few levels"),             # 512 and 513 blocks of the last query: one, four a thread
+    (32768, 64, 8, "few levels"), (32769, 64, 8, "few levels"),
+    (82000, 64, 16, "random"), (110000, 64, 33, "few levels"),              # live blocks in the later waves
+    (131070, 64, 16, "random"), (131071, 64, 16, "random"),                 # 2048 blocks of the last query, and one too many
+    (131070, 64, 16, "equal"), (131070, 64, 32, "few levels"), (131070, 64, 64, "ascending"), (131070, 64, 64, "few levels"),
+    (131072, 64, 16, "random"), (131073, 64, 16, "random"),
     (65536, 256, 16, "ascending"), (65500, 128, 16, "equal"), (9000, 64, 64, "few levels"), (9000, 128, 3, "negative")])
-def test_mm_pick_by_one_wave(hip, orc, limit, block, keep, kind):
-    """A selection of blocks by one wave: as many blocks as lanes, candidates for the threshold that fit its lanes and
-    that do not, ties that do not all fit, and the line to the workgroup's radix select; three queries of growing
-    limits.  The scores are set by one dimension, so that whole blocks agree."""
+def test_mm_pick_of_few_blocks(hip, orc, limit, block, keep, kind):
+    """A selection of up to 64 of up to 2048 blocks: as many blocks as lanes, candidates for the threshold that fit a wave's
+    lanes and that do not, ties that do not all fit, and the line to the radix select of longer rows; three queries
+    of growing limits (the last one's blocks pick the kernel).  The scores are set by one dimension, so that whole blocks agree."""
     import torch
     say("[case] mm pick", limit, block, keep, kind)
     g = synth.rng(91)
