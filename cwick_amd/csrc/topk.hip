@@ -53,16 +53,16 @@ constexpr int TOPK_MW_MAX_WGS = 64;                              // per row
 
 struct TopkMwState { uint32_t prefix, remaining; };
 
-// sum of p[w * stride] over w < count with thirty-two loads in flight (the slices sit in L2: a
+// sum of p[256 w] over w < count with thirty-two loads in flight (the slices sit in L2: a
 // dependent chain of loads would cost a round trip each, and so does every further batch)
-__device__ __forceinline__ uint32_t topk_mw_colsum(const uint32_t *__restrict__ p, int count, int stride = 256) {
+__device__ __forceinline__ uint32_t topk_mw_colsum(const uint32_t *__restrict__ p, int count) {
     uint32_t c = 0u;
     for (int w0 = 0; w0 < count; w0 += 32) {
         uint32_t v[32];
 #pragma unroll
         for (int j = 0; j < 32; j++) {
             const int w = w0 + j < count ? w0 + j : count - 1;      // clamped, not guarded: a guarded load is a branch
-            v[j] = p[(size_t)w * stride];
+            v[j] = p[(size_t)w * 256];
         }
 #pragma unroll
         for (int j = 0; j < 32; j++) c += w0 + j < count ? v[j] : 0u;
