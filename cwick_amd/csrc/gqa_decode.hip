@@ -10,8 +10,11 @@
 //   serves every head of its group, src/q35_model.c:1417-1423).  A wave takes tiles of 16 keys.
 //   At any time the workgroups read neighbouring steps, which lie in all channels of the memory.
 //   (A contiguous slice each: where its length is a multiple of a power of two, the slices are in the same
-//   channels at the same time.  64 heads on 8 x 128: 65536 keys 57.1 us, 50.5 so; 131072 103.0 and 95.3; 100003
-//   77.8 and 73.9; 33000 29.1 and 28.5.)
+//   channels at the same time.  64 heads on 8 x 128, a call on the caches of one layer after the other, some 6 GB of
+//   them: 65536 keys 58.0 us, 50.3 so; 131072 103.3 and 94.7; 100003 76.2 and 70.3; 33000 29.9 and 28.9; on the same
+//   caches again 57.1, 50.5; 103.0, 95.3; 77.8, 73.9; 29.1, 28.5.  Alone behind 512 MB written to other memory, 100003
+//   142 and 137.  The one place where it is the slower: alone on caches that were written whole just before, so that
+//   what the chip's memory cache still has is read in another order, 109.5 and 114.)
 //
 //   scores:  S[key][head] = K Q^T, v_mfma_f32_16x16x32_bf16 straight from registers: lane l reads
 //            16 bytes of key l%16 per load, which is the A operand as it lies in the cache.  The

@@ -836,10 +836,11 @@ gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restr
 // 1.65 us, 2.1 with every compute unit at it (2048 cycles of it matrix instructions), and what is in the way is
 // the copies.  One buffer each for K and V: K(u + 1) is on its way during the softmax and the value products of
 // tile u, V(u + 1) during the next scores.
-// 1000 positions of 16 heads 47.7 -> 31.5 us, 360: 22.9 -> 17.5, 100: 16.5 -> 11.7, 16: 10.2 -> 7.6 (the
-// launches of a call); 1000 of 8 / 8 heads 41.4 -> 24.5; 2500 of 16 105 -> 87; 29 behind 3219 29 -> 21.8 (23.4 with
-// the merge of the slices alone), 128 of 8 / 8 behind 1800 30.4 -> 22.6.  Long chunks go the other way: 517
-// behind 7083 take 115 us on 132 such workgroups, 104 in two slices each.
+// The launches of a call, against workgroups of one wave for few rows and 256 rows for more, with the plans and the
+// merge of that time: 1000 positions of 16 heads 49.9 -> 33.4 us, 360: 22.8 -> 18.4, 100: 16.6 -> 12.3, 16: 10.6 -> 8.7;
+// 1000 of 8 / 8 heads 42.5 -> 25.6; 2500 of 16 105 -> 89; 29 behind 3219 26.4 -> 17.5, 128 of 8 / 8 behind 1800
+// 27.2 -> 16.7, 16 behind 16000 43.7 -> 24.2.  Long chunks go the other way: 517 behind 7083 take 115 us on 132 such
+// workgroups, 104 in two slices each.
 struct PfTeamSmem {
     unsigned char k[PF_WAVES][PF_TILE], v[PF_WAVES][PF_TILE];   // at the end: the accumulators that change hands
     unsigned char q[PF_TILE];                                   // query rows 32 .. 63 (block B)
@@ -1283,8 +1284,8 @@ gqa_prefill_team_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
 // Combines the slices of a block: out = sum_s 2^(m_s - M) acc_s / sum_s 2^(m_s - M) l_s.  A wave
 // takes 32 rows x 8 dims (one KiB of the partials per slice, one load), a workgroup a 32-dim output block.
 // What it waits for is the partials' way from memory, so the loads of BATCH slices are in flight at once and
-// few rows make many waves: 16 positions behind 16000 on four kv heads (64 slices) took 46.6 us of which this
-// kernel had 17, and take 32.3 (a wave for four times the dims, four slices at a time, before).  Blocks of up
+// few rows make many waves: 16 positions behind 16000 on four kv heads (64 slices) took 46.6 us, with their
+// preparation, of which this kernel had 17, and 32.3 so (a wave for four times the dims, four slices at a time, before).  Blocks of up
 // to eight slices are shorter with eight (2500 positions 103 us against 108): the registers of sixteen cost
 // waves.
 template <int GROUP, int WAVES, int BATCH>

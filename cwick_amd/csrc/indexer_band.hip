@@ -105,7 +105,8 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
     const uint8_t *kb = keys + (size_t)b * key_bstride;
     const float *ksb = kscale + (size_t)b * kscale_bstride;
     // (the waves' blocks of 32 keys side by side, 32 KB per turn of the workgroup: a stretch for each wave put all waves
-    // of the chip at the same place of a 32 KB piece.  8 rows of 65536 keys of 64 heads 50.7 -> 50.4 us, of 32 49.2 -> 47.6)
+    // of the chip at the same place of a 32 KB piece.  8 rows of 65536 keys of 64 heads again and again 52.3 -> 51.4 us, of
+    // 32 49.1 -> 48.5; on keys that the chip's memory cache does not have no difference, 56.4 to 57.7 and 53.3 to 54.8)
     const int64_t wbase = (int64_t)wg * IB_KEYS + wave * 32;
     constexpr int IB_TURN = IB_WAVES * 32, N_IT = IB_KEYS / IB_TURN;
     // the key bytes and the scale of an iteration are loaded two iterations ahead
