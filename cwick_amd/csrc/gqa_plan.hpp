@@ -30,100 +30,159 @@ __host__ __device__ inline int pf_slices(int tiles, int plain, int per) {
 }
 
 // What a kernel's workgroups take, in microseconds: the launch, a workgroup besides its tiles, a step of
-// `waves` tiles (with two-term weights; what it takes longer when every compute unit is at work all the time),
-// and, where there are slices, the second launch, more for each slice of a block, and each slice's partials
-// (written and read).  Fitted to 150 times of 21 shapes for the first and 170 of 52 for the second (16 to 8192
-// positions behind 0 to 16000, between none and sixty slices); the times of list scheduling with these
-// figures are 3.4 and 5.5 % off them (rms).
+// `waves` tiles (with two-term weights; what it takes longer where every compute unit of its XCD is at work all the
+// time, and from which share of them on it takes longer at all), and, where there are slices, the second launch, more
+// for each slice of a block, and each slice's partials (written and read).
+// Fitted to 20500 times of 1049 shapes (1 to 8192 positions behind 0 to 16000 of one to eight heads on one to
+// eight kv heads, whole and in slices): of the plans of a shape the one with the least price is 0.3 % behind the
+// fastest on the mean, 10 % at the worst; the prices of plans near the fastest are 3.6 and 5.4 % off (rms).
+// What counts is the share of an XCD's own units that are at work, and up to a third or a half of them it adds nothing:
+// 1.21 us a tile with up to half of them, 1.33 with 64 %, 1.55 with 90.  With the mean of the chip, and in
+// proportion from the first unit on, two slices a block (the long ones of which lie on half of the XCDs, where there
+// are four kv heads) looked shorter than four, and whole blocks of 64 rows shorter than slices: 2500 positions
+// behind 4000 of 16 / 4 heads 287 us, now 252; 2800 298, 271; 4000 of 8 / 8 240, 211.
 struct PfCost {
     int waves, least;                       // tiles of a step; the fewest tiles of a slice
-    float launch, item, step, step2, crowd, merge, merge_slice, merge_part;
+    float launch, item, step, step2, crowd, alone, merge, merge_slice, merge_part;
 };
-constexpr PfCost PF_COST_WIDE = {1, 4, 7.0f, 5.0f, 1.19f, 2.19f, 0.45f, 3.7f, 0.05f, 0.085f};       // 256 rows
-constexpr PfCost PF_COST_TEAM = {4, 4, 2.3f, 7.1f, 1.64f, 2.3f, 0.46f, 2.2f, 0.065f, 0.023f};       // 64 rows
+constexpr PfCost PF_COST_WIDE = {1, 4, 0.8f, 9.6f, 1.22f, 2.135f, 0.411f, 0.36f, 4.8f, 0.021f, 0.063f};      // 256 rows
+constexpr PfCost PF_COST_TEAM = {4, 4, 2.5f, 7.25f, 1.815f, 2.46f, 0.362f, 0.44f, 2.5f, 0.072f, 0.016f};      // 64 rows
 
 struct PfBlocks {
     int count, n_kv_heads, n_prec, cus;     // the first n_prec blocks take two-term weights
     int tiles[PF_MAX_BLOCKS], plain[PF_MAX_BLOCKS];     // by rank
 };
 
-// The time of a plan, or anything from `limit` on where it takes at least that, and its slices of blocks that are
-// cut.  The kernels hand their workgroups out in the order of the ranks, each to the compute unit that is
-// free first.
-inline float pf_time(const PfBlocks &b, const PfCost &c, int per, float limit, int &parts) {
-    int items = 0, most = 1;
-    parts = 0;
-    uint16_t cut[PF_MAX_BLOCKS];            // slices of each block
+// What a plan comes to: its slices of each block, how many of them belong to blocks that are cut, the time of their
+// merge, and with their sums the least time: the even share or the longest, with the units of all XCDs at
+// work alike (seldom more than it is).
+struct PfSums {
+    int items, parts;
+    float end, sum, sum_steps, least;
+    uint16_t cut[PF_MAX_BLOCKS];
+};
+inline float pf_steps(const PfCost &c, int tiles) { return (float)(c.waves == 1 ? tiles : (tiles + 3) / 4); }
+inline float pf_slice_time(const PfBlocks &b, const PfCost &c, int r, int tiles) {
+    return c.item + (b.count - 1 - r < b.n_prec ? c.step2 : c.step) * pf_steps(c, tiles);
+}
+// what a step takes longer, from the share of the units at work when they start and the mean of it: it falls evenly
+inline float pf_slower(const PfCost &c, float at_first, float mean) {
+    const float at_last = 2.0f * mean - at_first, room = 1.0f - c.alone;
+    if (at_last >= c.alone || at_first <= at_last) return mean > c.alone ? c.crowd * (mean < 1.0f ? mean - c.alone : room) / room : 0.0f;
+    if (at_first <= c.alone) return 0.0f;
+    const float over = at_first - c.alone;
+    return c.crowd * over * over / (2.0f * (at_first - at_last) * room);
+}
+inline void pf_sums(const PfBlocks &b, const PfCost &c, int per, PfSums &p) {
+    int most = 1;
+    float longest = 0.0f, longest_steps = 0.0f;
+    const float full_steps = pf_steps(c, per);
+    p.items = p.parts = 0;
+    p.sum = p.sum_steps = 0.0f;
     for (int r = 0; r < b.count; r++) {
-        const int k = per && b.tiles[r] > per ? pf_slices(b.tiles[r], b.plain[r], per) : 1;
-        cut[r] = (uint16_t)k;
-        items += k;
-        if (k > 1) parts += k;
+        const int k = per && b.tiles[r] > per ? pf_slices(b.tiles[r], b.plain[r], per) : 1, left = b.tiles[r] - (k - 1) * per;
+        const float rest = pf_slice_time(b, c, r, left), rest_steps = pf_steps(c, left);
+        p.cut[r] = (uint16_t)k;
+        p.items += k;
+        p.sum += rest;
+        p.sum_steps += rest_steps;
+        if (rest > longest) longest = rest, longest_steps = rest_steps;
+        if (k == 1) continue;
+        const float full = pf_slice_time(b, c, r, per);
+        p.parts += k;
+        p.sum += full * (float)(k - 1);
+        p.sum_steps += full_steps * (float)(k - 1);
         if (k > most) most = k;
+        if (full > longest) longest = full, longest_steps = full_steps;
     }
-    const int n = items * b.n_kv_heads;
-    const float end = parts ? c.merge + c.merge_slice * (float)most + c.merge_part * (float)(parts * b.n_kv_heads) : 0.0f;
-    auto steps = [&](int tiles) { return (float)(c.waves == 1 ? tiles : (tiles + 3) / 4); };
-    auto step = [&](int r) { return b.count - 1 - r < b.n_prec ? c.step2 : c.step; };
-    float sum = 0.0f, sum_steps = 0.0f, longest = 0.0f, longest_steps = 0.0f;
-    auto add = [&](int r, int tiles, int times) {
-        const float x = steps(tiles), t = c.item + step(r) * x;
-        sum += t * (float)times;
-        sum_steps += x * (float)times;
-        if (t > longest) longest = t, longest_steps = x;
-    };
-    for (int r = 0; r < b.count; r++) {
-        const int k = cut[r];
-        add(r, b.tiles[r] - (k - 1) * per, 1);
-        if (k > 1) add(r, per, k - 1);
-    }
-    const float share = (float)b.n_kv_heads / (float)b.cus;
-    const float crowd = c.crowd * (sum * share < longest ? sum * share / longest : 1.0f);
-    const float even = (sum + crowd * sum_steps) * share, alone = longest + crowd * longest_steps;
-    const float least = even > alone ? even : alone;
-    auto cost = [&](int r, int tiles) { return c.item + (step(r) + crowd) * steps(tiles); };
-    if (n <= b.cus || c.launch + least + end >= limit) return c.launch + least + end;
-    // list scheduling, the kv heads of a slice as one where they go into the compute units evenly
-    const bool joint = b.cus % b.n_kv_heads == 0;
+    p.end = p.parts ? c.merge + c.merge_slice * (float)most + c.merge_part * (float)(p.parts * b.n_kv_heads) : 0.0f;
+    const float part_of = (float)b.n_kv_heads / (float)b.cus, even = p.sum * part_of;
+    const float x = pf_slower(c, (float)p.items * part_of < 1.0f ? (float)p.items * part_of : 1.0f, even / longest);
+    const float even_x = even + x * p.sum_steps * part_of, longest_x = longest + x * longest_steps;
+    p.least = c.launch + (even_x > longest_x ? even_x : longest_x) + p.end;
+}
+
+// The time of a plan, or anything from `limit` on where it takes at least that.  The kernels hand their workgroups out
+// in the order of the ranks, the first to the XCDs in turn and the others each to the compute unit that is free first.
+inline float pf_time(const PfBlocks &b, const PfCost &c, int per, const PfSums &p, float limit) {
+    const bool joint = b.cus % b.n_kv_heads == 0;       // the kv heads of a slice as one where they go into the units evenly
     const int machines = joint ? b.cus / b.n_kv_heads : b.cus, copies = joint ? 1 : b.n_kv_heads;
-    float heap[1024];                       // when each is free, the first to be at the top
-    if (machines > 1024) return c.launch + least + end;
-    int used = 0;
-    float last = 0.0f;
-    auto deal = [&](float t) {
-        if (used < machines) {              // one that has had nothing yet (the heap is made when there is none left)
-            heap[used++] = t;
-            last = t > last ? t : last;
-            if (used < machines) return;
-            for (int i = machines / 2 - 1; i >= 0; i--) {
-                const float v = heap[i];
-                int j = i;
-                for (int ch; (ch = 2 * j + 1) < machines; j = ch) {
-                    if (ch + 1 < machines && heap[ch + 1] < heap[ch]) ch++;
-                    if (heap[ch] >= v) break;
-                    heap[j] = heap[ch];
-                }
-                heap[j] = v;
+    const int kv = b.n_kv_heads, groups = !joint || kv % 8 == 0 ? 1 : kv % 4 == 0 ? 2 : kv % 2 == 0 ? 4 : 8;
+    const bool at_once = p.items * copies <= machines;
+    if (machines > 1024 || (at_once && groups == 1)) return p.least;
+    // what the XCDs of each group (those of the slices with its remainder) do, and until when
+    float busy[8] = {}, last[8] = {}, start[8] = {};
+    if (at_once) {
+        int i = 0;
+        for (int g = 0; g < groups; g++) start[g] = (float)((p.items - g + groups - 1) / groups * groups) / (float)machines;
+        for (int r = 0; r < b.count; r++) {
+            const int k = p.cut[r];
+            const float rest = pf_slice_time(b, c, r, b.tiles[r] - (k - 1) * per), full = k > 1 ? pf_slice_time(b, c, r, per) : 0.0f;
+            for (int g = 0; g < groups && g < k - 1; g++) {
+                const int to = (i + g) % groups;
+                busy[to] += full * (float)((k - 2 - g) / groups + 1);
+                last[to] = full > last[to] ? full : last[to];
             }
-            return;
+            i += k;
+            const int to = (i - 1) % groups;
+            busy[to] += rest;
+            last[to] = rest > last[to] ? rest : last[to];
         }
-        const float v = heap[0] + t;
-        last = v > last ? v : last;
-        int j = 0;
-        for (int ch; (ch = 2 * j + 1) < machines; j = ch) {
-            if (ch + 1 < machines && heap[ch + 1] < heap[ch]) ch++;
-            if (heap[ch] >= v) break;
-            heap[j] = heap[ch];
+    } else {
+        // list scheduling
+        for (int g = 0; g < groups; g++) start[g] = 1.0f;
+        float free_at[1024], latest = 0.0f;             // the first to be free at the top, once each has had a slice
+        uint8_t of[1024];
+        int used = 0;
+        auto sink = [&](int at) {
+            const float v = free_at[at];
+            const uint8_t g = of[at];
+            int j = at;
+            for (int ch; (ch = 2 * j + 1) < machines; j = ch) {
+                if (ch + 1 < machines && free_at[ch + 1] < free_at[ch]) ch++;
+                if (free_at[ch] >= v) break;
+                free_at[j] = free_at[ch];
+                of[j] = of[ch];
+            }
+            free_at[j] = v;
+            of[j] = g;
+        };
+        auto deal = [&](float t) {
+            const bool first = used < machines;
+            const int at = first ? used : 0;
+            if (first) free_at[at] = 0.0f, of[at] = (uint8_t)(used % groups);
+            const float until = free_at[at] + t;
+            const int g = of[at];
+            free_at[at] = until;
+            busy[g] += t;
+            last[g] = until > last[g] ? until : last[g];
+            latest = until > latest ? until : latest;
+            if (!first) sink(0);
+            else if (++used == machines)
+                for (int i = machines / 2 - 1; i >= 0; i--) sink(i);
+        };
+        for (int r = 0; r < b.count && c.launch + latest + p.end < limit; r++) {
+            const int k = p.cut[r];
+            const float rest = pf_slice_time(b, c, r, b.tiles[r] - (k - 1) * per), full = k > 1 ? pf_slice_time(b, c, r, per) : 0.0f;
+            for (int i = 0; i < k; i++)
+                for (int n = 0; n < copies; n++) deal(i + 1 < k ? full : rest);
         }
-        heap[j] = v;
-    };
-    for (int r = 0; r < b.count && c.launch + last + end < limit; r++) {
-        const int k = cut[r];
-        const float rest = cost(r, b.tiles[r] - (k - 1) * per), full = k > 1 ? cost(r, per) : rest;
-        for (int i = 0; i < k; i++)
-            for (int x = 0; x < copies; x++) deal(i + 1 < k ? full : rest);
     }
-    return c.launch + last + end;
+    float t = 0.0f;
+    for (int g = 0; g < groups; g++) {
+        if (last[g] == 0.0f) continue;
+        const float until = last[g] * (1.0f + pf_slower(c, start[g], busy[g] * (float)groups / ((float)machines * last[g])) * p.sum_steps / p.sum);
+        t = until > t ? until : t;
+    }
+    return c.launch + t + p.end;
+}
+
+// the same with the sums of the plan, and its slices of blocks that are cut
+inline float pf_time(const PfBlocks &b, const PfCost &c, int per, float limit, int &parts) {
+    PfSums p;
+    pf_sums(b, c, per, p);
+    parts = p.parts;
+    return p.least >= limit ? p.least : pf_time(b, c, per, p, limit);
 }
 
 // The best plan of one kernel for a chunk whose blocks have `positions` positions each (at most PF_MAX_BLOCKS of
@@ -150,17 +209,17 @@ inline float pf_plan(int64_t pos0, int64_t n, int positions, int n_kv_heads, int
         total += b.tiles[r];
     }
     const int most = b.tiles[0];
-    float best_t = limit;
-    int best_per = -1;
-    int best_parts = 0;
-    // (Of two plans within 2 % the one with fewer slices: 700 positions behind 12000 take 157 us in 220 slices and
-    // 159 to 171, for the same by these figures, in 244.)
+    // the plans to try: their slice lengths, and what each takes at least
+    int tries = 0, pers[24];
+    float least[24];
+    PfSums sums;
     auto look = [&](int per) {
-        if (per && (per < c.least || per >= most)) return;
-        int parts;
-        const float t = pf_time(b, c, per, 1.02f * best_t, parts);
-        if (t < limit && (best_per < 0 ? t < best_t : parts < best_parts ? t < 1.02f * best_t : t < 0.98f * best_t))
-            best_t = t, best_per = per, best_parts = parts;
+        if ((per && (per < c.least || per >= most)) || tries == 24) return;
+        for (int i = 0; i < tries; i++)
+            if (pers[i] == per) return;
+        pf_sums(b, c, per, sums);
+        pers[tries] = per;
+        least[tries++] = sums.least;
     };
     look(0);
     const int room = cus / n_kv_heads;      // slices for one round
@@ -184,14 +243,31 @@ inline float pf_plan(int64_t pos0, int64_t n, int positions, int n_kv_heads, int
             while (!fits(fit)) fit = round_up(fit + 1 + fit / 16);
             for (int back = fit / 16; back > 0 && fit - c.waves >= c.least && fits(fit - c.waves); back -= c.waves) fit -= c.waves;
             look(fit);
-            const int cuts = pf_slices(most, b.plain[0], fit);      // one slice fewer for the longest block, if that is even
-            if (cuts > 1 && cuts < 12) look(round_up((most + cuts - 2) / (cuts - 1)));
+            const int cuts = pf_slices(most, b.plain[0], fit);      // as many even slices for the longest block, and one fewer
+            if (cuts > 1 && cuts < 12) look(round_up((most + cuts - 1) / cuts)), look(round_up((most + cuts - 2) / (cuts - 1)));
             if (rounds == 1)
                 for (int quarters : {5, 6, 8, 12}) look(round_up((int64_t)fit * quarters / 4));
         }
     }
     if (!whole && 2 * b.count >= room && 2 * b.count <= 3 * room)
         for (int eighths : {7, 6, 5, 4}) look((most * eighths + 7) / 8);
+    // The ones that may be the shortest first.  (Of the plans within 2 % of the shortest the one with the fewest slices: 700
+    // positions behind 12000 take 157 us in 220 slices and 159 to 171, for the same by these figures, in 244.)
+    float low = limit, best_t = limit;
+    int best_per = -1, best_parts = 0;
+    for (;;) {
+        int next = -1;
+        for (int i = 0; i < tries; i++)
+            if (least[i] >= 0.0f && (next < 0 || least[i] < least[next])) next = i;
+        if (next < 0 || least[next] >= limit || least[next] >= 1.02f * low) break;
+        least[next] = -1.0f;
+        int parts;
+        const float t = pf_time(b, c, pers[next], 1.02f * low, parts);
+        if (t >= limit || t >= 1.02f * low) continue;
+        low = t < low ? t : low;
+        if (best_per < 0 || best_t >= 1.02f * low || parts < best_parts || (parts == best_parts && t < best_t))
+            best_t = t, best_per = pers[next], best_parts = parts;
+    }
     if (best_per < 0) return limit;
     best.per = best_per;
     best.first[0] = 0;

@@ -261,7 +261,7 @@ int cwick_hip_dsa_decode(cwick_hip_ikeys *ik, cwick_hip_latent *lat, int slot0, 
  * each call once before capturing it, or size the workspace up front with
  * cwick_hip_reserve_dev().  A decode asks for what any shorter one needs as well;
  * a prefill may take more than a longer one, which fills the chip uncut: at most
- * 256 MiB for the GQA prefill (64 for 517 positions behind 7083) and 132 for the
+ * 258 MiB for the GQA prefill (64 for 517 positions behind 7083) and 132 for the
  * MLA chunk (15 for 8 queries of 128 heads behind 20000 rows).  The split-K partials and the
  * ticket counters of the GQA prefill and of GQA decodes of up to 16 splits belong to the stream: two calls
  * that use one stream's workspace at the same time (a graph replayed on another stream

@@ -148,6 +148,48 @@ int main() {
 }"""))
 
 
+def test_gqa_prefill_prices_follow_measured_plans(tmp_path):
+    """The prices of plans that were timed (us): the faster of two has the lesser price, and none is a tenth off.  Two
+    slices a block where the long ones lie on half of the XCDs; few units at work; the plan made of such a shape
+    is within 5 % of the faster one (not all slice lengths are tried)."""
+    print(run_cpp(tmp_path, "gqa_plan.hpp", r"""
+struct Timed { int rows, per; float us; };
+int main() {
+    const struct { int64_t n, pos0; int heads, kv; Timed fast, slow; } shapes[] = {
+        {2500, 4000, 16, 4, {256, 68, 251.4f}, {256, 152, 275.6f}}, {2500, 4000, 16, 2, {256, 59, 242.5f}, {256, 152, 270.7f}},
+        {2800, 8000, 16, 4, {256, 0, 447.3f}, {256, 282, 480.9f}}, {2800, 8000, 16, 2, {256, 113, 446.1f}, {256, 282, 477.9f}},
+        {3900, 6000, 8, 8, {256, 155, 267.4f}, {64, 0, 307.0f}}, {4000, 4000, 8, 8, {256, 125, 207.8f}, {64, 0, 237.6f}},
+        {3700, 4000, 8, 8, {256, 121, 195.7f}, {64, 0, 213.4f}}, {1000, 16000, 8, 8, {256, 67, 138.5f}, {256, 66, 145.7f}},
+    };
+    for (auto &s : shapes) {
+        static PfBlocks b[2];
+        float t[2], best = INFINITY;
+        for (int i = 0; i < 2; i++) {
+            const Timed &p = i ? s.slow : s.fast;
+            const int P = p.rows * s.kv / s.heads;
+            b[i].count = (int)((s.n + P - 1) / P), b[i].n_kv_heads = s.kv, b[i].n_prec = 0, b[i].cus = 256;
+            for (int r = 0; r < b[i].count; r++) {
+                const int64_t pb = b[i].count - 1 - r;
+                b[i].tiles[r] = (int)((pf_keys(s.pos0, s.n, P, pb) + PF_TK - 1) / PF_TK);
+                b[i].plain[r] = (int)((s.pos0 + pb * P + 1) / PF_TK);
+            }
+            int parts;
+            t[i] = pf_time(b[i], p.rows == 64 ? PF_COST_TEAM : PF_COST_WIDE, p.per, INFINITY, parts);
+            if (std::fabs(t[i] / p.us - 1.0f) > 0.1f) { printf("%d behind %d: %d rows, %d tiles %.1f, took %.1f\n", (int)s.n, (int)s.pos0, p.rows, p.per, t[i], p.us); return 1; }
+        }
+        if (t[0] >= t[1]) { printf("%d behind %d of %d / %d: %.1f and %.1f\n", (int)s.n, (int)s.pos0, s.heads, s.kv, t[0], t[1]); return 1; }
+        for (int rows : {64, 256}) {
+            PfPlan p;
+            const int P = rows * s.kv / s.heads;
+            if ((s.n + P - 1) / P > PF_MAX_BLOCKS) continue;
+            best = std::fmin(best, pf_plan(s.pos0, s.n, P, s.kv, 0, 256, rows == 64 ? PF_COST_TEAM : PF_COST_WIDE, INFINITY, p));
+        }
+        if (best > 1.05f * t[0]) { printf("%d behind %d of %d / %d: planned %.1f, there is %.1f\n", (int)s.n, (int)s.pos0, s.heads, s.kv, best, t[0]); return 1; }
+    }
+    return 0;
+}"""))
+
+
 def test_gqa_prefill_plans_are_sound_and_quick(tmp_path):
     """The plans of both prefill kernels: the slices of every block cover its tiles, each begins below the
     diagonal and none is empty, there is room for the partials' numbers; less than a
