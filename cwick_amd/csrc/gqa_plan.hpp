@@ -218,6 +218,7 @@ inline float pf_plan(int64_t pos0, int64_t n, int positions, int n_kv_heads, int
         for (int i = 0; i < tries; i++)
             if (pers[i] == per) return;
         pf_sums(b, c, per, sums);
+        if (per && sums.items * n_kv_heads > 4 * cus) return;   // (memory for the partials: 258 MiB for 1024 slices of 256 rows)
         pers[tries] = per;
         least[tries++] = sums.least;
     };

@@ -223,6 +223,7 @@ int main() {
                                 b.plain[r] = (int)((pos0 + pb * P + 1) / PF_TK);
                                 const int k = p.first[r + 1] - p.first[r];
                                 ok = ok && k >= 1 && (p.per || k == 1);
+                                ok = ok && (!p.per || p.first[b.count] * kv <= 4 * cus);       // the most that the header names
                                 if (k > 1) ok = ok && (int64_t)(k - 1) * p.per < b.tiles[r] && (int64_t)(k - 1) * p.per * PF_TK <= pos0 + pb * P + 1;
                             }
                             if (!ok) { printf("bad plan: %d rows, %d at %d, %d kv heads of %d\n", rows, (int)n, (int)pos0, kv, group); return 1; }
