@@ -238,7 +238,7 @@ inline float pf_plan(int64_t pos0, int64_t n, int positions, int n_kv_heads, int
             fit = fit < c.least ? c.least : fit;
             auto fits = [&](int per) {
                 int items = 0;
-                for (int r = 0; r < b.count; r++) items += b.tiles[r] > per ? pf_slices(b.tiles[r], b.plain[r], per) : 1;
+                for (int r = 0; r < b.count && items <= rounds * room; r++) items += b.tiles[r] > per ? pf_slices(b.tiles[r], b.plain[r], per) : 1;
                 return items <= rounds * room;
             };
             while (!fits(fit)) fit = round_up(fit + 1 + fit / 16);
