@@ -79,21 +79,12 @@ typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
 typedef __attribute__((address_space(3))) float lds_f32;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
-struct WideParams {
-    const uint8_t *rows;
-    const float *scales;
-    const uint16_t *q;        // [nq][nh][576] bf16
+// What a workgroup needs late; the rest are arguments of the kernel's own, in registers (see mla_roles.hip).
+struct WideRest {
     float *out;               // [nq][nh][512]
-    int pos0;                 // query y sees rows 0 .. pos0 + y
-    int nh;
-    uint32_t nhb, nhb_inv;    // 16-head blocks of a query; 2^31 / nhb, rounded up
-    uint32_t n_rb;            // row blocks of the chunk: block rb is heads 16 (rb % nhb) .. of query rb / nhb
-    uint32_t gsz;             // row blocks of a group: four, or fewer where groups of four leave the chip idle
-    uint32_t n_whole;         // the last groups, a workgroup each; the first n_rest
-    uint32_t n_rest, n_slices, slices_inv;    // groups take n_slices workgroups each and leave partials
-    float scale;
     float *part_ml;           // as in mla_roles.hip, [group of n_rest][slice][row block of the group]
     float *part_acc;
+    float scale;
 };
 
 // what a position past the end of a query's keys is fetched from (see mla_roles.hip)
@@ -180,12 +171,22 @@ __device__ __forceinline__ void scaled_by_row_lane(float &d, float r, float x, i
 // code.  A compute unit starts a launch with a cold instruction cache, and straight-line code costs it
 // about 150 cycles per 64 bytes: unrolled, what lies around the loops took 20 000 cycles of a
 // workgroup whose key tile takes 4 000.
+// q: [nq][nh][576] bf16; query y sees rows 0 .. pos0 + y.  shape: the heads nh of a query in the low eight bits,
+// above them the row blocks of a group, gsz: four, or fewer where groups of four leave the chip idle.
+// nhb_inv: 2^31 / nhb, rounded up, for the nhb = 16-head blocks of a query.  n_rb: row blocks of the chunk, block rb
+// is heads 16 (rb % nhb) .. of query rb / nhb.  The last n_whole groups take a workgroup each; the first n_rest
+// take p_slices workgroups each and leave partials; slices_inv as nhb_inv.
 template <bool SPAN>
-__global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams p) {
+__global__ void __launch_bounds__(THREADS)
+mla_prefill64_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all_rows, const float *__restrict__ all_scales,
+                     int pos0, uint32_t shape, uint32_t nhb_inv, uint32_t n_rb, uint32_t n_whole, uint32_t n_rest,
+                     uint32_t p_slices, uint32_t slices_inv, const WideRest p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     Smem &sm = *reinterpret_cast<Smem *>(smem_raw);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void *)smem_raw;
 
+    const int nh = (int)(shape & 255u);
+    const uint32_t gsz = shape >> 8, nhb = (uint32_t)(nh + 15) / 16;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -201,29 +202,29 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
     // contiguous eighth of the queries per XCD left the XCD with the longest ones 6 % behind).
     // The queries with the most keys start first, the groups in slices last.
     uint32_t grp, slice = 0, n_slices = 1;
-    const bool sliced = blockIdx.x >= p.n_whole;
+    const bool sliced = blockIdx.x >= n_whole;
     if (!sliced) {
         uint32_t i = blockIdx.x;
-        const uint32_t lg = p.nhb == 2 * p.gsz ? 4 : 3, lot = i >> lg, r = i & ((1u << lg) - 1);     // eight queries of one or two groups
-        if (((lot + 1) << lg) <= p.n_whole) i = ((8 * lot + r % 8) << (lg - 3)) + r / 8;
-        grp = p.n_rest + p.n_whole - 1 - i;
+        const uint32_t lg = nhb == 2 * gsz ? 4 : 3, lot = i >> lg, r = i & ((1u << lg) - 1);     // eight queries of one or two groups
+        if (((lot + 1) << lg) <= n_whole) i = ((8 * lot + r % 8) << (lg - 3)) + r / 8;
+        grp = n_rest + n_whole - 1 - i;
     } else {
-        n_slices = p.n_slices;
-        const uint32_t i = blockIdx.x - p.n_whole, above = div_by(i, p.slices_inv);
-        grp = p.n_rest - 1 - above;
+        n_slices = p_slices;
+        const uint32_t i = blockIdx.x - n_whole, above = div_by(i, slices_inv);
+        grp = n_rest - 1 - above;
         slice = i - above * n_slices;
     }
     // the query of row block h of the group (past the end of the chunk: its last row block again, not stored)
     // (and past the end of a smaller group its last one)
     auto rb_of = [&](uint32_t h) -> uint32_t {
-        const uint32_t rb = p.gsz * grp + (h < p.gsz ? h : p.gsz - 1);
-        return rb < p.n_rb ? rb : p.n_rb - 1;
+        const uint32_t rb = gsz * grp + (h < gsz ? h : gsz - 1);
+        return rb < n_rb ? rb : n_rb - 1;
     };
-    const int keys_hi = p.pos0 + 1 + (int)div_by(rb_of(NHQ - 1), p.nhb_inv);      // of the group's last query
+    const int keys_hi = pos0 + 1 + (int)div_by(rb_of(NHQ - 1), nhb_inv);      // of the group's last query
     const uint32_t all_tiles = ((uint32_t)keys_hi + TK - 1) / TK;
     uint32_t t_first = 0, t_end = all_tiles;
     if (sliced) {
-        const uint32_t per = div_by(all_tiles + n_slices - 1, p.slices_inv);
+        const uint32_t per = div_by(all_tiles + n_slices - 1, slices_inv);
         t_first = slice * per < all_tiles ? slice * per : all_tiles;
         t_end = t_first + per < all_tiles ? t_first + per : all_tiles;
     }
@@ -231,9 +232,9 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
     // from here on positions count from the slice's first key
     const int key0 = (int)t_first * TK;
     const int n_keys = t_end == all_tiles ? keys_hi - key0 : n_tiles * TK;
-    auto keys_of = [&](uint32_t h) -> int { return p.pos0 + 1 + (int)div_by(rb_of(h), p.nhb_inv) - key0; };
-    const uint8_t *rows = p.rows + (size_t)key0 * KDIM;
-    const float *scales = p.scales + (size_t)key0 * NBLK;
+    auto keys_of = [&](uint32_t h) -> int { return pos0 + 1 + (int)div_by(rb_of(h), nhb_inv) - key0; };
+    const uint8_t *rows = all_rows + (size_t)key0 * KDIM;
+    const float *scales = all_scales + (size_t)key0 * NBLK;
 
     uint64_t zrow = (uint64_t)(uintptr_t)g_zero_row64, zsc = (uint64_t)(uintptr_t)g_zero_scales64;
     asm volatile("" : "+s"(zrow), "+s"(zsc));
@@ -313,15 +314,15 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
     // Piece x (16 bytes) of head h sits at place x ^ h of the head's sixteen, so that the sixteen heads of
     // a fragment read come from different banks.
 #pragma clang loop unroll(disable)
-    for (int u = wave; u < 5 * (int)p.gsz; u += NWAVES) {
+    for (int u = wave; u < 5 * (int)gsz; u += NWAVES) {
         const int hqu = (u * 13) >> 6, b = u - 5 * hqu;           // u / 5 for u < 20
-        const uint32_t rb = rb_of((uint32_t)hqu), y = div_by(rb, p.nhb_inv);
-        const int head0 = 16 * (int)(rb - y * p.nhb);
-        const uint64_t base = (uint64_t)(uintptr_t)(p.q + (size_t)y * p.nh * KDIM + 128 * b);
+        const uint32_t rb = rb_of((uint32_t)hqu), y = div_by(rb, nhb_inv);
+        const int head0 = 16 * (int)(rb - y * nhb);
+        const uint64_t base = (uint64_t)(uintptr_t)(q + (size_t)y * nh * KDIM + 128 * b);
         const uint32_t pu = lds0 + PARK + (uint32_t)u * PARK_UNIT;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const int h = 4 * c + g, head = head0 + h < p.nh ? head0 + h : p.nh - 1;
+            const int h = 4 * c + g, head = head0 + h < nh ? head0 + h : nh - 1;
             const int x = (n ^ h) & (b < 4 ? 15 : 7);             // the rope block has eight pieces: fetched twice
             dma16(base + (uint64_t)(uint32_t)head * (KDIM * 2) + (uint32_t)(16 * x), pu + (uint32_t)c * 1024);
         }
@@ -334,7 +335,7 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
     }
     {
 #pragma clang loop unroll(disable)
-        for (int u = wave; u < 5 * (int)p.gsz; u += NWAVES) {
+        for (int u = wave; u < 5 * (int)gsz; u += NWAVES) {
             const uint32_t pu = lds0 + PARK + (uint32_t)u * PARK_UNIT, pr = pu + (uint32_t)lane * 16;
             u32x4 w[4];                                           // head n, pieces 4 g .. (rope: 4 (g & 1) ..)
 #pragma unroll
@@ -378,7 +379,7 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
             const u32x4 x = LDS_AT(lds_u32x4, a), y = LDS_AT(lds_u32x4, a + 1024);
             return (i32x8){(int)x[0], (int)x[1], (int)x[2], (int)x[3], (int)y[0], (int)y[1], (int)y[2], (int)y[3]};
         };
-        const uint32_t hp = (uint32_t)hq < p.gsz ? (uint32_t)hq : p.gsz - 1;
+        const uint32_t hp = (uint32_t)hq < gsz ? (uint32_t)hq : gsz - 1;
         const uint32_t pq = lds0 + PARK + 5 * hp * PARK_UNIT + (uint32_t)lane * 16;
         const uint32_t pc = lds0 + PARK_SC + 5 * hp * 256 + (uint32_t)lane * 4;
 #pragma unroll
@@ -698,10 +699,10 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
         // ---- every value wave owns its dims: write the result, or the slice's partial ----
         const float unit_f = e_run == E_NONE ? 0.0f : pow2i(e_run - WEXP);   // the accumulators are in units of 2^(e_run - WEXP)
 #pragma clang loop unroll(disable)
-        for (int h = 0; h < (int)p.gsz; h++) {
+        for (int h = 0; h < (int)gsz; h++) {
             const float L = lsum[h * 16 + n];
             if (!sliced) {
-                const uint32_t rb = p.gsz * grp + h, y = div_by(rb, p.nhb_inv);
+                const uint32_t rb = gsz * grp + h, y = div_by(rb, nhb_inv);
                 // Through the wave's own stretch of LDS (the tiles are done with), so that a store
                 // writes 512 bytes of two heads and not 64 of sixteen, whose rows are 2 KB apart and
                 // meet in two channels of the L2.
@@ -710,14 +711,14 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
 #pragma unroll
                 for (int j = 0; j < 8; j++)
                     LDS_AT(lds_f32x4, ow + (uint32_t)(64 * j)) = oacc[0][j] * fin;   // register i <-> dim 16 (8 cw + j) + 4 g + i
-                if (rb < p.n_rb) {
-                    const int head0 = 16 * (int)(rb - y * p.nhb) + (lane >> 5);
-                    float *dst = p.out + ((size_t)y * p.nh + head0) * VDIM + 128 * cw + 4 * (lane & 31);
+                if (rb < n_rb) {
+                    const int head0 = 16 * (int)(rb - y * nhb) + (lane >> 5);
+                    float *dst = p.out + ((size_t)y * nh + head0) * VDIM + 128 * cw + 4 * (lane & 31);
                     const uint32_t orow = ob + (uint32_t)((lane >> 5) * 528 + (lane & 31) * 16);
                     f32x4 v[8];
 #pragma unroll
                     for (int k = 0; k < 8; k++) v[k] = LDS_AT(lds_f32x4, orow + (uint32_t)(2 * k * 528));
-                    const int rows_left = p.nh - head0;           // (a scalar branch for whole blocks: eight predicated stores are slower)
+                    const int rows_left = nh - head0;           // (a scalar branch for whole blocks: eight predicated stores are slower)
                     if (__all(rows_left > 14)) {
 #pragma unroll
                         for (int k = 0; k < 8; k++) *(f32x4 *)(dst + 2 * k * VDIM) = v[k];
@@ -731,7 +732,7 @@ __global__ void __launch_bounds__(THREADS) mla_prefill64_kernel(const WideParams
                 // The layout and the write-through stores of mla_roles.hip's partials, but the accumulators as
                 // they are: the sums of an uncut chunk stay in fp32 from the first product to the output, and
                 // so do those that meet in the merge.
-                const size_t pb = ((size_t)grp * n_slices + slice) * p.gsz + h;
+                const size_t pb = ((size_t)grp * n_slices + slice) * gsz + h;
                 float *pq = p.part_acc + ((pb * (VDIM / 16) + 8 * cw) * 64 + lane) * 4;   // [dim block][lane][4]
 #pragma unroll
                 for (int j = 0; j < 8; j++) store_through16(pq + j * 256, __builtin_bit_cast(u32x4, oacc[0][j]));
@@ -768,12 +769,10 @@ int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, i
             attr_err = hipFuncSetAttribute((const void *)mla_prefill64_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     });
     CWICK_HIP_CALL(attr_err);
-    WideParams p{};
-    p.rows = rows; p.scales = scales; p.pos0 = (int)pos0; p.q = q; p.nh = n_heads; p.scale = scale; p.out = out;
-    p.nhb = (uint32_t)(n_heads + 15) / 16;
-    p.n_rb = (uint32_t)n * p.nhb;               // below 2^25
-    p.nhb_inv = div_inverse(p.nhb);
-    WidePlan plan = plan_wide((int64_t)p.n_rb, (pos0 + 1 + TK - 1) / TK, (pos0 + n + TK - 1) / TK, num_cus());
+    WideRest p{};
+    p.scale = scale; p.out = out;
+    const uint32_t nhb = (uint32_t)(n_heads + 15) / 16, n_rb = (uint32_t)n * nhb;               // below 2^25
+    WidePlan plan = plan_wide((int64_t)n_rb, (pos0 + 1 + TK - 1) / TK, (pos0 + n + TK - 1) / TK, num_cus());
     if (plan.whole < plan.groups) {
         const size_t blocks = (size_t)(plan.groups - plan.whole) * plan.slices * plan.gsz;
         const size_t acc_b = blocks * 16 * VDIM * sizeof(float);
@@ -781,22 +780,18 @@ int launch_mla_prefill(const uint8_t *rows, const float *scales, int64_t pos0, i
         p.part_acc = (float *)ws;
         p.part_ml = (float *)(ws + acc_b);
         // no room for partials (a stream that is being captured and has not run the shape before): uncut
-        if (!ws) plan = WidePlan{NHQ, (p.n_rb + NHQ - 1) / NHQ, (p.n_rb + NHQ - 1) / NHQ, 1, 0.0f};
+        if (!ws) plan = WidePlan{NHQ, (n_rb + NHQ - 1) / NHQ, (n_rb + NHQ - 1) / NHQ, 1, 0.0f};
     }
-    p.gsz = plan.gsz;
-    p.n_whole = plan.whole;
-    p.n_rest = plan.groups - plan.whole;
-    p.n_slices = plan.slices;
-    p.slices_inv = div_inverse(plan.slices);
+    const uint32_t n_rest = plan.groups - plan.whole;
     {
         ProfKernel pk(CWICK_HIP_PROF_MLA_PREFILL, s);
-        const dim3 grid(p.n_whole + p.n_rest * p.n_slices);
-        if (p.nhb % p.gsz == 0) pk.launch(mla_prefill64_kernel<false>, grid, dim3(THREADS), smem, p);
-        else pk.launch(mla_prefill64_kernel<true>, grid, dim3(THREADS), smem, p);
+        pk.launch(nhb % plan.gsz == 0 ? mla_prefill64_kernel<false> : mla_prefill64_kernel<true>, dim3(plan.whole + n_rest * plan.slices),
+                  dim3(THREADS), smem, q, rows, scales, (int)pos0, (uint32_t)n_heads | plan.gsz << 8, div_inverse(nhb), n_rb, plan.whole,
+                  n_rest, plan.slices, div_inverse(plan.slices), p);
     }
     CWICK_HIP_CALL(hipGetLastError());
-    if (p.n_rest)
-        return launch_mla_merge((const f32x4 *)p.part_acc, p.part_ml, (int)p.n_slices, (int)p.n_rest, (int)p.gsz, (int)p.nhb, (int64_t)p.n_rb,
+    if (n_rest)
+        return launch_mla_merge((const f32x4 *)p.part_acc, p.part_ml, (int)plan.slices, (int)n_rest, (int)plan.gsz, (int)nhb, (int64_t)n_rb,
                                 n_heads, nullptr, out, CWICK_HIP_PROF_MLA_MERGE, s);
     return 1;
 }

@@ -92,21 +92,26 @@ typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
 typedef __attribute__((address_space(3))) void lds_void;
 
-struct Params {
-    const uint8_t *rows;
-    const float *scales;
-    int64_t row_bstride, scale_bstride, n_rows;
-    const int32_t *sel;
-    int64_t n_list;
-    const uint16_t *q;
-    int nh, nq;
-    uint32_t n_hb_inv, n_splits_inv;    // 2^31 / n, rounded up, of the head blocks and the splits
-    float scale;
-    int n_splits;
-    int64_t keys_per_split;   // multiple of TK
+// What a workgroup's first copies need comes as arguments of its own, which arrive in registers with the
+// waves (the first fourteen dwords, and no struct among them: a struct is fetched through the scalar cache,
+// which a launch finds cold); the rest comes in this, fetched while the first copies are on their way.
+struct Rest {
+    int64_t row_bstride, scale_bstride;
     const float *sink;        // per head, natural-log units of the scaled scores, or null
     float *out, *part_ml;
     uint32_t *part_acc;
+    float scale;
+};
+struct Params {
+    const uint8_t *rows;
+    const float *scales;
+    int64_t n_rows;
+    const int32_t *sel;
+    int64_t n_list;
+    const uint16_t *q;
+    int nh, nq, n_splits;
+    int64_t keys_per_split;   // multiple of TK
+    Rest rest;
 };
 
 // What a masked position of a tile (past the end of the list, a -1 or out-of-range entry of
@@ -197,8 +202,13 @@ constexpr uint32_t XCH_B = sizeof(Xch);
 constexpr uint32_t XM_OFF = 2 * 2 * 4 * 16 * 4 * 4;               // Xch::m
 constexpr uint32_t XF_OFF = XM_OFF + 2 * 16 * 4 * 4;              // Xch::moved
 
+// shape: the heads of a query in the low eight bits, the splits above.  splits_inv: 2^31 / splits, rounded up.
+// eighth: an eighth of the workgroups, 0 if they are no multiple of eight.
 template <bool SEL>
-__global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
+__global__ void __launch_bounds__(THREADS)
+mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all_rows, const float *__restrict__ all_scales,
+                 const int32_t *__restrict__ all_sel, uint32_t n_list, uint32_t n_rows, uint32_t keys_per_split, uint32_t shape,
+                 uint32_t splits_inv, uint32_t eighth, const Rest p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     Smem &sm = *reinterpret_cast<Smem *>(smem_raw);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void *)smem_raw;
@@ -213,22 +223,26 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
     const int n = lane & 15;         // head column / key row of a 16-block / dim row
     const int g = lane >> 4;         // 32-wide contraction block (QK) / 8-wide (PV)
 
-    const uint32_t total = gridDim.x;
+    const int nh = (int)(shape & 255u), n_splits = (int)(shape >> 8);
     // Workgroups go to the eight XCDs round robin: an XCD takes a contiguous eighth of the units (the
     // head blocks of a slice, the slices of a query: what they share stays in one L2).
     // (divisions by multiplication: each is thirty instructions in front of the first load otherwise)
     uint32_t unit = blockIdx.x;
-    if (total % 8 == 0) unit = (unit % 8) * (total / 8) + unit / 8;
-    const uint32_t n_hb = (uint32_t)(p.nh + HW - 1) / HW, slice = div_by(unit, p.n_hb_inv), uy = div_by(slice, p.n_splits_inv);
-    const int hb = (int)(unit - slice * n_hb), split = (int)(slice - uy * (uint32_t)p.n_splits), y = (int)uy;
+    if (eighth) unit = (unit & 7) * eighth + unit / 8;
+    const uint32_t n_hb = (uint32_t)(nh + HW - 1) / HW;                    // one to four: 2^31 / n_hb, rounded up, without a table
+    const uint32_t slice = div_by(unit, n_hb == 3 ? 0x2AAAAAABu : 0x80000000u >> (n_hb >> 1)), y = div_by(slice, splits_inv);
+    const int hb = (int)(unit - slice * n_hb), split = (int)(slice - y * (uint32_t)n_splits);
 
-    const uint8_t *rows = p.rows + (size_t)y * p.row_bstride;
-    const float *scales = p.scales + (size_t)y * p.scale_bstride;
-    const int32_t *sel = SEL ? p.sel + (size_t)y * p.n_list : nullptr;
-    const int64_t k_begin = (int64_t)split * p.keys_per_split;
-    int64_t k_end = k_begin + p.keys_per_split;
-    if (k_end > p.n_list) k_end = p.n_list;
-    const int n_keys = k_end > k_begin ? (int)(k_end - k_begin) : 0;     // of this workgroup
+    const uint8_t *rows = all_rows;
+    const float *scales = all_scales;
+    if (y) {                                               // (the first query waits for nothing)
+        rows += (size_t)y * p.row_bstride;
+        scales += (size_t)y * p.scale_bstride;
+    }
+    const int32_t *sel = SEL ? all_sel + (size_t)y * n_list : nullptr;
+    const uint32_t k_begin = (uint32_t)split * keys_per_split;             // below n_list
+    const uint32_t left = n_list - k_begin;
+    const int n_keys = (int)(left < keys_per_split ? left : keys_per_split);     // of this workgroup
     const int n_tiles = (n_keys + TK - 1) / TK;
 
     // The zero row and its scales: where masked positions of a tile are fetched from.  The
@@ -244,7 +258,7 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
         int r = -1;
         if (t < n_tiles && i < n_keys) {
             r = sel[k_begin + i];
-            if (r < 0 || r >= p.n_rows) r = -1;
+            if ((uint32_t)r >= n_rows) r = -1;
         }
         return r;
     };
@@ -314,10 +328,10 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
     const int hhu = wave >= 5 ? 1 : 0, bu = wave - 5 * hhu;
     const uint32_t unit_lds = lds0 + PARK + (uint32_t)wave * PARK_UNIT;
     if (has_unit) {
-        const uint64_t base = (uint64_t)(uintptr_t)(p.q + (size_t)y * p.nh * KDIM + 128 * bu);
+        const uint64_t base = (uint64_t)(uintptr_t)(q + (size_t)(y * (uint32_t)nh) * KDIM + 128 * bu);
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const int h = 4 * c + g, head0 = hb * HW + 16 * hhu + h, head = head0 < p.nh ? head0 : p.nh - 1;
+            const int h = 4 * c + g, head0 = hb * HW + 16 * hhu + h, head = head0 < nh ? head0 : nh - 1;
             const int x = (n ^ h) & (bu < 4 ? 15 : 7);             // the rope block has eight pieces: fetched twice
             dma16(base + (uint64_t)(uint32_t)head * (KDIM * 2) + (uint32_t)(16 * x), unit_lds + (uint32_t)c * 1024);
         }
@@ -329,7 +343,7 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
     auto first_rows = [&](int t) -> int {
         if (!SEL) return row_of(t);
         const int r = list_entry[t];
-        return t < n_tiles && t * TK + lane < n_keys && r >= 0 && r < p.n_rows ? r : -1;
+        return t < n_tiles && t * TK + lane < n_keys && (uint32_t)r < n_rows ? r : -1;
     };
     if (n_tiles > 0) share(first_rows(0), lds0);
     if (has_unit) {
@@ -673,20 +687,20 @@ __global__ void __launch_bounds__(THREADS) mla_roles_kernel(const Params p) {
             const f32x4 lv = *(const f32x4 *)&lsum[(h2 * 16 + n) * 4];
             float L = (lv[0] + lv[1]) + (lv[2] + lv[3]);
             const int head = hb * HW + 16 * h2 + n;
-            if (head >= p.nh) continue;
+            if (head >= nh) continue;
             // the attention sink of src/ds_model.c:946: one more term in the denominator, no value
             // (with several splits the merge kernel adds it)
-            if (p.sink && p.n_splits == 1 && m_ref[h2] > -INFINITY)
+            if (p.sink && n_splits == 1 && m_ref[h2] > -INFINITY)
                 L += __builtin_amdgcn_exp2f(p.sink[head] * 1.44269504088896340736f - m_ref[h2]);
             const float unit_f = e_run == E_NONE ? 0.0f : pow2i(e_run - WEXP);   // the accumulators are in units of 2^(e_run - WEXP)
-            const float fin = p.n_splits == 1 ? (L > 0.0f ? unit_f / L : 0.0f) : unit_f;
-            const size_t pb = ((size_t)y * p.n_splits + split) * (2 * n_hb) + 2 * hb + h2;
-            if (p.n_splits == 1) {
+            const float fin = n_splits == 1 ? (L > 0.0f ? unit_f / L : 0.0f) : unit_f;
+            const size_t pb = (size_t)(y * (uint32_t)n_splits + (uint32_t)split) * (2 * n_hb) + 2 * hb + h2;
+            if (n_splits == 1) {
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
                     // accumulator register i <-> dim 16 db + 4 g + i
                     const f32x4 v = oacc[h2][j] * fin;
-                    *(f32x4 *)(p.out + ((size_t)y * p.nh + head) * VDIM + 16 * (8 * cw + j) + 4 * g) = v;
+                    *(f32x4 *)(p.out + (size_t)(y * (uint32_t)nh + (uint32_t)head) * VDIM + 16 * (8 * cw + j) + 4 * g) = v;
                 }
                 continue;
             }
@@ -948,8 +962,6 @@ int run(Params &p, int most_splits, hipStream_t s, bool fixed) {
     CWICK_HIP_CALL(attr_err);
     const int n_hb = (p.nh + HW - 1) / HW;
     const int64_t total = (int64_t)n_hb * p.n_splits * p.nq;     // below 2^25: n_hb <= 4, and splits only up to the compute units
-    p.n_hb_inv = div_inverse((uint32_t)n_hb);
-    p.n_splits_inv = div_inverse((uint32_t)p.n_splits);
     CWICK_REQUIRE(total < (1 << 25), "mla: grid of %lld workgroups is too large", (long long)total);
     if (p.n_splits > 1) {
         const size_t acc_b = (size_t)p.nq * p.n_splits * n_hb * HW * VDIM * sizeof(int16_t);
@@ -967,18 +979,20 @@ int run(Params &p, int most_splits, hipStream_t s, bool fixed) {
             ws = (char *)workspace(s, (acc_b + ml_b) / p.n_splits * most_splits);
             if (!ws) return 0;                      // workspace() has recorded why
         }
-        p.part_acc = (uint32_t *)ws;
-        p.part_ml = (float *)(ws + acc_b);
+        p.rest.part_acc = (uint32_t *)ws;
+        p.rest.part_ml = (float *)(ws + acc_b);
     }
     {
         ProfKernel pk(fixed ? -1 : CWICK_HIP_PROF_MLA, s);
-        if (p.sel) pk.launch(mla_roles_kernel<true>, dim3((unsigned)total), dim3(THREADS), smem, p);
-        else pk.launch(mla_roles_kernel<false>, dim3((unsigned)total), dim3(THREADS), smem, p);
+        pk.launch(p.sel ? mla_roles_kernel<true> : mla_roles_kernel<false>, dim3((unsigned)total), dim3(THREADS), smem,
+                  p.q, p.rows, p.scales, p.sel, (uint32_t)p.n_list, (uint32_t)p.n_rows, (uint32_t)p.keys_per_split,
+                  (uint32_t)p.nh | (uint32_t)p.n_splits << 8, div_inverse((uint32_t)p.n_splits),
+                  total % 8 == 0 ? (uint32_t)(total / 8) : 0u, p.rest);
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (p.n_splits > 1)
-        return launch_mla_merge((const u32x2 *)p.part_acc, p.part_ml, p.n_splits, p.nq, 2 * n_hb, 2 * n_hb, (int64_t)p.nq * 2 * n_hb, p.nh,
-                                p.sink, p.out, fixed ? -1 : CWICK_HIP_PROF_MLA_MERGE, s);
+        return launch_mla_merge((const u32x2 *)p.rest.part_acc, p.rest.part_ml, p.n_splits, p.nq, 2 * n_hb, 2 * n_hb, (int64_t)p.nq * 2 * n_hb, p.nh,
+                                p.rest.sink, p.rest.out, fixed ? -1 : CWICK_HIP_PROF_MLA_MERGE, s);
     return 1;
 }
 
@@ -1011,9 +1025,10 @@ int launch_mla_decode(const uint8_t *rows, const float *scales, int64_t row_bstr
                       (uintptr_t)out % 16 == 0 && (uintptr_t)scales % 4 == 0,
                   "mla_decode: rows, q and out must be 16-byte aligned");
     Params p{};
-    p.rows = rows; p.scales = scales; p.row_bstride = row_bstride; p.scale_bstride = scale_bstride;
-    p.n_rows = n_rows; p.sel = sel; p.n_list = n_list;
-    p.q = q; p.nh = n_heads; p.nq = batch; p.scale = scale; p.out = out; p.sink = sink;
+    p.rows = rows; p.scales = scales; p.n_rows = n_rows; p.sel = sel; p.n_list = n_list;
+    p.q = q; p.nh = n_heads; p.nq = batch;
+    p.rest.row_bstride = row_bstride; p.rest.scale_bstride = scale_bstride;
+    p.rest.scale = scale; p.rest.out = out; p.rest.sink = sink;
     const int n_hb = (n_heads + HW - 1) / HW;
     const int64_t tiles = (n_list + TK - 1) / TK, want = mla_decode_most_splits(n_hb * batch, splits_per_cu(), num_cus());
     const int64_t per = (int64_t)TK * mla_decode_tiles(tiles, n_hb * batch, sel != nullptr, splits_per_cu(), num_cus());
