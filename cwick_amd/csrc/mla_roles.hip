@@ -23,37 +23,31 @@
 //   every wave reads the eight flags: all clear (almost always) means nothing to do; otherwise
 //   the accumulating waves (and the scorers, for their sums) bring everything to the common
 //   maximum.  Each scoring lane keeps the sum of its own keys; the sums meet once, after the loop.
-//   Tiles are copied global -> LDS by global_load_lds (no registers) into four stages.  Tiles 0 and 1
-//   are fetched by all twelve waves around the preparation of Q, tile 2 by the value waves while the
-//   scoring waves read their Q back; from step 0
-//   on every wave copies its share of tile t+3 during step t
-//   (three sixteen-byte columns of the 64 rows, plus a scale block for five of the waves): the
-//   value waves at the top of the step, the scoring waves at the end of theirs, when they would
-//   otherwise wait at the barrier.  The copies are issued from inline assembly and the barrier
+//   Tiles are copied global -> LDS by global_load_lds (no registers) into four stages.  Tiles 0 to 2
+//   are fetched by all twelve waves around the preparation of Q; from step 0 on every wave copies its share of
+//   tile t+3 during step t (a scoring wave the 512 latent bytes of eight keys, a value wave the rope bytes of
+//   sixteen and a scale block): the value waves at the top of the step, the scoring waves at the end of theirs,
+//   when they would otherwise wait at the barrier.  The copies are issued from inline assembly and the barrier
 //   waits for LDS traffic only, so the compiler never makes anything wait for the tiles in
 //   flight.  LDS is addressed by integer byte offsets throughout (a generic pointer into LDS costs
 //   a null check and a 64-bit add per use), and the kernel exists in two instantiations: dense
 //   lists (rows are k_begin + i, only the last tile can be ragged) and lists given by sel[].
 //
-//   Where the time goes (counters and ablation builds, 12 waves on 256 CUs): a 64-key step takes
-//   about 3 000 cycles against 1 088 of matrix-core work.  Leaving out the tile copies, the score
-//   MFMAs or the value MFMAs with their conversions takes about a quarter off each, all three
-//   together two thirds; what remains (barrier, exchange, softmax, weights) is the last third.
-//   No single unit is saturated: vector ALU 56 % busy, matrix core 37 %, LDS 32 %.  A copy
-//   instruction here has one lane per row (64 cache lines touched); alone on the machine that
-//   pattern moves 54 bytes per ns and compute unit from L2 and 18 from HBM, a pattern that walks
-//   along the rows 125 and 25.  Inside this kernel it makes no difference: tile layouts filled
-//   sixteen lines per instruction ([16-key block][piece][key]) or row by row were built, pass
-//   parity and run 4 to 7 % slower, because they spend more vector instructions per copy on
-//   addresses, and the vector ALU, not the copy path, is what a step waits for most.  With 32
-//   query rows per tile the per-tile work that does not depend on the rows (copies, scale
-//   handling, conversions of V) is paid per 1 088 matrix cycles; 64 rows would halve it per
-//   flop.  Eight or sixteen waves per workgroup (the same work split differently) were measured
-//   and are no faster.
-//
-//   LDS tile layout [16-byte column][key 0..63][16 B]: the K fragment is two 16-byte reads per
-//   lane, 256 B contiguous per 16 keys; the V^T fragment of 32 keys x 16 dims is one
-//   ds_read_b64_tr_b8, 128 B contiguous per 16-lane group (keys 8 g..8 g+7 of the half).
+//   Where the time goes (cycle stamps, 12 waves on 256 CUs): a 64-key step has 1 088 cycles of matrix work on
+//   a SIMD and takes about 2 500.  No unit is saturated: the two scoring waves and the value wave of a SIMD are
+//   chains of instructions, each of which takes its wave five cycles whatever its kind, of LDS round trips and of
+//   products.  So what pays is fewer instructions in the chain and fewer waits in it: the steps with a whole tile
+//   to copy have no condition and no 64-bit multiplication in them (running addresses; the step as a function of its
+//   kind), everything a step reads is requested before the first product, the keys' scales are two registers
+//   out of which the folds take their factor by DPP, eight flags are eight bytes.  32768 rows of 128 heads, the
+//   whole call: 25.2 -> 23.5 us, and 22.7 with the partial's scale found two values an instruction and its stores
+//   on their way before the sums meet.
+//   A copy instruction that has one lane per row touches 64 cache lines and moves a tile into LDS in 3 100 cycles when
+//   every compute unit does it, one that walks along the rows in 1 900 (copy-only kernels; a list of rows 3 600 and
+//   3 450), hence the tile's layout (see Tile).  With 32 query rows per tile the per-tile work that does not
+//   depend on the rows (copies, scale handling, conversions of V) is paid per 1 088 matrix cycles; 64 rows would
+//   halve it per flop.  Eight or sixteen waves per workgroup (the same work split differently) were measured
+//   and are no faster; nor are other priorities of the two roles.
 //
 //   Split-K partials are stored per 16 heads in accumulator-fragment order
 //   [split][16-head block][dim block][lane][4] (every store 1 KiB contiguous);
@@ -82,6 +76,8 @@ constexpr int NDB = VDIM / 16;                // 32 sixteen-dim output blocks
 constexpr float LAZY = 4.0f;                  // the reference moves when a tile exceeds it by 2^LAZY
 constexpr int WEXP = 10;                      // fp16 weights are p * scale * 2^(WEXP - e), scale < 2^e
 constexpr int E_NONE = -1000;                 // no scale seen yet
+// the steps of the loop: before tile 0, with the copy of a whole tile, with whatever there is, behind the last tile
+constexpr int FIRST = 0, STEADY_ = 1, TAIL = 2, LAST = 3;
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
@@ -121,8 +117,20 @@ struct Params {
 __device__ __attribute__((aligned(16))) uint8_t g_zero_row[KDIM + 64] = {0};
 __device__ __attribute__((aligned(16))) float g_zero_scales[8] = {0.0f};
 
+// A tile is 36 blocks of 1 KiB, each what one copy instruction fetches: block 8 cg + kg is the eight columns of
+// sixteen bytes 8 cg .. of the keys 8 kg .. +7, block 32 + kq the four rope columns of the keys 16 kq .. +15.
+// Byte of column c of a key in its block: the four columns of a quarter of the row stay together (four neighbouring
+// lanes of the copy fetch 64 bytes of it), keys are 64 bytes apart, and within its four columns a key takes places
+// that depend on which four of the sixteen it belongs to.  The bytes in flight through LDS at a time are those of
+// lanes 0..3, 12..15, 20..23, 24..27 (then the others, then the upper half) of a sixteen-byte read and of 32 lanes of a
+// transpose read: the Gray code of the four takes them to different banks in both (3.3 and 2.0 cycles a read; keys in order
+// 6.0 and 6.0, the number of the four itself 6.0 and 2.0).
+__device__ __forceinline__ uint32_t swap_of(uint32_t key) { return ((key >> 2) ^ (key >> 3 & 1)) & 3; }
+__device__ __forceinline__ uint32_t place(uint32_t c, uint32_t key, uint32_t keys) {          // keys: of the block, 8 or 16
+    return 512 * (c >> 2) + 64 * (key & (keys - 1)) + 16 * ((c & 3) ^ swap_of(key));
+}
 struct Tile {
-    uint8_t kv[NCOL][TK][16];     // [16-byte column][key][16]     36864 B
+    uint8_t kv[NCOL][1024];
     float sc[NBLK][TK];           // [block][key]                   1280 B
     uint32_t valid[2];            // list kernels: bit k = position k of the tile holds a row
     uint32_t pad[2];
@@ -133,7 +141,8 @@ struct Xch {                       // what the scoring waves publish per tile
     // half is key 8 g + j of that half
     uint32_t p[2][2][4][16][4];
     float m[2][16][4];            // [head half][head][key block]: the reference m they are relative to
-    uint32_t moved[8];            // per scoring wave: its reference for this tile is not the common one
+    uint8_t moved[8];             // per scoring wave: its reference for this tile is not the common one
+    uint8_t pad[8];
 };
 struct Smem {
     Tile tile[NST];
@@ -178,9 +187,10 @@ __device__ __forceinline__ float vmax3(float a, float b, float c) {
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
-__device__ __forceinline__ uint32_t umax3(uint32_t a, uint32_t b, uint32_t c) {
-    uint32_t r;
-    asm("v_max3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+// max(|a|, |b|, |c|), NaN if any of them is one
+__device__ __forceinline__ float maximum3_abs(float a, float b, float c) {
+    float r;
+    asm("v_maximum3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
@@ -189,6 +199,7 @@ typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
 typedef __attribute__((address_space(3))) float lds_f32;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
 // LDS is addressed by byte offsets held in ordinary integers (a generic pointer into LDS costs a
 // null check and a 64-bit add at every use)
 #define LDS_AT(type, a) (*(type *)(size_t)(uint32_t)(a))
@@ -251,9 +262,9 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
     uint64_t zrow = (uint64_t)(uintptr_t)g_zero_row, zsc = (uint64_t)(uintptr_t)g_zero_scales;
     asm volatile("" : "+s"(zrow), "+s"(zsc));
 
-    // copy role: lane = key of the tile; row of the cache or -1
-    auto row_of = [&](int t) -> int {
-        const int i = t * TK + lane;
+    // the row of the cache behind position k of tile t, or -1
+    auto row_of = [&](int t, int k) -> int {
+        const int i = t * TK + k;
         if (!SEL) return (t < n_tiles && i < n_keys) ? (int)(k_begin + i) : -1;    // rows fit 31 bits (checked by the launcher)
         int r = -1;
         if (t < n_tiles && i < n_keys) {
@@ -276,54 +287,99 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
     };
     auto row_ptr = [&](int r) -> uint64_t { return r >= 0 ? (uint64_t)(uintptr_t)rows + (uint64_t)(uint32_t)r * KDIM : zrow; };
     auto sc_ptr = [&](int r) -> uint64_t { return r >= 0 ? (uint64_t)(uintptr_t)scales + (uint64_t)(uint32_t)r * (NBLK * 4) : zsc; };
-    // this wave's share of a tile: three columns, and a scale block for the first five waves
     // which of the 64 positions of the tile hold a row (the scoring waves mask the others)
     auto mark = [&](int r, uint32_t tile_off) {
         const uint64_t v = __ballot(r >= 0);
         LDS_AT(lds_u32x2, tile_off + VALID_OFF) = (u32x2){(uint32_t)v, (uint32_t)(v >> 32)};
     };
-    auto share = [&](int r, uint32_t tile_off) {
-        const uint64_t rp = row_ptr(r), sp = sc_ptr(r);
-        // columns wave, wave + 12, wave + 24 (all below 36) and, for the first five waves, scale block `wave`
-        const uint32_t col_off = tile_off + (uint32_t)wave * (TK * 16);
-        const uint64_t col_src = rp + 16 * wave;
-        // (the 192 and 384 bytes to the lane's source are the instruction's immediate offset, which
-        // the hardware also adds to the LDS address: M0 is set that much below the column)
-        dma16(col_src, col_off);
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:192"
-                     ::"v"(col_src), "s"(col_off + 12 * (TK * 16) - 192u) : "memory");
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:384"
-                     ::"v"(col_src), "s"(col_off + 24 * (TK * 16) - 384u) : "memory");
-        if (wave < NBLK) dma4(sp + 4 * wave, tile_off + SC_OFF + (uint32_t)wave * (TK * 4));
-        if (SEL && wave == 0) mark(r, tile_off);
+    // A wave's share of a tile.  Scoring wave w: the blocks of keys 8 w .. +7, lane l key (l / 4) % 8 and column
+    // 4 (l / 32) + .. of each of the four.  Value wave cw: the rope block of keys 16 cw .. +15, lane l key l / 4, and
+    // the scales of dim block cw (the first one: of the rope block too), lane = key.
+    const int key_of = scorer ? 8 * wave + ((lane >> 2) & 7) : 16 * cw + (lane >> 2);
+    const uint32_t col_of = (scorer ? (uint32_t)(4 * (lane >> 5)) : 32u) + ((uint32_t)(lane & 3) ^ swap_of(key_of));
+    const uint32_t lane_row = (uint32_t)key_of * KDIM + 16u * col_of, lane_sc = (uint32_t)lane * (NBLK * 4);
+    // rk: the row of the lane's key, rl: of key `lane` (value waves); whole: a dense tile without a masked position,
+    // whose place is a scalar
+    struct RowPair { int k, l; };
+    // (128 cg bytes to the source are the instruction's immediate offset, which the hardware also adds to the LDS
+    // address: M0 is set that much below the block)
+#define CWICK_ROLES_BLK(cg, ...) asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, " __VA_ARGS__ " offset:128*" #cg
+    auto copy_whole = [&](uint64_t rp, uint64_t sp, uint32_t tile_off) {
+        if (scorer) {
+            const uint32_t blk = tile_off + (uint32_t)wave * 1024;
+#define CWICK_ROLES_COPY(cg) CWICK_ROLES_BLK(cg, "%2") ::"v"(lane_row), "s"(blk + (8 * 1024 - 128) * cg), "s"(rp) : "memory")
+            CWICK_ROLES_COPY(0); CWICK_ROLES_COPY(1); CWICK_ROLES_COPY(2); CWICK_ROLES_COPY(3);
+#undef CWICK_ROLES_COPY
+        } else {
+            const uint32_t rope = tile_off + (32u + (uint32_t)cw) * 1024, sc = tile_off + SC_OFF + (uint32_t)cw * (TK * 4);
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" ::"v"(lane_row), "s"(rope), "s"(rp) : "memory");
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2" ::"v"(lane_sc), "s"(sc), "s"(sp + 4 * cw) : "memory");
+            if (cw == 0)
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2" ::"v"(lane_sc), "s"(sc + 4 * (TK * 4)), "s"(sp + 16) : "memory");
+        }
     };
-    // a quarter of a tile: columns cw, cw + 4, .. and scale block cw (the first value wave: block 4 too)
-    auto quarter = [&](int r, uint32_t tile_off) {
-        const uint64_t rp = row_ptr(r) + 16 * cw, sp = sc_ptr(r);
-#pragma clang loop unroll(disable)
-        for (uint32_t k = 0; k < 9; k++) dma16(rp + 64 * k, tile_off + (4 * k + (uint32_t)cw) * (TK * 16));
-        dma4(sp + 4 * cw, tile_off + SC_OFF + (uint32_t)cw * (TK * 4));
-        if (cw == 0) dma4(sp + 16, tile_off + SC_OFF + 4u * (TK * 4));
-        if (SEL && cw == 0) mark(r, tile_off);
+    auto share = [&](int t, RowPair r, uint32_t tile_off) {
+        if (!SEL && (t + 1) * TK <= n_keys) {
+            copy_whole((uint64_t)(uintptr_t)rows + (uint64_t)(k_begin + (uint32_t)t * TK) * KDIM,
+                       (uint64_t)(uintptr_t)scales + (uint64_t)(k_begin + (uint32_t)t * TK) * (NBLK * 4), tile_off);
+        } else if (scorer) {
+            const uint32_t blk = tile_off + (uint32_t)wave * 1024;
+            const uint64_t rp = row_ptr(r.k) + 16 * col_of;
+#define CWICK_ROLES_COPY(cg) CWICK_ROLES_BLK(cg, "off") ::"v"(rp), "s"(blk + (8 * 1024 - 128) * cg) : "memory")
+            CWICK_ROLES_COPY(0); CWICK_ROLES_COPY(1); CWICK_ROLES_COPY(2); CWICK_ROLES_COPY(3);
+#undef CWICK_ROLES_COPY
+        } else {
+            const uint32_t rope = tile_off + (32u + (uint32_t)cw) * 1024, sc = tile_off + SC_OFF + (uint32_t)cw * (TK * 4);
+            const uint64_t sp = sc_ptr(r.l);
+            dma16(row_ptr(r.k) + 16 * col_of, rope);
+            dma4(sp + 4 * cw, sc);
+            if (cw == 0) dma4(sp + 16, sc + 4 * (TK * 4));
+            if (SEL && cw == 0) mark(r.l, tile_off);
+        }
     };
-    // What comes first.  A copy takes the memory pipeline a cycle per cache line it touches: 64 for a column
-    // of a tile (a lane per row), 2600 for a tile.  So: the query, whose preparation the first barrier
-    // waits for, along its rows (ten to sixteen lines per instruction; a head's 256 bytes of a unit in
-    // sixteen pieces, piece x of head h at place x ^ h, so that the heads of a fragment read come from
-    // different banks); tile 0; tile 1 when the wave has converted its unit; tile 2 by the value waves while
-    // the scoring waves read Q back.  From step 0 on tile t+3 is fetched during step t.  The loads of the
-    // list entries are in assembly like the copies, so that the wait for them leaves the query in flight.
-    // (Q loaded into registers with a lane per row, tile 1 whole by two waves in front of it, Q parked a
-    // dword at a time: 8 400 cycles to the loop instead of 6 000.)
-    int list_entry[3];
-    auto list_at = [&](int t) -> const int32_t * {
-        const int i = t * TK + lane;
-        return sel + k_begin + (i < n_keys ? i : 0);
+#undef CWICK_ROLES_BLK
+    // The same in the steps t < n_steady, in which tile t+3 is whole (dense: a running address; a list: entries
+    // without a look at its end).
+    const int n_steady = n_keys / TK - 3;
+    uint64_t next_rows = (uint64_t)(uintptr_t)rows + (uint64_t)(k_begin + 3 * TK) * KDIM, next_sc = (uint64_t)(uintptr_t)scales + (uint64_t)(k_begin + 3 * TK) * (NBLK * 4);
+    auto list_row = [&](int t, int k) -> int {
+        const int r = sel[k_begin + (uint32_t)(t * TK + k)];
+        return (uint32_t)r < n_rows ? r : -1;
     };
-    if (SEL)                                          // (a workgroup has at least one key)
-        asm volatile("global_load_dword %0, %3, off\n\tglobal_load_dword %1, %4, off\n\tglobal_load_dword %2, %5, off"
-                     : "=&v"(list_entry[0]), "=&v"(list_entry[1]), "=&v"(list_entry[2])
-                     : "v"(list_at(0)), "v"(list_at(1)), "v"(list_at(2)) : "memory");
+    auto share_steady = [&](int t, RowPair r, uint32_t tile_off) {
+        if (SEL) {
+            share(t, r, tile_off);
+            return;
+        }
+        copy_whole(next_rows, next_sc, tile_off);
+        next_rows += TK * KDIM;
+        next_sc += TK * NBLK * 4;
+    };
+    // copies of a wave's share
+#define CWICK_ROLES_WAIT(extra_s, extra_v, extra_v0)                                         \
+    do {                                                                                     \
+        if (scorer) asm volatile("s_waitcnt vmcnt(" #extra_s ")" ::: "memory");               \
+        else if (cw) asm volatile("s_waitcnt vmcnt(" #extra_v ")" ::: "memory");              \
+        else asm volatile("s_waitcnt vmcnt(" #extra_v0 ")" ::: "memory");                     \
+    } while (0)
+    // What comes first.  A copy takes the memory pipeline a cycle for every 64 bytes of a row that it touches.  The
+    // query, whose preparation the first barrier waits for, goes along its rows (ten to sixteen lines per instruction; a
+    // head's 256 bytes of a unit in sixteen pieces, piece x of head h at place x ^ h, so that the heads of a fragment
+    // read come from different banks); then tile 0; tiles 1 and 2 when the wave has converted its unit.  From step 0
+    // on tile t+3 is fetched during step t.  The loads of the list entries are in assembly like the copies, so that
+    // the wait for them leaves the query in flight.
+    int entry_k[3], entry_l[3];
+    if (SEL) {                                        // (a workgroup has at least one key)
+        auto list_at = [&](int t, int k) -> const int32_t * {
+            const int i = t * TK + k;
+            return sel + k_begin + (i < n_keys ? i : 0);
+        };
+        asm volatile("global_load_dword %0, %6, off\n\tglobal_load_dword %1, %7, off\n\tglobal_load_dword %2, %8, off\n\t"
+                     "global_load_dword %3, %9, off\n\tglobal_load_dword %4, %10, off\n\tglobal_load_dword %5, %11, off"
+                     : "=&v"(entry_k[0]), "=&v"(entry_k[1]), "=&v"(entry_k[2]), "=&v"(entry_l[0]), "=&v"(entry_l[1]), "=&v"(entry_l[2])
+                     : "v"(list_at(0, key_of)), "v"(list_at(1, key_of)), "v"(list_at(2, key_of)),
+                       "v"(list_at(0, lane)), "v"(list_at(1, lane)), "v"(list_at(2, lane)) : "memory");
+    }
     const bool has_unit = wave < 10;
     const int hhu = wave >= 5 ? 1 : 0, bu = wave - 5 * hhu;
     const uint32_t unit_lds = lds0 + PARK + (uint32_t)wave * PARK_UNIT;
@@ -339,22 +395,21 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
     } else if (SEL) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    if (SEL) asm volatile("" : "+v"(list_entry[0]), "+v"(list_entry[1]), "+v"(list_entry[2])::"memory");
-    auto first_rows = [&](int t) -> int {
-        if (!SEL) return row_of(t);
-        const int r = list_entry[t];
-        return t < n_tiles && t * TK + lane < n_keys && (uint32_t)r < n_rows ? r : -1;
+    if (SEL) asm volatile("" : "+v"(entry_k[0]), "+v"(entry_k[1]), "+v"(entry_k[2]), "+v"(entry_l[0]), "+v"(entry_l[1]), "+v"(entry_l[2])::"memory");
+    auto rows_of = [&](int t) -> RowPair { return {row_of(t, key_of), scorer ? -1 : row_of(t, lane)}; };
+    auto first_rows = [&](int t) -> RowPair {
+        if (!SEL) return rows_of(t);
+        auto row = [&](int r, int k) { return t < n_tiles && t * TK + k < n_keys && (uint32_t)r < n_rows ? r : -1; };
+        return {row(entry_k[t], key_of), row(entry_l[t], lane)};
     };
-    if (n_tiles > 0) share(first_rows(0), lds0);
+    share(0, first_rows(0), lds0);
     if (has_unit) {
         // ---- the wave's unit as two E4M3 terms with one E8M0 scale per head (the hardware pairs the scale of
         // lane (n, g) with k-elements that live in other lanes of the same head, so the four lanes must
         // agree; both terms use it).  lane (n, g) holds head n of the half, dims 128 b + 32 g + [0, 32);
         // the rope block is one register set: lanes g < 2 hold the hi term of dims 512 + 32 g.., lanes
         // g >= 2 the lo term of dims 512 + 32 (g - 2).. (the key side repeats its bytes).
-        if (n_tiles <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if (wave < NBLK) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");      // the share of tile 0 stays in flight
-        else asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+        CWICK_ROLES_WAIT(4, 2, 3);                        // the share of tile 0 stays in flight
         u32x4 w[4], hi[2], lo[2];
 #pragma unroll
         for (int c = 0; c < 4; c++) w[c] = LDS_AT(lds_u32x4, unit_lds + (uint32_t)(n * 256 + (((4 * g + c) ^ n) & 15) * 16));
@@ -367,16 +422,18 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
         }
         LDS_AT(lds_u32, lds0 + PARK_SC + (uint32_t)(wave * 256 + lane * 4)) = unit_byte;
     }
-    if (n_tiles > 1) {
-        share(first_rows(1), lds0 + TILE_B);
-        // tile 0 has landed (this wave's share), the share of tile 1 stays in flight
-        if (wave < NBLK) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+    // tile 0 has landed (this wave's share), what comes behind it stays in flight
+    if (n_tiles > 2) {
+        share(1, first_rows(1), lds0 + TILE_B);
+        share(2, first_rows(2), lds0 + 2 * TILE_B);
+        CWICK_ROLES_WAIT(8, 4, 6);
+    } else if (n_tiles > 1) {
+        share(1, first_rows(1), lds0 + TILE_B);
+        CWICK_ROLES_WAIT(4, 2, 3);
     } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        CWICK_ROLES_WAIT(0, 0, 0);
     }
     LDS_BARRIER();
-    static_assert(NCOL + NBLK == 41, "the counts of copies in flight above and below");
 
     const float c0 = p.scale * 1.44269504088896340736f;   // scores in log2 units
     float m_ref[2] = {-INFINITY, -INFINITY};          // of head 16 h2 + n; every wave tracks the same values
@@ -405,29 +462,84 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
 
         float l_priv = 0.0f, l_pend = 0.0f;               // sum over this lane's keys (head 16 hh + n), relative to m_ref / to the tile's m_loc
         float mr = -INFINITY;                             // m_ref of this wave's head half
-        // per-lane LDS offsets inside a tile: K fragment (key 16 kb + n, columns 8 b + 2 g and the
-        // next), the rope block's (columns 32 + 2 (g & 1)), this lane's four keys' scales
-        const uint32_t k_off = (uint32_t)((2 * g) * (TK * 16) + (16 * kb + n) * 16);
-        const uint32_t kr_off = (uint32_t)((32 + 2 * (g & 1)) * (TK * 16) + (16 * kb + n) * 16);
-        const uint32_t s_off = SC_OFF + (uint32_t)((16 * kb + 4 * g) * 4);
+        // per-lane LDS offsets inside a tile: K fragment (key 16 kb + n, columns 8 b + 2 g and, 16 bytes to either side,
+        // the next), the rope block's (columns 32 + 2 (g & 1)); the scales of this lane's row of sixteen lanes, place
+        // 4 b + i that of dim block b and key 16 kb + 4 g + i (the rope block's by itself)
+        const uint32_t k_off = (uint32_t)(2 * kb + (n >> 3)) * 1024 + place(2 * g, n, 8);
+        const uint32_t kr_off = (uint32_t)(32 + kb) * 1024 + place(2 * (g & 1), n, 16);
+        const uint32_t s_off = SC_OFF + (uint32_t)(((n >> 2) * TK + 16 * kb + 4 * g + (n & 3)) * 4);
+        const uint32_t sr_off = SC_OFF + (uint32_t)((4 * TK + 16 * kb + 4 * g + (n & 3)) * 4);
         // where this lane's four probabilities go: keys 16 (kb & 1) + 4 g + i of half kb >> 1
         const uint32_t xp_off = (uint32_t)(((((hh * 2 + (kb >> 1)) * 4 + 2 * (kb & 1) + (g >> 1)) * 16 + n) * 4 + 2 * (g & 1)) * 4);
         const uint32_t xm_off = XM_OFF + (uint32_t)(((hh * 16 + n) * 4 + kb) * 4);
         const uint32_t xmr_off = XM_OFF + (uint32_t)((hh * 16 + n) * 4 * 4);
-        const uint32_t xf_off = XF_OFF + (uint32_t)(wave * 4);
+        const uint32_t xf_off = XF_OFF + (uint32_t)wave;
         const int tail_tile = n_tiles - 1;
         const bool ragged = (n_keys & (TK - 1)) != 0;
 
-#pragma clang loop unroll(disable)
-        for (int t = -1; t < n_tiles; t++) {
+        auto step = [&](int t, auto kind) {
+            constexpr bool FLAGS = decltype(kind)::value != FIRST, SCORE = decltype(kind)::value != LAST, STEADY = decltype(kind)::value == STEADY_;
             const uint32_t xb = lds0 + X_OFF + (uint32_t)(t & 1) * XCH_B;         // exchange area of tile t
-            const bool do_copy = t >= 0 && t + 3 < n_tiles;
-            const int r_cp = do_copy ? row_of(t + 3) : -1;    // fetched here (a list entry is a load), used at the end of the step
-            if (t >= 0) {
+            const bool do_copy = STEADY || (FLAGS && SCORE && t + 3 < n_tiles);
+            int r_cp = -1;                                // fetched here (a list entry is a load), used at the end of the step
+            if (SEL && do_copy) r_cp = STEADY ? list_row(t + 3, key_of) : row_of(t + 3, key_of);
+            u32x2 fl = {0u, 0u};
+            if (FLAGS) fl = LDS_AT(lds_u32x2, xb + XF_OFF);
+            const uint32_t tb = lds0 + (uint32_t)((t + 1) & (NST - 1)) * TILE_B;
+            const uint32_t xn = lds0 + X_OFF + (uint32_t)((t + 1) & 1) * XCH_B;
+            f32x4 S;
+            if constexpr (SCORE) {
+                // ---- scores S^T[key][head] for keys 16 kb.., heads 16 hh.. of tile t+1 ----
+                // All that is read is requested first: eight waves read at the same time, and a fragment requested when the
+                // one before it is used costs a round trip each (S ready 1 700 cycles behind the barrier that way).
+                // The products are in assembly, which the compiler does not space from what reads them: the folds stand behind
+                // all of them and wait states.
+                const uint32_t ka = tb + k_off, kA = tb + (k_off ^ 16u), kr = tb + kr_off, kR = tb + (kr_off ^ 16u);
+                u32x4 k0[NBLK], k1[NBLK];
+                float r0, r1;
+                k0[0] = LDS_AT(lds_u32x4, ka), k1[0] = LDS_AT(lds_u32x4, kA);
+                k0[1] = LDS_AT(lds_u32x4, ka + 8192), k1[1] = LDS_AT(lds_u32x4, kA + 8192);
+                r0 = LDS_AT(lds_f32, tb + s_off);
+                k0[2] = LDS_AT(lds_u32x4, ka + 16384), k1[2] = LDS_AT(lds_u32x4, kA + 16384);
+                k0[3] = LDS_AT(lds_u32x4, ka + 24576), k1[3] = LDS_AT(lds_u32x4, kA + 24576);
+                k0[4] = LDS_AT(lds_u32x4, kr), k1[4] = LDS_AT(lds_u32x4, kR);
+                r1 = LDS_AT(lds_f32, tb + sr_off);
+                __builtin_amdgcn_sched_barrier(0);
+                auto key = [&](int b) -> i32x8 {
+                    return (i32x8){(int)k0[b][0], (int)k0[b][1], (int)k0[b][2], (int)k0[b][3], (int)k1[b][0], (int)k1[b][1], (int)k1[b][2], (int)k1[b][3]};
+                };
+                const int one_scales = 0x7F7F7F7F;
+                f32x4 acc[NBLK];
+#define CWICK_ROLES_PAIR(b, SEL_)                                                                                  \
+    asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %4, %5 " SEL_ "\n\t"                             \
+                 "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %3, %0, %4, %5 " SEL_                                    \
+                 : "=&v"(acc[b]) : "v"(key(b)), "v"(qhi[b]), "v"(qlo[b]), "v"(one_scales), "v"(qsc0))
+                // S (+)= product * scale of the key: out of place 4 b + i of the row, inside the multiply-add
+                float sum[4];
+#define CWICK_ROLES_FOLD(OP, C, i, r, pl, b) asm volatile(OP " %0, %1, %2 row_newbcast:" #pl " row_mask:0xf bank_mask:0xf" : C(sum[i]) : "v"(r), "v"(acc[b][i]))
+#define CWICK_ROLES_FOLD4(OP, C, r, p0, p1, p2, p3, b)                                                                                         \
+    CWICK_ROLES_FOLD(OP, C, 0, r, p0, b); CWICK_ROLES_FOLD(OP, C, 1, r, p1, b); CWICK_ROLES_FOLD(OP, C, 2, r, p2, b); CWICK_ROLES_FOLD(OP, C, 3, r, p3, b)
+                CWICK_ROLES_PAIR(0, "op_sel:[0,0,0] op_sel_hi:[0,0,0]");
+                CWICK_ROLES_PAIR(1, "op_sel:[0,1,0] op_sel_hi:[0,0,0]");
+                CWICK_ROLES_PAIR(2, "op_sel:[0,0,0] op_sel_hi:[0,1,0]");
+                CWICK_ROLES_PAIR(3, "op_sel:[0,1,0] op_sel_hi:[0,1,0]");
+                asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %3, %4 op_sel:[0,0,0] op_sel_hi:[0,0,0]"
+                             : "=&v"(acc[4]) : "v"(key(4)), "v"(qrope), "v"(one_scales), "v"(qsc1));
+                // (fourteen instructions behind the last product of block 0, and more behind the others')
+                asm volatile("s_nop 6" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4])::"memory");
+                CWICK_ROLES_FOLD4("v_mul_f32_dpp", "=v", r0, 0, 1, 2, 3, 0);
+                CWICK_ROLES_FOLD4("v_fmac_f32_dpp", "+v", r0, 4, 5, 6, 7, 1);
+                CWICK_ROLES_FOLD4("v_fmac_f32_dpp", "+v", r0, 8, 9, 10, 11, 2);
+                CWICK_ROLES_FOLD4("v_fmac_f32_dpp", "+v", r0, 12, 13, 14, 15, 3);
+                CWICK_ROLES_FOLD4("v_fmac_f32_dpp", "+v", r1, 0, 1, 2, 3, 4);
+#undef CWICK_ROLES_FOLD4
+#undef CWICK_ROLES_FOLD
+#undef CWICK_ROLES_PAIR
+                S = (f32x4){sum[0], sum[1], sum[2], sum[3]};
+            }
+            if constexpr (FLAGS) {
                 // did any scoring wave move its reference in tile t?  (rare after the first tiles)
-                const u32x4 f0 = LDS_AT(lds_u32x4, xb + XF_OFF), f1 = LDS_AT(lds_u32x4, xb + XF_OFF + 16);
-                const uint32_t any_moved = (f0[0] | f0[1] | f0[2] | f0[3]) | (f1[0] | f1[1] | f1[2] | f1[3]);
-                if (__builtin_amdgcn_readfirstlane(any_moved) != 0u) {
+                if (__builtin_amdgcn_readfirstlane(fl[0] | fl[1]) != 0u) {
                     const f32x4 ml = LDS_AT(lds_f32x4, xb + xmr_off);
                     const float m_new = fmaxf(mr, fmaxf(fmaxf(ml[0], ml[1]), fmaxf(ml[2], ml[3])));
                     const float mo = kb == 0 ? ml[0] : kb == 1 ? ml[1] : kb == 2 ? ml[2] : ml[3];
@@ -439,58 +551,17 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                     l_priv += l_pend;
                 }
             }
-            if (t + 1 < n_tiles) {
-                // ---- scores S^T[key][head] for keys 16 kb.., heads 16 hh.. of tile t+1 ----
-                const uint32_t tb = lds0 + (uint32_t)((t + 1) & (NST - 1)) * TILE_B;
-                const uint32_t xn = lds0 + X_OFF + (uint32_t)((t + 1) & 1) * XCH_B;
-                const uint32_t ka = tb + k_off, kr = tb + kr_off, sa = tb + s_off;
-                auto kfrag = [&](int b) -> i32x8 {
-                    const uint32_t a = b < 4 ? ka + (uint32_t)(8 * b) * (TK * 16) : kr;
-                    const u32x4 k0 = LDS_AT(lds_u32x4, a);
-                    const u32x4 k1 = LDS_AT(lds_u32x4, a + TK * 16);
-                    return (i32x8){(int)k0[0], (int)k0[1], (int)k0[2], (int)k0[3], (int)k1[0], (int)k1[1], (int)k1[2], (int)k1[3]};
-                };
-                const f32x4 z4 = {0.0f, 0.0f, 0.0f, 0.0f};
-                f32x4 S;
-                i32x8 kA = kfrag(0);
-#pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    const i32x8 kN = kfrag(b + 1);
-                    const f32x4 scb = LDS_AT(lds_f32x4, sa + (uint32_t)b * (TK * 4));
-                    f32x4 acc;
-                    if (b == 0) {
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qhi[b], z4, 0, 0, 0, 0x7F7F7F7F, 0, qsc0);
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qlo[b], acc, 0, 0, 0, 0x7F7F7F7F, 0, qsc0);
-                    } else if (b == 1) {
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qhi[b], z4, 0, 0, 0, 0x7F7F7F7F, 1, qsc0);
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qlo[b], acc, 0, 0, 0, 0x7F7F7F7F, 1, qsc0);
-                    } else if (b == 2) {
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qhi[b], z4, 0, 0, 0, 0x7F7F7F7F, 2, qsc0);
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qlo[b], acc, 0, 0, 0, 0x7F7F7F7F, 2, qsc0);
-                    } else {
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qhi[b], z4, 0, 0, 0, 0x7F7F7F7F, 3, qsc0);
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qlo[b], acc, 0, 0, 0, 0x7F7F7F7F, 3, qsc0);
-                    }
-                    if (b == 0) S = acc * scb;
-                    else S += acc * scb;
-                    kA = kN;
-                }
-                {
-                    const f32x4 scb = LDS_AT(lds_f32x4, sa + 4u * (TK * 4));
-                    const f32x4 acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kA, qrope, z4, 0, 0, 0, 0x7F7F7F7F, 0, qsc1);
-                    S += acc * scb;
-                }
-                S *= c0;
+            if constexpr (SCORE) {
                 // masked positions: past the end of the list (only the last tile of a dense list),
                 // or entries of sel[] that name no row
-                if (SEL ? true : (ragged && t + 1 == tail_tile)) {
+                if (SEL ? true : (!STEADY && ragged && t + 1 == tail_tile)) {
                     uint64_t valid;
                     if (SEL) {
                         const u32x2 vw = LDS_AT(lds_u32x2, tb + VALID_OFF);
                         valid = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)vw[0]) |
                                 ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)vw[1]) << 32);
                     } else {
-                        valid = __ballot(row_of(t + 1) >= 0);
+                        valid = __ballot(row_of(t + 1, lane) >= 0);
                     }
                     if (valid != ~0ull) {
                         const uint32_t bits = (uint32_t)(valid >> (16 * kb)) >> (4 * g);
@@ -499,7 +570,7 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                             if (!((bits >> i) & 1u)) S[i] = -INFINITY;
                     }
                 }
-                float lmax = vmax3(S[0], S[1], vmax(S[2], S[3]));
+                float lmax = vmax3(S[0], S[1], vmax(S[2], S[3])) * c0;    // S stays unscaled: c0 > 0 goes into the exponent's multiply-add
                 float m_loc = mr;
                 const bool moves = __any(lmax > mr + LAZY);   // rare after the first tiles: only then the lanes of a head confer
                 if (moves) {
@@ -510,7 +581,7 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 const float m_use = m_loc == -INFINITY ? 0.0f : m_loc;
                 f32x4 P;
 #pragma unroll
-                for (int i = 0; i < 4; i++) P[i] = __builtin_amdgcn_exp2f(S[i] - m_use);
+                for (int i = 0; i < 4; i++) P[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[i], c0, -m_use));
                 l_pend = (P[0] + P[1]) + (P[2] + P[3]);   // of this lane's four keys, relative to m_loc
                 {
                     u32x2 d;
@@ -521,14 +592,23 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 // the reference this key block used (the four lanes of a head write the same word)
                 // and whether it differs from the one every wave holds
                 LDS_AT(lds_f32, xn + xm_off) = m_loc;
-                LDS_AT(lds_u32, xn + xf_off) = moves ? 1u : 0u;
+                LDS_AT(lds_u8, xn + xf_off) = moves ? 1 : 0;
             }
-            // the copies this wave issued a step ago (its share of tile t+2) have long landed; its
-            // share of tile t+3 goes out now, when the wave would otherwise wait at the barrier
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            if (do_copy) share(r_cp, lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B);
+            // the copies this wave issued a step ago (its share of tile t+2) have long landed (in step -1 tile 1 is
+            // needed); its share of tile t+3 goes out now, when the wave would otherwise wait at the barrier
+            if (!FLAGS && n_tiles > 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            else if (SCORE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (STEADY) share_steady(t + 3, {r_cp, -1}, lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B);
+            else if (do_copy) share(t + 3, {SEL ? r_cp : row_of(t + 3, key_of), -1}, lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B);
             LDS_BARRIER();
-        }
+        };
+        int t = 0;
+        step(-1, std::integral_constant<int, FIRST>{});
+#pragma clang loop unroll(disable)
+        for (; t < n_steady; t++) step(t, std::integral_constant<int, STEADY_>{});
+#pragma clang loop unroll(disable)
+        for (; t + 1 < n_tiles; t++) step(t, std::integral_constant<int, TAIL>{});
+        step(t, std::integral_constant<int, LAST>{});
 
         // ---- the sums of the scoring role meet in LDS (the exchange area is free now) ----
         float *lsum = reinterpret_cast<float *>(&sm.x[0]);            // [head half][head][key block]
@@ -537,9 +617,6 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
         if (g == 0) lsum[(hh * 16 + n) * 4 + kb] = ls;
         LDS_BARRIER();
     } else {
-        // tile 2 (stage 2; Q is parked in the last stage and the exchange area): pieces cw, cw + 4, ...
-        const bool quarter_of_2 = n_tiles > 2;
-        if (quarter_of_2) quarter(first_rows(2), lds0 + 2 * TILE_B);        // 11 copies for cw = 0, else 10
         LDS_BARRIER();                                // before copies or weights land in the park area
         f32x4 oacc[2][8];                                 // [head half][dim block]: dims 128 cw + 16 j + 4 g + i, head n
 #pragma unroll
@@ -554,22 +631,32 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
         __builtin_amdgcn_s_setprio(3);
         // transpose-read addressing for V^T: lane i of 16-lane group g supplies key 8 g + (i >> 1),
         // bytes 8 (i & 1) .. +7 of the sixteen-byte column
-        const uint32_t tr_off = (uint32_t)((8 * cw) * (TK * 16) + (8 * g + (n >> 1)) * 16 + 8 * (n & 1));
+        // (columns 8 cw + j and j + 4 of keys 8 g .. and 32 + 8 g ..: one offset for each j < 4)
+        uint32_t tr_off[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) tr_off[j] = (uint32_t)(8 * cw + g) * 1024 + place(j, 8 * (g & 1) + (n >> 1), 8) + 8 * (n & 1);
         // the two scales this lane turns into a pair of factors (see the loop)
         const uint32_t sv_off = SC_OFF + (uint32_t)(cw * (TK * 4) + (32 * ((n & 7) >> 2) + 8 * g + 2 * (n & 3)) * 4);
         // the probabilities of this lane's slots: [head half][key half][g][n][4 dwords]
         const uint32_t pw_off = (uint32_t)((g * 16 + n) * 16);
         const uint32_t xml_off = XM_OFF + (uint32_t)(n * 16);
         asm volatile("" ::: "memory");
-        int r_cp = row_of(3);                             // rows of the tile copied in step 0; a list entry is a load: fetched a step ahead
-#pragma clang loop unroll(disable)
-        for (int t = -1; t < n_tiles; t++) {
-            const bool do_copy = t >= 0 && t + 3 < n_tiles;
-            if (do_copy) {
-                share(r_cp, lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B);   // the stage tile t-1 left at the last barrier
-                r_cp = row_of(t + 4);
+        // step -1: tile 1 must be whole at the barrier
+        if (n_tiles > 2) CWICK_ROLES_WAIT(0, 2, 3);
+        else CWICK_ROLES_WAIT(0, 0, 0);
+        RowPair r_cp = {-1, -1};
+        if (SEL) r_cp = rows_of(3);                       // rows of the tile copied in step 0; a list entry is a load: fetched a step ahead
+        LDS_BARRIER();
+        auto step = [&](int t, auto kind) {
+            constexpr bool STEADY = decltype(kind)::value == STEADY_;
+            const bool do_copy = STEADY || t + 3 < n_tiles;
+            {
+                const uint32_t stage = lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B;   // which tile t-1 left at the last barrier
+                if (STEADY) share_steady(t + 3, r_cp, stage);
+                else if (do_copy) share(t + 3, SEL ? r_cp : rows_of(t + 3), stage);
+                if (SEL && do_copy) r_cp = rows_of(t + 4);
             }
-            if (t >= 0) {
+            {
                 // ---- values O^T[dim][head] += V^T W^T for dims 128 cw.., all 32 heads, tile t ----
                 const uint32_t tb = lds0 + (uint32_t)(t & (NST - 1)) * TILE_B;
                 const uint32_t xb = lds0 + X_OFF + (uint32_t)(t & 1) * XCH_B;
@@ -583,7 +670,17 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 for (int h2 = 0; h2 < 2; h2++)
 #pragma unroll
                     for (int kh = 0; kh < 2; kh++) pw[h2][kh] = LDS_AT(lds_u32x4, xb + pw_off + (uint32_t)((h2 * 2 + kh) * 1024));
-                const u32x4 f0 = LDS_AT(lds_u32x4, xb + XF_OFF), f1 = LDS_AT(lds_u32x4, xb + XF_OFF + 16);
+                const u32x2 fl = LDS_AT(lds_u32x2, xb + XF_OFF);
+                // V^T, fragment q of the tile: dim block (q >> 1) & 7 of the wave's, key half q & 1
+                const uint32_t va[4] = {tb + tr_off[0], tb + tr_off[1], tb + tr_off[2], tb + tr_off[3]};
+                i32x2 vt[16];
+                auto vfetch = [&](int q) {
+                    const int j = q >> 1;
+                    vt[q] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2 *)(size_t)(va[j & 3] + (uint32_t)(512 * (j >> 2) + 4096 * (q & 1))));
+                };
+#pragma unroll
+                for (int q = 0; q < 8; q++) vfetch(q);
+                __builtin_amdgcn_sched_barrier(0);
                 // normaliser of the fp16 weights: a power of two above every scale seen so far (it
                 // only grows, and only then the lanes confer).  Scales are compared as integers:
                 // they are positive, and a negative or NaN scale has the larger bit pattern too.
@@ -613,8 +710,7 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 sw[1][1] = row_place<5>(my_pair);
                 sw[1][2] = row_place<6>(my_pair);
                 sw[1][3] = row_place<7>(my_pair);
-                const uint32_t any_moved = (f0[0] | f0[1] | f0[2] | f0[3]) | (f1[0] | f1[1] | f1[2] | f1[3]);
-                if (__builtin_amdgcn_readfirstlane(any_moved) != 0u || ecorr != 1.0f) {
+                if (__builtin_amdgcn_readfirstlane(fl[0] | fl[1]) != 0u || ecorr != 1.0f) {
                     // a scoring wave left the common reference in this tile (or the weights'
                     // normaliser grew): bring accumulators and probabilities to the new maximum
 #pragma unroll
@@ -626,8 +722,9 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                         for (int k = 0; k < 4; k++) f[k] = ml[k] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[k] - m_new);
                         const float c = (m_ref[h2] == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_ref[h2] - m_new)) * ecorr;
                         m_ref[h2] = m_new;
+                        if (t > 0)
 #pragma unroll
-                        for (int j = 0; j < 8; j++) oacc[h2][j] *= c;
+                            for (int j = 0; j < 8; j++) oacc[h2][j] *= c;
                         // probabilities were taken relative to each key block's own reference: bring
                         // them to m_new (slot group g of half kh holds keys of key block 2 kh + g / 2)
                         const float fsel0 = (g >> 1) ? f[1] : f[0];
@@ -644,101 +741,99 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                     for (int kh = 0; kh < 2; kh++)
 #pragma unroll
                         for (int d = 0; d < 4; d++) pw[h2][kh][d] = mul_f16x2(pw[h2][kh][d], sw[kh][d]);
-                const uint32_t va0 = tb + tr_off;
 #pragma unroll
-                for (int j0 = 0; j0 < 8; j0 += 4) {
-                    i32x2 vt[4][2];
+                for (int q = 8; q < 16; q++) vfetch(q);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int j = 0; j < 4; j++)
-#pragma unroll
-                        for (int kh = 0; kh < 2; kh++)
-                            vt[j][kh] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2 *)(size_t)(va0 + (uint32_t)((j0 + j) * (TK * 16) + kh * (32 * 16))));
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-#pragma unroll
-                        for (int kh = 0; kh < 2; kh++) {
-                            u32x4 vh;
-                            vh[0] = e4m3x2_to_f16x2<false>((uint32_t)vt[j][kh][0]);
-                            vh[1] = e4m3x2_to_f16x2<true>((uint32_t)vt[j][kh][0]);
-                            vh[2] = e4m3x2_to_f16x2<false>((uint32_t)vt[j][kh][1]);
-                            vh[3] = e4m3x2_to_f16x2<true>((uint32_t)vt[j][kh][1]);
-                            const f16x8 va = __builtin_bit_cast(f16x8, vh);
-                            oacc[0][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, __builtin_bit_cast(f16x8, pw[0][kh]), oacc[0][j0 + j], 0, 0, 0);
-                            oacc[1][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, __builtin_bit_cast(f16x8, pw[1][kh]), oacc[1][j0 + j], 0, 0, 0);
-                        }
+                for (int q = 0; q < 16; q++) {
+                    const int j = q >> 1, kh = q & 1;
+                    u32x4 vh;
+                    vh[0] = e4m3x2_to_f16x2<false>((uint32_t)vt[q][0]);
+                    vh[1] = e4m3x2_to_f16x2<true>((uint32_t)vt[q][0]);
+                    vh[2] = e4m3x2_to_f16x2<false>((uint32_t)vt[q][1]);
+                    vh[3] = e4m3x2_to_f16x2<true>((uint32_t)vt[q][1]);
+                    const f16x8 v = __builtin_bit_cast(f16x8, vh);
+                    oacc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, __builtin_bit_cast(f16x8, pw[0][kh]), oacc[0][j], 0, 0, 0);
+                    oacc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, __builtin_bit_cast(f16x8, pw[1][kh]), oacc[1][j], 0, 0, 0);
                 }
             }
-            // tile t+2 must be whole at the next barrier; the share of tile t+3 issued in this
-            // step (three copies) may stay in flight, and in step -1 this wave's quarter of tile 2,
-            // which is needed one step later than tile 1
-            if (do_copy) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-            else if (t < 0 && quarter_of_2) {
-                if (cw == 0) asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
-                else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
-            } else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            // tile t+2 must be whole at the next barrier; the share of the tile behind it may stay in flight
+            if (do_copy) CWICK_ROLES_WAIT(0, 2, 3);
+            else CWICK_ROLES_WAIT(0, 0, 0);
             LDS_BARRIER();
-        }
+        };
+        int t = 0;
+#pragma clang loop unroll(disable)
+        for (; t < n_steady; t++) step(t, std::integral_constant<int, STEADY_>{});
+#pragma clang loop unroll(disable)
+        for (; t < n_tiles; t++) step(t, std::integral_constant<int, TAIL>{});
 
-        const float *lsum = reinterpret_cast<const float *>(&sm.x[0]);
-        LDS_BARRIER();
         // ---- every value wave owns its dims: write the partial (or the result) directly ----
+        const float *lsum = reinterpret_cast<const float *>(&sm.x[0]);
+        const float unit_f = e_run == E_NONE ? 0.0f : pow2i(e_run - WEXP);   // the accumulators are in units of 2^(e_run - WEXP)
+        if (n_splits == 1) {
+            LDS_BARRIER();                                // the sums
 #pragma unroll
-        for (int h2 = 0; h2 < 2; h2++) {
-            const f32x4 lv = *(const f32x4 *)&lsum[(h2 * 16 + n) * 4];
-            float L = (lv[0] + lv[1]) + (lv[2] + lv[3]);
-            const int head = hb * HW + 16 * h2 + n;
-            if (head >= nh) continue;
-            // the attention sink of src/ds_model.c:946: one more term in the denominator, no value
-            // (with several splits the merge kernel adds it)
-            if (p.sink && n_splits == 1 && m_ref[h2] > -INFINITY)
-                L += __builtin_amdgcn_exp2f(p.sink[head] * 1.44269504088896340736f - m_ref[h2]);
-            const float unit_f = e_run == E_NONE ? 0.0f : pow2i(e_run - WEXP);   // the accumulators are in units of 2^(e_run - WEXP)
-            const float fin = n_splits == 1 ? (L > 0.0f ? unit_f / L : 0.0f) : unit_f;
-            const size_t pb = (size_t)(y * (uint32_t)n_splits + (uint32_t)split) * (2 * n_hb) + 2 * hb + h2;
-            if (n_splits == 1) {
+            for (int h2 = 0; h2 < 2; h2++) {
+                const f32x4 lv = *(const f32x4 *)&lsum[(h2 * 16 + n) * 4];
+                float L = (lv[0] + lv[1]) + (lv[2] + lv[3]);
+                const int head = hb * HW + 16 * h2 + n;
+                if (head >= nh) continue;
+                // the attention sink of src/ds_model.c:946: one more term in the denominator, no value
+                // (with several splits the merge kernel adds it)
+                if (p.sink && m_ref[h2] > -INFINITY)
+                    L += __builtin_amdgcn_exp2f(p.sink[head] * 1.44269504088896340736f - m_ref[h2]);
+                const float fin = L > 0.0f ? unit_f / L : 0.0f;
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
                     // accumulator register i <-> dim 16 db + 4 g + i
                     const f32x4 v = oacc[h2][j] * fin;
                     *(f32x4 *)(p.out + (size_t)(y * (uint32_t)nh + (uint32_t)head) * VDIM + 16 * (8 * cw + j) + 4 * g) = v;
                 }
-                continue;
             }
-            // The partial leaves as 16-bit fixed point: this wave's 128 dims of the head share one
-            // scale, their largest magnitude, so every value is off by at most 2^-16 of that.  A
-            // non-finite value makes the scale NaN and with it the head's merged output.
-            // (the largest magnitude as an integer maximum of the bit patterns without their signs:
-            // infinities and NaNs compare above every finite value; four chains, because each link
-            // waits for the one before it, and the four lanes of a head meet without a trip
-            // through LDS)
-            uint32_t b0 = 0u, b1 = 0u, b2 = 0u, b3 = 0u;
+            return;
+        }
+        // The partial leaves as 16-bit fixed point: this wave's 128 dims of the head share one scale, their largest
+        // magnitude, so every value is off by at most 2^-16 of that.  A non-finite value makes the scale NaN and with it
+        // the head's merged output (v_maximum3 hands a NaN on; two values and their signs an instruction, four
+        // chains, because each link waits for the one before it; the four lanes of a head meet without a trip through
+        // LDS).  None of it needs the sums: they are met behind it, when the stores are on their way.
+        float big[2];
+        const size_t pb0 = (size_t)(y * (uint32_t)n_splits + (uint32_t)split) * (2 * n_hb) + 2 * hb;
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const u32x4 a = __builtin_bit_cast(u32x4, oacc[h2][j]) & 0x7FFFFFFFu;
-                b0 = a[0] > b0 ? a[0] : b0;
-                b1 = a[1] > b1 ? a[1] : b1;
-                b2 = a[2] > b2 ? a[2] : b2;
-                b3 = a[3] > b3 ? a[3] : b3;
+        for (int h2 = 0; h2 < 2; h2++) {
+            float m[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const f32x4 a = oacc[h2][2 * c], b = oacc[h2][2 * c + 1];
+                m[c] = maximum3_abs(a[0], a[1], a[2]);
+                m[c] = maximum3_abs(m[c], a[3], b[0]);
+                m[c] = maximum3_abs(m[c], b[1], b[2]);
+                m[c] = maximum3_abs(m[c], b[3], b[3]);
             }
-            uint32_t bm = b0 > b1 ? b0 : b1;
-            const uint32_t bn = b2 > b3 ? b2 : b3;
-            bm = bm > bn ? bm : bn;
-            bm = lanes_xor16_max(bm);
+            uint32_t bm = __builtin_bit_cast(uint32_t, maximum3_abs(maximum3_abs(m[0], m[1], m[2]), m[3], m[3])) & 0x7FFFFFFFu;
+            bm = lanes_xor16_max(bm);                     // (as integers: NaNs and infinities are above every finite value)
             bm = lanes_xor32_max(bm);
-            float big = bm > 0x7F7FFFFFu ? __builtin_nanf("") : __builtin_bit_cast(float, bm);   // in accumulator units
-            const float to_unit = big > 0.0f ? 1.0f / big : 0.0f;
-            uint32_t *pq = p.part_acc + (pb * NDB + 8 * cw) * 128 + lane * 2;   // [db][lane][4 x i16]
+            big[h2] = bm > 0x7F7FFFFFu ? __builtin_nanf("") : __builtin_bit_cast(float, bm);   // in accumulator units
+            const float to_unit = big[h2] > 0.0f ? 1.0f / big[h2] : 0.0f;
+            if (hb * HW + 16 * h2 + n < nh) {
+                uint32_t *pq = p.part_acc + ((pb0 + h2) * NDB + 8 * cw) * 128 + lane * 2;   // [db][lane][4 x i16]
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const f32x4 v = oacc[h2][j] * to_unit;
-                u32x2 w;
-                w[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(v[0], v[1]));
-                w[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(v[2], v[3]));
-                store_through8(pq + j * 128, w);
+                for (int j = 0; j < 8; j++) {
+                    const f32x4 v = oacc[h2][j] * to_unit;
+                    u32x2 w;
+                    w[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(v[0], v[1]));
+                    w[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(v[2], v[3]));
+                    store_through8(pq + j * 128, w);
+                }
             }
-            if (g == 0)
-                *(f32x4 *)(p.part_ml + ((pb * 4 + cw) * HB + n) * 4) =
-                    (f32x4){m_ref[h2] * 0.69314718055994530942f, L, big * fin * (1.0f / 32767.0f), 0.0f};
+        }
+        LDS_BARRIER();                                    // the sums
+        if (g < 2 && hb * HW + 16 * g + n < nh) {
+            const f32x4 lv = *(const f32x4 *)&lsum[lane * 4];
+            const float L = (lv[0] + lv[1]) + (lv[2] + lv[3]);
+            *(f32x4 *)(p.part_ml + (((pb0 + (uint32_t)g) * 4 + cw) * HB + n) * 4) =
+                (f32x4){(g ? m_ref[1] : m_ref[0]) * 0.69314718055994530942f, L, (g ? big[1] : big[0]) * unit_f * (1.0f / 32767.0f), 0.0f};
         }
     }
 }

@@ -15,7 +15,7 @@ import pytest
 
 from cwick_amd import build as B
 
-ASM_MFMA_SOURCES = ["gqa_prefill.hip", "indexer_band.hip", "mla_prefill64.hip"]
+ASM_MFMA_SOURCES = ["gqa_prefill.hip", "indexer_band.hip", "mla_prefill64.hip", "mla_roles.hip"]
 
 
 def _regs(tok):
