@@ -142,15 +142,54 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
         }
         return dead;
     };
+    // The waves of the workgroup meet here at the end; until then a wave's part holds its queries.
+    __shared__ __attribute__((aligned(16))) float sh_acc[NW][GROUP][HD];
+    // The group's queries come whole, 1 KiB a load, and go through LDS to the lanes (sixteen-byte piece p of head h at
+    // place p ^ h, so that the heads of a read come from different banks).  Loads of what each lane needs touch a line
+    // for every lane and occupy the memory pipeline as long as the tile behind them, which a workgroup with one tile
+    // per wave waits for.  (With the folds below in one statement and no rescale before the first tile, replayed from a
+    // graph: 300 keys of 4 x 256 with sixteen heads 7.99 -> 7.04 us, 4096 keys 9.15 -> 8.65; 5000 of 4 x 128 with 32
+    // heads 9.12 -> 8.52, 4096 of 8 x 128 with 64 9.13 -> 8.74; 20000 and more keys the same to 1 %.)
+    // (Not sixteen heads x 256: as many loads either way, and two registers more than there are.)
+    constexpr bool Q_WHOLE = HD * GROUP < 4096;
+    constexpr int Q_LOADS = Q_WHOLE ? (GROUP * HD * 2 + 1023) / 1024 : NK;
+    constexpr int PIECES = HD / 8;                      // of a head
+    u32x4 q_raw[Q_LOADS];
+    auto request_q = [&]() {
+        if constexpr (!Q_WHOLE) {
+#pragma unroll
+            for (int j = 0; j < NK; j++) q_raw[j] = *(const u32x4 *)(Q + (size_t)(g * GROUP + l16) * HD + 32 * j + 8 * lg);
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < Q_LOADS; i++) {
+            const int piece = 64 * i + lane;
+            q_raw[i] = *(const u32x4 *)(Q + (size_t)g * (GROUP * HD) + 8 * (piece < GROUP * PIECES ? piece : 0));
+        }
+    };
     // this lane's part of the queries: head `col`, dims 32j + 8 lg .. +8
     const int col = QUADS ? l16 % GROUP : l16;
     bf16x8 q[NK];
+    auto place_q = [&]() {
+        if constexpr (!Q_WHOLE) {
 #pragma unroll
-    for (int j = 0; j < NK; j++) {
-        u32x4 w = {0u, 0u, 0u, 0u};
-        if (col < GROUP) w = *(const u32x4 *)(Q + (size_t)(g * GROUP + col) * HD + 32 * j + 8 * lg);
-        q[j] = __builtin_bit_cast(bf16x8, w);
-    }
+            for (int j = 0; j < NK; j++) q[j] = __builtin_bit_cast(bf16x8, q_raw[j]);
+            return;
+        }
+        unsigned char *mine = (unsigned char *)&sh_acc[wave][0][0];
+#pragma unroll
+        for (int i = 0; i < Q_LOADS; i++) {
+            const int piece = 64 * i + lane, h = piece / PIECES;
+            if (GROUP * PIECES % 64 == 0 || piece < GROUP * PIECES) *(u32x4 *)(mine + 16 * (piece ^ (h & 15))) = q_raw[i];
+        }
+        const unsigned char *from = mine + (col < GROUP ? col : 0) * (HD * 2);
+#pragma unroll
+        for (int j = 0; j < NK; j++) {
+            u32x4 w = *(const u32x4 *)(from + 16 * ((4 * j + lg) ^ (col & 15)));
+            if (!QUADS && GROUP < 16 && col >= GROUP) w = (u32x4){0u, 0u, 0u, 0u};
+            q[j] = __builtin_bit_cast(bf16x8, w);
+        }
+    };
 
     // acc[.][8h + i]: dim 128 h + 8 l16 + i; heads 4 lg .. +4, with QUADS heads 4 qd .. +4 over the
     // lane group's keys
@@ -174,16 +213,18 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
         if (__any(top > m + SLACK)) {                   // the first tile, and hardly ever again
             top = fmaxf(m, xor32_max(xor16_max(top)));
             const float corr = top > -INFINITY ? __builtin_amdgcn_exp2f(m - top) : 1.0f;
+            const bool some = __any(m > -INFINITY);     // (before that nothing has been added up)
             m = top;
             l *= corr;
+            if (some)
 #pragma unroll
-            for (int qd = 0; qd < NQ; qd++) {
-                f32x4 c;                                // the factors of the accumulators' heads
+                for (int qd = 0; qd < NQ; qd++) {
+                    f32x4 c;                            // the factors of the accumulators' heads
 #pragma unroll
-                for (int r = 0; r < 4; r++) c[r] = __shfl(corr, QUADS ? 4 * qd + r : 4 * lg + r, 64);
+                    for (int r = 0; r < 4; r++) c[r] = __shfl(corr, QUADS ? 4 * qd + r : 4 * lg + r, 64);
 #pragma unroll
-                for (int i = 0; i < 8 * NV; i++) acc[qd][i] *= c;
-            }
+                    for (int i = 0; i < 8 * NV; i++) acc[qd][i] *= c;
+                }
         }
         const float mu = m == -INFINITY ? 0.0f : m;
 #pragma unroll
@@ -220,7 +261,9 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
     if (t < count) {
         GqaDecTile<HD> a, b;
         if (LIST) names_next = entries(t);
+        request_q();
         uint32_t dead_a = load(a, t), dead_b = 0;
+        place_q();
         for (;;) {
             if (t + STRIDE < count) dead_b = load(b, t + STRIDE);
             step(a, dead_a);
@@ -235,15 +278,31 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
     l = xor32_sum(xor16_sum(l));
 
     // the waves of the workgroup through LDS
-    __shared__ __attribute__((aligned(16))) float sh_acc[NW][GROUP][HD];
     __shared__ float sh_m[NW][GROUP], sh_l[NW][GROUP];
     if constexpr (QUADS) {
         // the lane groups' sums meet on the way: a swap of two registers leaves one half of the lanes
         // with both parts of the first and the other half with both parts of the second
-        auto fold = [](float x, float y, auto swap) {
-            uint32_t a = __builtin_bit_cast(uint32_t, x), b = __builtin_bit_cast(uint32_t, y);
-            swap(a, b);
-            return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+        // (one statement for four or two swaps: each by itself has two wait states in front of it)
+        auto fold32 = [](const float (&x)[4], const float (&y)[4], float *t) {
+            float a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) a[i] = x[i], b[i] = y[i];
+            asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %4\n\tv_permlane32_swap_b32 %1, %5\n\tv_permlane32_swap_b32 %2, %6\n\tv_permlane32_swap_b32 %3, %7"
+                         : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
+#pragma unroll
+            for (int i = 0; i < 4; i++) t[i] = a[i] + b[i];
+        };
+        auto fold16 = [](float *t, int half) {          // t[0 .. half) and t[half .. 2 half), half 2 or 4
+            float a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) a[i] = t[i % half], b[i] = t[half + i % half];
+            if (half == 4)
+                asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %4\n\tv_permlane16_swap_b32 %1, %5\n\tv_permlane16_swap_b32 %2, %6\n\tv_permlane16_swap_b32 %3, %7"
+                             : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
+            else
+                asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %2\n\tv_permlane16_swap_b32 %1, %3" : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]));
+#pragma unroll
+            for (int i = 0; i < half; i++) t[i] = a[i] + b[i];
         };
 #pragma unroll
         for (int qd = 0; qd < NQ; qd++)
@@ -251,11 +310,12 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
             for (int r = 0; r < (GROUP < 4 ? GROUP : 4); r++) {
                 float t[4 * NV];
 #pragma unroll
-                for (int i = 0; i < 4 * NV; i++)
-                    t[i] = fold(acc[qd][i][r], acc[qd][i + 4 * NV][r], [](uint32_t &a, uint32_t &b) { lanes_swap32(a, b); });
-#pragma unroll
-                for (int i = 0; i < 2 * NV; i++)
-                    t[i] = fold(t[i], t[i + 2 * NV], [](uint32_t &a, uint32_t &b) { lanes_swap16(a, b); });
+                for (int i = 0; i < 4 * NV; i += 4) {
+                    const float x[4] = {acc[qd][i][r], acc[qd][i + 1][r], acc[qd][i + 2][r], acc[qd][i + 3][r]};
+                    const float y[4] = {acc[qd][i + 4 * NV][r], acc[qd][i + 4 * NV + 1][r], acc[qd][i + 4 * NV + 2][r], acc[qd][i + 4 * NV + 3][r]};
+                    fold32(x, y, t + i);
+                }
+                fold16(t, 2 * NV);
                 // this lane: accumulators 4 NV (lg / 2) + 2 NV (lg % 2) .. + 2 NV
                 const int first = 4 * NV * (lg >> 1) + 2 * NV * (lg & 1);
                 float *dst = &sh_acc[wave][4 * qd + r][128 * (first >> 3) + 8 * l16 + (first & 7)];
