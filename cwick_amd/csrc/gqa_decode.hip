@@ -66,9 +66,10 @@ constexpr int GQA_DEC_QUADS = GROUP <= 4 ? 1 : GROUP == 8 && HD == 128 ? 2 : 0; 
 template <int HD, int GROUP, bool LIST>
 __global__ void __launch_bounds__(GQA_DEC_THREADS, HD == 256 || GROUP == 8 ? 2 : 3)
 gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-                        const uint16_t *__restrict__ Q, int64_t n_keys, int n_kv_heads,
-                        const int32_t *__restrict__ sel, int64_t n_rows,
+                        const uint16_t *__restrict__ Q, int n_keys, int n_kv_heads, int n_splits,
                         float scale_log2e,
+                        const int32_t *__restrict__ sel, int64_t n_rows,
+                        // (up to here they arrive in registers: what the first loads need is among them)
                         float *__restrict__ part_acc,   // [n_splits][n_heads][HD]
                         float *__restrict__ part_ml,    // [n_splits][n_heads][2]
                         float *__restrict__ out,        // [n_heads][HD], one split only; host memory where there are flags
@@ -83,12 +84,12 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
     const int l16 = lane & 15, lg = lane >> 4;
     const uint32_t row_stride = (uint32_t)n_kv_heads * HD;
     const int64_t k_begin = (int64_t)split * (NW * GQA_DEC_TILE);
-    const int count = (int)(n_keys - k_begin);          // from its first key to the end (negative: none)
+    const int count = n_keys - (int)k_begin;          // from its first key to the end (negative: none)
     const uint16_t *Kg = K + (LIST ? 0 : k_begin * row_stride) + (size_t)g * HD + lg * 8;
     const uint16_t *Vg = V + (LIST ? 0 : k_begin * row_stride) + (size_t)g * HD + l16 * 8;
     const int32_t *list = LIST ? sel + k_begin : nullptr;
 
-    const int STRIDE = (int)gridDim.x * (NW * GQA_DEC_TILE);
+    const int STRIDE = n_splits * (NW * GQA_DEC_TILE);
     int t = wave * GQA_DEC_TILE;
     // List entries, those of four of the wave's tiles in one register: lane 16 j + i has key i of the j-th.
     // A tile takes what it needs (key l16, whose K row this lane reads, and keys 4 lg .. +4 of the V rows)
@@ -361,7 +362,7 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
             }
         }
         const int h = g * GROUP + j;
-        if (gridDim.x == 1) {
+        if (n_splits == 1) {
             a *= ls > 0.0f ? 1.0f / ls : 0.0f;
             if (flags) store_through16(&out[(size_t)h * HD + d], __builtin_bit_cast(u32x4, a));
             else *(f32x4 *)&out[(size_t)h * HD + d] = a;
@@ -379,9 +380,8 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
         __syncthreads();
         if (threadIdx.x == 0) sh_ticket = __hip_atomic_fetch_add(&tickets[g], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
-        if (sh_ticket != gridDim.x - 1) return;
+        if (sh_ticket != (uint32_t)n_splits - 1) return;
         if (threadIdx.x == 0) __hip_atomic_store(&tickets[g], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int n_splits = (int)gridDim.x;
         for (int i4 = threadIdx.x; i4 < GROUP * HD / 4; i4 += GQA_DEC_THREADS) {
             const int h = g * GROUP + i4 / (HD / 4), d = (i4 % (HD / 4)) * 4;
             const float *pa = part_acc + (size_t)h * HD + d, *pm = part_ml + 2 * h;
@@ -410,7 +410,7 @@ gqa_decode_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
             else *(f32x4 *)&out[(size_t)h * HD + d] = r;
         }
     }
-    if (flags && (tickets || gridDim.x == 1)) {
+    if (flags && (tickets || n_splits == 1)) {
         stores_done();
         __syncthreads();
         if (threadIdx.x == 0) host_flag(flags, g, epoch);
@@ -455,8 +455,8 @@ static int run_gqa_decode(const uint16_t *k, const uint16_t *v, int64_t n_keys, 
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_DECODE, s);
         pk.launch(sel ? gqa_decode_split_kernel<HD, GROUP, true> : gqa_decode_split_kernel<HD, GROUP, false>,
-                  dim3(n_splits, n_kv_heads), dim3(GQA_DEC_THREADS), 0, k, v, q, n_keys, n_kv_heads, sel, n_rows,
-                  scale * 1.44269504088896340736f, part_acc, part_ml, out, flags, epoch, tickets);
+                  dim3(n_splits, n_kv_heads), dim3(GQA_DEC_THREADS), 0, k, v, q, (int)n_keys, n_kv_heads, n_splits,
+                  scale * 1.44269504088896340736f, sel, n_rows, part_acc, part_ml, out, flags, epoch, tickets);
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (one_launch) return 1;

@@ -402,20 +402,33 @@ indexer_approx_kernel(const uint8_t *__restrict__ keys, const float *__restrict_
 // (the q values of a head come to the FMAs through DPP row broadcasts); the 64 weighted terms
 // of a candidate meet in LDS and one lane adds them in head order.
 __global__ void __launch_bounds__(256)
-indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict__ kscale,
-                       int64_t key_bstride, int64_t kscale_bstride, int64_t n_keys,
+indexer_rescore_kernel(const int32_t *__restrict__ cand, const IndexerBandRow *__restrict__ rows, int n_keys32, int cap,
                        const uint16_t *__restrict__ q, const float *__restrict__ w, int ih,
-                       const int32_t *__restrict__ cand, int cap,
-                       const IndexerBandRow *__restrict__ rows, float *__restrict__ scores,
+                       // (up to here they arrive in registers)
+                       const uint8_t *__restrict__ keys, const float *__restrict__ kscale,
+                       int64_t key_bstride, int64_t kscale_bstride, float *__restrict__ scores,
                        float *__restrict__ cand_score) {   // [batch][cap]: the same scores in list order
     __shared__ __attribute__((aligned(16))) float terms[16][68];
     const int b = blockIdx.y, tid = threadIdx.x;
+    const int64_t n_keys = n_keys32;
     int c0 = blockIdx.x * 16;
     const int j = tid & 15, hg = tid >> 4;                          // candidate, head group
     // The list entry is fetched next to the row's state, not behind it (one round trip less in
     // front of the key's bytes): an entry past the end of the list is whatever the workspace
     // held, so it is clamped to a key of the row; what is computed for it is not stored.
     int64_t t_guess = cand[(size_t)b * cap + c0 + j];
+    // q of the group's four heads, on its way beside them: lane j holds q[h][8 j .. 8 j + 7]
+    const uint16_t *qb = q + (size_t)b * ih * IB_HD;
+    const float *wb = w + (size_t)b * ih;
+    u32x4 qraw[4];
+    float wh[4];
+#pragma unroll
+    for (int hh = 0; hh < 4; hh++) {
+        const int h = hg * 4 + hh;
+        const int hc = h < ih ? h : ih - 1;
+        qraw[hh] = *(const u32x4 *)(qb + (size_t)hc * IB_HD + 8 * j);
+        wh[hh] = wb[hc];
+    }
     IndexerBandRow st;                                              // the two words in use, not the padding
     st.n_cand = rows[b].n_cand;
     st.fallback = rows[b].fallback;
@@ -438,8 +451,6 @@ indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict
     }
     const uint8_t *krow = keys + (size_t)b * key_bstride + (size_t)t * IB_HD;
     const float ks = kscale[(size_t)b * kscale_bstride + t];
-    const uint16_t *qb = q + (size_t)b * ih * IB_HD;
-    const float *wb = w + (size_t)b * ih;
     float e[IB_HD];
 #pragma unroll
     for (int c = 0; c < IB_HD / 16; c++) {
@@ -453,16 +464,6 @@ indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict
             e[c * 16 + jj * 4 + 2] = hi[0];
             e[c * 16 + jj * 4 + 3] = hi[1];
         }
-    }
-    // q of the group's four heads, all loads in flight at once: lane j holds q[h][8 j .. 8 j + 7]
-    u32x4 qraw[4];
-    float wh[4];
-#pragma unroll
-    for (int hh = 0; hh < 4; hh++) {
-        const int h = hg * 4 + hh;
-        const int hc = h < ih ? h : ih - 1;
-        qraw[hh] = *(const u32x4 *)(qb + (size_t)hc * IB_HD + 8 * j);
-        wh[hh] = wb[hc];
     }
     f32x4 mine;
 #pragma unroll
@@ -508,7 +509,7 @@ indexer_rescore_kernel(const uint8_t *__restrict__ keys, const float *__restrict
         float s = 0.0f;
 #pragma unroll
         for (int h = 0; h < 64; h++) s = s + x[h >> 2][h & 3];
-        scores[(size_t)b * n_keys + cand[(size_t)b * cap + c0 + tid]] = s;
+        scores[(size_t)b * n_keys + t] = s;                         // (candidate j is thread j's own)
         cand_score[(size_t)b * cap + c0 + tid] = s;
     }
     __syncthreads();                                                // before the next round's terms
@@ -584,7 +585,7 @@ int launch_indexer_banded(const uint8_t *keys, const float *kscale, int64_t key_
     int rescore_wgs = num_cus() / batch;
     rescore_wgs = rescore_wgs < 8 ? 8 : (rescore_wgs > cap / 16 ? cap / 16 : rescore_wgs);
     indexer_rescore_kernel<<<dim3(rescore_wgs, batch), 256, 0, s>>>(
-        keys, kscale, key_bstride, kscale_bstride, n_keys, q_idx, w, n_idx_heads, cand, cap, rows, scores, cand_score);
+        cand, rows, (int)n_keys, cap, q_idx, w, n_idx_heads, keys, kscale, key_bstride, kscale_bstride, scores, cand_score);
     CWICK_HIP_CALL(hipGetLastError());
     }
     return launch_topk_band_finish(scores, batch, n_keys, k, cand, cand_score, cap, rows, hi_count, out_idx, s);
