@@ -384,12 +384,13 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
     const int hhu = wave >= 5 ? 1 : 0, bu = wave - 5 * hhu;
     const uint32_t unit_lds = lds0 + PARK + (uint32_t)wave * PARK_UNIT;
     if (has_unit) {
-        const uint64_t base = (uint64_t)(uintptr_t)(q + (size_t)(y * (uint32_t)nh) * KDIM + 128 * bu);
+        const uint64_t base = (uint64_t)(uintptr_t)(q + (size_t)(y * (uint32_t)nh) * KDIM + 128 * bu);      // (a scalar)
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             const int h = 4 * c + g, head0 = hb * HW + 16 * hhu + h, head = head0 < nh ? head0 : nh - 1;
             const int x = (n ^ h) & (bu < 4 ? 15 : 7);             // the rope block has eight pieces: fetched twice
-            dma16(base + (uint64_t)(uint32_t)head * (KDIM * 2) + (uint32_t)(16 * x), unit_lds + (uint32_t)c * 1024);
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" ::"v"((uint32_t)head * (KDIM * 2) + (uint32_t)(16 * x)),
+                         "s"(unit_lds + (uint32_t)c * 1024), "s"(base) : "memory");
         }
         if (SEL) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
     } else if (SEL) {
@@ -600,6 +601,13 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
             else if (SCORE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (STEADY) share_steady(t + 3, {r_cp, -1}, lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B);
             else if (do_copy) share(t + 3, {SEL ? r_cp : row_of(t + 3, key_of), -1}, lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B);
+            if constexpr (!SCORE) {
+                // the sums of the scoring role go where tile t + 1 would have its weights
+                float *lsum = reinterpret_cast<float *>(&sm.x[(t + 1) & 1]);      // [head half][head][key block]
+                float ls = xor16_sum(l_priv);
+                ls = xor32_sum(ls);
+                if (g == 0) lsum[(hh * 16 + n) * 4 + kb] = ls;
+            }
             LDS_BARRIER();
         };
         int t = 0;
@@ -609,13 +617,6 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
 #pragma clang loop unroll(disable)
         for (; t + 1 < n_tiles; t++) step(t, std::integral_constant<int, TAIL>{});
         step(t, std::integral_constant<int, LAST>{});
-
-        // ---- the sums of the scoring role meet in LDS (the exchange area is free now) ----
-        float *lsum = reinterpret_cast<float *>(&sm.x[0]);            // [head half][head][key block]
-        float ls = xor16_sum(l_priv);
-        ls = xor32_sum(ls);
-        if (g == 0) lsum[(hh * 16 + n) * 4 + kb] = ls;
-        LDS_BARRIER();
     } else {
         LDS_BARRIER();                                // before copies or weights land in the park area
         f32x4 oacc[2][8];                                 // [head half][dim block]: dims 128 cw + 16 j + 4 g + i, head n
@@ -641,7 +642,58 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
         const uint32_t pw_off = (uint32_t)((g * 16 + n) * 16);
         const uint32_t xml_off = XM_OFF + (uint32_t)(n * 16);
         asm volatile("" ::: "memory");
-        // step -1: tile 1 must be whole at the barrier
+        // What a tile's values need besides the probabilities is fetched and prepared a step ahead, when the tile is whole
+        // already: behind the barrier a step has the probabilities and flags to wait for, and nothing else.  (In step 0
+        // that is a round trip to LDS, the first normaliser and eight pairs of factors, 1 200 of the 15 700 cycles of a
+        // workgroup with one tile: the value waves have nothing to do while that tile is scored.)
+        i32x2 vt[16];                                     // V^T, fragment q: dim block (q >> 1) & 7 of the wave's, key half q & 1
+        u32x4 sw[2];                                      // scale * 2^(WEXP - e_run) of the slots' keys, fp16 pairs
+        float ecorr = 1.0f;
+        auto prepare = [&](int t) {
+            const uint32_t tb = lds0 + (uint32_t)(t & (NST - 1)) * TILE_B;
+            // The sixteen lanes of a row share their contraction slots (keys 8 g .. 8 g + 7 of each
+            // half), so a row needs eight fp16 pairs of scale factors per tile: lane (g, n) reads
+            // the two scales of pair n & 7 (half (n & 7) >> 2, keys 8 g + 2 (n & 3) and the next),
+            // forms that one pair, and every lane takes the eight pairs out of the row by DPP.
+            const f32x2 sv = LDS_AT(lds_f32x2, tb + sv_off);
+            const uint32_t va[4] = {tb + tr_off[0], tb + tr_off[1], tb + tr_off[2], tb + tr_off[3]};
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const int j = q >> 1;
+                vt[q] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2 *)(size_t)(va[j & 3] + (uint32_t)(512 * (j >> 2) + 4096 * (q & 1))));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // normaliser of the fp16 weights: a power of two above every scale seen so far (it
+            // only grows, and only then the lanes confer).  Scales are compared as integers:
+            // they are positive, and a negative or NaN scale has the larger bit pattern too.
+            ecorr = 1.0f;
+            {
+                const uint32_t b0 = __builtin_bit_cast(uint32_t, sv[0]) & 0x7FFFFFFFu, b1 = __builtin_bit_cast(uint32_t, sv[1]) & 0x7FFFFFFFu;
+                const uint32_t smax = b0 > b1 ? b0 : b1;
+                if (__any(smax >= thr_bits && smax != 0u)) {
+                    float sm_f = __builtin_bit_cast(float, smax);
+                    sm_f = wave_max(sm_f);
+                    const int e_tile = (int)((__builtin_bit_cast(uint32_t, sm_f) >> 23) & 0xFFu) - 126;
+                    if (e_tile > e_run) {
+                        if (e_run != E_NONE) ecorr = pow2i(e_run - e_tile);
+                        e_run = e_tile;
+                        thr_bits = __builtin_bit_cast(uint32_t, pow2i(e_run));
+                        wfac = pow2i(WEXP - e_run);
+                    }
+                }
+            }
+            const uint32_t my_pair = pack_f16_rne(sv[0] * wfac, sv[1] * wfac);
+            sw[0][0] = row_place<0>(my_pair);
+            sw[0][1] = row_place<1>(my_pair);
+            sw[0][2] = row_place<2>(my_pair);
+            sw[0][3] = row_place<3>(my_pair);
+            sw[1][0] = row_place<4>(my_pair);
+            sw[1][1] = row_place<5>(my_pair);
+            sw[1][2] = row_place<6>(my_pair);
+            sw[1][3] = row_place<7>(my_pair);
+        };
+        // step -1: tile 1 must be whole at the barrier (tile 0 is)
+        prepare(0);
         if (n_tiles > 2) CWICK_ROLES_WAIT(0, 2, 3);
         else CWICK_ROLES_WAIT(0, 0, 0);
         RowPair r_cp = {-1, -1};
@@ -651,65 +703,19 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
             constexpr bool STEADY = decltype(kind)::value == STEADY_;
             const bool do_copy = STEADY || t + 3 < n_tiles;
             {
-                const uint32_t stage = lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B;   // which tile t-1 left at the last barrier
-                if (STEADY) share_steady(t + 3, r_cp, stage);
-                else if (do_copy) share(t + 3, SEL ? r_cp : rows_of(t + 3), stage);
-                if (SEL && do_copy) r_cp = rows_of(t + 4);
-            }
-            {
                 // ---- values O^T[dim][head] += V^T W^T for dims 128 cw.., all 32 heads, tile t ----
-                const uint32_t tb = lds0 + (uint32_t)(t & (NST - 1)) * TILE_B;
                 const uint32_t xb = lds0 + X_OFF + (uint32_t)(t & 1) * XCH_B;
-                // The sixteen lanes of a row share their contraction slots (keys 8 g .. 8 g + 7 of each
-                // half), so a row needs eight fp16 pairs of scale factors per tile: lane (g, n) reads
-                // the two scales of pair n & 7 (half (n & 7) >> 2, keys 8 g + 2 (n & 3) and the next),
-                // forms that one pair, and every lane takes the eight pairs out of the row by DPP.
-                const f32x2 sv = LDS_AT(lds_f32x2, tb + sv_off);
+                const u32x2 fl = LDS_AT(lds_u32x2, xb + XF_OFF);
                 u32x4 pw[2][2];                           // [head half][key half]
 #pragma unroll
                 for (int h2 = 0; h2 < 2; h2++)
 #pragma unroll
                     for (int kh = 0; kh < 2; kh++) pw[h2][kh] = LDS_AT(lds_u32x4, xb + pw_off + (uint32_t)((h2 * 2 + kh) * 1024));
-                const u32x2 fl = LDS_AT(lds_u32x2, xb + XF_OFF);
-                // V^T, fragment q of the tile: dim block (q >> 1) & 7 of the wave's, key half q & 1
-                const uint32_t va[4] = {tb + tr_off[0], tb + tr_off[1], tb + tr_off[2], tb + tr_off[3]};
-                i32x2 vt[16];
-                auto vfetch = [&](int q) {
-                    const int j = q >> 1;
-                    vt[q] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2 *)(size_t)(va[j & 3] + (uint32_t)(512 * (j >> 2) + 4096 * (q & 1))));
-                };
-#pragma unroll
-                for (int q = 0; q < 8; q++) vfetch(q);
                 __builtin_amdgcn_sched_barrier(0);
-                // normaliser of the fp16 weights: a power of two above every scale seen so far (it
-                // only grows, and only then the lanes confer).  Scales are compared as integers:
-                // they are positive, and a negative or NaN scale has the larger bit pattern too.
-                float ecorr = 1.0f;
-                {
-                    const uint32_t b0 = __builtin_bit_cast(uint32_t, sv[0]) & 0x7FFFFFFFu, b1 = __builtin_bit_cast(uint32_t, sv[1]) & 0x7FFFFFFFu;
-                    const uint32_t smax = b0 > b1 ? b0 : b1;
-                    if (__any(smax >= thr_bits && smax != 0u)) {
-                        float sm_f = __builtin_bit_cast(float, smax);
-                        sm_f = wave_max(sm_f);
-                        const int e_tile = (int)((__builtin_bit_cast(uint32_t, sm_f) >> 23) & 0xFFu) - 126;
-                        if (e_tile > e_run) {
-                            if (e_run != E_NONE) ecorr = pow2i(e_run - e_tile);
-                            e_run = e_tile;
-                            thr_bits = __builtin_bit_cast(uint32_t, pow2i(e_run));
-                            wfac = pow2i(WEXP - e_run);
-                        }
-                    }
-                }
-                const uint32_t my_pair = pack_f16_rne(sv[0] * wfac, sv[1] * wfac);
-                u32x4 sw[2];                              // scale * 2^(WEXP - e_run) of the slots' keys, fp16 pairs
-                sw[0][0] = row_place<0>(my_pair);
-                sw[0][1] = row_place<1>(my_pair);
-                sw[0][2] = row_place<2>(my_pair);
-                sw[0][3] = row_place<3>(my_pair);
-                sw[1][0] = row_place<4>(my_pair);
-                sw[1][1] = row_place<5>(my_pair);
-                sw[1][2] = row_place<6>(my_pair);
-                sw[1][3] = row_place<7>(my_pair);
+                const uint32_t stage = lds0 + (uint32_t)((t + 3) & (NST - 1)) * TILE_B;   // which tile t-1 left at the last barrier
+                if (STEADY) share_steady(t + 3, r_cp, stage);
+                else if (do_copy) share(t + 3, SEL ? r_cp : rows_of(t + 3), stage);
+                if (SEL && do_copy) r_cp = rows_of(t + 4);
                 if (__builtin_amdgcn_readfirstlane(fl[0] | fl[1]) != 0u || ecorr != 1.0f) {
                     // a scoring wave left the common reference in this tile (or the weights'
                     // normaliser grew): bring accumulators and probabilities to the new maximum
@@ -742,9 +748,6 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
 #pragma unroll
                         for (int d = 0; d < 4; d++) pw[h2][kh][d] = mul_f16x2(pw[h2][kh][d], sw[kh][d]);
 #pragma unroll
-                for (int q = 8; q < 16; q++) vfetch(q);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
                 for (int q = 0; q < 16; q++) {
                     const int j = q >> 1, kh = q & 1;
                     u32x4 vh;
@@ -757,6 +760,7 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                     oacc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, __builtin_bit_cast(f16x8, pw[1][kh]), oacc[1][j], 0, 0, 0);
                 }
             }
+            if (STEADY || t + 1 < n_tiles) prepare(t + 1);
             // tile t+2 must be whole at the next barrier; the share of the tile behind it may stay in flight
             if (do_copy) CWICK_ROLES_WAIT(0, 2, 3);
             else CWICK_ROLES_WAIT(0, 0, 0);
@@ -769,10 +773,9 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
         for (; t < n_tiles; t++) step(t, std::integral_constant<int, TAIL>{});
 
         // ---- every value wave owns its dims: write the partial (or the result) directly ----
-        const float *lsum = reinterpret_cast<const float *>(&sm.x[0]);
+        const float *lsum = reinterpret_cast<const float *>(&sm.x[n_tiles & 1]);   // written in front of the last barrier
         const float unit_f = e_run == E_NONE ? 0.0f : pow2i(e_run - WEXP);   // the accumulators are in units of 2^(e_run - WEXP)
         if (n_splits == 1) {
-            LDS_BARRIER();                                // the sums
 #pragma unroll
             for (int h2 = 0; h2 < 2; h2++) {
                 const f32x4 lv = *(const f32x4 *)&lsum[(h2 * 16 + n) * 4];
@@ -797,7 +800,7 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
         // magnitude, so every value is off by at most 2^-16 of that.  A non-finite value makes the scale NaN and with it
         // the head's merged output (v_maximum3 hands a NaN on; two values and their signs an instruction, four
         // chains, because each link waits for the one before it; the four lanes of a head meet without a trip through
-        // LDS).  None of it needs the sums: they are met behind it, when the stores are on their way.
+        // LDS).
         float big[2];
         const size_t pb0 = (size_t)(y * (uint32_t)n_splits + (uint32_t)split) * (2 * n_hb) + 2 * hb;
 #pragma unroll
@@ -828,7 +831,6 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 }
             }
         }
-        LDS_BARRIER();                                    // the sums
         if (g < 2 && hb * HW + 16 * g + n < nh) {
             const f32x4 lv = *(const f32x4 *)&lsum[lane * 4];
             const float L = (lv[0] + lv[1]) + (lv[2] + lv[3]);
