@@ -424,45 +424,56 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// 32 bf16 values of a query (16 dwords) as two E4M3 terms, hi + lo, in units of a power of two that the
-// four lanes l, l ^ 16, l ^ 32, l ^ 48 (a head's 128 dims) share; returns the unit's E8M0 byte.
-// The bf16 pairs go straight into the scaled conversions: nine instructions per pair, where widening,
+// bf16 values of a query as two E4M3 terms, hi + lo, in units of a power of two that the lanes which hold the same
+// head's block share.  The bf16 pairs go straight into the scaled conversions: nine instructions per pair, where widening,
 // scaling and the plain conversions took thirteen (the same bits for every bf16 value below the unit's
 // overflow).  The largest magnitude is an integer maximum of the bit patterns without their signs.
-__device__ __forceinline__ uint32_t q_two_terms(const u32x4 (&w)[4], u32x4 (&hi)[2], u32x4 (&lo)[2]) {
+typedef __attribute__((ext_vector_type(2))) unsigned short q_u16x2;
+__device__ __forceinline__ q_u16x2 q_larger(q_u16x2 m, uint32_t pair) {
+    return __builtin_elementwise_max(m, __builtin_bit_cast(q_u16x2, pair & 0x7FFF7FFFu));
+}
+// the unit's E8M0 byte, from the largest magnitude's bits
+__device__ __forceinline__ uint32_t q_unit(uint32_t top) {
+    const int s = top ? (int)(top >> 7) - 127 - 7 : 0;
+    return (uint32_t)(127 + (s < -110 ? -110 : s));
+}
+// four values, two pairs
+__device__ __forceinline__ void q_two_terms(uint32_t x0, uint32_t x1, uint32_t unit_byte, uint32_t &hi, uint32_t &lo) {
     typedef __attribute__((ext_vector_type(2))) short s16x2;
-    typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
     typedef __attribute__((ext_vector_type(2))) __bf16 b16x2;
-    u16x2 m[4] = {};
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int d = 0; d < 4; d++) m[d] = __builtin_elementwise_max(m[d], __builtin_bit_cast(u16x2, w[c][d] & 0x7FFF7FFFu));
-    const u16x2 mm = __builtin_elementwise_max(__builtin_elementwise_max(m[0], m[1]), __builtin_elementwise_max(m[2], m[3]));
-    uint32_t top = mm[0] > mm[1] ? mm[0] : mm[1];
-    top = lanes_xor32_max(lanes_xor16_max(top));
-    int s = top ? (int)(top >> 7) - 127 - 7 : 0;
-    s = s < -110 ? -110 : s;
-    const float unit = __builtin_bit_cast(float, (uint32_t)(s + 127) << 23);
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int d = 0; d < 4; d++) {
-            s16x2 h = {0, 0}, l = {0, 0};
-#define CWICK_Q_PAIR(HALF)                                                                                              \
+    const float unit = __builtin_bit_cast(float, unit_byte << 23);
+    s16x2 h = {0, 0}, l = {0, 0};
+#define CWICK_Q_PAIR(x, HALF)                                                                                           \
     do {                                                                                                                \
-        const uint32_t x = w[2 * c + (d >> 1)][2 * (d & 1) + HALF];                                                     \
         h = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(h, __builtin_bit_cast(b16x2, x), unit, HALF);                     \
         const f32x2 back = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(__builtin_bit_cast(uint32_t, h), unit, HALF);       \
         l = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(l, bf16lo_to_f32(x) - back[0], bf16hi_to_f32(x) - back[1], unit, HALF); \
     } while (0)
-            CWICK_Q_PAIR(0);
-            CWICK_Q_PAIR(1);
+    CWICK_Q_PAIR(x0, 0);
+    CWICK_Q_PAIR(x1, 1);
 #undef CWICK_Q_PAIR
-            hi[c][d] = __builtin_bit_cast(uint32_t, h);
-            lo[c][d] = __builtin_bit_cast(uint32_t, l);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, l);
+}
+// 32 values (16 dwords) per lane, the head's 128 dims in lanes l, l ^ 16, l ^ 32, l ^ 48; returns the unit's E8M0 byte
+__device__ __forceinline__ uint32_t q_two_terms(const u32x4 (&w)[4], u32x4 (&hi)[2], u32x4 (&lo)[2]) {
+    q_u16x2 m[4] = {};
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) m[d] = q_larger(m[d], w[c][d]);
+    const q_u16x2 mm = __builtin_elementwise_max(__builtin_elementwise_max(m[0], m[1]), __builtin_elementwise_max(m[2], m[3]));
+    const uint32_t unit_byte = q_unit(lanes_xor32_max(lanes_xor16_max(mm[0] > mm[1] ? mm[0] : mm[1])));
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            uint32_t h, l;
+            q_two_terms(w[2 * c + (d >> 1)][2 * (d & 1)], w[2 * c + (d >> 1)][2 * (d & 1) + 1], unit_byte, h, l);
+            hi[c][d] = h;
+            lo[c][d] = l;
         }
-    return (uint32_t)(127 + s);
+    return unit_byte;
 }
 
 // Sixteen bytes of host memory past every cache: plain accesses may find a line that an earlier kernel left

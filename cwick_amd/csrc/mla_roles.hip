@@ -187,6 +187,14 @@ __device__ __forceinline__ float vmax3(float a, float b, float c) {
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
+// the maximum over eight neighbouring lanes
+__device__ __forceinline__ uint32_t lanes8_max(uint32_t v) {
+    auto meet = [&](uint32_t o) { v = o > v ? o : v; };
+    meet(dpp_u32<0xB1, 0xF>(v));                          // quad_perm [1, 0, 3, 2]
+    meet(dpp_u32<0x4E, 0xF>(v));                          // quad_perm [2, 3, 0, 1]
+    meet(dpp_u32<0x141, 0xF>(v));                         // row_half_mirror
+    return v;
+}
 // max(|a|, |b|, |c|), NaN if any of them is one
 __device__ __forceinline__ float maximum3_abs(float a, float b, float c) {
     float r;
@@ -380,21 +388,22 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                      : "v"(list_at(0, key_of)), "v"(list_at(1, key_of)), "v"(list_at(2, key_of)),
                        "v"(list_at(0, lane)), "v"(list_at(1, lane)), "v"(list_at(2, lane)) : "memory");
     }
-    const bool has_unit = wave < 10;
-    const int hhu = wave >= 5 ? 1 : 0, bu = wave - 5 * hhu;
-    const uint32_t unit_lds = lds0 + PARK + (uint32_t)wave * PARK_UNIT;
-    if (has_unit) {
-        const uint64_t base = (uint64_t)(uintptr_t)(q + (size_t)(y * (uint32_t)nh) * KDIM + 128 * bu);      // (a scalar)
+    // scoring wave (kb, hh): dims 128 kb .. of the head half; value wave: the rope dims of heads 8 cw .. of the 32, eight dims a lane
+    const uint32_t unit_lds = lds0 + PARK + (uint32_t)(5 * hh + kb) * PARK_UNIT;
+    const uint64_t q_base = (uint64_t)(uintptr_t)(q + (size_t)(y * (uint32_t)nh) * KDIM + 128 * (scorer ? kb : 4));      // (a scalar)
+    auto head_off = [&](int h) -> uint32_t { return (uint32_t)(hb * HW + h < nh ? hb * HW + h : nh - 1) * (KDIM * 2); };
+    u32x4 rope;
+    if (scorer) {
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const int h = 4 * c + g, head0 = hb * HW + 16 * hhu + h, head = head0 < nh ? head0 : nh - 1;
-            const int x = (n ^ h) & (bu < 4 ? 15 : 7);             // the rope block has eight pieces: fetched twice
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" ::"v"((uint32_t)head * (KDIM * 2) + (uint32_t)(16 * x)),
-                         "s"(unit_lds + (uint32_t)c * 1024), "s"(base) : "memory");
+            const int h = 4 * c + g;
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" ::"v"(head_off(16 * hh + h) + (uint32_t)(16 * (n ^ h))),
+                         "s"(unit_lds + (uint32_t)c * 1024), "s"(q_base) : "memory");
         }
         if (SEL) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    } else if (SEL) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else {
+        asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(rope) : "v"(head_off(8 * cw + (lane >> 3)) + 16u * (uint32_t)(lane & 7)), "s"(q_base) : "memory");
+        if (SEL) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
     }
     if (SEL) asm volatile("" : "+v"(entry_k[0]), "+v"(entry_k[1]), "+v"(entry_k[2]), "+v"(entry_l[0]), "+v"(entry_l[1]), "+v"(entry_l[2])::"memory");
     auto rows_of = [&](int t) -> RowPair { return {row_of(t, key_of), scorer ? -1 : row_of(t, lane)}; };
@@ -404,24 +413,44 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
         return {row(entry_k[t], key_of), row(entry_l[t], lane)};
     };
     share(0, first_rows(0), lds0);
-    if (has_unit) {
-        // ---- the wave's unit as two E4M3 terms with one E8M0 scale per head (the hardware pairs the scale of
-        // lane (n, g) with k-elements that live in other lanes of the same head, so the four lanes must
-        // agree; both terms use it).  lane (n, g) holds head n of the half, dims 128 b + 32 g + [0, 32);
-        // the rope block is one register set: lanes g < 2 hold the hi term of dims 512 + 32 g.., lanes
-        // g >= 2 the lo term of dims 512 + 32 (g - 2).. (the key side repeats its bytes).
-        CWICK_ROLES_WAIT(4, 2, 3);                        // the share of tile 0 stays in flight
+    // ---- the wave's part of the query as two E4M3 terms with one E8M0 scale per head and block (the hardware pairs the
+    // scale of lane (n, g) with k-elements that live in other lanes of the same head, so the four lanes must
+    // agree; both terms use it).  Eight dim blocks for eight waves, two a SIMD, and the rope block, half as wide, dealt
+    // to the value waves: a SIMD is through with its conversions, 600 cycles of it a dim block, when it has done 2.25.
+    CWICK_ROLES_WAIT(4, 2, 3);                            // the share of tile 0 stays in flight
+    if (scorer) {
+        // lane (n, g) holds head n of the half, dims 128 b + 32 g + [0, 32)
         u32x4 w[4], hi[2], lo[2];
 #pragma unroll
         for (int c = 0; c < 4; c++) w[c] = LDS_AT(lds_u32x4, unit_lds + (uint32_t)(n * 256 + (((4 * g + c) ^ n) & 15) * 16));
         const uint32_t unit_byte = q_two_terms(w, hi, lo);
-        const bool rope_lo = bu == 4 && g >= 2;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            LDS_AT(lds_u32x4, unit_lds + (uint32_t)(c * 1024 + lane * 16)) = rope_lo ? lo[c] : hi[c];
+            LDS_AT(lds_u32x4, unit_lds + (uint32_t)(c * 1024 + lane * 16)) = hi[c];
             LDS_AT(lds_u32x4, unit_lds + PARK_LO + (uint32_t)(c * 1024 + lane * 16)) = lo[c];
         }
-        LDS_AT(lds_u32, lds0 + PARK_SC + (uint32_t)(wave * 256 + lane * 4)) = unit_byte;
+        LDS_AT(lds_u32, lds0 + PARK_SC + (uint32_t)((5 * hh + kb) * 256 + lane * 4)) = unit_byte;
+    } else {
+        // the rope block is one register set: lanes g < 2 hold the hi term of dims 512 + 32 g.., lanes g >= 2 the lo term
+        // of dims 512 + 32 (g - 2).. (the key side repeats its bytes); eight lanes here hold a head
+        asm volatile("" : "+v"(rope)::"memory");
+        q_u16x2 m = {};
+#pragma unroll
+        for (int d = 0; d < 4; d++) m = q_larger(m, rope[d]);
+        uint32_t top = m[0] > m[1] ? m[0] : m[1];
+        top = lanes8_max(top);
+        const uint32_t unit_byte = q_unit(top), h = 8 * (cw & 1) + (uint32_t)(lane >> 3), d8 = (uint32_t)lane & 7;
+        u32x2 hi, lo;
+#pragma unroll
+        for (int d = 0; d < 2; d++) {
+            uint32_t a, b;
+            q_two_terms(rope[2 * d], rope[2 * d + 1], unit_byte, a, b);
+            hi[d] = a, lo[d] = b;
+        }
+        const uint32_t at = lds0 + PARK + (5 * (uint32_t)(cw >> 1) + 4) * PARK_UNIT + ((d8 >> 1) & 1) * 1024 + ((d8 >> 2) * 16 + h) * 16 + 8 * (d8 & 1);
+        LDS_AT(lds_u32x2, at) = hi;
+        LDS_AT(lds_u32x2, at + 32 * 16) = lo;
+        if (d8 < 4) LDS_AT(lds_u32, lds0 + PARK_SC + (5 * (uint32_t)(cw >> 1) + 4) * 256 + (d8 * 16 + h) * 4) = unit_byte;
     }
     // tile 0 has landed (this wave's share), what comes behind it stays in flight
     if (n_tiles > 2) {
