@@ -44,9 +44,15 @@ __host__ __device__ inline int pf_slices(int tiles, int plain, int per) {
 struct PfCost {
     int waves, least;                       // tiles of a step; the fewest tiles of a slice
     float launch, item, step, step2, crowd, alone, merge, merge_slice, merge_part;
+    // workgroups of up to `few` steps (`few2` with two-term weights), where another body is the shorter one
+    int few, few2;
+    float few_item, few_step, few_step2;
 };
-constexpr PfCost PF_COST_WIDE = {1, 4, 0.8f, 9.6f, 1.22f, 2.135f, 0.411f, 0.36f, 4.8f, 0.021f, 0.063f};      // 256 rows
-constexpr PfCost PF_COST_TEAM = {4, 4, 2.5f, 7.25f, 1.815f, 2.46f, 0.362f, 0.44f, 2.5f, 0.072f, 0.016f};      // 64 rows
+constexpr int PF_ROUNDS = 7, PF_ROUNDS2 = 5;        // steps of a workgroup up to which that is so
+                                                    // (100 positions behind 7000, seven steps: 32.2 us, 33.8 the other way; 1000 at the
+                                                    // beginning, up to eight: 34.1 with all of them so, 31.8 with five)
+constexpr PfCost PF_COST_WIDE = {1, 4, 0.8f, 9.6f, 1.22f, 2.135f, 0.411f, 0.36f, 4.8f, 0.021f, 0.063f, 0, 0, 0.0f, 0.0f, 0.0f};      // 256 rows
+constexpr PfCost PF_COST_TEAM = {4, 4, 2.5f, 7.25f, 1.815f, 2.46f, 0.362f, 0.44f, 2.5f, 0.072f, 0.016f, PF_ROUNDS, PF_ROUNDS2, 3.9f, 2.3f, 3.3f};      // 64 rows
 
 struct PfBlocks {
     int count, n_kv_heads, n_prec, cus;     // the first n_prec blocks take two-term weights
@@ -63,7 +69,9 @@ struct PfSums {
 };
 inline float pf_steps(const PfCost &c, int tiles) { return (float)(c.waves == 1 ? tiles : (tiles + 3) / 4); }
 inline float pf_slice_time(const PfBlocks &b, const PfCost &c, int r, int tiles) {
-    return c.item + (b.count - 1 - r < b.n_prec ? c.step2 : c.step) * pf_steps(c, tiles);
+    const bool two = b.count - 1 - r < b.n_prec;
+    const float steps = pf_steps(c, tiles);
+    return steps <= (float)(two ? c.few2 : c.few) ? c.few_item + (two ? c.few_step2 : c.few_step) * steps : c.item + (two ? c.step2 : c.step) * steps;
 }
 // what a step takes longer, from the share of the units at work when they start and the mean of it: it falls evenly
 inline float pf_slower(const PfCost &c, float at_first, float mean) {
@@ -197,7 +205,7 @@ inline float pf_plan(int64_t pos0, int64_t n, int positions, int n_kv_heads, int
     b.count = (int)((n + positions - 1) / positions);
     // (the even share of all tiles with one-term weights: nothing takes less)
     const float keys = (float)b.count * (float)pos0 + 0.5f * (float)n * (float)b.count;
-    if (c.launch + ((float)b.count * c.item + keys / (float)(PF_TK * c.waves) * c.step) * (float)n_kv_heads / (float)cus >= limit) return limit;
+    if (c.launch + ((float)b.count * (c.few ? c.few_item : c.item) + keys / (float)(PF_TK * c.waves) * c.step) * (float)n_kv_heads / (float)cus >= limit) return limit;
     b.n_kv_heads = n_kv_heads;
     b.n_prec = (int)n_prec;
     b.cus = cus;

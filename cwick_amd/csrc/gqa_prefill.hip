@@ -910,11 +910,9 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory");
         }
     }
-    const bool single = n_tiles == 1 && !part;
-    const int first_tile = single ? 0 : wave;
-    if (first_tile < n_tiles) {
-        issue(Kg, lds_k, first_tile);
-        if (wave != PF_WAVES - 1) issue(Vg, lds_v, first_tile);
+    if (wave < n_tiles) {
+        issue(Kg, lds_k, wave);
+        if (wave != PF_WAVES - 1) issue(Vg, lds_v, wave);
     }
     f32x16 oacc[2][8];
     auto clear = [&]() {
@@ -937,7 +935,7 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
         for (int ks = 0; ks < 16; ks++) qf[ks] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(a + 32 * ks));
     }
     PF_LDS_BARRIER();
-    if (wave == PF_WAVES - 1 && first_tile < n_tiles) issue(Vg, lds_v, first_tile);
+    if (wave == PF_WAVES - 1 && wave < n_tiles) issue(Vg, lds_v, wave);
 
     const unsigned char *kfrag = &sm.k[wave][pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
     const unsigned char *qfrag = &sm.q[pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
@@ -1077,56 +1075,6 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
         if (u < my_tiles) issue(base, lds_tile, wave + PF_WAVES * u);
     };
 
-    // A block of one tile: every wave scores it, and takes a quarter of the dims of the value products to the output
-    // (16 positions: 7.6 us, 11.0 where one wave takes them all and the meeting below follows).
-    if (single) {
-        f32x16 s[2], acc[2][2];
-        u32x4 pw[2][2], pl[2][2];
-        landed(false);
-        scores(s);
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            (void)move_ref(c, prep(0, c, s[c]));
-            finish(c, s[c], pw[c], pl[c]);
-#pragma unroll
-            for (int d = 0; d < 2; d++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc[c][d][i] = 0.0f;
-        }
-        typedef __attribute__((ext_vector_type(8))) short s16x8;
-#pragma unroll
-        for (int st = 0; st < 4; st++) {
-            const int ks2 = st >> 1, d = st & 1, off = wave * 128 + d * 64 + ks2 * 512;
-            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vfrag[0] + off));
-            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vfrag[1] + off));
-            const bf16x8 va = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                acc[c][d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8, pw[c][ks2]), acc[c][d], 0, 0, 0);
-                if (PRECISE)
-                    acc[c][d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8, pl[c][ks2]), acc[c][d], 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const float l = xor32_sum(l_part[c]), inv = l > 0.0f ? 1.0f / l : 0.0f;
-            const int r = 32 * c + l32;
-            if (t0 + r % P < n) {
-                float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 64 * wave + 4 * g;
-#pragma unroll
-                for (int d = 0; d < 2; d++)
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        f32x4 w;
-#pragma unroll
-                        for (int i = 0; i < 4; i++) w[i] = acc[c][d][4 * b + i] * inv;
-                        *(f32x4 *)(o + 32 * d + 8 * b) = w;
-                    }
-            }
-        }
-        return;
-    }
-
     // All of the wave's tiles.  FOLLOW: the reference follows the maximum and the accumulators are rescaled every
     // tile; without, the reference stays at the first tile's maximum, and a tile with a row that outgrew it ends the
     // attempt (false).  (A row whose keys of a tile are all masked sees nothing of later tiles either: every row
@@ -1243,6 +1191,429 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
     if (part && dw == 0 && g == 0) *(f32x2 *)(part_ml + r * 2) = (f32x2){top, sum};
 }
 
+// The same for workgroups of few steps (PF_ROUNDS, PF_ROUNDS2).  Four waves with accumulators of their own clear, and at the
+// end meet in, 256 KB of them: 11 500 cycles of the 27 000 of a block of one step, LDS takes 64 bytes of the writes a
+// cycle.  Here the waves score a tile each as there, but hand the weights round in LDS, and each accumulates a quarter of the
+// dims over all four tiles: nothing meets at the end but the weight sums, and the query's second block has room in
+// registers.  For that they go in step, two barriers a round (four with two-term weights, whose LDS has room for one block of
+// rows at a time), with one reference for a row; K(u + 1) is copied beside the value products, V(u) beside the scores.  A
+// round takes 6 000 cycles (8 300 with two-term weights), a step of the other 4 400 and 5 900: the copies, 500 cycles of
+// the compute unit's memory pipeline for a tile, find the other's waves at different places.  (The scores of round u + 1
+// beside the softmax of round u as well, out of two sets of score registers: the copies no longer land in time, 1000
+// positions 34.1 -> 35.5 us.  The operands of the next tile's products fetched ahead: equal.)
+// Replayed from a graph, 16 heads on 4 kv heads: 16 positions 7.9 -> 6.9 us, 100 11.8 -> 9.7, 360 17.9 -> 16.8, 700
+// 25.5 -> 24.6; 50 of 8 / 8 10.5 -> 8.3; 200 of 16 / 2 14.8 -> 12.9; 29 behind 3219, with their preparation, 21.4 -> 18.0, 128 of
+// 8 / 8 behind 1800 20.3 -> 17.5, 16 behind 16000 27.3 -> 25.5, 300 of 16 / 2 behind 500 28.9 -> 27.1.  For all steps: 1000
+// positions 31.8 -> 34.1, 900 behind 3000 79 -> 84.5.
+struct PfRoundsSmem {
+    unsigned char k[PF_WAVES][PF_TILE], v[PF_WAVES][PF_TILE];
+    // query rows 32 .. 63 on their way into registers, then the weights of four tiles: [tile][four fragments][lane]
+    union {
+        unsigned char q[PF_TILE];
+        u32x4 w[PF_WAVES][4][64];
+    };
+    float top[PF_WAVES][64];                                    // a wave's maximum of every row, at the end its weight sum
+    uint32_t outgrown[PF_WAVES];
+};
+static_assert(sizeof(PfRoundsSmem) <= 160 * 1024 - 64, "LDS");
+constexpr size_t PF_TEAM_LDS = sizeof(PfRoundsSmem) > sizeof(PfTeamSmem) ? sizeof(PfRoundsSmem) : sizeof(PfTeamSmem);
+
+template <int GROUP, bool PRECISE>
+__device__ __forceinline__ void
+gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
+                      const uint16_t *__restrict__ Q, int64_t pos0, int64_t n, int64_t wg_keys, int n_kv_heads,
+                      float scale_log2e, float *__restrict__ out, int64_t pblk, int kvh, float *part, float *part_ml) {
+    constexpr int P = 64 / GROUP;           // positions per workgroup
+    constexpr int NI = 16;                  // copies of a tile
+    PfRoundsSmem &sm = *reinterpret_cast<PfRoundsSmem *>(smem_raw);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));           // (see gqa_prefill_body)
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31;
+    const int g = lane >> 5;                // 0/1
+
+    const int64_t t0 = pblk * P;
+    const int n_heads = n_kv_heads * GROUP;
+    const int64_t q_stride = (int64_t)n_heads * PF_HD;
+    const int n_tiles = (int)((wg_keys + PF_TK - 1) / PF_TK);
+    const int64_t first_masked_key = pos0 + t0;
+
+    const uint32_t row_bytes = (uint32_t)n_kv_heads * (PF_HD * 2);
+    uint32_t cp_off = (uint32_t)(16 * g) * row_bytes + (uint32_t)l32 * 16;
+    asm volatile("" : "+v"(cp_off));
+    const unsigned char *Kg = (const unsigned char *)(K + (size_t)kvh * PF_HD);
+    const unsigned char *Vg = (const unsigned char *)(V + (size_t)kvh * PF_HD);
+    const uint32_t lds_k = (uint32_t)(uintptr_t)(pf_lds_void *)&sm.k[wave][0];
+    const uint32_t lds_v = (uint32_t)(uintptr_t)(pf_lds_void *)&sm.v[wave][0];
+    // copy i of a tile takes rows i and i + 16 (gqa_prefill_body's copies)
+    struct TileSrc {
+        const unsigned char *base;
+        uint32_t last;
+    };
+    auto tile_src = [&](const unsigned char *base, int tile) -> TileSrc {
+        const uint32_t key0 = (uint32_t)tile * PF_TK;
+        const uint32_t left = (uint32_t)wg_keys - 1 - key0;
+        const uint64_t first = (uint64_t)base + (uint64_t)key0 * row_bytes;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)first), hi = __builtin_amdgcn_readfirstlane((uint32_t)(first >> 32));
+        return {(const unsigned char *)((uint64_t)hi << 32 | lo), (left < PF_TK ? left : PF_TK - 1) * row_bytes + (PF_HD * 2 - 16)};
+    };
+    auto copy_one = [&](const TileSrc &src, uint32_t lds_tile, int i) {
+        const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_tile + (uint32_t)(i * PF_PAIR));
+        uint32_t off = (i >= 8 ? cp_off ^ 16 : cp_off) + (uint32_t)i * row_bytes;
+        off = off < src.last ? off : src.last;
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src.base), "s"(m0) : "memory");
+    };
+    auto issue = [&](const unsigned char *base, uint32_t lds_tile, int tile) {
+        const TileSrc src = tile_src(base, tile);
+#pragma unroll
+        for (int i = 0; i < NI; i++) copy_one(src, lds_tile, i);
+    };
+
+    // Query rows, sixteen pairs of rows of either block, dealt to the waves; block A goes through the last
+    // wave's V buffer on its way into fragments.  The first tiles are requested with them.
+    {
+        const int c = wave >> 1;
+        const uint32_t lds_q = (uint32_t)(uintptr_t)(pf_lds_void *)(c ? &sm.q[0] : &sm.v[PF_WAVES - 1][0]);
+        const int64_t left = n - 1 - t0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int m = 8 * (wave & 1) + j;
+            const int r = 32 * c + m + 16 * g;
+            const uint32_t t = (uint32_t)(r % P) < left ? (uint32_t)(r % P) : (uint32_t)left;
+            const unsigned char *src = (const unsigned char *)(Q + t0 * q_stride + (size_t)kvh * GROUP * PF_HD) +
+                                       (uint64_t)t * ((uint32_t)n_heads * (PF_HD * 2)) + (r / P) * (PF_HD * 2) + ((uint32_t)l32 ^ pf_swap(m)) * 16;
+            const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_q + (uint32_t)(m * PF_PAIR));
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory");
+        }
+    }
+    const bool single = n_tiles == 1 && !part;
+    const int first_tile = single ? 0 : wave;
+    if (first_tile < n_tiles) {
+        issue(Kg, lds_k, first_tile);
+        if (wave != PF_WAVES - 1) issue(Vg, lds_v, first_tile);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    PF_LDS_BARRIER();
+    bf16x8 qf[2][16];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const unsigned char *a = (c ? &sm.q[0] : &sm.v[PF_WAVES - 1][0]) + pf_row(l32) + ((g ^ pf_swap(l32)) << 4);
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) qf[c][ks] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(a + 32 * ks));
+    }
+    PF_LDS_BARRIER();
+    if (wave == PF_WAVES - 1 && first_tile < n_tiles) issue(Vg, lds_v, first_tile);
+
+    const unsigned char *kfrag = &sm.k[wave][pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
+    const int grp = lane >> 4, gi = lane & 15;
+    const int v_key0 = 4 * (grp >> 1) + (gi >> 2);
+    const int v_col = 2 * (grp & 1) + ((gi & 3) >> 1);
+    const unsigned char *vfrag[2] = {&sm.v[wave][pf_row(v_key0) + (v_col << 4) + (gi & 1) * 8],
+                                     &sm.v[wave][pf_row(v_key0 + 8) + ((v_col ^ 1) << 4) + (gi & 1) * 8]};
+    float m_ref[2] = {-INFINITY, -INFINITY}, l_part[2] = {0.0f, 0.0f};
+
+    // after_step(ks) is called behind every pair of products
+    auto scores = [&](f32x16 (&s)[2], auto after_step) {
+        u32x4 ka[PF_PRE];
+#pragma unroll
+        for (int ks = 0; ks < PF_PRE; ks++) ka[ks] = *(const u32x4 *)(kfrag + 32 * ks);
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) {
+            const bf16x8 kf = __builtin_bit_cast(bf16x8, ka[ks % PF_PRE]);
+            if (ks + PF_PRE < 16) ka[ks % PF_PRE] = *(const u32x4 *)(kfrag + 32 * (ks + PF_PRE));
+            if (ks == 0) {
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s[0]) : "v"(kf), "a"(qf[0][ks]));
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s[1]) : "v"(kf), "a"(qf[1][ks]));
+            } else {
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[0]) : "v"(kf), "a"(qf[0][ks]));
+                asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s[1]) : "v"(kf), "a"(qf[1][ks]));
+            }
+            after_step(ks);
+        }
+        // (the wait carries the scores: without, nothing keeps the first instruction that reads them behind it)
+        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s[0]), "+v"(s[1])::"memory");
+    };
+    // masks the raw scores of a tile and returns this lane's maximum in log2 units
+    auto prep = [&](int tile, int c, f32x16 &s) -> float {
+        const int64_t key0 = (int64_t)tile * PF_TK;
+        float tmax = -INFINITY;
+        if (key0 + PF_TK - 1 > first_masked_key) {
+            const int left = (int)(n - 1 - t0 < P ? n - 1 - t0 : P), tr = (32 * c + l32) % P;
+            const int lim = (int)(first_masked_key - key0) + (tr < left ? tr : left) - 4 * g;
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if ((i >> 2) * 8 + (i & 3) > lim) s[i] = -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) tmax = fmaxf(tmax, s[i]);
+        return tmax * scale_log2e;
+    };
+    auto finish = [&](int c, f32x16 &s, u32x4 (&pw)[2], u32x4 (&pl)[2]) {
+        const float m_use = m_ref[c] == -INFINITY ? 0.0f : m_ref[c];
+        float psum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], scale_log2e, -m_use));
+            if (PRECISE) psum += s[i];
+        }
+#pragma unroll
+        for (int ks2 = 0; ks2 < 2; ks2++)
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                pw[ks2][h] = pack_bf16_rne(s[8 * ks2 + 2 * h], s[8 * ks2 + 2 * h + 1]);
+                if (PRECISE)
+                    pl[ks2][h] = pack_bf16_rne(s[8 * ks2 + 2 * h] - bf16lo_to_f32(pw[ks2][h]),
+                                               s[8 * ks2 + 2 * h + 1] - bf16hi_to_f32(pw[ks2][h]));
+                else
+                    psum = pair_sum_bf16(pw[ks2][h], psum);
+            }
+        l_part[c] += psum;
+    };
+    constexpr float SLACK = 64.0f;
+    auto move_ref = [&](int c, float tmax) -> float {
+        tmax = xor32_max(tmax);
+        float corr = 1.0f;
+        if (tmax > m_ref[c] + 8.0f) {
+            corr = __builtin_amdgcn_exp2f(m_ref[c] - tmax);
+            m_ref[c] = tmax;
+            l_part[c] *= corr;
+        }
+        return corr;
+    };
+    // A block of one tile: every wave scores it, and takes a quarter of the dims of the value products to the output
+    // (16 positions: 7.6 us, 11.0 where one wave took them all).
+    if (single) {
+        f32x16 s[2], acc[2][2];
+        u32x4 pw[2][2], pl[2][2];
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        scores(s, [](int) {});
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            (void)move_ref(c, prep(0, c, s[c]));
+            finish(c, s[c], pw[c], pl[c]);
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[c][d][i] = 0.0f;
+        }
+        typedef __attribute__((ext_vector_type(8))) short s16x8;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            const int ks2 = st >> 1, d = st & 1, off = wave * 128 + d * 64 + ks2 * 512;
+            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vfrag[0] + off));
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vfrag[1] + off));
+            const bf16x8 va = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                acc[c][d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8, pw[c][ks2]), acc[c][d], 0, 0, 0);
+                if (PRECISE)
+                    acc[c][d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(bf16x8, pl[c][ks2]), acc[c][d], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const float l = xor32_sum(l_part[c]), inv = l > 0.0f ? 1.0f / l : 0.0f;
+            const int r = 32 * c + l32;
+            if (t0 + r % P < n) {
+                float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 64 * wave + 4 * g;
+#pragma unroll
+                for (int d = 0; d < 2; d++)
+#pragma unroll
+                    for (int b = 0; b < 4; b++) {
+                        f32x4 w;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) w[i] = acc[c][d][4 * b + i] * inv;
+                        *(f32x4 *)(o + 32 * d + 8 * b) = w;
+                    }
+            }
+        }
+        return;
+    }
+
+    // Round by round, four tiles at a time.  FOLLOW: the reference follows the maximum and the accumulators are rescaled
+    // every round; without, the reference stays at the first round's maximum, and a round with a row that outgrew it ends the
+    // attempt of all waves (false).  (A row whose keys of a tile are all masked sees nothing of later tiles either: every row
+    // has its reference from the first round.)
+    auto values_done = [&]() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); };     // before a VALU read of the accumulators
+    const int rounds = (n_tiles + PF_WAVES - 1) / PF_WAVES;
+    const unsigned char *vquarter[2] = {vfrag[0] - wave * (PF_TILE - 128), vfrag[1] - wave * (PF_TILE - 128)};     // of tile 0
+    f32x16 oacc[2][2];                                      // rows of block c, dims 64 wave + 32 d ..
+    auto tiles = [&](auto follow) -> bool {
+        constexpr bool FOLLOW = decltype(follow)::value;
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) asm volatile("v_accvgpr_write_b32 %0, 0" : "=a"(oacc[c][d][i]));
+        for (int u = 0;; u++) {
+            const int tile = wave + PF_WAVES * u, here = n_tiles - PF_WAVES * u < PF_WAVES ? n_tiles - PF_WAVES * u : PF_WAVES;
+            const bool mine = wave < here, more = tile + PF_WAVES < n_tiles;
+            f32x16 s[2];
+            u32x4 pw[2][2], pl[2][2];
+            float x[2] = {-INFINITY, -INFINITY};
+            if (mine) {
+                // K(u) has landed; V(u), whose place the round before has left, comes beside the scores
+                if (u == 0) {
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");
+                    scores(s, [](int) {});
+                } else {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    const TileSrc src = tile_src(Vg, tile);
+                    scores(s, [&](int i) { copy_one(src, lds_v, i); });
+                }
+                x[0] = prep(tile, 0, s[0]), x[1] = prep(tile, 1, s[1]);
+            }
+            float corr[2] = {1.0f, 1.0f};
+            if (FOLLOW || u == 0) {
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    const float t = xor32_max(x[c]);
+                    if (g == 0) sm.top[wave][32 * c + l32] = t;
+                }
+                PF_LDS_BARRIER();
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    const int r = 32 * c + l32;
+                    const float t = fmaxf(fmaxf(sm.top[0][r], sm.top[1][r]), fmaxf(sm.top[2][r], sm.top[3][r]));
+                    if (t > m_ref[c] + 8.0f) {
+                        corr[c] = __builtin_amdgcn_exp2f(m_ref[c] - t);         // first round: exp2(-inf) = 0
+                        m_ref[c] = t;
+                        l_part[c] *= corr[c];
+                    }
+                }
+                if (FOLLOW && u > 0) {
+                    values_done();
+#pragma unroll
+                    for (int c = 0; c < 2; c++)
+#pragma unroll
+                        for (int d = 0; d < 2; d++)
+#pragma unroll
+                            for (int i = 0; i < 16; i++) {          // (in place: see gqa_prefill_body)
+                                float tmp;
+                                asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\ts_nop 0\n\t"
+                                             "v_accvgpr_write_b32 %0, %1"
+                                             : "+a"(oacc[c][d][i]), "=&v"(tmp)
+                                             : "v"(corr[c]));
+                            }
+                }
+            } else {
+                const bool out = __any(x[0] > m_ref[0] + SLACK || x[1] > m_ref[1] + SLACK);
+                if (lane == 0) sm.outgrown[wave] = out;
+            }
+            if (mine) {
+                finish(0, s[0], pw[0], pl[0]);
+                finish(1, s[1], pw[1], pl[1]);
+            }
+            // The weights change hands in the order the registers hold them: lane l of every wave reads what lane l wrote.
+            // Weights of single precision go all at once, two-term ones a block of rows after the other.
+            typedef __attribute__((ext_vector_type(8))) short s16x8;
+            const TileSrc next_k = tile_src(Kg, more ? tile + PF_WAVES : 0);
+            auto values = [&](int j, int first_c) {         // tile j of the round; beside the first two K(u + 1) comes
+                u32x4 w[4];
+                bf16x8 va[2][2];                            // [16 keys][32 dims]
+#pragma unroll
+                for (int f = 0; f < 4; f++) w[f] = sm.w[j][f][lane];
+#pragma unroll
+                for (int ks2 = 0; ks2 < 2; ks2++)
+#pragma unroll
+                    for (int d = 0; d < 2; d++) {
+                        const int off = j * PF_TILE + d * 64 + ks2 * 512;
+                        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vquarter[0] + off));
+                        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vquarter[1] + off));
+                        va[ks2][d] = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                    }
+#pragma unroll
+                for (int f = 0; f < 4; f++) {
+                    const int c = PRECISE ? first_c : f >> 1;
+#pragma unroll
+                    for (int d = 0; d < 2; d++)
+                        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(oacc[c][d]) : "v"(va[f & 1][d]), "v"(w[f]));
+                    if (j < 2 && (!PRECISE || first_c == 0) && more) {
+                        copy_one(next_k, lds_k, 8 * j + 2 * f);
+                        copy_one(next_k, lds_k, 8 * j + 2 * f + 1);
+                    }
+                }
+            };
+            if (mine) {
+#pragma unroll
+                for (int f = 0; f < 4; f++) sm.w[wave][f][lane] = PRECISE ? (f < 2 ? pw[0][f & 1] : pl[0][f & 1]) : pw[f >> 1][f & 1];
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // V(u) has landed
+            }
+            PF_LDS_BARRIER();
+            if (!FOLLOW && u > 0) {
+                const u32x4 o = *(const u32x4 *)sm.outgrown;
+                if (__builtin_amdgcn_readfirstlane(o[0] | o[1] | o[2] | o[3])) return false;
+            }
+            auto all_values = [&](int c) {
+#pragma unroll
+                for (int j = 0; j < PF_WAVES; j++)
+                    if (j < here) values(j, c);
+            };
+            all_values(0);
+            if (PRECISE) {
+                PF_LDS_BARRIER();
+                if (mine)
+#pragma unroll
+                    for (int f = 0; f < 4; f++) sm.w[wave][f][lane] = f < 2 ? pw[1][f & 1] : pl[1][f & 1];
+                PF_LDS_BARRIER();
+                all_values(1);
+            }
+            if (u + 1 == rounds) return true;
+            PF_LDS_BARRIER();                               // everybody is done with the round's values and weights
+        }
+    };
+    if (!tiles(std::false_type{})) {
+        // a row outgrew its reference (rare): from the first tile again
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        PF_LDS_BARRIER();
+        m_ref[0] = m_ref[1] = -INFINITY;
+        l_part[0] = l_part[1] = 0.0f;
+        if (wave < n_tiles) {
+            issue(Kg, lds_k, wave);
+            issue(Vg, lds_v, wave);
+        }
+        (void)tiles(std::true_type{});
+    }
+
+    // ---- the waves' sums meet; a wave has all that there is of its 64 dims ----
+    asm volatile("s_nop 15\n\ts_nop 15" : "+a"(oacc[0][0]), "+a"(oacc[0][1]), "+a"(oacc[1][0]), "+a"(oacc[1][1])::"memory");
+    PF_LDS_BARRIER();
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const float l = xor32_sum(l_part[c]);
+        if (g == 0) sm.top[wave][32 * c + l32] = l;
+    }
+    PF_LDS_BARRIER();
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int r = 32 * c + l32;
+        const float l = (sm.top[0][r] + sm.top[1][r]) + (sm.top[2][r] + sm.top[3][r]);
+        if (part) {
+            float *po = part + ((c * 8 + 2 * wave) * 4 * 64 + lane) * 4;
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+#pragma unroll
+                for (int b = 0; b < 4; b++)
+                    *(f32x4 *)(po + (d * 4 + b) * 256) = (f32x4){oacc[c][d][4 * b], oacc[c][d][4 * b + 1], oacc[c][d][4 * b + 2], oacc[c][d][4 * b + 3]};
+            if (wave == c && g == 0) *(f32x2 *)(part_ml + r * 2) = (f32x2){m_ref[c], l};
+        } else if (t0 + r % P < n) {
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 64 * wave + 4 * g;
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    f32x4 w;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) w[i] = oacc[c][d][4 * b + i] * inv;
+                    *(f32x4 *)(o + 32 * d + 8 * b) = w;
+                }
+        }
+    }
+}
+
 template <int GROUP>
 __global__ void __launch_bounds__(64 * PF_WAVES, 1)
 gqa_prefill_team_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
@@ -1270,8 +1641,14 @@ gqa_prefill_team_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
         if (slice + 1 < n_slices) keys = (int64_t)plan.per * PF_TK;
         const size_t row0 = (size_t)k0 * n_kv_heads * PF_HD;
         float *p = n_slices > 1 ? part + item * PF_PART<1> : nullptr, *pml = part_ml + (size_t)item * (64 * 2);
-        if (pblk < n_prec) gqa_prefill_team_body<GROUP, true>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh, p, pml);
-        else gqa_prefill_team_body<GROUP, false>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh, p, pml);
+        auto body = [&](auto f) { f(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh, p, pml); };
+        if (pblk < n_prec) {
+            if (keys <= PF_ROUNDS2 * PF_WAVES * PF_TK) body([](auto... a) { gqa_prefill_rounds_body<GROUP, true>(a...); });
+            else body([](auto... a) { gqa_prefill_team_body<GROUP, true>(a...); });
+        } else {
+            if (keys <= PF_ROUNDS * PF_WAVES * PF_TK) body([](auto... a) { gqa_prefill_rounds_body<GROUP, false>(a...); });
+            else body([](auto... a) { gqa_prefill_team_body<GROUP, false>(a...); });
+        }
         if (gridDim.x >= total) break;                  // one item each: nothing to draw
         if (threadIdx.x == 0) sh_item = gridDim.x + atomicAdd(&tickets[0], 1u);
         __syncthreads();
@@ -1370,13 +1747,13 @@ template <int GROUP>
 static int run_gqa_prefill_team(const uint16_t *k, const uint16_t *v, int64_t pos0, int64_t n, int n_kv_heads, const uint16_t *q,
                                 float scale, float *out, int64_t n_prec, int pblocks, const PfPlan &plan, float *part,
                                 uint32_t *tickets, hipStream_t s) {
-    CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_team_kernel<GROUP>>(sizeof(PfTeamSmem))));
+    CWICK_HIP_CALL((pf_allow_lds<gqa_prefill_team_kernel<GROUP>>(PF_TEAM_LDS)));
     const int slices = plan.first[pblocks] * n_kv_heads;
     float *part_ml = part ? part + (size_t)slices * PF_PART<1> : nullptr;
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_PREFILL, s);
         pk.launch(gqa_prefill_team_kernel<GROUP>, dim3((unsigned)(slices < num_cus() ? slices : num_cus())), dim3(64 * PF_WAVES),
-                  sizeof(PfTeamSmem), k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, plan,
+                  PF_TEAM_LDS, k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, plan,
                   part, part_ml, tickets);
     }
     CWICK_HIP_CALL(hipGetLastError());
