@@ -775,6 +775,30 @@ gqa_prefill_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ 
     pf_tickets_done(tickets);
 }
 
+// What the first loads of a workgroup need comes in the arguments that arrive in registers; the plan, which whole blocks
+// do without, is searched through the scalar cache (2 900 cycles from a kernel's first instruction to its first load; in
+// one trip of a vector load, eight entries a lane: 3 % slower).
+struct PfWork {
+    int kvh, rank, slice, n_slices;
+};
+__device__ __forceinline__ PfWork pf_work(uint32_t item, uint32_t n_kv_heads, int pblocks, int per, const PfPlan &plan) {
+    uint32_t slice_no;
+    if (n_kv_heads & (n_kv_heads - 1)) slice_no = item / n_kv_heads;
+    else slice_no = item >> __builtin_ctz(n_kv_heads);
+    PfWork w = {(int)(item - slice_no * n_kv_heads), (int)slice_no, 0, 1};
+    if (!per) return w;
+    int lo = 0, hi = pblocks;                           // the rank with first[rank] <= slice_no < first[rank + 1]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if ((uint32_t)plan.first[mid] <= slice_no) lo = mid;
+        else hi = mid;
+    }
+    w.rank = lo;
+    w.slice = (int)slice_no - plan.first[lo];
+    w.n_slices = plan.first[lo + 1] - plan.first[lo];
+    return w;
+}
+
 // The same for chunks whose position blocks do not fill the chip: a block's keys are dealt to several
 // workgroups, each with whole tiles, and gqa_prefill_merge_kernel combines what they leave.
 // What it costs is the partials: 256 KB written and read per slice of 256 rows, 252 slices of 34 tiles
@@ -785,29 +809,24 @@ template <int WAVES> constexpr size_t PF_PART = (size_t)64 * WAVES * PF_HD;     
 template <int GROUP>
 __global__ void __launch_bounds__(64 * PF_WAVES, 1)
 gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-                         const uint16_t *__restrict__ Q, int64_t pos0, int64_t n, int n_kv_heads,
-                         float scale_log2e, float *__restrict__ out, int64_t n_prec, int pblocks,
-                         const PfPlan plan, float *__restrict__ part, float *__restrict__ part_ml,
+                         const uint16_t *__restrict__ Q, int pos0_, int n_, uint32_t n_kv_heads_, int pblocks, int per, int n_prec,
+                         float scale_log2e,
+                         // (up to here they arrive in registers)
+                         float *__restrict__ out, const PfPlan plan, float *__restrict__ part, float *__restrict__ part_ml,
                          uint32_t *__restrict__ tickets) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     __shared__ uint32_t sh_item;
     __shared__ PfSlice sh_slice;
-    const uint32_t total = (uint32_t)plan.first[pblocks] * (uint32_t)n_kv_heads;
-    uint32_t item = blockIdx.x;
+    const int64_t pos0 = pos0_, n = n_;
+    const int n_kv_heads = (int)n_kv_heads_;
+    uint32_t item = blockIdx.x;                         // (no more workgroups than items)
     for (;;) {
-        if (item >= total) break;
-        const int slice_no = (int)(item / (uint32_t)n_kv_heads), kvh = (int)(item % (uint32_t)n_kv_heads);
-        int lo = 0, hi = pblocks;                       // the rank with first[rank] <= slice_no < first[rank + 1]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if ((int)plan.first[mid] <= slice_no) lo = mid;
-            else hi = mid;
-        }
-        const int64_t pblk = pblocks - 1 - lo;
-        const int slice = slice_no - plan.first[lo], n_slices = plan.first[lo + 1] - plan.first[lo];
-        const int64_t k0 = (int64_t)slice * plan.per * PF_TK;
+        const PfWork w = pf_work(item, n_kv_heads_, pblocks, per, plan);
+        const int kvh = w.kvh, slice = w.slice, n_slices = w.n_slices;
+        const int64_t pblk = pblocks - 1 - w.rank;
+        const int64_t k0 = (int64_t)slice * per * PF_TK;
         int64_t keys = pf_block_keys<GROUP, PF_WAVES>(pos0, n, pblk) - k0;
-        if (slice + 1 < n_slices) keys = (int64_t)plan.per * PF_TK;
+        if (slice + 1 < n_slices) keys = (int64_t)per * PF_TK;
         const size_t row0 = (size_t)k0 * n_kv_heads * PF_HD;
         // (read behind the body's barriers; the last item's reads are behind the draw's)
         if (threadIdx.x == 0) sh_slice = {n_slices > 1 ? part + item * PF_PART<PF_WAVES> : nullptr, part_ml + (size_t)item * (64 * PF_WAVES * 2)};
@@ -818,13 +837,15 @@ gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restr
             gqa_prefill_body<GROUP, false, true>(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads,
                                                  scale_log2e, out, pblk, kvh, &sh_slice);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (gridDim.x >= total) break;                  // one item each: nothing to draw
+        const uint32_t total = (uint32_t)(per ? (int)plan.first[pblocks] : pblocks) * n_kv_heads_;
+        if (gridDim.x >= total) return;                  // one item each: nothing to draw
         if (threadIdx.x == 0) sh_item = gridDim.x + atomicAdd(&tickets[0], 1u);
         __syncthreads();
         item = __builtin_amdgcn_readfirstlane(sh_item);
         __syncthreads();
+        if (item >= total) break;
     }
-    if (gridDim.x < total) pf_tickets_done(tickets);
+    pf_tickets_done(tickets);
 }
 
 // ---- workgroups whose four waves share one block of 64 rows ----
@@ -841,6 +862,16 @@ gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restr
 // 1000 of 8 / 8 heads 42.5 -> 25.6; 2500 of 16 105 -> 89; 29 behind 3219 26.4 -> 17.5, 128 of 8 / 8 behind 1800
 // 27.2 -> 16.7, 16 behind 16000 43.7 -> 24.2.  Long chunks go the other way: 517 behind 7083 take 115 us on 132 such
 // workgroups, 104 in two slices each.
+// One copy global -> LDS: 16 bytes a lane from a scalar base and the lane's offset, to a scalar place and a constant beyond it.
+// (The constant is added inside: outside, sixteen places a tile are sixteen scalars that live through the loops, more than
+// there are, and go in and out of lanes of vector registers.  With this and the arguments in registers: 16 positions of 16
+// heads 6.94 -> 6.61 us, 100 9.67 -> 9.10, 64 of 16 / 2 8.99 -> 8.39, 1500 44.1 -> 42.3, 2500 of 16 / 4 85.1 -> 82.2.)
+#define PF_COPY(off, base, place, by)                                                                                    \
+    do {                                                                                                                 \
+        uint32_t at_;                                                                                                    \
+        asm volatile("s_add_u32 %0, %3, %4\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"              \
+                     : "=&s"(at_) : "v"(off), "s"(base), "s"(place), "n"(by) : "memory", "scc");                         \
+    } while (0)
 struct PfTeamSmem {
     unsigned char k[PF_WAVES][PF_TILE], v[PF_WAVES][PF_TILE];   // at the end: the accumulators that change hands
     unsigned char q[PF_TILE];                                   // query rows 32 .. 63 (block B)
@@ -886,10 +917,9 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
         const uint32_t last = (left < PF_TK ? left : PF_TK - 1) * row_bytes + (PF_HD * 2 - 16);
 #pragma unroll
         for (int i = 0; i < NI; i++) {
-            const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_tile + (uint32_t)(i * PF_PAIR));
             uint32_t off = (i >= 8 ? cp_off ^ 16 : cp_off) + (uint32_t)i * row_bytes;
             off = off < last ? off : last;
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src), "s"(m0) : "memory");
+            PF_COPY(off, src, lds_tile, i * PF_PAIR);
         }
     };
 
@@ -904,10 +934,8 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
             const int m = 8 * (wave & 1) + j;
             const int r = 32 * c + m + 16 * g;
             const uint32_t t = (uint32_t)(r % P) < left ? (uint32_t)(r % P) : (uint32_t)left;
-            const unsigned char *src = (const unsigned char *)(Q + t0 * q_stride + (size_t)kvh * GROUP * PF_HD) +
-                                       (uint64_t)t * ((uint32_t)n_heads * (PF_HD * 2)) + (r / P) * (PF_HD * 2) + ((uint32_t)l32 ^ pf_swap(m)) * 16;
-            const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_q + (uint32_t)(m * PF_PAIR));
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory");
+            const uint32_t off = t * ((uint32_t)n_heads * (PF_HD * 2)) + (uint32_t)(r / P) * (PF_HD * 2) + ((uint32_t)l32 ^ pf_swap(m)) * 16;
+            PF_COPY(off, Q + t0 * q_stride + (size_t)kvh * GROUP * PF_HD, lds_q + (uint32_t)(8 * (wave & 1) * PF_PAIR), j * PF_PAIR);
         }
     }
     if (wave < n_tiles) {
@@ -1259,10 +1287,9 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
         return {(const unsigned char *)((uint64_t)hi << 32 | lo), (left < PF_TK ? left : PF_TK - 1) * row_bytes + (PF_HD * 2 - 16)};
     };
     auto copy_one = [&](const TileSrc &src, uint32_t lds_tile, int i) {
-        const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_tile + (uint32_t)(i * PF_PAIR));
         uint32_t off = (i >= 8 ? cp_off ^ 16 : cp_off) + (uint32_t)i * row_bytes;
         off = off < src.last ? off : src.last;
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src.base), "s"(m0) : "memory");
+        PF_COPY(off, src.base, lds_tile, i * PF_PAIR);
     };
     auto issue = [&](const unsigned char *base, uint32_t lds_tile, int tile) {
         const TileSrc src = tile_src(base, tile);
@@ -1281,10 +1308,8 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
             const int m = 8 * (wave & 1) + j;
             const int r = 32 * c + m + 16 * g;
             const uint32_t t = (uint32_t)(r % P) < left ? (uint32_t)(r % P) : (uint32_t)left;
-            const unsigned char *src = (const unsigned char *)(Q + t0 * q_stride + (size_t)kvh * GROUP * PF_HD) +
-                                       (uint64_t)t * ((uint32_t)n_heads * (PF_HD * 2)) + (r / P) * (PF_HD * 2) + ((uint32_t)l32 ^ pf_swap(m)) * 16;
-            const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_q + (uint32_t)(m * PF_PAIR));
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory");
+            const uint32_t off = t * ((uint32_t)n_heads * (PF_HD * 2)) + (uint32_t)(r / P) * (PF_HD * 2) + ((uint32_t)l32 ^ pf_swap(m)) * 16;
+            PF_COPY(off, Q + t0 * q_stride + (size_t)kvh * GROUP * PF_HD, lds_q + (uint32_t)(8 * (wave & 1) * PF_PAIR), j * PF_PAIR);
         }
     }
     const bool single = n_tiles == 1 && !part;
@@ -1617,28 +1642,23 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
 template <int GROUP>
 __global__ void __launch_bounds__(64 * PF_WAVES, 1)
 gqa_prefill_team_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-                        const uint16_t *__restrict__ Q, int64_t pos0, int64_t n, int n_kv_heads,
-                        float scale_log2e, float *__restrict__ out, int64_t n_prec, int pblocks,
-                        const PfPlan plan, float *__restrict__ part, float *__restrict__ part_ml,
-                        uint32_t *__restrict__ tickets) {
+                         const uint16_t *__restrict__ Q, int pos0_, int n_, uint32_t n_kv_heads_, int pblocks, int per, int n_prec,
+                         float scale_log2e,
+                         // (up to here they arrive in registers)
+                         float *__restrict__ out, const PfPlan plan, float *__restrict__ part, float *__restrict__ part_ml,
+                         uint32_t *__restrict__ tickets) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     __shared__ uint32_t sh_item;
-    const uint32_t total = (uint32_t)plan.first[pblocks] * (uint32_t)n_kv_heads;
-    uint32_t item = blockIdx.x;
+    const int64_t pos0 = pos0_, n = n_;
+    const int n_kv_heads = (int)n_kv_heads_;
+    uint32_t item = blockIdx.x;                         // (no more workgroups than items)
     for (;;) {
-        if (item >= total) break;
-        const int slice_no = (int)(item / (uint32_t)n_kv_heads), kvh = (int)(item % (uint32_t)n_kv_heads);
-        int lo = 0, hi = pblocks;                       // the rank with first[rank] <= slice_no < first[rank + 1]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if ((int)plan.first[mid] <= slice_no) lo = mid;
-            else hi = mid;
-        }
-        const int64_t pblk = pblocks - 1 - lo;
-        const int slice = slice_no - plan.first[lo], n_slices = plan.first[lo + 1] - plan.first[lo];
-        const int64_t k0 = (int64_t)slice * plan.per * PF_TK;
+        const PfWork w = pf_work(item, n_kv_heads_, pblocks, per, plan);
+        const int kvh = w.kvh, slice = w.slice, n_slices = w.n_slices;
+        const int64_t pblk = pblocks - 1 - w.rank;
+        const int64_t k0 = (int64_t)slice * per * PF_TK;
         int64_t keys = pf_block_keys<GROUP, 1>(pos0, n, pblk) - k0;
-        if (slice + 1 < n_slices) keys = (int64_t)plan.per * PF_TK;
+        if (slice + 1 < n_slices) keys = (int64_t)per * PF_TK;
         const size_t row0 = (size_t)k0 * n_kv_heads * PF_HD;
         float *p = n_slices > 1 ? part + item * PF_PART<1> : nullptr, *pml = part_ml + (size_t)item * (64 * 2);
         auto body = [&](auto f) { f(smem_raw, K + row0, V + row0, Q, pos0 - k0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh, p, pml); };
@@ -1649,13 +1669,15 @@ gqa_prefill_team_kernel(const uint16_t *__restrict__ K, const uint16_t *__restri
             if (keys <= PF_ROUNDS * PF_WAVES * PF_TK) body([](auto... a) { gqa_prefill_rounds_body<GROUP, false>(a...); });
             else body([](auto... a) { gqa_prefill_team_body<GROUP, false>(a...); });
         }
-        if (gridDim.x >= total) break;                  // one item each: nothing to draw
+        const uint32_t total = (uint32_t)(per ? (int)plan.first[pblocks] : pblocks) * n_kv_heads_;
+        if (gridDim.x >= total) return;                  // one item each: nothing to draw
         if (threadIdx.x == 0) sh_item = gridDim.x + atomicAdd(&tickets[0], 1u);
         __syncthreads();
         item = __builtin_amdgcn_readfirstlane(sh_item);
         __syncthreads();
+        if (item >= total) break;
     }
-    if (gridDim.x < total) pf_tickets_done(tickets);
+    pf_tickets_done(tickets);
 }
 
 // Combines the slices of a block: out = sum_s 2^(m_s - M) acc_s / sum_s 2^(m_s - M) l_s.  A wave
@@ -1753,8 +1775,8 @@ static int run_gqa_prefill_team(const uint16_t *k, const uint16_t *v, int64_t po
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_PREFILL, s);
         pk.launch(gqa_prefill_team_kernel<GROUP>, dim3((unsigned)(slices < num_cus() ? slices : num_cus())), dim3(64 * PF_WAVES),
-                  PF_TEAM_LDS, k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, plan,
-                  part, part_ml, tickets);
+                  PF_TEAM_LDS, k, v, q, (int)pos0, (int)n, (uint32_t)n_kv_heads, pblocks, plan.per, (int)n_prec, scale * 1.44269504088896340736f, out,
+                  plan, part, part_ml, tickets);
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (!plan.per) return 1;
@@ -1775,8 +1797,8 @@ static int run_gqa_prefill_split(const uint16_t *k, const uint16_t *v, int64_t p
     {
         ProfKernel pk(CWICK_HIP_PROF_GQA_PREFILL, s);
         pk.launch(gqa_prefill_split_kernel<GROUP>, dim3((unsigned)(slices < num_cus() ? slices : num_cus())), dim3(64 * PF_WAVES),
-                  sizeof(PfSmem), k, v, q, pos0, n, n_kv_heads, scale * 1.44269504088896340736f, out, n_prec, pblocks, plan,
-                  part, part_ml, tickets);
+                  sizeof(PfSmem), k, v, q, (int)pos0, (int)n, (uint32_t)n_kv_heads, pblocks, plan.per, (int)n_prec, scale * 1.44269504088896340736f, out,
+                  plan, part, part_ml, tickets);
     }
     CWICK_HIP_CALL(hipGetLastError());
     if (!plan.per) return 1;
