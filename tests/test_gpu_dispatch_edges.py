@@ -753,3 +753,56 @@ def test_mla_decode_fewer_workgroups(hip, orc, n, nh):
     ref = orc.mla_decode(c["q"], c["rows"], c["scales"], c["scale"], nthreads=0)
     assert_close(got, ref, "mla decode, fewer workgroups", strict=False)
     lat.free()
+
+
+@pytest.mark.parametrize("n_keys", [64, 65, 128, 129, 192, 193, 256, 257, 320, 383])
+@pytest.mark.parametrize("listed", [False, True])
+def test_mla_decode_tiles_of_a_workgroup(hip, orc, n_keys, listed):
+    """One to six tiles in a workgroup, the last one whole and not (256 blocks of 32 heads leave one workgroup to each): the
+    steps that copy a whole tile, the ones that copy what there is, and those behind the last copy."""
+    import torch
+    say("[case] mla decode, tiles of a workgroup", n_keys, listed)
+    batch, nh, n_rows = 64, 128, 400
+    c = synth.cfg3_mla_decode(n_rows, nh, seed=96)
+    g = synth.rng(97)
+    q = synth.f32_to_bf16(g.standard_normal((batch, nh, synth.KDIM), dtype=np.float32))
+    q[0] = c["q"]
+    sel = np.stack([g.permutation(n_rows)[:n_keys] for _ in range(batch)]).astype(np.int32)
+    sel[:, n_keys // 3] = -1
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    rows, scales, dq, dsel = d(c["rows"].view(np.uint8)), d(c["scales"]), d(q.view(np.int16)), d(sel)
+    out = torch.zeros((batch, nh, synth.VDIM), dtype=torch.float32, device="cuda")
+    hip.mla_decode_dev(rows, scales, 0, 0, n_rows, batch, dsel if listed else None, n_keys, dq, nh, c["scale"], out,
+                       torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for y in (0, batch - 1):
+        if listed:
+            ref = orc.mla_decode(q[y], c["rows"], c["scales"], c["scale"], sel=sel[y], nthreads=0)
+        else:
+            ref = orc.mla_decode(q[y], c["rows"][:n_keys], c["scales"][:n_keys], c["scale"], nthreads=0)
+        assert_close(out[y].cpu().numpy(), ref, "mla decode, tiles of a workgroup", strict=False)
+
+
+@pytest.mark.parametrize("n,pos0,nh,nkv", [
+    (656, 0, 16, 4),         # blocks of 20 tiles and one more: the last of five rounds, and the other body
+    (645, 0, 8, 8),          # diagonals that begin in one round and end in the next
+    (100, 7000, 16, 4),      # slices of seven rounds
+    (9, 8191, 16, 2),        # slices, the last one short
+    (5, 508, 4, 2),          # exactly four rounds, rows of one block only
+])
+@pytest.mark.parametrize("late", [0, 1, 4])
+def test_gqa_prefill_rounds(hip, orc, n, pos0, nh, nkv, late):
+    """Workgroups whose waves pass their weights round, at the number of rounds up to which they do; with keys that outgrow
+    every reference before them in several rounds, so that the workgroup starts over."""
+    say("[case] gqa prefill, rounds", n, pos0, nh, nkv, late)
+    c = synth.cfg2_gqa_prefill(n, nh, nkv, 256, pos0, seed=98)
+    k = synth.bf16_to_f32(c["k"])
+    for i in range(late):
+        k[(pos0 + n) * (i + 1) // (late + 1)] = 20.0 * (i + 1) * synth.bf16_to_f32(c["q"])[n - 1].reshape(nkv, nh // nkv, 256)[:, 0]
+    k = synth.f32_to_bf16(k)
+    cache = hip.KVCache(pos0 + n, nkv, 256)
+    cache.write(0, k.reshape(pos0 + n, -1), c["v"].reshape(pos0 + n, -1))
+    got = hip.gqa_prefill(cache, pos0, c["q"], c["scale"])
+    ref = orc.gqa_prefill(c["q"], k, c["v"], pos0, c["scale"], nthreads=0)
+    assert_close(got, ref, "gqa prefill, rounds", strict=False)
+    cache.free()
