@@ -523,8 +523,9 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 // ---- scores S^T[key][head] for keys 16 kb.., heads 16 hh.. of tile t+1 ----
                 // All that is read is requested first: eight waves read at the same time, and a fragment requested when the
                 // one before it is used costs a round trip each (S ready 1 700 cycles behind the barrier that way).
-                // The products are in assembly, which the compiler does not space from what reads them: the folds stand behind
-                // all of them and wait states.
+                // The products are in assembly, which the compiler spaces neither from what reads them nor from what writes what
+                // they read: the folds stand behind all of them and wait states, and a statement begins with the two wait states
+                // between a vector-ALU write (the constant of the scales, wherever the compiler loads it) and a product.
                 const uint32_t ka = tb + k_off, kA = tb + (k_off ^ 16u), kr = tb + kr_off, kR = tb + (kr_off ^ 16u);
                 u32x4 k0[NBLK], k1[NBLK];
                 float r0, r1;
@@ -542,7 +543,7 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 const int one_scales = 0x7F7F7F7F;
                 f32x4 acc[NBLK];
 #define CWICK_ROLES_PAIR(b, SEL_)                                                                                  \
-    asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %4, %5 " SEL_ "\n\t"                             \
+    asm volatile("s_nop 1\n\tv_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %4, %5 " SEL_ "\n\t"                   \
                  "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %3, %0, %4, %5 " SEL_                                    \
                  : "=&v"(acc[b]) : "v"(key(b)), "v"(qhi[b]), "v"(qlo[b]), "v"(one_scales), "v"(qsc0))
                 // S (+)= product * scale of the key: out of place 4 b + i of the row, inside the multiply-add
@@ -554,7 +555,7 @@ mla_roles_kernel(const uint16_t *__restrict__ q, const uint8_t *__restrict__ all
                 CWICK_ROLES_PAIR(1, "op_sel:[0,1,0] op_sel_hi:[0,0,0]");
                 CWICK_ROLES_PAIR(2, "op_sel:[0,0,0] op_sel_hi:[0,1,0]");
                 CWICK_ROLES_PAIR(3, "op_sel:[0,1,0] op_sel_hi:[0,1,0]");
-                asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %3, %4 op_sel:[0,0,0] op_sel_hi:[0,0,0]"
+                asm volatile("s_nop 1\n\tv_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, 0, %3, %4 op_sel:[0,0,0] op_sel_hi:[0,0,0]"
                              : "=&v"(acc[4]) : "v"(key(4)), "v"(qrope), "v"(one_scales), "v"(qsc1));
                 // (fourteen instructions behind the last product of block 0, and more behind the others')
                 asm volatile("s_nop 6" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4])::"memory");

@@ -6,6 +6,7 @@ rule on what the compiler scheduled: no vector-ALU instruction that writes an MF
 may be one of the two instructions in front of it, and no instruction may read an MFMA's result
 within nineteen wait states of it (thirteen for the eight-pass scaled FP8 instruction) unless it is an MFMA accumulating into it.  (Violations give wrong numbers only now and
 then, depending on timing, which is why the rule is checked on the code and not on results.)"""
+import functools
 import os
 import re
 import subprocess
@@ -24,6 +25,106 @@ def _regs(tok):
         return set(range(int(m.group(1)), int(m.group(2)) + 1))
     m = re.match(r"v(\d+)$", tok)
     return {int(m.group(1))} if m else set()
+
+
+def _operands(text):
+    """Registers of every operand, "v7", "a12", "s3" ("vcc" is its two halves), an operand's in one set."""
+    out = []
+    for o in re.split(r",(?![^\[]*\])", text):
+        o = re.sub(r"^-?\|?|\|$", "", o.strip().split(" ")[0])
+        m = re.match(r"([vas])(?:(\d+)|\[(\d+):(\d+)\])$", o)
+        if m:
+            lo, hi = (m.group(2), m.group(2)) if m.group(2) else (m.group(3), m.group(4))
+            out.append({m.group(1) + str(i) for i in range(int(lo), int(hi) + 1)})
+        else:
+            out.append({"vcc_lo", "vcc_hi"} if o == "vcc" else {o} if o in ("vcc_lo", "vcc_hi") else set())
+    return out
+
+
+class _Code:
+    """A function's instructions, and which may be the one executed before each."""
+
+    def __init__(self, name):
+        self.name, self.text, self.op, self.regs, self.asm, self.label = name, [], [], [], [], {}
+
+    def link(self):
+        self.before = [[] for _ in self.text]
+        for k, op in enumerate(self.op):
+            if op.startswith(("s_branch", "s_cbranch")):
+                self.before[self.label[self.text[k].split()[-1]]].append(k)
+            if not op.startswith(("s_branch", "s_endpgm")) and k + 1 < len(self.text):
+                self.before[k + 1].append(k)
+        self.behind = [[] for _ in self.text]
+        for k, b in enumerate(self.before):
+            for j in b:
+                self.behind[j].append(k)
+
+    def valu(self, k):
+        return self.op[k].startswith("v_") and not self.op[k].startswith("v_mfma")
+
+    def written(self, k):
+        """by a vector-ALU instruction (carries and exchanges have a second result)"""
+        return set().union(*self.regs[k][:2 if re.search(r"swap|_co_|div_scale|mad_[iu]64", self.op[k]) else 1])
+
+    def in_front(self, k, states):
+        """(instruction, wait states in between) of all that may run less than so many in front, whatever the branches"""
+        least, todo = {}, [(j, 0) for j in self.before[k]]
+        while todo:
+            j, w = todo.pop()
+            if w < states and w < least.get(j, states):
+                least[j] = w
+                w += int(self.text[j].split()[1], 0) + 1 if self.op[j] == "s_nop" else 1
+                todo += [(i, w) for i in self.before[j]]
+        return least.items()
+
+    def where(self, j, k, w):
+        return "%s: %s | %s (%d in between)" % (self.name[:60], self.text[j][:80], self.text[k][:80], w)
+
+
+@functools.lru_cache(maxsize=None)
+def _functions(src):
+    with tempfile.TemporaryDirectory() as tmp:
+        out = os.path.join(tmp, "k.s")
+        cmd = [B._hipcc()] + B.COMMON + B.PER_FILE.get(src, []) + ["-w", "-S", "--cuda-device-only", os.path.join(B.CSRC, src), "-o", out]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:]
+        lines = open(out).read().splitlines()
+    found, cur, in_asm = [], None, False
+    for line in lines:
+        t = line.strip()
+        if t.startswith(";;#ASM"):
+            in_asm = t.startswith(";;#ASMSTART")
+        elif re.match(r"\w+:", line):
+            cur = _Code(line.split(":")[0])
+            found.append(cur)
+        elif t.startswith((".section", ".set")):
+            cur = None
+        elif cur and re.match(r"\.LBB\w+:", t):
+            cur.label[t.split(":")[0]] = len(cur.text)
+        elif cur and t and t[0] not in ";.":
+            t = t.split(";")[0].strip()
+            op, _, rest = t.partition(" ")
+            cur.text.append(t), cur.op.append(op), cur.regs.append(_operands(rest)), cur.asm.append(in_asm)
+    found = [f for f in found if f.text]
+    for f in found:
+        f.link()
+    assert found
+    return found
+
+
+@pytest.mark.parametrize("src", ASM_MFMA_SOURCES)
+def test_no_operand_of_an_mfma_is_written_right_before_it(src):
+    """The first rule for everything that an MFMA from assembly reads: the two factors, the sum and the two registers of
+    scales, whichever half of the register file they are in, and along every branch that leads to it."""
+    n_mfma, bad = 0, []
+    for f in _functions(src):
+        for k, op in enumerate(f.op):
+            if op.startswith("v_mfma") and f.asm[k]:
+                n_mfma += 1
+                read = set().union(*f.regs[k][1:6])
+                bad += [f.where(j, k, w) for j, w in f.in_front(k, 2) if f.valu(j) and f.written(j) & read]
+    assert n_mfma > 0
+    assert not bad, "%d written within two wait states of the MFMA that reads it: %s" % (len(bad), bad[:3])
 
 
 @pytest.mark.parametrize("src", ASM_MFMA_SOURCES)
