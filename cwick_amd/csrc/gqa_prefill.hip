@@ -1460,10 +1460,14 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
     // every round; without, the reference stays at the first round's maximum, and a round with a row that outgrew it ends the
     // attempt of all waves (false).  (A row whose keys of a tile are all masked sees nothing of later tiles either: every row
     // has its reference from the first round.)
-    auto values_done = [&]() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); };     // before a VALU read of the accumulators
+    f32x16 oacc[2][2];                                      // rows of block c, dims 64 wave + 32 d ..
+    // The wait behind the value products carries the accumulators: the compiler moves them about as well, where a loop
+    // around the rescaling takes them out of the accumulation registers.
+    auto values_done = [&]() {
+        asm volatile("s_nop 15\n\ts_nop 15" : "+a"(oacc[0][0]), "+a"(oacc[0][1]), "+a"(oacc[1][0]), "+a"(oacc[1][1])::"memory");
+    };
     const int rounds = (n_tiles + PF_WAVES - 1) / PF_WAVES;
     const unsigned char *vquarter[2] = {vfrag[0] - wave * (PF_TILE - 128), vfrag[1] - wave * (PF_TILE - 128)};     // of tile 0
-    f32x16 oacc[2][2];                                      // rows of block c, dims 64 wave + 32 d ..
     auto tiles = [&](auto follow) -> bool {
         constexpr bool FOLLOW = decltype(follow)::value;
 #pragma unroll
@@ -1509,7 +1513,6 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
                     }
                 }
                 if (FOLLOW && u > 0) {
-                    values_done();
 #pragma unroll
                     for (int c = 0; c < 2; c++)
 #pragma unroll
@@ -1585,6 +1588,7 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
                 PF_LDS_BARRIER();
                 all_values(1);
             }
+            if (FOLLOW) values_done();
             if (u + 1 == rounds) return true;
             PF_LDS_BARRIER();                               // everybody is done with the round's values and weights
         }
@@ -1603,7 +1607,7 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
     }
 
     // ---- the waves' sums meet; a wave has all that there is of its 64 dims ----
-    asm volatile("s_nop 15\n\ts_nop 15" : "+a"(oacc[0][0]), "+a"(oacc[0][1]), "+a"(oacc[1][0]), "+a"(oacc[1][1])::"memory");
+    values_done();
     PF_LDS_BARRIER();
 #pragma unroll
     for (int c = 0; c < 2; c++) {

@@ -128,6 +128,24 @@ def test_no_operand_of_an_mfma_is_written_right_before_it(src):
 
 
 @pytest.mark.parametrize("src", ASM_MFMA_SOURCES)
+def test_no_result_of_an_mfma_is_touched_too_early(src):
+    """The other direction along every branch that leads away from an MFMA from assembly: what it leaves, in vector or in
+    accumulation registers, may be neither read nor written over before it is there, except by an MFMA that goes on from it
+    (the figures of test_no_valu_write_right_before_an_mfma_reads_it)."""
+    n_mfma, bad = 0, []
+    for f in _functions(src):
+        for k in range(len(f.text)):
+            onward = f.op[k].startswith("v_mfma")
+            touched = set().union(*(f.regs[k][1:3] + f.regs[k][4:6] if onward else f.regs[k]))
+            n_mfma += onward and f.asm[k]
+            for j, w in f.in_front(k, 19):
+                if f.op[j].startswith("v_mfma") and f.asm[j] and w < (13 if "16x16x128" in f.op[j] else 19) and f.regs[j][0] & touched:
+                    bad.append(f.where(j, k, w))
+    assert n_mfma > 0
+    assert not bad, "%d touch an MFMA's result before the matrix pipe has written it: %s" % (len(bad), bad[:3])
+
+
+@pytest.mark.parametrize("src", ASM_MFMA_SOURCES)
 def test_no_valu_write_right_before_an_mfma_reads_it(src):
     with tempfile.TemporaryDirectory() as tmp:
         out = os.path.join(tmp, "k.s")
