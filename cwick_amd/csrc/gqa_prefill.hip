@@ -752,7 +752,9 @@ gqa_prefill_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ 
     for (;;) {
         if (item >= total) break;
         const int64_t rank = (int64_t)item / n_kv_heads;
-        const int kvh = (int)(item % (uint32_t)n_kv_heads);
+        // (a scalar for good: the division leaves it in a vector register, and what the copies' addresses are made of with it)
+        uint32_t kvh = item % (uint32_t)n_kv_heads;
+        asm volatile("" : "+s"(kvh));
         int64_t pblk = -1, before = 0;                  // precise blocks ranked before this one
         for (int64_t pp = n_prec - 1; pp >= 0; pp--) {
             int64_t qmin = 16 * (pp + 1) / 10;          // plain blocks q >= qmin cost more than precise block pp
@@ -763,8 +765,8 @@ gqa_prefill_kernel(const uint16_t *__restrict__ K, const uint16_t *__restrict__ 
         }
         if (pblk < 0) pblk = pblocks - 1 - (rank - before);
         const int64_t keys = pf_block_keys<GROUP, PF_WAVES>(pos0, n, pblk);
-        if (pblk < n_prec) gqa_prefill_body<GROUP, true, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh);
-        else gqa_prefill_body<GROUP, false, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, kvh);
+        if (pblk < n_prec) gqa_prefill_body<GROUP, true, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, (int)kvh);
+        else gqa_prefill_body<GROUP, false, false>(smem_raw, K, V, Q, pos0, n, keys, n_kv_heads, scale_log2e, out, pblk, (int)kvh);
         // nothing of the last item may still be on its way into LDS
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (threadIdx.x == 0) sh_item = gridDim.x + atomicAdd(&tickets[0], 1u);

@@ -145,6 +145,22 @@ def test_no_result_of_an_mfma_is_touched_too_early(src):
     assert not bad, "%d touch an MFMA's result before the matrix pipe has written it: %s" % (len(bad), bad[:3])
 
 
+@pytest.mark.parametrize("src", ["mla_roles.hip", "mla_prefill64.hip", "gqa_prefill.hip"])
+def test_scalar_addresses_of_copies_come_from_the_scalar_unit(src):
+    """A copy from assembly may take its base address out of scalar registers that a vector-ALU instruction wrote
+    (v_readfirstlane, v_readlane) only five wait states later: the compiler, which keeps that distance for its own loads, does
+    not for what a statement holds."""
+    n_copies, bad = 0, []
+    for f in _functions(src):
+        for k, op in enumerate(f.op):
+            if f.asm[k] and op.startswith(("global_", "buffer_", "flat_", "scratch_")):
+                read = {r for r in set().union(*f.regs[k]) if r[0] == "s" or r.startswith("vcc")}
+                n_copies += bool(read)
+                bad += [f.where(j, k, w) for j, w in f.in_front(k, 5) if f.valu(j) and f.written(j) & read]
+    assert n_copies > 0
+    assert not bad, "%d scalar addresses are used before they are there: %s" % (len(bad), bad[:3])
+
+
 @pytest.mark.parametrize("src", ASM_MFMA_SOURCES)
 def test_no_valu_write_right_before_an_mfma_reads_it(src):
     with tempfile.TemporaryDirectory() as tmp:
