@@ -84,6 +84,12 @@ __device__ __forceinline__ uint32_t pf_swap(uint32_t row) { return (row >> 3) & 
 // workgroup barrier that orders LDS traffic only (the copies of later tiles stay in flight)
 #define PF_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
+// Of the sum of a row's weights.  A score that overflows when it is scaled leaves a reference of infinity and weights of
+// zero: its row is NaN, as with a score that overflows by itself and where slices or waves meet (infinity minus infinity).
+__device__ __forceinline__ float pf_reciprocal(float l, float m_ref) {
+    return m_ref == INFINITY ? __builtin_nanf("") : l > 0.0f ? 1.0f / l : 0.0f;
+}
+
 // PRECISE: the bf16 rounding residual of the weights goes through the matrix core as well
 // (position blocks that see at most 1024 keys; see the launcher).  The body of one workgroup.
 // K and V start at the first key of the item's slice and pos0 counts from there (a whole item: the
@@ -691,8 +697,7 @@ gqa_prefill_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const 
     }
 #pragma unroll
     for (int c = 0; c < 2; c++) {
-        const float l = l_part[c] + __shfl_xor(l_part[c], 32, 64);
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const float inv = pf_reciprocal(l_part[c] + __shfl_xor(l_part[c], 32, 64), m_ref[c]);
         const int r = wave * 64 + 32 * c + l32;
         if (t0 + r % P < n) {
             float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 4 * g;
@@ -1440,7 +1445,7 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
         }
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            const float l = xor32_sum(l_part[c]), inv = l > 0.0f ? 1.0f / l : 0.0f;
+            const float inv = pf_reciprocal(xor32_sum(l_part[c]), m_ref[c]);
             const int r = 32 * c + l32;
             if (t0 + r % P < n) {
                 float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 64 * wave + 4 * g;
@@ -1630,7 +1635,7 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
                     *(f32x4 *)(po + (d * 4 + b) * 256) = (f32x4){oacc[c][d][4 * b], oacc[c][d][4 * b + 1], oacc[c][d][4 * b + 2], oacc[c][d][4 * b + 3]};
             if (wave == c && g == 0) *(f32x2 *)(part_ml + r * 2) = (f32x2){m_ref[c], l};
         } else if (t0 + r % P < n) {
-            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            const float inv = pf_reciprocal(l, m_ref[c]);
             float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 64 * wave + 4 * g;
 #pragma unroll
             for (int d = 0; d < 2; d++)

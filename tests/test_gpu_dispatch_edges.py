@@ -806,3 +806,33 @@ def test_gqa_prefill_rounds(hip, orc, n, pos0, nh, nkv, late):
     ref = orc.gqa_prefill(c["q"], k, c["v"], pos0, c["scale"], nthreads=0)
     assert_close(got, ref, "gqa prefill, rounds", strict=False)
     cache.free()
+
+
+@pytest.mark.parametrize("n,pos0,nh,nkv", [
+    (16, 0, 16, 4),          # one tile
+    (100, 0, 16, 4),         # few steps, whole blocks
+    (9, 8191, 16, 2),        # few steps, slices
+    (1025, 0, 16, 4),        # more steps, whole blocks
+    (300, 5000, 16, 4),      # more steps, slices
+    (517, 7083, 16, 4),      # 256 rows, slices
+    (2000, 0, 32, 4),        # 256 rows, whole blocks
+])
+@pytest.mark.parametrize("early", [False, True])
+def test_gqa_prefill_score_that_overflows_when_scaled(hip, orc, n, pos0, nh, nkv, early):
+    """A score that fp32 holds and whose scaled value it does not: the row is NaN, as it is with a score that overflows by
+    itself (infinity minus infinity), whichever workgroup it falls to; the other rows are what they are."""
+    say("[case] gqa prefill, overflow when scaled", n, pos0, nh, nkv, early)
+    c = synth.cfg2_gqa_prefill(n, nh, nkv, 256, pos0, seed=101)
+    scale, dim, key, head, row = 3.0, 17, 3 if early else 2 * (pos0 + n) // 3, 1, n - 1
+    q, k = synth.bf16_to_f32(c["q"]) * (c["scale"] / scale), synth.bf16_to_f32(c["k"])
+    q[:, :, dim] = 0.0
+    q[row, head, dim] = k[key, head // (nh // nkv), dim] = 1.2e19           # the score is 1.4e38, three times that no fp32 value
+    q, k = synth.f32_to_bf16(q), synth.f32_to_bf16(k)
+    cache = hip.KVCache(pos0 + n, nkv, 256)
+    cache.write(0, k.reshape(pos0 + n, -1), c["v"].reshape(pos0 + n, -1))
+    got = hip.gqa_prefill(cache, pos0, q, scale)
+    ref = orc.gqa_prefill(q, k, c["v"], pos0, scale, nthreads=0)
+    assert np.isnan(ref[row, head]).all() and np.isnan(got[row, head]).all()
+    others = ~((np.arange(n) == row)[:, None] & (np.arange(nh) == head))
+    assert_close(got[others], ref[others], "gqa prefill, the other rows", strict=False)
+    cache.free()
