@@ -808,6 +808,31 @@ def test_gqa_prefill_rounds(hip, orc, n, pos0, nh, nkv, late):
     cache.free()
 
 
+@pytest.mark.parametrize("listed", [False, True])
+@pytest.mark.parametrize("n_keys,nh", [(64, 16), (300, 40), (9000, 64)])
+def test_mla_decode_score_that_overflows_when_scaled(hip, orc, n_keys, nh, listed):
+    """A score that fp32 holds and whose scaled value it does not: the head's row is NaN, as it is with a score that overflows
+    by itself (infinity minus infinity), whether its keys are one slice or several; the other heads' rows are what they are."""
+    say("[case] mla decode, overflow when scaled", n_keys, nh, listed)
+    c = synth.cfg3_mla_decode(n_keys, nh, seed=99)
+    scale, dim, key, head = 3.0, 520, 2 * n_keys // 3, 1          # (a rope dim: no part of any value)
+    q, rows, scales = synth.bf16_to_f32(c["q"]) * (c["scale"] / scale), c["rows"].copy(), c["scales"].copy()
+    q[:, dim] = 0.0
+    q[head, dim] = 5e17
+    rows[key, 512:], scales[key, 4] = 0, 1e18
+    rows[key, dim] = 0x78                                           # 256: the score is 1.28e38, three times that no fp32 value
+    q = synth.f32_to_bf16(q)
+    sel = synth.rng(100).permutation(n_keys).astype(np.int32) if listed else None
+    lat = hip.LatentCache(1, n_keys)
+    lat.write(0, 0, rows, scales)
+    got = hip.mla_decode(lat, 0, q, scale, sel=sel, n_list=n_keys)
+    ref = orc.mla_decode(q, rows, scales, scale, sel=sel, nthreads=0)
+    others = np.arange(nh) != head
+    assert np.isnan(ref[head]).all() and np.isnan(got[head]).all()
+    assert_close(got[others], ref[others], "mla decode, the other heads", strict=False)
+    lat.free()
+
+
 @pytest.mark.parametrize("n,pos0,nh,nkv", [
     (16, 0, 16, 4),          # one tile
     (100, 0, 16, 4),         # few steps, whole blocks
