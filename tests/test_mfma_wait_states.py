@@ -5,7 +5,9 @@ place `s_nop 1` where such a write comes last; this test compiles them to assemb
 rule on what the compiler scheduled: no vector-ALU instruction that writes an MFMA's A or B operand
 may be one of the two instructions in front of it, and no instruction may read an MFMA's result
 within nineteen wait states of it (thirteen for the eight-pass scaled FP8 instruction) unless it is an MFMA accumulating into it.  (Violations give wrong numbers only now and
-then, depending on timing, which is why the rule is checked on the code and not on results.)"""
+then, depending on timing, which is why the rule is checked on the code and not on results.)  The same
+goes for the other distances the compiler keeps for its own instructions only: scalar registers that a
+vector-ALU instruction writes and a copy from assembly takes its address from, and registers that a load from assembly fills."""
 import functools
 import os
 import re
@@ -222,11 +224,9 @@ def test_no_valu_write_right_before_an_mfma_reads_it(src):
     assert not early, "MFMA result read before the matrix pipe has written it: %r" % early[:3]
 
 
-@pytest.mark.parametrize("src,kernel", [("gqa_prefill.hip", "gqa_prefill_team_kernel"), ("indexer_band.hip", "indexer_approx_kernel")])
-def test_the_wait_behind_the_matrix_instructions_carries_their_results(src, kernel):
-    """The rule above holds for what the compiler happened to schedule.  That it may not schedule otherwise takes the results
-    through the wait: in the compiler's input to the scheduler, nothing but a further MFMA or the `s_nop 15` statement
-    may use what an MFMA from assembly leaves in VGPRs."""
+@functools.lru_cache(maxsize=None)
+def _ir(src, kernel):
+    """The lines of each instantiation of a kernel in the compiler's input to the scheduler, and what uses each value."""
     with tempfile.TemporaryDirectory() as tmp:
         out = os.path.join(tmp, "k.ll")
         cmd = [B._hipcc()] + B.COMMON + B.PER_FILE.get(src, []) + [
@@ -234,7 +234,7 @@ def test_the_wait_behind_the_matrix_instructions_carries_their_results(src, kern
         r = subprocess.run(cmd, capture_output=True, text=True)
         assert r.returncode == 0, r.stderr[-2000:]
         functions = [f.splitlines() for f in open(out).read().split("\ndefine ")[1:]]
-    n_mfma, loose = 0, []
+    found = []
     for lines in functions:
         if kernel not in lines[0]:
             continue
@@ -242,13 +242,50 @@ def test_the_wait_behind_the_matrix_instructions_carries_their_results(src, kern
         for t in lines[1:]:
             for name in set(re.findall(r"%[\w.]+", t.split(" = ", 1)[-1])):
                 users.setdefault(name, []).append(t.strip())
+        found.append((lines, users))
+    return found
+
+
+@pytest.mark.parametrize("src,kernel,wait", [("gqa_prefill.hip", "gqa_prefill_team_kernel", "s_nop 15"),
+                                             ("indexer_band.hip", "indexer_approx_kernel", "s_nop 15"),
+                                             ("mla_roles.hip", "mla_roles_kernel", "s_nop 6")])
+def test_the_wait_behind_the_matrix_instructions_carries_their_results(src, kernel, wait):
+    """The rule above holds for what the compiler happened to schedule.  That it may not schedule otherwise takes the results
+    through the wait: in the compiler's input to the scheduler, nothing but a further MFMA or the statement that waits
+    may use what an MFMA from assembly leaves in VGPRs."""
+    n_mfma, loose = 0, []
+    for lines, users in _ir(src, kernel):
         for t in lines:
-            m = re.match(r'\s+(%\w+) = .*\basm .*"v_mfma.*", "=&?v', t)
+            m = re.match(r'\s+(%\w+) = .*\basm .*"(?:s_nop 1\\0A\\09)?v_mfma.*", "=&?v', t)
             if m:
                 n_mfma += 1
-                loose += [u for u in users.get(m.group(1), ()) if not re.search(r'\basm .*"(v_mfma|s_nop 15)', u)]
+                loose += [u for u in users.get(m.group(1), ()) if not re.search(r'\basm .*"(v_mfma|%s)' % wait, u)]
     assert n_mfma > 0
     assert not loose, "an MFMA's result is used by what no wait is in front of: %r" % loose[:3]
+
+
+def test_what_a_load_from_assembly_brings_is_used_behind_its_wait():
+    """The first loads of the latent decode (the query's rope block, the list's entries) are statements whose wait is a later
+    one, so that the copies behind them stay in flight; to the compiler their values are there at once.  In its input to the
+    scheduler nothing may use them but the empty statement behind the wait, wherever branches meet on the way to it."""
+    n_loads, loose = 0, []
+    for lines, users in _ir("mla_roles.hip", "mla_roles_kernel"):
+        for t in lines:
+            m = re.match(r'\s+(%\w+) = .*\basm .*"global_load_dword', t)
+            if not m:
+                continue
+            n_loads += 1
+            todo, seen = [m.group(1)], set()
+            while todo:
+                name = todo.pop()
+                seen.add(name)
+                for u in users.get(name, ()):
+                    if re.search(r" = (extractvalue|phi) ", u):
+                        todo += {u.split(" = ")[0]} - seen
+                    elif not re.search(r'\basm sideeffect "",', u):
+                        loose.append(u)
+    assert n_loads == 2 + 1, "a rope block in both instantiations, the list's entries in one: %d" % n_loads
+    assert not loose, "a load's result is used by what its wait is not in front of: %r" % loose[:3]
 
 
 def test_decode_kernels_keep_their_tiles_in_registers():
