@@ -783,13 +783,21 @@ def test_mla_decode_tiles_of_a_workgroup(hip, orc, n_keys, listed):
         assert_close(out[y].cpu().numpy(), ref, "mla decode, tiles of a workgroup", strict=False)
 
 
-@pytest.mark.parametrize("n,pos0,nh,nkv", [
-    (656, 0, 16, 4),         # blocks of 20 tiles and one more: the last of five rounds, and the other body
-    (645, 0, 8, 8),          # diagonals that begin in one round and end in the next
-    (100, 7000, 16, 4),      # slices of seven rounds
-    (9, 8191, 16, 2),        # slices, the last one short
-    (5, 508, 4, 2),          # exactly four rounds, rows of one block only
-])
+# chunks that 64-row workgroups take, and the steps of four tiles those have, with one-term and with two-term weights (up to
+# seven and five of them are rounds; tests/test_host_rules.py holds the plan to these figures)
+PREFILL_ROUNDS = [
+    ((656, 0, 16, 4), (), range(1, 4)),              # slices, the last ones of one to three tiles
+    ((645, 0, 8, 8), (), (1, 2)),
+    ((1025, 0, 16, 4), (9,), range(1, 9)),           # whole blocks: five rounds with two-term weights, and the other body from six steps on
+    ((1300, 200, 8, 8), (9, 10, 11, 12), range(3, 9)),      # diagonals that begin in one round and end in the next, of up to five
+    ((100, 7000, 16, 4), (6, 7), ()),                # slices of seven rounds
+    ((200, 7000, 16, 4), (10, 11, 12, 15), ()),      # and of more than seven: the other body
+    ((9, 8191, 16, 2), (1, 2), ()),                  # slices, the last one of a tile
+    ((5, 508, 4, 2), (), (1, 2)),                    # rows of one block only
+]
+
+
+@pytest.mark.parametrize("n,pos0,nh,nkv", [shape for shape, _, _ in PREFILL_ROUNDS])
 @pytest.mark.parametrize("late", [0, 1, 4])
 def test_gqa_prefill_rounds(hip, orc, n, pos0, nh, nkv, late):
     """Workgroups whose waves pass their weights round, at the number of rounds up to which they do; with keys that outgrow

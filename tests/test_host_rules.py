@@ -4,6 +4,7 @@ import os
 import subprocess
 
 from cwick_amd import build as B
+from tests.test_gpu_dispatch_edges import PREFILL_ROUNDS
 
 
 def run_cpp(tmp_path, header, body):
@@ -188,6 +189,35 @@ int main() {
     }
     return 0;
 }"""))
+
+
+def test_gqa_prefill_shapes_of_the_rounds_test(tmp_path):
+    """What the plans make of the chunks that test_gqa_prefill_rounds runs: on 256 compute units the 64-row workgroups take
+    them, and their steps are the ones that the test names."""
+    out = run_cpp(tmp_path, "gqa_plan.hpp", r"""
+int main() {
+    static const int shapes[][4] = {SHAPES};
+    for (auto &s : shapes) {
+        const int n = s[0], pos0 = s[1], kv = s[3], group = s[2] / kv, rows[2] = {256 / group, 64 / group};
+        int prec[2] = {0, 0}, blocks[2];
+        static PfPlan wide, team;
+        for (int k = 0; k < 2; k++) {
+            blocks[k] = (n + rows[k] - 1) / rows[k];
+            while (prec[k] < blocks[k] && pf_keys(pos0, n, rows[k], prec[k]) <= 1024) prec[k]++;
+        }
+        const float t = pf_plan(pos0, n, rows[0], kv, prec[0], 256, PF_COST_WIDE, INFINITY, wide);
+        if (pf_plan(pos0, n, rows[1], kv, prec[1], 256, PF_COST_TEAM, t, team) >= t) { printf("%d at %d: not the 64-row workgroups\n", n, pos0); return 1; }
+        unsigned steps[2] = {0, 0};
+        for (int r = 0; r < blocks[1]; r++) {
+            const int tiles = (int)(pf_keys(pos0, n, rows[1], blocks[1] - 1 - r) + PF_TK - 1) / PF_TK, cuts = team.first[r + 1] - team.first[r];
+            for (int i = 0; i < cuts; i++) steps[blocks[1] - 1 - r < prec[1]] |= 1u << (((i + 1 < cuts ? team.per : tiles - i * team.per) + 3) / 4);
+        }
+        printf("%u %u\n", steps[0], steps[1]);
+    }
+}
+""".replace("SHAPES", ", ".join("{%d, %d, %d, %d}" % shape for shape, _, _ in PREFILL_ROUNDS)))
+    seen = [tuple([i for i in range(32) if int(w) >> i & 1] for w in line.split()) for line in out.splitlines()]
+    assert seen == [(list(one), list(two)) for _, one, two in PREFILL_ROUNDS]
 
 
 def test_gqa_prefill_plans_are_sound_and_quick(tmp_path):
