@@ -864,11 +864,11 @@ gqa_prefill_split_kernel(const uint16_t *__restrict__ K, const uint16_t *__restr
 // 1.65 us, 2.1 with every compute unit at it (2048 cycles of it matrix instructions), and what is in the way is
 // the copies.  One buffer each for K and V: K(u + 1) is on its way during the softmax and the value products of
 // tile u, V(u + 1) during the next scores.
-// The launches of a call, against workgroups of one wave for few rows and 256 rows for more, with the plans and the
-// merge of that time: 1000 positions of 16 heads 49.9 -> 33.4 us, 360: 22.8 -> 18.4, 100: 16.6 -> 12.3, 16: 10.6 -> 8.7;
-// 1000 of 8 / 8 heads 42.5 -> 25.6; 2500 of 16 105 -> 89; 29 behind 3219 26.4 -> 17.5, 128 of 8 / 8 behind 1800
-// 27.2 -> 16.7, 16 behind 16000 43.7 -> 24.2.  Long chunks go the other way: 517 behind 7083 take 115 us on 132 such
-// workgroups, 104 in two slices each.
+// Calls replayed from a graph, in the best plan of workgroups of 256 rows and as they are dealt, those of few steps to the
+// other body: 1000 positions of 16 heads on 4 kv heads 47.0 and 31.3 us, 360 29.9 and 17.3, 100 20.6 and 10.0, 16 11.7 and 7.7;
+// 1000 of 8 / 8 43.7 and 25.4; 2500 of 16 98.1 and 80.5; 29 behind 3219 31.8 and 15.8, 128 of 8 / 8 behind 1800 29.4 and 14.9,
+// 16 behind 16000 43.3 and 24.0.  Long chunks go the other way: 517 behind 7083 take 109 us in the best plan of such workgroups,
+// 84.7 in workgroups of 256 rows.
 // One copy global -> LDS: 16 bytes a lane from a scalar base and the lane's offset, to a scalar place and a constant beyond it.
 // (The constant is added inside: outside, sixteen places a tile are sixteen scalars that live through the loops, more than
 // there are, and go in and out of lanes of vector registers.  With this and the arguments in registers: 16 positions of 16
@@ -885,6 +885,8 @@ struct PfTeamSmem {
     f32x2 ml[PF_WAVES][64];                                     // a wave's reference and weight sum of every row
 };
 
+// For more than PF_ROUNDS2 or PF_ROUNDS steps of four tiles (gqa_prefill_rounds_body has the others): every wave has tiles.
+static_assert(PF_ROUNDS >= 1 && PF_ROUNDS2 >= 1, "a wave without a tile");
 template <int GROUP, bool PRECISE>
 __device__ __forceinline__ void
 gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
@@ -945,10 +947,8 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
             PF_COPY(off, Q + t0 * q_stride + (size_t)kvh * GROUP * PF_HD, lds_q + (uint32_t)(8 * (wave & 1) * PF_PAIR), j * PF_PAIR);
         }
     }
-    if (wave < n_tiles) {
-        issue(Kg, lds_k, wave);
-        if (wave != PF_WAVES - 1) issue(Vg, lds_v, wave);
-    }
+    issue(Kg, lds_k, wave);
+    if (wave != PF_WAVES - 1) issue(Vg, lds_v, wave);
     f32x16 oacc[2][8];
     auto clear = [&]() {
 #pragma unroll
@@ -970,7 +970,7 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
         for (int ks = 0; ks < 16; ks++) qf[ks] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(a + 32 * ks));
     }
     PF_LDS_BARRIER();
-    if (wave == PF_WAVES - 1 && wave < n_tiles) issue(Vg, lds_v, wave);
+    if (wave == PF_WAVES - 1) issue(Vg, lds_v, wave);
 
     const unsigned char *kfrag = &sm.k[wave][pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
     const unsigned char *qfrag = &sm.q[pf_row(l32) + ((g ^ pf_swap(l32)) << 4)];
@@ -1140,7 +1140,7 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
             if (++u == my_tiles) return true;
         }
     };
-    if (my_tiles > 0 && !tiles(std::false_type{})) {
+    if (!tiles(std::false_type{})) {
         // a row outgrew its reference (rare): from the first tile again
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
         clear();
@@ -1181,15 +1181,11 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
     const bool row = t0 + r % P < n;
     float *o = out + (t0 + r % P) * q_stride + (size_t)(kvh * GROUP + r / P) * PF_HD + 32 * dw + 4 * g;
     float *po = part + ((cw * 8 + dw) * 4 * 64 + lane) * 4;
-    const int live = n_tiles < PF_WAVES ? n_tiles : PF_WAVES;       // waves that had tiles
     f32x4 *put = (f32x4 *)smem_raw + wave * 16 * 64 + lane;
     const f32x4 *get = (const f32x4 *)smem_raw + (cw * 2 + dw) * 4 * 64 + lane;
-    // (of one or two waves' accumulators all quarters have a place at once)
-    const bool few = live <= 2;
-    auto place = [&](int qd) { return (few ? 2 * qd : PF_WAVES * (qd & 1)) * 16 * 64; };
 #pragma unroll
     for (int qd = 0; qd < 4; qd++) {
-        if (wave < live)
+        const int place = PF_WAVES * (qd & 1) * 16 * 64;
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
@@ -1203,24 +1199,20 @@ gqa_prefill_team_body(unsigned char *smem_raw, const uint16_t *__restrict__ K, c
                         asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(oacc[c][2 * qd + d][4 * b + i]));
                         w[i] = x * f[c];
                     }
-                    put[place(qd) + ((c * 2 + d) * 4 + b) * 64] = w;
+                    put[place + ((c * 2 + d) * 4 + b) * 64] = w;
                 }
-        if (few && qd < 3) continue;
         PF_LDS_BARRIER();
-        for (int q = few ? 0 : qd; q <= qd; q++) {
-            f32x4 w[4];
+        f32x4 w[4];
 #pragma unroll
-            for (int b = 0; b < 4; b++) w[b] = get[place(q) + b * 64];
+        for (int b = 0; b < 4; b++) w[b] = get[place + b * 64];
 #pragma unroll
-            for (int v = 1; v < PF_WAVES; v++)
-                if (v < live)
+        for (int v = 1; v < PF_WAVES; v++)
 #pragma unroll
-                    for (int b = 0; b < 4; b++) w[b] += get[place(q) + (v * 16 + b) * 64];
+            for (int b = 0; b < 4; b++) w[b] += get[place + (v * 16 + b) * 64];
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                if (part) *(f32x4 *)(po + (2 * q * 4 + b) * 256) = w[b];
-                else if (row) *(f32x4 *)(o + 64 * q + 8 * b) = w[b] * inv;
-            }
+        for (int b = 0; b < 4; b++) {
+            if (part) *(f32x4 *)(po + (2 * qd * 4 + b) * 256) = w[b];
+            else if (row) *(f32x4 *)(o + 64 * qd + 8 * b) = w[b] * inv;
         }
     }
     if (part && dw == 0 && g == 0) *(f32x2 *)(part_ml + r * 2) = (f32x2){top, sum};
@@ -1414,7 +1406,7 @@ gqa_prefill_rounds_body(unsigned char *smem_raw, const uint16_t *__restrict__ K,
         return corr;
     };
     // A block of one tile: every wave scores it, and takes a quarter of the dims of the value products to the output
-    // (16 positions: 7.6 us, 11.0 where one wave took them all).
+    // (16 positions: 11.0 us where one wave took them all, 7.6 so, 6.8 with all that came later).
     if (single) {
         f32x16 s[2], acc[2][2];
         u32x4 pw[2][2], pl[2][2];
