@@ -34,8 +34,12 @@ __host__ __device__ inline int pf_slices(int tiles, int plain, int per) {
 // time, and from which share of them on it takes longer at all), and, where there are slices, the second launch, more
 // for each slice of a block, and each slice's partials (written and read).
 // Fitted to 20500 times of 1049 shapes (1 to 8192 positions behind 0 to 16000 of one to eight heads on one to
-// eight kv heads, whole and in slices): of the plans of a shape the one with the least price is 0.3 % behind the
-// fastest on the mean, 10 % at the worst; the prices of plans near the fastest are 3.6 and 5.4 % off (rms).
+// eight kv heads, whole and in slices) when workgroups of few steps had no body of their own; its prices (few_*) came with it, the
+// others stayed.  12791 times of 984 such shapes, of the kernels as they are: of the plans of a shape the one with the least price
+// is 0.5 % behind the fastest on the mean, 15 % at the worst (129 positions at the beginning of 16 / 4 heads, cut in two and
+// whole: 13.1 and 11.4 us) but for six kv heads (84 behind 13135 of 12 / 6: 47.8, in slices an eighth longer 34.4).  The prices of
+// plans near the fastest are 4.0 % off (rms) with 256 rows, with 64 rows 3.2 in slices of more steps, 8.4 of few, and 25 for
+// whole blocks, whose calls of 8 to 15 us they have 14 % too long on the mean.
 // What counts is the share of an XCD's own units that are at work, and up to a third or a half of them it adds nothing:
 // 1.21 us a tile with up to half of them, 1.33 with 64 %, 1.55 with 90.  With the mean of the chip, and in
 // proportion from the first unit on, two slices a block (the long ones of which lie on half of the XCDs, where there
@@ -48,11 +52,18 @@ struct PfCost {
     int few, few2;
     float few_item, few_step, few_step2;
 };
-constexpr int PF_ROUNDS = 7, PF_ROUNDS2 = 5;        // steps of a workgroup up to which that is so
-                                                    // (100 positions behind 7000, seven steps: 32.2 us, 33.8 the other way; 1000 at the
-                                                    // beginning, up to eight: 34.1 with all of them so, 31.8 with five)
+// Steps of a workgroup up to which that is so: where the prices below cross.  (Four and five steps with two-term weights, in
+// that body and the other: 500 positions of 32 / 4 heads 20.7 and 19.8 us, 560 24.1 and 23.1, 411 behind 210 23.4 and 22.0,
+// 236 of 64 / 8 behind 334 23.4 and 22.2; seven with one-term weights the same to 0.5 %: 100 behind 7000 27.4 and 27.5.)
+constexpr int PF_ROUNDS = 6, PF_ROUNDS2 = 3;
 constexpr PfCost PF_COST_WIDE = {1, 4, 0.8f, 9.6f, 1.22f, 2.135f, 0.411f, 0.36f, 4.8f, 0.021f, 0.063f, 0, 0, 0.0f, 0.0f, 0.0f};      // 256 rows
 constexpr PfCost PF_COST_TEAM = {4, 4, 2.5f, 7.25f, 1.815f, 2.46f, 0.362f, 0.44f, 2.5f, 0.072f, 0.016f, PF_ROUNDS, PF_ROUNDS2, 3.9f, 2.3f, 3.3f};      // 64 rows
+constexpr bool pf_crosses(int steps, float few_step, float step) {
+    const PfCost &c = PF_COST_TEAM;
+    return c.few_item + few_step * (float)steps <= c.item + step * (float)steps && c.few_item + few_step * (float)(steps + 1) > c.item + step * (float)(steps + 1);
+}
+static_assert(pf_crosses(PF_ROUNDS, PF_COST_TEAM.few_step, PF_COST_TEAM.step) && pf_crosses(PF_ROUNDS2, PF_COST_TEAM.few_step2, PF_COST_TEAM.step2),
+              "the limits of the other body are not where its prices end to be the lesser ones");
 
 struct PfBlocks {
     int count, n_kv_heads, n_prec, cus;     // the first n_prec blocks take two-term weights

@@ -784,14 +784,15 @@ def test_mla_decode_tiles_of_a_workgroup(hip, orc, n_keys, listed):
 
 
 # chunks that 64-row workgroups take, and the steps of four tiles those have, with one-term and with two-term weights (up to
-# seven and five of them are rounds; tests/test_host_rules.py holds the plan to these figures)
+# six and three of them are rounds; tests/test_host_rules.py holds the plan to these figures)
 PREFILL_ROUNDS = [
     ((656, 0, 16, 4), (), range(1, 4)),              # slices, the last ones of one to three tiles
     ((645, 0, 8, 8), (), (1, 2)),
-    ((1025, 0, 16, 4), (9,), range(1, 9)),           # whole blocks: five rounds with two-term weights, and the other body from six steps on
-    ((1300, 200, 8, 8), (9, 10, 11, 12), range(3, 9)),      # diagonals that begin in one round and end in the next, of up to five
-    ((100, 7000, 16, 4), (6, 7), ()),                # slices of seven rounds
-    ((200, 7000, 16, 4), (10, 11, 12, 15), ()),      # and of more than seven: the other body
+    ((1025, 0, 16, 4), (9,), range(1, 9)),           # whole blocks: three rounds with two-term weights, and the other body from four steps on
+    ((1300, 200, 8, 8), (9, 10, 11, 12), range(3, 9)),      # diagonals that begin in one round and end in the next
+    ((100, 7000, 16, 4), (6, 7), ()),                # slices of six rounds, and of seven steps of the other body
+    ((90, 6000, 16, 4), (2, 3, 5), ()),              # slices of five rounds
+    ((200, 7000, 16, 4), (10, 11, 12, 15), ()),
     ((9, 8191, 16, 2), (1, 2), ()),                  # slices, the last one of a tile
     ((5, 508, 4, 2), (), (1, 2)),                    # rows of one block only
 ]
