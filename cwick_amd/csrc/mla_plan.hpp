@@ -105,12 +105,13 @@ inline int64_t mla_decode_most_splits(int64_t blocks, int per_cu, int cus) {
 }
 // The tiles of 64 keys of a workgroup.  With up to three of them each, fewer workgroups of a tile or more in addition
 // are often the shorter ones: a further tile takes 1.1 us (out of a list 1.5), while all workgroups start, write their
-// partials and have them merged at the same time, 2.5 us for 128 of them and 6.2 for 256 (fitted to 150 times; left
-// alone from four tiles on, where the end of the workgroups spreads).  us, with the workgroups of a full round and as
-// chosen here: 64 heads, 8192 keys 16.5 and 12.7, 16384 17.1 and 15.5; 128 heads, 4096 15.8 and 12.6, 12288 17.1 and
-// 16.2; 16 heads, 32768 18.9 and 16.2; 8 x 600 keys of 64 heads 13.5 and 11.6; 4 x 2048 selected keys of 64 heads, the
-// whole step, 31.9 and 29.7.  (A percent behind the full round where it is closest, 16 heads x 49000 and
-// 2 x 12000 of 64.)  Two tiles in one workgroup take less than the merge (100 keys of 16 heads: 8.8 and 7.8).
+// partials and have them merged at the same time, 2.5 us for 128 of them and 6.2 for 256 (fitted to 150 times when a step took
+// 2 800 cycles, now 2 200; left alone from four tiles on, where the end of the workgroups spreads).  Of the kernels as they are, 250
+// shapes: 0.7 % behind the fastest number of tiles on the mean, 11 % at the worst (8 lists of 1280 rows for 48 heads); a full
+// round 1.9 % and 17.  us, replayed from a graph, with the workgroups of a full round and as chosen here: 64 heads, 8192 keys
+// 15.1 and 12.1, 16384 16.2 and 14.0; 128 heads, 4096 14.3 and 11.9, 12288 16.1 and 15.4; 16 heads, 32768 16.1 and 14.4; 8 x 600
+// keys of 64 heads 12.6 and 11.1; 4 x 2048 out of lists of 64 heads 14.7 and 12.5; equal where it is closest, 2 x 12000 of 64.
+// Two tiles in one workgroup take less than the merge (100 keys of 16 heads: 8.3 and 7.4).
 inline int64_t mla_decode_tiles(int64_t tiles, int64_t blocks, bool list, int per_cu, int cus) {
     const int64_t want = mla_decode_most_splits(blocks, per_cu, cus);
     int64_t per = (tiles + want - 1) / want;

@@ -34,7 +34,7 @@
 //   lists (rows are k_begin + i, only the last tile can be ragged) and lists given by sel[].
 //
 //   Where the time goes (cycle stamps, 12 waves on 256 CUs): a 64-key step has 1 088 cycles of matrix work on
-//   a SIMD and takes about 2 500.  No unit is saturated: the two scoring waves and the value wave of a SIMD are
+//   a SIMD and takes 2 100 to 2 300.  No unit is saturated: the two scoring waves and the value wave of a SIMD are
 //   chains of instructions, each of which takes its wave five cycles whatever its kind, of LDS round trips and of
 //   products.  So what pays is fewer instructions in the chain and fewer waits in it: the steps with a whole tile
 //   to copy have no condition and no 64-bit multiplication in them (running addresses; the step as a function of its
@@ -42,7 +42,8 @@
 //   out of which the folds take their factor by DPP, eight flags are eight bytes.  32768 rows of 128 heads, the
 //   whole call: 25.2 -> 23.5 us, 22.7 with the partial's scale found two values an instruction and its stores
 //   on their way early, 21.0 (of 21.6, from a graph) with a tile's values prepared a step ahead.  Before the first step a
-//   workgroup takes 7 000 cycles, behind the last 4 500 (a layer's 3037 rows of 64 heads, one tile each: 14 000 in all).
+//   workgroup takes 7 200 cycles; behind the last, until its partial is written, 4 300 to 5 300, with 256 workgroups 9 200
+//   (a layer's 3037 rows of 64 heads, one tile each: 13 100 in all).
 //   A copy instruction that has one lane per row touches 64 cache lines and moves a tile into LDS in 3 100 cycles when
 //   every compute unit does it, one that walks along the rows in 1 900 (copy-only kernels; a list of rows 3 600 and
 //   3 450), hence the tile's layout (see Tile).  With 32 query rows per tile the per-tile work that does not
